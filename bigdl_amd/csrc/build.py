@@ -28,7 +28,10 @@ HIP_SOURCES = sorted((CSRC / "hip").glob("*.hip"))
 
 HOST_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-fopenmp", "-march=x86-64-v3", "-Wall", "-Wno-unused-function"]
 HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-Wall", "-Wno-unused-function",
-             "-Wno-unused-variable", "-DNDEBUG"]
+             "-Wno-unused-variable", "-DNDEBUG",
+             # no packed fp32 arithmetic (v_pk_add_f32 and its like), as in ops/ragged.py: some forms of these instructions
+             # have given wrong results now and then on this hardware
+             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # per-file additions.  attn_prefill: MFMA accumulators in ordinary VGPRs -- the online softmax rescales them with VALU
 # multiplies, and accumulators kept in AGPRs are copied out and back around every such pass (64 moves per key tile).
 HIP_FILE_FLAGS = {"attn_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
@@ -79,7 +82,8 @@ def build_hip(jobs=8, force=False) -> Path | None:
     if not HIP_SOURCES:
         return None
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    headers = list((CSRC / "hip").glob("*.h")) + list((CSRC / "hip").glob("*.hpp"))
+    # (this file counts as a header: a change of the flags rebuilds every object)
+    headers = list((CSRC / "hip").glob("*.h")) + list((CSRC / "hip").glob("*.hpp")) + [Path(__file__)]
     objs, changed = _compile_all(hipcc, HIP_FLAGS, HIP_SOURCES, headers, "hip", jobs, HIP_FILE_FLAGS)
     if changed or force or not out.exists():
         LIB.mkdir(exist_ok=True)

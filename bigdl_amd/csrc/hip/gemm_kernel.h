@@ -1,4 +1,4 @@
-// Dequant-fused MFMA GEMM for mid-size row counts on gfx950:  y[M,N] = f(x[M,K] . dequant(W)[N,K]^T), 16 < M <= ~512,
+// Dequant-fused MFMA GEMM for mid-size row counts on gfx950:  y[M,N] = f(x[M,K] . dequant(W)[N,K]^T), 64 < M <= ~512,
 // and its grouped (mixture-of-experts) form where every 64/128-row block of x belongs to one expert.
 //
 // Takes the place of the reference's closed xe_linear.forward_new for prefill-sized inputs / xe_batch.batch_forward
@@ -420,10 +420,9 @@ static int gemm_launch_mt(const GemmArgs& a, int mblocks, hipStream_t st) {
   return HIP_CHECK_LAUNCH();
 }
 
-// bm: rows per block (16 / 32 / 64 / 128); bn: columns per block (128).  64-column blocks were measured too (more
-// workgroups streaming weights at few rows): slower or equal on every Llama-2-7B projection shape.  The row block
-// follows the row count: every workgroup re-reads the x rows of its K range, and with 64-row blocks that x tile (16 KiB
-// per k-tile) is twice the weight tile (8 KiB) whatever the real row count is.
+// bm: rows per block (64 / 128); bn: columns per block (128).  64-column blocks were measured too (more workgroups
+// streaming weights at few rows): slower or equal on every Llama-2-7B projection shape.  Up to 64 rows the dense products
+// run on gemm_rows_kernel.h.
 template <int QT>
 static int gemm_launch_qt(const GemmArgs& a, int bm, int bn, int mblocks, hipStream_t st) {
   if (bn != 128) return -4;
@@ -434,12 +433,8 @@ static int gemm_launch_qt(const GemmArgs& a, int bm, int bn, int mblocks, hipStr
   }
   static const int lw = getenv("BIGDL_GEMM_LOADER") ? atoi(getenv("BIGDL_GEMM_LOADER")) : 1;
   if (lw && (a.K & 127) == 0) {
-    if (bm == 16) return gemm_launch_mt<QT, 1, 2, false, 4, true>(a, mblocks, st);
-    if (bm == 32) return gemm_launch_mt<QT, 2, 2, false, 4, true>(a, mblocks, st);
     if (bm == 64) return gemm_launch_mt<QT, 4, 2, false, 4, true>(a, mblocks, st);
   }
-  if (bm == 16) return gemm_launch_mt<QT, 1, 2>(a, mblocks, st);
-  if (bm == 32) return gemm_launch_mt<QT, 2, 2>(a, mblocks, st);
   if (bm == 64) return gemm_launch_mt<QT, 4, 2>(a, mblocks, st);
   if (bm == 128) return gemm_launch_mt<QT, 8, 2>(a, mblocks, st);
   return -4;

@@ -2,6 +2,8 @@
 // format: gemm_inst_*.hip), its split-K reduce/epilogue kernel and the device-side block table of the grouped
 // (mixture-of-experts) form.
 #include "gemm_kernel.h"
+#include "gemm_rows_kernel.h"
+#include "gemm_rows.h"
 #include <stdlib.h>
 
 namespace bigdl {
@@ -196,22 +198,42 @@ static int pick_bn(int M) {
   return 128;
 }
 
-extern "C" int bigdl_gemm_lowbit_splitk(int M, int N, int K) {
+// Up to 64 rows the few-row kernel (gemm_rows_kernel.h) replaces the tile kernel: Llama-2-7B shapes, sym_int4, one MI355X, tile
+// kernel with its reduce launch -> few-row kernel, us: 64 rows qkv 25.3 -> 16.9, o 16.6 -> 12.4, gate / up 32.8 -> 23.7, down
+// 22.2 -> 23 (the one equal: K = 11008 makes x the larger stream, it runs in two K splits); 32 rows 19.8 -> 12.1, 12.8 -> 9.0,
+// 26.2 -> 17.6, 17.7 -> 17.8; 14336-wide shapes, asym_int4: 64 rows qkv 25.6 -> 14.1, gate / up 43.8 -> 35.5.
+static bool takes_rows_kernel(const void* x, int ldx, int M, int N, int K, int qtype, bool pair, RowsPlan* plan) {
+  if (M > 64 || !is_t16(qtype)) return false;
+  if (x != nullptr && !rows_ok(x, ldx)) return false;
+  *plan = rows_plan(M, N, K, qtype, pair, !pair);
+  return true;
+}
+static int launch_rows(const GemmArgs& a, int qtype, const RowsPlan& p, hipStream_t stream) {
+  RowsArgs b = {};
+  b.x = a.x; b.w = a.w; b.w2 = a.w2; b.out = a.out; b.partial = a.partial; b.bias = a.bias; b.bias2 = a.bias2; b.residual = a.residual;
+  b.M = a.M; b.N = a.N; b.K = a.K; b.ldx = a.ldx; b.ldo = a.ldo; b.act = a.act; b.out_type = a.out_type;
+  b.splitk = p.splitk; b.kt_per_split = p.kt_per_split;
+  const int rc = rows_launch(b, p, qtype, stream);
+  return rc != 0 || p.splitk == 1 ? rc : launch_reduce(a, stream);
+}
+
+// qtype: the format as the caller knows it
+extern "C" int bigdl_gemm_lowbit_splitk(int M, int N, int K, int qtype) {
   int sk, per;
+  RowsPlan p;
+  // (the workspace has to do for whichever kernel the alignment of x allows)
+  const int rows_sk = takes_rows_kernel(nullptr, 0, M, N, K, t16_kernel_qtype(qtype), false, &p) ? p.splitk : 1;
   const int bm = bigdl_gemm_lowbit_bm(M);
   plan((M + bm - 1) / bm, pick_bn(M), N, K, &sk, &per);
-  return sk;
+  return sk > rows_sk ? sk : rows_sk;
 }
 
 extern "C" int bigdl_gemm_lowbit_bm(int M) {
+  (void)M;
   static const int forced = getenv("BIGDL_GEMM_BM") ? atoi(getenv("BIGDL_GEMM_BM")) : 0;
-  if (forced == 16 || forced == 32 || forced == 64 || forced == 128) return forced;
+  if (forced == 64 || forced == 128) return forced;
   // 64-row blocks keep two or more wavefronts per SIMD (170 VGPRs): measured 10-40 % faster than 128-row blocks at
-  // every M between 64 and 1024 on the Llama-2-7B projection shapes; 16 / 32-row blocks for row counts that fit them
-  // (a quarter / half of the x tile traffic of a 64-row block)
-  static const int small = getenv("BIGDL_GEMM_SMALL_BM") ? atoi(getenv("BIGDL_GEMM_SMALL_BM")) : 1;
-  if (small && M <= 16) return 16;
-  if (small && M <= 32) return 32;
+  // every M between 64 and 1024 on the Llama-2-7B projection shapes
   return 64;
 }
 
@@ -226,6 +248,12 @@ extern "C" int bigdl_gemm_lowbit(const void* x, const void* w, void* out, const 
   GemmArgs a = {};
   a.x = (const _Float16*)x; a.w = w; a.out = out; a.bias = bias; a.residual = residual; a.partial = workspace;
   a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldo = ldo; a.act = act; a.out_type = out_type;
+  RowsPlan p;
+  if (takes_rows_kernel(x, ldx, M, N, K, qtype, false, &p)) {
+    a.splitk = p.splitk;
+    if (p.splitk > 1 && (workspace == nullptr || workspace_floats < (int64_t)p.splitk * M * N)) return -5;
+    return launch_rows(a, qtype, p, stream);
+  }
   const int bm = bigdl_gemm_lowbit_bm(M);
   const int bn = pick_bn(M);
   const int mblocks = (M + bm - 1) / bm;
@@ -254,6 +282,12 @@ extern "C" int bigdl_gemm_lowbit_ex(const void* x, const void* w, const void* w2
   a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldo = ldo; a.act = act; a.out_type = out_type;
   a.gamma = (const _Float16*)gamma; a.gamma_offset = gamma_offset; a.eps = eps; a.row_ssq = gamma != nullptr ? row_ssq : nullptr;
   a.ssq_out = ssq_out; a.w2 = w2; a.bias2 = bias2;
+  RowsPlan p;
+  if (gamma == nullptr && ssq_out == nullptr && takes_rows_kernel(x, ldx, M, N, K, qtype, w2 != nullptr, &p)) {
+    a.splitk = p.splitk;
+    if (p.splitk > 1 && (workspace == nullptr || workspace_floats < (int64_t)p.splitk * M * N)) return -5;
+    return launch_rows(a, qtype, p, stream);
+  }
   const int bm = gamma != nullptr ? (bigdl_gemm_lowbit_bm(M) < 64 ? 64 : bigdl_gemm_lowbit_bm(M)) : bigdl_gemm_lowbit_bm(M);
   const int bn = pick_bn(M);
   const int mblocks = (M + bm - 1) / bm;
@@ -268,11 +302,13 @@ extern "C" int bigdl_gemm_lowbit_ex(const void* x, const void* w, const void* w2
 }
 
 // splits the extended form will use (workspace sizing): pair = 1 when w2 is given
-extern "C" int bigdl_gemm_lowbit_ex_splitk(int M, int N, int K, int pair) {
+extern "C" int bigdl_gemm_lowbit_ex_splitk(int M, int N, int K, int pair, int qtype) {
   int sk, per;
+  RowsPlan p;
+  const int rows_sk = takes_rows_kernel(nullptr, 0, M, N, K, t16_kernel_qtype(qtype), pair != 0, &p) ? p.splitk : 1;
   const int bm = bigdl_gemm_lowbit_bm(M);
   plan(((M + bm - 1) / bm) * (pair ? 2 : 1), pick_bn(M), N, K, &sk, &per);
-  return sk;
+  return sk > rows_sk ? sk : rows_sk;
 }
 
 // Grouped form: `rows` sorted rows in total; row i uses the weights of the expert that the block table assigns

@@ -1,0 +1,5 @@
+// Instantiation unit of the few-row low-bit product for one weight format.
+#include "gemm_rows_kernel.h"
+namespace bigdl {
+int gemm_rows_launch_fp8_e5m2(const RowsArgs& a, int mt, int nt, hipStream_t st) { return gemm_rows_launch_qt<Q_FP8_E5M2>(a, mt, nt, st); }
+}  // namespace bigdl

@@ -1,0 +1,5 @@
+// Instantiation unit of the few-row low-bit product for one weight format.
+#include "gemm_rows_kernel.h"
+namespace bigdl {
+int gemm_rows_launch_sym_int5(const RowsArgs& a, int mt, int nt, hipStream_t st) { return gemm_rows_launch_qt<Q_SYM_INT5>(a, mt, nt, st); }
+}  // namespace bigdl

@@ -1,6 +1,7 @@
 // Host entry point of the dequant-fused skinny GEMM (kernel: gemv_kernel.h; one instantiation
 // unit per weight format: gemv_inst_*.hip).
-#include "gemv_kernel.h"
+#include "gemm_rows_kernel.h"
+#include "gemm_rows.h"
 
 namespace bigdl {
 int gemv_launch_sym_int4(const GemvArgs& a, bool gate_up, hipStream_t st);
@@ -34,6 +35,35 @@ static int dispatch(const GemvArgs& a, int qtype, hipStream_t stream) {
     case Q_FP8_E5M2: return gemv_launch_fp8_e5m2(a, gu, stream);
     default: return -2;
   }
+}
+
+// Whether up to 16 rows take the few-row kernel (gemm_rows_kernel.h) instead of the skinny one.  The skinny kernel gives a
+// workgroup 16 columns, and every workgroup stages all rows of x; the few-row kernel shares x among up to 64 columns but
+// needs more registers a column, so it streams a single row slower (qkv 12288 x 4096 sym_int4, 1 row: 8.7 us against
+// 10.8).  What decides is therefore the x that a CU stages, rows x column tiles per CU, counted 1.5 times for a gate / up
+// pair, whose skinny form fits fewer workgroups on a CU.  Measured pairs (skinny / few-row, us): at 6: qkv 6144 x 4096
+// asym_int4 4 rows 11.6 / 11.7; at 8: pair 5632 x 2048 4 rows 9.6 / 9.7; at 12: 6144 x 4096 8 rows 13.5 / 11.7, 4096 x 4096
+// 12 rows 8.0 / 8.0; at 18: 12288 x 4096 6 rows 14.7 / 11.7; at 21: pair 14336 x 4096 4 rows 23.6 / 19.8; at 63: pair
+// 14336 x 4096 asym_int4 12 rows 50.6 / 23.5.  Two exceptions: x that no longer fits the LDS of the skinny kernel (4096 x 14336
+// asym_int4, 8 rows: 25.9 / 18.2) goes over at once, and the CU-resident form of 8 to 11 rows keeps the widest products (32000
+// x 4096 asym_int4, 8 rows: 25.7 / 29.7; 12 rows: 31.8 / 29.7).
+static bool takes_rows_kernel(const GemvArgs& a) {
+  if (a.M > 16 || a.M < 3 || a.att_ws != nullptr || a.ln_c1 != nullptr || !rows_ok(a.x, a.ldx)) return false;
+  const int tiles = (a.N + 15) / 16, cus = gemv_cu_count();
+  const size_t xbytes = (size_t)a.M * ((a.K + 127) / 128 * 128 + XTAIL + XPAD) * 2;
+  if (xbytes > GEMV_XLDS_LIMIT_FEW_ROWS) return true;
+  if (tiles > 4 * cus && a.M >= 8 && a.M <= 11) return false;
+  return (int64_t)a.M * tiles * (a.w2 != nullptr ? 3 : 2) >= 20ll * cus;
+}
+
+static int launch_rows(const GemvArgs& a, int qtype, hipStream_t stream) {
+  const RowsPlan p = rows_plan(a.M, a.N, a.K, qtype, a.w2 != nullptr, false);
+  RowsArgs b = {};
+  b.x = a.x; b.w = a.w; b.w2 = a.w2; b.out = a.out; b.bias = a.bias; b.bias2 = a.bias2; b.residual = a.residual;
+  b.gamma = a.gamma; b.gamma_offset = a.gamma_offset; b.eps = a.eps;
+  b.M = a.M; b.N = a.N; b.K = a.K; b.ldx = a.ldx; b.ldo = a.ldo; b.act = a.act; b.out_type = a.out_type;
+  b.splitk = p.splitk; b.kt_per_split = p.kt_per_split;
+  return rows_launch(b, p, qtype, stream);
 }
 
 // Returns 0 on success; negative = rejected on the host before any launch.
@@ -72,6 +102,7 @@ static int gemv_lowbit_impl(const void* x, const void* w, const void* w2, void* 
   a.att_qlen = att_qlen; a.att_rows_alloc = att_rows_alloc;
   a.ln_c1 = ln_c1; a.ln_c2 = ln_c2; a.ln2_c1 = ln2_c1; a.ln2_c2 = ln2_c2;
   a.slot_expert = nullptr; a.slot_scale = nullptr; a.n_total = 0; a.slot_xdiv = 1; a.n_slots = 0; a.slot_cat = 0;
+  if (is_t16(qtype) && takes_rows_kernel(a)) return launch_rows(a, qtype, stream);
   return dispatch(a, qtype, stream);
 }
 

@@ -1,0 +1,104 @@
+"""The few-row low-bit product (csrc/hip/gemm_rows_kernel.h) against a float64 product of the dequantized weight."""
+import pytest
+import torch
+
+from bigdl_amd import qtypes as Q
+from bigdl_amd.ops import host
+
+pytestmark = pytest.mark.gpu
+FORMATS = ["sym_int4", "asym_int4", "woq_int4", "fp4", "nf4", "sym_int5", "asym_int5", "fp6", "sym_int8", "fp8_e4m3", "fp8_e5m2"]
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from bigdl_amd.ops import hip as h
+    h.lib()
+    return h
+
+
+def _weight(n, k, qt, seed):
+    w = torch.randn(n, k, generator=torch.Generator().manual_seed(seed)) * 0.05
+    raw = host.quantize(w, qt)
+    raw = raw.view(torch.uint8) if raw.dtype != torch.uint8 else raw
+    return host.relayout_to_device(raw, qt, n, k).cuda(), host.dequantize(raw, qt, w.shape).double()
+
+
+def _x(m, k, seed):
+    """[m, k] rows inside a buffer of NaN: what lies behind a row or below the last one must not be read as data"""
+    buf = torch.full((m + 2, k + 24), float("nan"), dtype=torch.float16)
+    buf[:m, :k] = torch.randn(m, k, generator=torch.Generator().manual_seed(seed)).half()
+    return buf.cuda()[:m, :k], buf[:m, :k].double()
+
+
+def _close(out, x, w, ref, m, extra=0.0, nf4=False):
+    # up to 16 rows the codes are exact in fp16 and the scale is applied in fp32: fp32 sums only (k * 2^-24 of the absolute
+    # sum, bounded loosely), but for nf4, whose code values are a table in fp16 (2^-11 each).  More rows round
+    # code * scale (+ min) to fp16: 2^-11 of a weight's larger term, on top of the table's, times two.
+    bound = (2.0 ** -9 if m > 16 else 2.0 ** -11 if nf4 else 2.0 ** -16) * (x.abs() @ w.abs().t()) + 1e-5 + extra
+    assert torch.isfinite(out).all()
+    assert ((out.double().cpu() - ref).abs() <= bound).all()
+
+
+# (rows, N, K): tile edges of rows and columns, a last k-tile that is cut, fewer k-tiles than wavefronts, one more than
+# the tiles in flight
+SHAPES = [(1, 16, 32), (6, 37, 2080), (16, 200, 1024), (17, 48, 96), (32, 65, 2304), (33, 130, 3232), (64, 80, 1184), (70, 33, 1024)]
+
+
+@pytest.mark.parametrize("name", FORMATS)
+@pytest.mark.parametrize("shape", SHAPES)
+def test_every_tiling_matches_float64(hip, name, shape):
+    m, n, k = shape
+    k = k if name not in ("nf4", "woq_int4") else (k + 127) // 128 * 128
+    qt = Q.ggml_tensor_qtype[name]
+    dev, w = _weight(n, k, qt, 1)
+    x, xd = _x(m, k, 2)
+    ref = xd @ w.t()
+    mt = 1 if m <= 16 else 2 if m <= 32 else 4
+    for nt in (0, 1, 2, 3) + ((4,) if mt < 4 else ()):
+        _close(hip.gemm_rows(x, dev, qt, n, k, out_dtype=torch.float32, nt=nt), xd, w, ref, m, nf4=name == "nf4")
+    parts = hip.gemm_rows(x, dev, qt, n, k, out_dtype=torch.float32, nt=2, splitk=3)
+    if parts.dim() == 3:
+        _close(parts.sum(0), xd, w, ref, m, nf4=name == "nf4")
+
+
+@pytest.mark.parametrize("name", ["sym_int4", "asym_int5", "nf4", "sym_int8"])
+@pytest.mark.parametrize("m", [3, 16, 24, 61])
+def test_pairs_norm_bias_residual(hip, name, m):
+    n, k, eps = 104, 1280, 1e-5
+    qt = Q.ggml_tensor_qtype[name]
+    (dg, wg), (du, wu) = _weight(n, k, qt, 3), _weight(n, k, qt, 4)
+    x, xd = _x(m, k, 5)
+    b1, b2 = torch.randn(n).half(), torch.randn(n).half()
+    res = torch.randn(m, n).half()
+    gamma = (1 + 0.1 * torch.randn(k)).half()
+    silu = torch.nn.functional.silu
+    for nt in (0, 1, 2):
+        xn, kw = xd, {}
+        if m <= 16:
+            # x * gamma is rounded to fp16 before the product, so the reference multiplies those values
+            xn = (xd.half() * gamma).double() * torch.rsqrt(xd.pow(2).mean(-1, keepdim=True) + eps)
+            kw = dict(gamma=gamma.cuda(), eps=eps)
+        got = hip.gemm_rows(x, dg, qt, n, k, w2=du, bias=b1.cuda(), bias2=b2.cuda(), act="silu", out_dtype=torch.float32, nt=nt, **kw)
+        ref = silu(xn @ wg.t() + b1.double()) * (xn @ wu.t() + b2.double())
+        torch.testing.assert_close(got.cpu().double(), ref, rtol=4e-3, atol=8e-3)      # two products of 2^-9 and 2^-10 each, silu's slope 1.1
+        out = res.cuda()
+        hip.gemm_rows(x, dg, qt, n, k, bias=b1.cuda(), residual=out, out=out, nt=nt)    # in place, as on the residual stream
+        torch.testing.assert_close(out.cpu().double(), xd @ wg.t() + b1.double() + res.double(), rtol=2e-3, atol=8e-3)
+
+
+@pytest.mark.parametrize("name", ["sym_int4", "q4_k", "nf4", "sym_int8"])
+@pytest.mark.parametrize("m", [4, 8, 13, 16, 17, 40, 64])
+def test_public_products_at_their_row_limits(hip, name, m):
+    """gemv_lowbit / gemm_lowbit / gemm_lowbit_ex on either side of each change of kernel, K split included"""
+    qt = Q.ggml_tensor_qtype[name]
+    n, k = 272, 11008
+    dev, w = _weight(n, k, qt, 6)
+    x, xd = _x(m, k, 7)
+    f = hip.gemv_lowbit if m <= 16 else hip.gemm_lowbit
+    out = f(x, dev, qt, n, k, out_dtype=torch.float32)
+    # (q4_k: the tiled scale d * sc6 and min dmin * m6 are fp16, 2^-11 of terms up to the block's range, taken as 0.4)
+    _close(out, xd, w, xd @ w.t(), m if name != "q4_k" else 64, extra=0.0 if name != "q4_k" else 2.0 ** -11 * 0.4 * xd.abs().sum(-1, keepdim=True), nf4=name == "nf4")
+    if m > 16:
+        both = hip.gemm_lowbit_ex(x, dev, qt, n, k, w2=dev, act="silu")
+        y = xd @ w.t()
+        torch.testing.assert_close(both.cpu().double(), torch.nn.functional.silu(y) * y, rtol=1e-2, atol=0.15)     # y reaches 30: 2^-9 of y^2

@@ -7,11 +7,12 @@ namespace bigdl {
 #define ROWS_FORMATS(X)                                                                                                     \
   X(Q_SYM_INT4, sym_int4) X(Q_ASYM_INT4, asym_int4) X(Q_WOQ_INT4, woq_int4) X(Q_FP4, fp4) X(Q_NF4, nf4)                     \
   X(Q_SYM_INT5, sym_int5) X(Q_ASYM_INT5, asym_int5) X(Q_FP6, fp6) X(Q_SYM_INT8, sym_int8) X(Q_FP8_E4M3, fp8_e4m3)           \
-  X(Q_FP8_E5M2, fp8_e5m2)
+  X(Q_FP8_E5M2, fp8_e5m2) X(Q_Q6_K, q6_k)
 #define ROWS_DECLARE(id, name) int gemm_rows_launch_##name(const RowsArgs& a, int mt, int nt, hipStream_t st);
 ROWS_FORMATS(ROWS_DECLARE)
 
 static int tile_bytes(int qtype) {
+  if (qtype == Q_Q6_K) return 16 * 105;      // half of a 210-byte block a row
   return 256 * (lo_bits_of(qtype) + hi_bits_of(qtype)) + (has_min_of(qtype) ? 256 : 128);
 }
 
@@ -49,6 +50,7 @@ int rows_launch(const RowsArgs& a, const RowsPlan& p, int qtype, hipStream_t st)
 
 using namespace bigdl;
 
+// (q6_k: w holds the file's blocks row by row, K % 256 == 0, 4-byte aligned, no w2.)
 // y = act(norm?(x) W^T + bias) [* (x W2^T + bias2)] [+ residual] on an explicit tiling (nt weight tiles per workgroup, K
 // split over splitk workgroups); nt = 0: the planner's, unsplit.  workspace: fp32, splitk * M * N (twice that with w2) when split: the partial
 // sums stay there, nothing is written to out.  For tests and measurements; the public products choose by themselves.
@@ -57,7 +59,9 @@ extern "C" int bigdl_gemm_rows(const void* x, const void* w, const void* w2, voi
                                int64_t workspace_floats, int M, int N, int K, int ldx, int ldo, int qtype, int act, int out_type,
                                int nt, int splitk, hipStream_t stream) {
   qtype = t16_kernel_qtype(qtype);
-  if (M <= 0 || N <= 0 || K <= 0 || (K & 31) || !rows_ok(x, ldx) || ((uintptr_t)w & 15) || (w2 && ((uintptr_t)w2 & 15)) || splitk < 1) return -1;
+  const bool raw = qtype == Q_Q6_K;
+  if (raw && ((K & 255) || w2 != nullptr)) return -1;
+  if (M <= 0 || N <= 0 || K <= 0 || (K & 31) || !rows_ok(x, ldx) || ((uintptr_t)w & (raw ? 3 : 15)) || (w2 && ((uintptr_t)w2 & 15)) || splitk < 1) return -1;
   if (gamma != nullptr && (((uintptr_t)gamma & 15) || M > 16 || splitk > 1)) return -7;
   if (out_type < 0 || out_type > 2) return -3;
   RowsPlan p = rows_plan(M, N, K, qtype, w2 != nullptr, false);

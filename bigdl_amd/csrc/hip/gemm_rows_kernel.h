@@ -56,8 +56,8 @@ constexpr int rows_x_halves(int mt, int ns) { return mt * ns > 16 || mt * ns == 
 // k-tiles of weights requested ahead: about eight tiles per wavefront (72 KiB a CU), as far as the registers of two
 // wavefronts per SIMD hold them
 constexpr int rows_ahead(int qt, int mt, int ns) {
-  const int tile = lo_bits_of(qt) + hi_bits_of(qt) + 2 + (has_min_of(qt) ? 2 : 0);        // VGPRs of a weight tile
-  const int other = ns * mt * 4 + 8 * mt * rows_x_halves(mt, ns) + (mt == 4 ? 30 : mt == 1 ? 6 * ns : 0) + (lo_bits_of(qt) == 8 ? 120 : has_min_of(qt) || hi_bits_of(qt) == 2 ? 84 : 72);
+  const int tile = qt == Q_Q6_K ? 14 : lo_bits_of(qt) + hi_bits_of(qt) + 2 + (has_min_of(qt) ? 2 : 0);        // VGPRs of a weight tile
+  const int other = ns * mt * 4 + 8 * mt * rows_x_halves(mt, ns) + (mt == 4 ? 30 : mt == 1 ? 6 * ns : 0) + (lo_bits_of(qt) == 8 || qt == Q_Q6_K ? 120 : has_min_of(qt) || hi_bits_of(qt) == 2 ? 84 : 72);
   int ahead = 1;
   while (ahead < 4 && (ahead < 2 || ahead * ns < 6) && other + (ahead + 1) * ns * tile <= 250) ++ahead;
   return ahead;
@@ -96,6 +96,92 @@ struct RowsPlanes {
   }
 };
 
+// How a lane's share of a weight tile becomes MFMA operands.  T16 formats: fragment s holds k = 32 s + 8 g + j, one 32-element
+// scale block per fragment.
+template <int QT>
+__device__ __forceinline__ half8 rows_fragment(const Tile<QT>& t, int s, const _Float16* lut, int) { return decode_step<QT>(t, s, lut); }
+template <int QT>
+__device__ __forceinline__ float rows_scale(const Tile<QT>& t, int s) { return (float)t.d[s] * post_scale<QT>(); }
+template <int QT>
+__device__ __forceinline__ half8 rows_scaled(const Tile<QT>& t, half8 code, int s) {
+  _Float16 d = t.d[s];
+  if constexpr (post_scale<QT>() != 1.0f) d = (_Float16)fminf((float)d * post_scale<QT>(), 65504.0f);
+  if constexpr (has_min<QT>()) return code * d + t.m[s];
+  return code * d;
+}
+template <int QT>
+__device__ __forceinline__ int rows_chunk(int s, int g) { return 4 * (s & 1) + g; }     // 16-byte chunk of half an x tile
+
+// q6_k as the file's blocks hold it (210 bytes for 256 elements of a row: 128 of low nibbles, 64 of high bit pairs, 16 int8
+// sub-scales, fp16 d): a k-tile is half a block.  Lane group g takes bytes 16 g .. of the half's low nibbles -- 64 contiguous
+// bytes a row and request -- so that fragment s holds k = 32 ((g >> 1) + 2 (s >> 1)) + 16 (g & 1) + 8 (s & 1) + j, all of it
+// in sub-block g + 4 (s >> 1).  Code times sub-scale is exact in fp16 up to 2048 and within 2^-12 above; d multiplies the fp32
+// product (up to 16 rows).
+// Blocks start at even bytes, every other one between two dwords.  16-byte loads from there are split by the address unit
+// (4096 x 11008, 1 row: 34 us, 25 this way); so the dwords around them are loaded and shifted into place.  The last dword's address steps
+// back where it is not needed: nothing outside the block is touched.
+typedef uint4v rows_raw16 __attribute__((aligned(4)));
+typedef uint2v rows_raw8 __attribute__((aligned(4)));
+template <>
+struct Tile<Q_Q6_K> {
+  uint4v ql, qh;
+  uint32_t ql4, qh4, sc2;     // the dword behind each
+  uint2v sc;
+  _Float16 d;
+};
+template <>
+struct RowsPlanes<Q_Q6_K> {
+  const uint8_t* row[4];      // this lane's weight row of every column tile
+  template <int NT>
+  __device__ __forceinline__ void init(const void* w, int first, int N, int K, int lane) {
+#pragma unroll
+    for (int n = 0; n < NT; ++n) row[n] = (const uint8_t*)w + (int64_t)min((first + n) * 16 + (lane & 15), N - 1) * (K / 256 * 210);
+  }
+  __device__ __forceinline__ void load(Tile<Q_Q6_K>& t, int n, int kt, int lane) const {
+    const uint8_t* b = row[n] + (kt >> 1) * 210;
+    const int h = kt & 1, g = lane >> 4, odd = (int)((uintptr_t)b & 2);
+    const uint8_t* c = b - odd;          // (the pieces start at multiples of 8: they are all as far off a dword as the block)
+    const uint8_t* last = c + 2 * odd;   // + 4 where the shift needs one more dword
+    t.ql = *(const rows_raw16*)(c + 64 * h + 16 * g);
+    t.ql4 = *(const uint32_t*)(last + 64 * h + 16 * g + 12);
+    t.qh = *(const rows_raw16*)(c + 128 + 32 * h + 16 * (g & 1));
+    t.qh4 = *(const uint32_t*)(last + 128 + 32 * h + 16 * (g & 1) + 12);
+    t.sc = *(const rows_raw8*)(c + 192 + 8 * h);
+    t.sc2 = *(const uint32_t*)(last + 192 + 8 * h + 4);
+    t.d = *(const _Float16*)(b + 208);
+  }
+  // the tile with its pieces shifted into place
+  __device__ __forceinline__ void settle(Tile<Q_Q6_K>& t, int n, int kt) const {
+    const uint32_t odd = (uint32_t)((uintptr_t)(row[n] + (kt >> 1) * 210) & 2);
+    t.ql = uint4v{__builtin_amdgcn_alignbyte(t.ql[1], t.ql[0], odd), __builtin_amdgcn_alignbyte(t.ql[2], t.ql[1], odd),
+                  __builtin_amdgcn_alignbyte(t.ql[3], t.ql[2], odd), __builtin_amdgcn_alignbyte(t.ql4, t.ql[3], odd)};
+    t.qh = uint4v{__builtin_amdgcn_alignbyte(t.qh[1], t.qh[0], odd), __builtin_amdgcn_alignbyte(t.qh[2], t.qh[1], odd),
+                  __builtin_amdgcn_alignbyte(t.qh[3], t.qh[2], odd), __builtin_amdgcn_alignbyte(t.qh4, t.qh[3], odd)};
+    t.sc = uint2v{__builtin_amdgcn_alignbyte(t.sc[1], t.sc[0], odd), __builtin_amdgcn_alignbyte(t.sc2, t.sc[1], odd)};
+  }
+};
+template <>
+__device__ __forceinline__ half8 rows_fragment<Q_Q6_K>(const Tile<Q_Q6_K>& t, int s, const _Float16*, int g) {
+  H8 r;
+  const half2v off = {(_Float16)1056.0f, (_Float16)1056.0f};       // 1024 + 32
+  const _Float16 sc = (_Float16)(float)(int8_t)(t.sc[s >> 1] >> (8 * g));
+  const int up = 2 * (g >> 1) + 4 * (s >> 1);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const uint32_t lo = t.ql[2 * (s & 1) + i] >> (4 * (s >> 1)), hi = t.qh[2 * (s & 1) + i] >> up;
+    const uint32_t code = (lo & 0x0F0F0F0Fu) | ((hi & 0x03030303u) << 4);
+    r.h2[2 * i] = (u2h(__builtin_amdgcn_perm(0x64646464u, code, 0x04010400u)) - off) * sc;
+    r.h2[2 * i + 1] = (u2h(__builtin_amdgcn_perm(0x64646464u, code, 0x04030402u)) - off) * sc;
+  }
+  return r.v;
+}
+template <>
+__device__ __forceinline__ float rows_scale<Q_Q6_K>(const Tile<Q_Q6_K>& t, int) { return (float)t.d; }
+template <>
+__device__ __forceinline__ half8 rows_scaled<Q_Q6_K>(const Tile<Q_Q6_K>& t, half8 code, int) { return code * t.d; }
+template <>
+__device__ __forceinline__ int rows_chunk<Q_Q6_K>(int s, int g) { return 2 * g + (s & 1); }
+
 // MT = 16-row tiles of x, NT = 16-column tiles of a weight per workgroup, WD = k-tiles of weights requested ahead.
 template <int QT, int MT, int NT, bool PAIR, int NW = ROWS_NW, int WD = rows_ahead(QT, MT, PAIR ? 2 * NT : NT)>
 __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(RowsArgs a) {
@@ -122,7 +208,10 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(RowsAr
 
   const _Float16* lut = nullptr;
   RowsPlanes<QT> pl, pl2;
-  pl.init(t16_planes(a.w, QT, a.N, a.K), (int64_t)nb * NT * KT, min(NT, ntiles - nb * NT) * KT);
+  constexpr bool RAW = QT == Q_Q6_K;
+  static_assert(!RAW || !PAIR, "q6_k: single products");
+  if constexpr (RAW) pl.template init<NT>(a.w, nb * NT, a.N, a.K, lane);
+  else pl.init(t16_planes(a.w, QT, a.N, a.K), (int64_t)nb * NT * KT, min(NT, ntiles - nb * NT) * KT);
   if constexpr (PAIR) pl2.init(t16_planes(a.w2, QT, a.N, a.K), (int64_t)nb * NT * KT, min(NT, ntiles - nb * NT) * KT);
   int tbase[NT];                                     // first tile of the block's tile rows (past the last one: that again)
 #pragma unroll
@@ -140,7 +229,8 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(RowsAr
     const int kt = kmap(i), out = past(i);
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
-      pl.load(t[n], tbase[n] + kt, lane, out);
+      if constexpr (RAW) pl.load(t[n], n, kt, lane);        // (past the end: the last tile again, never multiplied)
+      else pl.load(t[n], tbase[n] + kt, lane, out);
       if constexpr (PAIR) pl2.load(t[NT + n], tbase[n] + kt, lane, out);
     }
   };
@@ -207,7 +297,7 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(RowsAr
     for (int s = 2 * h; s < 2 * h + 2; ++s) {
       half8 xa[MT];
 #pragma unroll
-      for (int j = 0; j < MT; ++j) xa[j] = *(const half8*)(xt + h * XB + (16 * j + r) * 128 + (((4 * (s & 1) + g) ^ (r & 7)) << 4));
+      for (int j = 0; j < MT; ++j) xa[j] = *(const half8*)(xt + h * XB + (16 * j + r) * 128 + ((rows_chunk<QT>(s, g) ^ (r & 7)) << 4));
       float4v sx[POST ? MT : 1];
       if constexpr (POST && has_min<QT>()) {
         // block sums of x in the layout of the product: a fragment of ones
@@ -217,9 +307,9 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(RowsAr
       }
 #pragma unroll
       for (int n = 0; n < NS; ++n) {
-        const half8 code = decode_step<QT>(t[n], s, lut);
+        const half8 code = rows_fragment<QT>(t[n], s, lut, g);
         if constexpr (POST) {
-          const float d = (float)t[n].d[s] * post_scale<QT>();
+          const float d = rows_scale<QT>(t[n], s);
 #pragma unroll
           for (int j = 0; j < MT; ++j) {
             const float4v c = mfma16(xa[j], code, float4v{0, 0, 0, 0});
@@ -232,11 +322,7 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(RowsAr
             }
           }
         } else {
-          _Float16 d = t[n].d[s];
-          if constexpr (post_scale<QT>() != 1.0f) d = (_Float16)fminf((float)d * post_scale<QT>(), 65504.0f);
-          half8 bf;
-          if constexpr (has_min<QT>()) bf = code * d + t[n].m[s];
-          else bf = code * d;
+          const half8 bf = rows_scaled<QT>(t[n], code, s);
 #pragma unroll
           for (int j = 0; j < MT; ++j) acc[n][j] = mfma16(xa[j], bf, acc[n][j]);
         }
@@ -255,6 +341,11 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(RowsAr
     for (int d = 0; d < WD; ++d) {
       // (only arithmetic stands under a condition: a load there would cost the counts of the waits)
       const bool live = d == 0 || i + d < nk, next = i + d + 1 < nk;
+      if constexpr (RAW) {
+        if (live)
+#pragma unroll
+          for (int n = 0; n < NT; ++n) pl.settle(tt[d][n], n, kmap(i + d));
+      }
       if constexpr (XH == 2) {
         if (live) stage_x(1);
         fetch_x(i + d + 1, 1);
@@ -390,10 +481,18 @@ static int gemm_rows_launch_mt(const RowsArgs& a, int nt, hipStream_t st) {
 template <int QT>
 static int gemm_rows_launch_qt(const RowsArgs& a, int mt, int nt, hipStream_t st) {
   const bool pair = a.w2 != nullptr;
+  if constexpr (QT == Q_Q6_K) {
+    if (pair) return -7;
+    if (mt == 1) return gemm_rows_launch_mt<QT, 1, false>(a, nt, st);
+    if (mt == 2) return gemm_rows_launch_mt<QT, 2, false>(a, nt, st);
+    if (mt == 4) return gemm_rows_launch_mt<QT, 4, false>(a, nt, st);
+    return -4;
+  } else {
   if (mt == 1) return pair ? gemm_rows_launch_mt<QT, 1, true>(a, nt, st) : gemm_rows_launch_mt<QT, 1, false>(a, nt, st);
   if (mt == 2) return pair ? gemm_rows_launch_mt<QT, 2, true>(a, nt, st) : gemm_rows_launch_mt<QT, 2, false>(a, nt, st);
   if (mt == 4) return pair ? gemm_rows_launch_mt<QT, 4, true>(a, nt, st) : gemm_rows_launch_mt<QT, 4, false>(a, nt, st);
   return -4;
+  }
 }
 
 }  // namespace bigdl

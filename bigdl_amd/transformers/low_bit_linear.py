@@ -32,6 +32,10 @@ TORCH_LINEAR_THRESHOLD = int(os.getenv("BIGDL_LLM_LINEAR_THRESHOLD", "512"))
 # up to 32 rows, inside the batched decode step the GEMM path is 20 % ahead at 32 rows), dequantize + hipBLASLt above
 GEMV_MAX_ROWS = int(os.getenv("BIGDL_GEMV_MAX_ROWS", "16"))
 GEMM_MAX_ROWS = 256
+# q6_k weights stay in their checkpoint blocks on the GPU.  Up to this many fp16 rows are multiplied from the blocks (csrc/hip/
+# gemm_rows_kernel.h); above, and for bf16 activations, whose range fp16 does not have, the weight is expanded for a dense
+# product.  4096 x 11008, one MI355X, expanded -> from the blocks: 1 row 100 -> 25 us, 64 rows 108 -> 35, 128 rows 128 -> 58.
+Q6K_MAX_ROWS = 128
 # forward of frozen low-bit linears inside a training step on the fused prompt GEMM (fp16 copy of the activations)
 # instead of dequantize + dense product
 _TRAIN_FUSED_FORWARD = os.getenv("BIGDL_TRAIN_FUSED_FORWARD", "0") == "1"
@@ -332,6 +336,12 @@ def lowbit_matmul(x_2d: torch.Tensor, weight: FP4Params, out_features: int, for_
             if xh.stride(1) != 1 or xh.stride(0) % 8 or xh.data_ptr() % 16:
                 xh = xh.contiguous()
             return lowbit_rows(xh, weight.data, weight.qtype, n, k, out_dtype=x_2d.dtype)
+        if weight.qtype == Q.Q6_K and m <= Q6K_MAX_ROWS and x_2d.dtype != torch.bfloat16 and not for_training and weight.data.data_ptr() % 4 == 0:
+            xh = x_2d.to(torch.float16)
+            if xh.stride(1) != 1 or xh.stride(0) % 8 or xh.data_ptr() % 16:
+                xh = xh.contiguous()
+            raw = weight.data.view(torch.uint8) if weight.data.dtype != torch.uint8 else weight.data
+            return hip.gemm_q6k(xh, raw, n, k, out_dtype=x_2d.dtype)
         cdt = x_2d.dtype if x_2d.dtype in (torch.float16, torch.bfloat16) else torch.float16
         w = dequant_weight(weight, cdt)
         xc = x_2d.to(cdt)

@@ -102,3 +102,36 @@ def test_public_products_at_their_row_limits(hip, name, m):
         both = hip.gemm_lowbit_ex(x, dev, qt, n, k, w2=dev, act="silu")
         y = xd @ w.t()
         torch.testing.assert_close(both.cpu().double(), torch.nn.functional.silu(y) * y, rtol=1e-2, atol=0.15)     # y reaches 30: 2^-9 of y^2
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 16, 256), (5, 37, 512), (16, 130, 2304), (17, 48, 4096), (40, 33, 2816), (64, 80, 1024), (70, 20, 512)])
+def test_q6k_blocks_without_expansion(hip, m, n, k):
+    w0 = torch.randn(n, k, generator=torch.Generator().manual_seed(8)) * 0.05
+    raw = host.quantize(w0, Q.Q6_K)
+    w = host.dequantize(raw, Q.Q6_K, w0.shape).double()
+    x, xd = _x(m, k, 9)
+    ref = xd @ w.t()
+    # code * sub-scale reaches 32 * 128: above 2048 it is rounded to 2^-11; more than 16 rows round the weight to fp16 once
+    for nt in (0, 1, 2, 3):
+        out = hip.gemm_rows(x, raw.cuda(), Q.Q6_K, n, k, out_dtype=torch.float32, nt=nt)
+        bound = (2.0 ** -11 if m <= 16 else 2.0 ** -10) * (xd.abs() @ w.abs().t()) + 1e-5
+        assert ((out.double().cpu() - ref).abs() <= bound).all()
+
+
+def test_q6k_linear_takes_the_blocks_for_few_rows(hip):
+    from bigdl_amd.transformers.low_bit_linear import FP4Params, Q6K_MAX_ROWS, lowbit_matmul
+    n, k = 96, 1024
+    w0 = torch.randn(n, k, generator=torch.Generator().manual_seed(10)) * 0.05
+    p = FP4Params(host.quantize(w0, Q.Q6_K), quantized=True, _shape=(n, k), qtype=Q.Q6_K).to("cuda")
+    w = host.dequantize(p.data.cpu(), Q.Q6_K, (n, k)).double()
+    for m in (1, Q6K_MAX_ROWS, Q6K_MAX_ROWS + 1):
+        for dt, tol in ((torch.float16, 2e-3), (torch.float32, 2e-3), (torch.bfloat16, 1e-2)):
+            x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(dt)
+            got = lowbit_matmul(x.cuda(), p, n)
+            ref = x.double() @ w.t()
+            assert got.dtype == dt
+            # inputs and outputs of 2^-11 (2^-9 in bf16) on values of about 1.6
+            torch.testing.assert_close(got.cpu().double(), ref, rtol=tol, atol=4 * tol)
+    # strides and an offset that the kernel's 16-byte loads do not take
+    x = torch.randn(3, k + 3, generator=torch.Generator().manual_seed(11)).half()[:, 3:]
+    torch.testing.assert_close(lowbit_matmul(x.cuda(), p, n).cpu().double(), x.double() @ w.t(), rtol=2e-3, atol=8e-3)

@@ -108,7 +108,7 @@ class FP4Params(torch.nn.Parameter):
     def qlayout(self) -> str:
         """"t16" (device tile order) or "host" (ggml block order).  Derived from where the bytes live, because
         ``nn.Module._apply`` swaps ``.data`` in place and drops attributes of the tensor ``to()`` returned."""
-        if self.quantized and self.data.device.type == "cuda" and self.qtype in Q.T16_QTYPES and not self.host_only:
+        if self.quantized and self.is_cuda and self.qtype in Q.T16_QTYPES and not self.host_only:
             return "t16"
         return "host"
 
@@ -311,17 +311,18 @@ def lowbit_matmul(x_2d: torch.Tensor, weight: FP4Params, out_features: int, for_
     forward of an autograd node whose backward will expand the weight anyway (bf16 activations): prompt-sized row
     counts then take the dense product in the activations' own dtype instead of the fp16 fused kernel."""
     n, k = weight._shape
-    if weight.data.device.type == "cuda":
+    if weight.is_cuda:
         from ..ops import hip
-        m = x_2d.shape[0]
-        if weight.qlayout == "t16" and m <= GEMM_MAX_ROWS:
-            xh = x_2d if x_2d.dtype == torch.float16 else x_2d.to(torch.float16)
+        m, dt = x_2d.shape[0], x_2d.dtype
+        t16 = weight.qlayout == "t16"
+        if t16 and m <= GEMM_MAX_ROWS:
+            xh = x_2d if dt == torch.float16 else x_2d.to(torch.float16)
             if xh.stride(1) != 1 or xh.stride(0) % 8 or xh.data_ptr() % 16:
                 xh = xh.contiguous()
             if m <= GEMV_MAX_ROWS:
-                return hip.gemv_lowbit(xh, weight.data, weight.qtype, n, k, out_dtype=x_2d.dtype)
-            return hip.gemm_lowbit(xh, weight.data, weight.qtype, n, k, out_dtype=x_2d.dtype)
-        if weight.qlayout == "t16" and (not for_training or _TRAIN_FUSED_FORWARD) and getattr(weight, "_dense_cache", None) is None:
+                return hip.gemv_lowbit(xh, weight, weight.qtype, n, k, out_dtype=dt)
+            return hip.gemm_lowbit(xh, weight, weight.qtype, n, k, out_dtype=dt)
+        if t16 and (not for_training or _TRAIN_FUSED_FORWARD) and getattr(weight, "_dense_cache", None) is None:
             # prompt-sized rows: the fused kernels take every row count (reference: one native op,
             # low_bit_linear.py:657-668); no fp16 copy of the weight is written and no library GEMM runs.  (Training keeps
             # the dense product below: its backward needs the expanded weight anyway, and its activations are bf16 --
@@ -445,28 +446,31 @@ class LowBitLinear(nn.Linear):
                 x = x.to(self.compute_dtype)
             elif torch.is_autocast_enabled():
                 x = x.to(torch.get_autocast_dtype(x.device.type))
-        if self.bias is not None and self.bias.dtype != x.dtype:
-            self.bias.data = self.bias.data.to(x.dtype)
+        bias, weight = self.bias, self.weight           # (each lookup on a module walks its tables)
+        if bias is not None and bias.dtype != x.dtype:
+            bias.data = bias.data.to(x.dtype)
         if self.optimize_lm_head and not (self.training and torch.is_grad_enabled()):
             x = reshape_lm_head_input(x)       # inference only: a training step needs the logits of every position
-        new_shape = x.shape[:-1] + (self.out_len,)
-        if 0 in x.shape:
-            return torch.empty(new_shape, dtype=x.dtype, device=x.device)
+        shape, dtype = x.shape, x.dtype
+        if 0 in shape:
+            return torch.empty(shape[:-1] + (self.out_len,), dtype=dtype, device=x.device)
         if self.act_order:
             x = x[..., self.g_idx_map]
-        x_2d = x.contiguous().view(-1, x.shape[-1])
-        if not self.weight.quantized:
-            self.weight = self.weight.to(self.weight.data.device)  # lazily quantize (CPU only)
+        flat = len(shape) == 2
+        x_2d = x.contiguous() if flat else x.contiguous().view(-1, shape[-1])
+        if not weight.quantized:
+            self.weight = weight = weight.to(weight.data.device)  # lazily quantize (CPU only)
         if is_training and x_2d.requires_grad:
-            result = MatMulLowBit.apply(x_2d, self.weight, self.out_len)
+            result = MatMulLowBit.apply(x_2d, weight, self.out_len)
         else:
-            result = lowbit_matmul(x_2d, self.weight, self.out_len)
-        result = result.view(new_shape)
+            result = lowbit_matmul(x_2d, weight, self.out_len)
+        if not flat or result.shape[1] != self.out_len:
+            result = result.view(shape[:-1] + (self.out_len,))
         if self.mp_group is not None:
             result = _all_reduce(result, self.mp_group)
-        if self.bias is not None:
-            result = result + self.bias
-        return result.to(x.dtype)
+        if bias is not None:
+            result = result + bias
+        return result if result.dtype == dtype else result.to(dtype)
 
     def extra_repr(self):
         return f"in={self.in_len}, out={self.out_len}, qtype={Q.qtype_name(self.qtype)}, bias={self.bias is not None}"

@@ -198,14 +198,17 @@ static int pick_bn(int M) {
   return 128;
 }
 
-// Up to 64 rows the few-row kernel (gemm_rows_kernel.h) replaces the tile kernel: Llama-2-7B shapes, sym_int4, one MI355X, tile
-// kernel with its reduce launch -> few-row kernel, us: 64 rows qkv 25.3 -> 16.9, o 16.6 -> 12.4, gate / up 32.8 -> 23.7, down
-// 22.2 -> 23 (the one equal: K = 11008 makes x the larger stream, it runs in two K splits); 32 rows 19.8 -> 12.1, 12.8 -> 9.0,
-// 26.2 -> 17.6, 17.7 -> 17.8; 14336-wide shapes, asym_int4: 64 rows qkv 25.6 -> 14.1, gate / up 43.8 -> 35.5.
+// Which products the few-row kernel (gemm_rows_kernel.h) takes from the tile kernel, one MI355X, tile kernel with its reduce
+// launch -> few-row kernel, us.  Llama-2-7B shapes, sym_int4: 64 rows qkv 25.3 -> 16.9, o 16.6 -> 12.4, gate / up 32.8 -> 23.7,
+// down 22.2 -> 23 (the one equal: K = 11008 makes x the larger stream, it runs in two K splits); 32 rows 19.8 -> 12.1,
+// 12.8 -> 9.0, 26.2 -> 17.6, 17.7 -> 17.8.  Llama-3-8B shapes, asym_int4, in blocks of 64 rows: 128 rows qkv 35.4 -> 16.8, o
+// 20.5 -> 13.8, gate / up 78 -> 70, down 38.7 -> 35.7; 192 rows 45.9 -> 30.3, 35.3 -> 25.1, 116 -> 93, 82.7 -> 68.7; 256 rows
+// 39.3 -> 31.0, 27.5 -> 25.0, 150 -> 117, and down 62.6 -> 69.5: every block reads all of x and of the weight, so four blocks
+// of a long K are the tile kernel's.
 static bool takes_rows_kernel(const void* x, int ldx, int M, int N, int K, int qtype, bool pair, RowsPlan* plan) {
-  if (M > 64 || !is_t16(qtype)) return false;
+  if (M > 256 || (M > 192 && K > 8192) || !is_t16(qtype)) return false;
   if (x != nullptr && !rows_ok(x, ldx)) return false;
-  *plan = rows_plan(M, N, K, qtype, pair, !pair);
+  *plan = rows_plan(M, N, K, qtype, pair, !pair && M <= 64);
   return true;
 }
 static int launch_rows(const GemmArgs& a, int qtype, const RowsPlan& p, hipStream_t stream) {

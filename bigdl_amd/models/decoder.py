@@ -671,6 +671,9 @@ class NativeDecoder:
                 # both input projections and act(g) * u in one launch: g and u never reach memory
                 g = hip.gemm_prompt_pair(x.contiguous(), gt.w, up.w, gt.qtype, gt.n, gt.k, bias=gt.bias, bias2=up.bias,
                                          act=cfg.act)
+            elif (gt.fused and up.fused and gt.qtype == up.qtype and gt.n == up.n and gt.k == up.k and x.dtype == torch.float16
+                    and GEMV_MAX_ROWS < x.shape[0] <= GEMM_MAX_ROWS):
+                g = hip.gemm_lowbit_ex(x.contiguous(), gt.w, gt.qtype, gt.n, gt.k, w2=up.w, bias=gt.bias, bias2=up.bias, act=cfg.act)
             else:
                 g = self._linear_dense(x, gt)
                 u = self._linear_dense(x, up)

@@ -87,7 +87,7 @@ def test_pairs_norm_bias_residual(hip, name, m):
 
 
 @pytest.mark.parametrize("name", ["sym_int4", "q4_k", "nf4", "sym_int8"])
-@pytest.mark.parametrize("m", [4, 8, 13, 16, 17, 40, 64])
+@pytest.mark.parametrize("m", [4, 8, 13, 16, 17, 40, 64, 65, 192, 193])
 def test_public_products_at_their_row_limits(hip, name, m):
     """gemv_lowbit / gemm_lowbit / gemm_lowbit_ex on either side of each change of kernel, K split included"""
     qt = Q.ggml_tensor_qtype[name]

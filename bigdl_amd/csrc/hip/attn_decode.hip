@@ -26,6 +26,7 @@
 // is exactly the k-slice its P^T fragment must hold for the O^T product.
 #include "common.h"
 #include <stdlib.h>
+#include <type_traits>
 
 namespace bigdl {
 
@@ -116,8 +117,16 @@ constexpr float P8_SCALE = 256.0f;     // probabilities are carried as 256 p (an
 // e5m2 path is bound by the number of memory instructions, not by bytes (batch 64, 1024 keys: 184 us per layer where
 // the fp16 cache needs 258 us for twice the bytes).  The MFMA k index <-> head channel assignment is free as long as
 // Q and K agree, so lane group g takes channels [16 (g + 4 c2), +16) of a row for the k-steps 2 c2 and 2 c2 + 1.
+//
+// The leading arguments arrive in scalar registers (build flag, see gemv_kernel.h): with them q and the length are requested
+// at once, and the rest of the arguments returns along with the length.  One sequence, 4 kv heads of 64, 50 keys: 8 steps of
+// 8 layers 1692 -> 1671 us, with the rows of q requested ahead of the append.
 template <int D, bool FP8, int RT, int KW, bool I4, int NWT = ATT_NW, int MINW = 1>
-__global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(AttnArgs a) {
+__global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* p_past, _Float16* p_qkv, int p_ld, int p_q_total,
+                                                                     int p_splits, int p_Hq, int p_Hkv, int p_nchunk, int p_gchunk,
+                                                                     int p_Lmax, void* p_kc, AttnArgs a) {
+  a.past_len = p_past; a.qkv = p_qkv; a.ld = p_ld; a.q_total = p_q_total; a.splits = p_splits; a.Hq = p_Hq; a.Hkv = p_Hkv;
+  a.nchunk = p_nchunk; a.gchunk = p_gchunk; a.Lmax = p_Lmax; a.kc = p_kc;
   constexpr int DC = D / 32;   // QK k-steps
   constexpr int DT = D / 16;   // O^T d-tiles
   constexpr int NW = NWT;
@@ -130,6 +139,10 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(AttnArgs a)
   constexpr bool F8M = FP8 && WIDE;
   static_assert(!WIDE || (FP8 && D % 128 == 0), "16-byte fragments: e5m2 cache, rotate-half partner in k-step c + DC/2");
   static_assert(!I4 || (!FP8 && KW == 32), "int4 caches: 32 keys per wavefront");
+  constexpr bool AHEAD = RT == 1 && D <= 128;              // registers for a second block's fragments
+  // fp16 caches: 12 sequences x 8 heads x 1900 keys 1.5 us a launch; e5m2 caches gain nothing (64 x 32 x 1000: 125 us either
+  // way), and the 32-key e5m2 form's 8-byte pieces would not make whole 64 bytes
+  constexpr bool FOLD = !I4 && !FP8;
   // first head channel of this lane's 8 values in k-step c.  int4: lane group g owns the D/4 contiguous channels
   // (D/4) g .. of a key, one load of D/8 bytes
   auto chan = [](int c, int g) {
@@ -187,6 +200,57 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(AttnArgs a)
       }
     }
   };
+  // the other caches: one block's K / V^T fragments as they lie in the cache
+  typedef typename std::conditional<FP8, uint2v, half8>::type Piece;
+  constexpr bool F16F = !F8M && !I4;
+  struct Frag { Piece k[F16F ? NU : 1][F16F ? DC : 1], v[F16F ? DT : 1]; };
+  auto piece = [&](const char* base, int64_t elem) { return *(const Piece*)(base + (FP8 ? elem : 2 * elem)); };
+  auto load_frag = [&](const int kb, Frag& f) {
+    const int key0 = kb + KL * (rr >> 2) + (rr & 3);
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+#pragma unroll
+      for (int c = 0; c < DC; ++c) f.k[u][c] = piece(kc, (int64_t)(key0 + 4 * u) * D + 32 * c + 8 * g);
+#pragma unroll
+    for (int d = 0; d < DT; ++d) f.v[d] = piece(vc, (int64_t)(16 * d + rr) * a.Lmax + kb + 8 * g);
+  };
+  auto widen = [&](const Piece& p) -> half8 {
+    if constexpr (FP8) return dec_e5m2(p.x, p.y);
+    else return p;
+  };
+  // A decode step's one new value row is not stored element by element (V^T: two bytes in each of D lines, which memory
+  // turns into a read and a write of every line) but put into the fragments of the block that holds its key, by the
+  // wavefront that multiplies that block, and stored with them: 64 whole bytes a channel.
+  const bool fold_v = FOLD && a.q_total == 1 && (a.rope != nullptr || a.rot == 0) && a.q_off == 0 && past < a.Lmax;
+  // bytes [16 g, 16 g + 16) of the block's 64 bytes of channel 16 d + rr are this lane's
+  auto fold_new_value = [&](const int kb, auto&& word) {
+    const int at = (past - kb) * 2;                             // byte of the new value within the 64
+    const _Float16* vrow = a.qkv + (int64_t)b * a.ld + (int64_t)(a.Hq + a.Hkv + hkv) * D;
+    _Float16 nv[DT];
+#pragma unroll
+    for (int d = 0; d < DT; ++d) nv[d] = vrow[16 * d + rr];
+    const bool mine = g == (at >> 4);
+    const int shift = 8 * (at & 3);
+    const uint32_t keep = ~(0xffffu << shift);
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      const uint32_t nb = (uint32_t)__builtin_bit_cast(uint16_t, nv[d]) << shift;
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+        if (mine && w == ((at >> 2) & 3)) word(d, w) = (word(d, w) & keep) | nb;
+      const uint4v out = {word(d, 0), word(d, 1), word(d, 2), word(d, 3)};
+      *(uint4v*)(vc + ((int64_t)(16 * d + rr) * a.Lmax + kb) * 2 + 16 * g) = out;
+    }
+  };
+  // The rows of q are requested ahead of the append: they depend on nothing it does, and its barrier waits for its stores
+  half8 qraw[RT][DC];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    const int row = min(16 * t + rr, rows - 1);
+    const _Float16* qp = a.qkv + (int64_t)(b * a.q_total + a.q_off + row / Gc) * a.ld + (hkv * G + g0 + row % Gc) * D;
+#pragma unroll
+    for (int c = 0; c < DC; ++c) qraw[t][c] = *(const half8*)(qp + chan(c, g));
+  }
   // ---- fused RoPE(k) + KV append for the new tokens that fall into this workgroup's key range ----
   if (a.rope != nullptr || a.rot == 0) {
     if (a.q_off == 0) {
@@ -269,15 +333,13 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(AttnArgs a)
           }
           continue;
         }
-        if constexpr (F8M)
-          if (a.ablate & 2) continue;   // (measurement: without the V^T byte stores, 128 partly written lines per key)
+        if (FOLD && fold_v) continue;
         for (int d = lane; d < D; d += 64) {
           if constexpr (FP8) ((uint8_t*)vc)[(int64_t)d * a.Lmax + p] = f16_to_e5m2(vrow[d]);
           else ((_Float16*)vc)[(int64_t)d * a.Lmax + p] = vrow[d];
         }
       }
     }
-    __syncthreads();   // appended keys become visible to the whole workgroup (vmcnt(0) + barrier)
   }
 
   const float qscale = a.softcap > 0.0f ? a.scale : a.scale * 1.4426950408889634f;
@@ -298,15 +360,11 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(AttnArgs a)
     const int tokidx = b * a.q_total + tok;
     lim[t] = valid ? past + tok : -1;
     lo_lim[t] = (a.window > 0 && valid) ? max(0, past + tok - a.window + 1) : 0;
-    const _Float16* qp = a.qkv + (int64_t)tokidx * a.ld + (hkv * G + gq) * D;
     float qv[DC][8];
 #pragma unroll
-    for (int c = 0; c < DC; ++c) {
-      half8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (valid) v = *(const half8*)(qp + chan(c, g));
+    for (int c = 0; c < DC; ++c)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) qv[c][j] = (float)v[j];
-    }
+      for (int j = 0; j < 8; ++j) qv[c][j] = valid ? (float)qraw[t][c][j] : 0.0f;
     if (a.rope != nullptr && valid) {
       const int pos = min(a.position_ids ? a.position_ids[tokidx] : past + tok, a.rope_max_pos - 1);
       const float* tab = a.rope + (int64_t)pos * half_rot * 2;
@@ -389,6 +447,8 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(AttnArgs a)
     }
   }
 
+  if (a.rope != nullptr || a.rot == 0) __syncthreads();   // appended keys become visible to the whole workgroup (vmcnt(0) + barrier)
+
   float m_run[RT], l_run[RT];
   float4v o[RT][DT];
 #pragma unroll
@@ -401,7 +461,7 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(AttnArgs a)
   const float4v zero4 = {0, 0, 0, 0};
 
   // the KW keys from kb on: K / V^T fragments loaded (e5m2: by load_raw) and folded into the running softmax state
-  auto process = [&](const int kb, const RawK& kr, const RawV& vr) {
+  auto process = [&](const int kb, const RawK& kr, const RawV& vr, const Frag& fr) {
     // ---- S^T = K . Q^T for NU 16-key tiles ----
     // A-row i of tile u  <->  key kb + KL*(i>>2) + 4*u + (i&3), so that lane group g ends up with the KL consecutive
     // keys kb + KL*g .. of every query row
@@ -435,7 +495,7 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(AttnArgs a)
 #pragma unroll
       for (int u = 0; u < NU; ++u)
 #pragma unroll
-        for (int c = 0; c < DC; ++c) kf[u][c] = load_kv8<FP8>(kc, (int64_t)(key0 + 4 * u) * D + 32 * c + 8 * g);
+        for (int c = 0; c < DC; ++c) kf[u][c] = widen(fr.k[u][c]);
     }
     // V^T fragments: lane (d_local, g) holds keys kb + KL*g .. of channel 16*dt + d_local (KL/8 k-steps)
     half8 vf[F8M ? 1 : DT][F8M ? 1 : KL / 8];
@@ -463,7 +523,7 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(AttnArgs a)
       (void)one;
     } else if constexpr (!F8M) {
 #pragma unroll
-      for (int d = 0; d < DT; ++d) vf[d][0] = load_kv8<FP8>(vc, (int64_t)(16 * d + rr) * a.Lmax + kb + 8 * g);
+      for (int d = 0; d < DT; ++d) vf[d][0] = widen(fr.v[d]);
     }
 
     if constexpr (F8M) {
@@ -605,13 +665,45 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(AttnArgs a)
       RawK kr;
       RawV vr;
       load_raw(kb, kr, vr);
-      process(kb, kr, vr);
+      process(kb, kr, vr, Frag{});
     }
-  } else {
+  } else if constexpr (I4) {
     for (int blk = blk0; blk < blk1; ++blk) {
       const int kb = blk * ATT_KEYS + wave * KW;
       if (kb >= kv_len) break;
-      process(kb, RawK{}, RawV{});
+      process(kb, RawK{}, RawV{}, Frag{});
+    }
+  } else {
+    int kb = blk0 * ATT_KEYS + wave * KW;
+    const int end = min(blk1 * ATT_KEYS, kv_len);
+    auto last_words = [&](Frag& f) {
+      if constexpr (FOLD)
+        if (fold_v && past >= kb && past < kb + KW)      // (the newest key: only ever in a wavefront's last block)
+          fold_new_value(kb, [&](int d, int w) -> uint32_t& { return ((uint32_t*)&f.v[d])[w]; });
+    };
+    if constexpr (AHEAD) {
+      // The next block is requested before this one is worked on; the asm statement keeps the compiler from moving the
+      // loads back to their use.  (The last block stands alone: a request under a condition would make every block wait
+      // for it.)
+      if (kb < end) {
+        Frag cur, nxt;
+        load_frag(kb, cur);
+        for (; kb + ATT_KEYS < end; kb += ATT_KEYS) {
+          load_frag(kb + ATT_KEYS, nxt);
+          asm volatile("" ::: "memory");
+          process(kb, RawK{}, RawV{}, cur);
+          cur = nxt;
+        }
+        last_words(cur);
+        process(kb, RawK{}, RawV{}, cur);
+      }
+    } else {
+      for (; kb < end; kb += ATT_KEYS) {
+        Frag cur;
+        load_frag(kb, cur);
+        last_words(cur);
+        process(kb, RawK{}, RawV{}, cur);
+      }
     }
   }
 
@@ -716,7 +808,8 @@ static int launch_one(const AttnArgs& a, size_t, hipStream_t st) {
       return -5;
     attr = true;
   }
-  hipLaunchKernelGGL((attn_decode_kernel<D, FP8, RT, KW, I4, NWT, MINW>), grid, block, smem, st, a);
+  hipLaunchKernelGGL((attn_decode_kernel<D, FP8, RT, KW, I4, NWT, MINW>), grid, block, smem, st, a.past_len, a.qkv, a.ld, a.q_total,
+                     a.splits, a.Hq, a.Hkv, a.nchunk, a.gchunk, a.Lmax, a.kc, a);
   return HIP_CHECK_LAUNCH();
 }
 

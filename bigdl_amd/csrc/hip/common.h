@@ -182,45 +182,37 @@ __device__ __forceinline__ half8 dec_fp6(uint32_t w, uint32_t hb) {
 }
 constexpr float FP6_POST = 4096.0f;
 
-__constant__ const float NF4_VALUES[16] = {
+__constant__ constexpr float NF4_VALUES[16] = {
     -1.0f, -0.6961928009986877f, -0.5250730514526367f, -0.39491748809814453f,
     -0.28444138169288635f, -0.18477343022823334f, -0.09105003625154495f, 0.0f,
     0.07958029955625534f, 0.16093020141124725f, 0.24611230194568634f, 0.33791524171829224f,
     0.44070982933044434f, 0.5626170039176941f, 0.7229568362236023f, 1.0f};
 
-// nf4: 16-entry table lookup; the table lives in LDS as 16 fp16 values replicated per lane
-// group to keep bank conflicts low (see gemv kernel)
-__device__ __forceinline__ half8 dec_nf4(uint32_t w, const _Float16* lut) {
+// byte `byte` of the fp16 values first .. first + 3, packed
+constexpr uint32_t nf4_bytes(int first, int byte) {
+  uint32_t v = 0;
+  for (int i = 0; i < 4; ++i)
+    v |= (uint32_t)((__builtin_bit_cast(uint16_t, (_Float16)NF4_VALUES[first + i]) >> (8 * byte)) & 0xff) << (8 * i);
+  return v;
+}
+// nf4: the 16 fp16 values lie in registers, low and high bytes apart, and v_perm_b32 looks four codes up at once: one lookup
+// in entries 0 - 7, one in 8 - 15, merged by a byte mask of the codes' top bits (selector 0x0c gives 0x00, 0x0d gives 0xff).
+// 25 vector instructions for 8 codes.  A table in LDS (8 reads and about 20 instructions) took a fifth of the LDS cycles
+// of the prompt product, which the fragment reads fill as far as the matrix cores are filled.
+__device__ __forceinline__ half8 dec_nf4(uint32_t w) {
   H8 r;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t t = w >> (4 * i);
-    half2v h = {lut[t & 15u], lut[(t >> 16) & 15u]};
-    r.h2[i] = h;
+  for (int i = 0; i < 2; ++i) {                      // even / odd codes of the word
+    const uint32_t at = (w >> (4 * i)) & 0x07070707u;
+    const uint32_t upper = __builtin_amdgcn_perm(0, 0, ((w >> (4 * i + 3)) & 0x01010101u) | 0x0c0c0c0cu);
+    const uint32_t lo = (upper & __builtin_amdgcn_perm(nf4_bytes(12, 0), nf4_bytes(8, 0), at)) |
+                        (~upper & __builtin_amdgcn_perm(nf4_bytes(4, 0), nf4_bytes(0, 0), at));
+    const uint32_t hi = (upper & __builtin_amdgcn_perm(nf4_bytes(12, 1), nf4_bytes(8, 1), at)) |
+                        (~upper & __builtin_amdgcn_perm(nf4_bytes(4, 1), nf4_bytes(0, 1), at));
+    r.u[i] = __builtin_amdgcn_perm(hi, lo, 0x06020400u);        // codes i, i + 4
+    r.u[2 + i] = __builtin_amdgcn_perm(hi, lo, 0x07030501u);    // codes i + 2, i + 6
   }
   return r.v;
-}
-
-// nf4 through a bank-private table: 16 entries x 32 dwords in LDS, entry i of lane l at dword i * 32 + (l & 31), the
-// fp16 value replicated in both halves of the dword.  Every lane only ever touches bank l & 31 (lanes l and l + 32
-// read the same dword: a broadcast), so the 8 lookups of a fragment are conflict free whatever the codes are; the
-// replicated halves let one v_bfi merge two lookups into a packed pair.  `lut` already points at the lane's column.
-__device__ __forceinline__ half8 dec_nf4_banked(uint32_t w, const uint32_t* lut) {
-  H8 r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t t = w >> (4 * i);
-    const uint32_t a = lut[(t & 15u) << 5], b = lut[((t >> 16) & 15u) << 5];
-    r.u[i] = (a & 0x0000ffffu) | (b & 0xffff0000u);
-  }
-  return r.v;
-}
-__device__ __forceinline__ void fill_nf4_banked(uint32_t* table, int tid, int nthreads) {
-  for (int i = tid; i < 16 * 32; i += nthreads) {
-    union { _Float16 h; uint16_t u; } c;
-    c.h = (_Float16)NF4_VALUES[i >> 5];
-    table[i] = (uint32_t)c.u | ((uint32_t)c.u << 16);
-  }
 }
 
 // int8 codes, 8 bytes (two words): value = (int8)code.  fp16 0x6400|b' = 1024 + b', b' = b ^ 0x80

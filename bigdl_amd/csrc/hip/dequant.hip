@@ -31,13 +31,8 @@ __device__ __forceinline__ void store8_out(void* p, int64_t idx, const float* v)
 template <int QT, int OUT>
 __global__ __launch_bounds__(256) void dequant_t16_kernel(const void* w, void* out, int N, int K, int64_t ldo, int n_planes,
                                                           int row0) {
-  __shared__ _Float16 nf4_lut[16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int KT = (K + 127) >> 7, NT = (N + 15) >> 4;
-  if constexpr (QT == Q_NF4) {
-    if (threadIdx.x < 16) nf4_lut[threadIdx.x] = (_Float16)NF4_VALUES[threadIdx.x];
-    __syncthreads();
-  }
   // rows [row0, row0 + N) of a [n_planes, K] buffer (row0 % 16 == 0) -> out rows [0, N)
   const int64_t ltile = (int64_t)blockIdx.x * 4 + wave;
   if (ltile >= (int64_t)NT * KT) return;
@@ -67,7 +62,7 @@ __global__ __launch_bounds__(256) void dequant_t16_kernel(const void* w, void* o
     if constexpr (QT == Q_SYM_INT4) f = dec_int4(lo0[s], 8.0f);
     else if constexpr (QT == Q_ASYM_INT4 || QT == Q_WOQ_INT4) f = dec_int4(lo0[s], 0.0f);
     else if constexpr (QT == Q_FP4) { f = dec_fp4(lo0[s]); post = FP4_POST; }
-    else if constexpr (QT == Q_NF4) f = dec_nf4(lo0[s], nf4_lut);
+    else if constexpr (QT == Q_NF4) f = dec_nf4(lo0[s]);
     else if constexpr (QT == Q_SYM_INT5) f = dec_int5(lo0[s], (hi0 >> (8 * s)) & 0xffu, 16.0f);
     else if constexpr (QT == Q_ASYM_INT5) f = dec_int5(lo0[s], (hi0 >> (8 * s)) & 0xffu, 0.0f);
     else if constexpr (QT == Q_FP6) { f = dec_fp6(lo0[s], ((s < 2 ? hi0 : hi1) >> (16 * (s & 1))) & 0xffffu); post = FP6_POST; }

@@ -114,7 +114,6 @@ __global__ __launch_bounds__((NW + (LW ? 1 : 0)) * 64, 2) void gemm_t16_kernel(G
   static_assert(BM % RP == 0 && RP % 16 == 0, "whole passes; the swizzle of a row is that of its pass-0 row");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   char* As = smem;                                               // [NSTAGE][BM][256 B]
-  _Float16* nf4_lut = (_Float16*)(smem + NSTAGE * BM * 256);      // [64][16] (nf4 only)
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -139,12 +138,6 @@ __global__ __launch_bounds__((NW + (LW ? 1 : 0)) * 64, 2) void gemm_t16_kernel(G
   const int kt0 = sp * a.kt_per_split, kt1 = min(KT, kt0 + a.kt_per_split);
   const bool second = a.w2 != nullptr && blockIdx.z == 1;
   const T16Planes pl = t16_planes(second ? a.w2 : a.w, QT, n_planes, a.K);
-
-  const _Float16* lut = nullptr;
-  if constexpr (QT == Q_NF4) {
-    fill_nf4_banked((uint32_t*)nf4_lut, threadIdx.x, (NW + (LW ? 1 : 0)) * 64);
-    lut = (const _Float16*)((const uint32_t*)nf4_lut + (lane & 31));
-  }
 
   // this wavefront's weight tile rows (clamped: a tile past N is loaded from the last valid one and never stored)
   const int ntiles = (a.N + 15) >> 4;
@@ -279,7 +272,7 @@ __global__ __launch_bounds__((NW + (LW ? 1 : 0)) * 64, 2) void gemm_t16_kernel(G
           bf[n] = __builtin_bit_cast(half8, uint4v{t[n].lo0[s], t[n].lo0[(s + 1) & 3], __builtin_bit_cast(uint32_t, half2v{t[n].d[s], t[n].d[s]}), 0x3c003c00u});
           continue;
         }
-        const half8 code = decode_step<QT>(t[n], s, lut);
+        const half8 code = decode_step<QT>(t[n], s);
         _Float16 d = t[n].d[s];
         if constexpr (post_scale<QT>() != 1.0f) d = (_Float16)fminf((float)d * post_scale<QT>(), 65504.0f);
         if constexpr (has_min<QT>()) bf[n] = code * d + t[n].m[s];
@@ -406,7 +399,7 @@ __global__ __launch_bounds__((NW + (LW ? 1 : 0)) * 64, 2) void gemm_t16_kernel(G
 template <int QT, int MT, int NT, bool NORM = false, int NW = 4, bool LW = false>
 static int gemm_launch_mt(const GemmArgs& a, int mblocks, hipStream_t st) {
   constexpr int BM = MT * 16;
-  const size_t lds = (LW ? 3 : 2) * BM * 256 + (QT == Q_NF4 ? 64 * 16 * 2 : 0);
+  const size_t lds = (LW ? 3 : 2) * BM * 256;
   static bool attr_set = false;
   if (!attr_set) {
     if (hipFuncSetAttribute((const void*)gemm_t16_kernel<QT, MT, NT, NORM, NW, LW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)

@@ -61,8 +61,8 @@ constexpr int waitcnt_vm_lgkm0(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0
 // one expansion unit = the 8 codes per lane of one (16-row weight tile, 32-deep k step) -> the fp16 fragment with the
 // block scale (and minimum) folded in.  `s` is the step inside the T16 tile (0 .. 3), static.
 template <int QT, int S>
-__device__ __forceinline__ half8 unit_expand(const Tile<QT>& t, const _Float16* lut) {
-  const half8 code = decode_step<QT>(t, S, lut);
+__device__ __forceinline__ half8 unit_expand(const Tile<QT>& t) {
+  const half8 code = decode_step<QT>(t, S);
   _Float16 d = t.d[S];
   if constexpr (post_scale<QT>() != 1.0f) d = (_Float16)fminf((float)d * post_scale<QT>(), 65504.0f);
   if constexpr (has_min<QT>()) return code * d + t.m[S];
@@ -111,14 +111,6 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_prompt_kernel(GemmArgs a
   const int nkt = kt1 - kt0, T = 2 * nkt;            // T16 k tiles / 64-deep tiles of this workgroup
   const T16Planes pl = t16_planes(a.w, QT, a.N, a.K);
   const T16Planes pl2 = t16_planes(pair ? a.w2 : a.w, QT, a.N, a.K);
-
-  const _Float16* lut = nullptr;
-  if constexpr (QT == Q_NF4) {
-    uint32_t* table = (uint32_t*)(smem + prompt_lds_tiles(BM, BN, NW, MTW, NTW));
-    fill_nf4_banked(table, threadIdx.x, 64 * NW);
-    lut = (const _Float16*)(table + (lane & 31));
-    __syncthreads();       // every wavefront fills a share of the table and the first expansion reads all of it
-  }
 
   // ---- x tile: every wavefront stages rows of its own row half (the half it reads fragments from, so that the two
   // halves of the workgroup may run out of step); instruction p fills rows 8 (p WN + wn) .. + 7 of the half; lane i
@@ -176,8 +168,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_prompt_kernel(GemmArgs a
       if (i >= FULL && half_sel != h) continue;        // wave-uniform
       half8 v0, v1;
       // (both steps of the parity are instantiated, the static one is kept: decode_step wants a constant step)
-      if (u & 1) v0 = unit_expand<QT, 2 * h + 1>(rawC[i], lut);
-      else v0 = unit_expand<QT, 2 * h>(rawC[i], lut);
+      if (u & 1) v0 = unit_expand<QT, 2 * h + 1>(rawC[i]);
+      else v0 = unit_expand<QT, 2 * h>(rawC[i]);
       if constexpr (PROMPT_ABL & 4) v0 = __builtin_bit_cast(half8, uint4v{rawC[i].lo0[0], rawC[i].lo0[1], 0x3c003c00u, 0x3c003c00u});
       (void)v1;
       *(half8*)(base + slot_rt[i] * 2048 + frag_off[u & 1]) = v0;
@@ -528,7 +520,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_prompt_kernel(GemmArgs a
 template <int QT, int WM, int WN, int MTW, int NTW, int PH>
 static int gemm_prompt_launch_cfg(const GemmArgs& a, hipStream_t st) {
   constexpr int NW = WM * WN, BM = WM * MTW * 16, BN = WN * NTW * 16;
-  const size_t lds = prompt_lds_tiles(BM, BN, NW, MTW, NTW) + (QT == Q_NF4 ? 16 * 32 * 4 : 0);
+  const size_t lds = prompt_lds_tiles(BM, BN, NW, MTW, NTW);
   static bool attr_set = false;
   if (!attr_set) {
     if (hipFuncSetAttribute((const void*)gemm_prompt_kernel<QT, WM, WN, MTW, NTW, PH>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)

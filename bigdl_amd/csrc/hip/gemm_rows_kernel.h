@@ -47,8 +47,8 @@ constexpr int ROWS_NW = 8;            // wavefronts per workgroup
 // partial sums of all wavefronts at once, or of one half after the other where they do not fit
 constexpr bool rows_two_phase(int mt, int ns, int nw) { return nw * mt * ns > 144; }
 constexpr int rows_red_kib(int mt, int ns, int nw) { return rows_two_phase(mt, ns, nw) ? nw * mt * ns / 2 : nw * mt * ns; }
-constexpr int rows_lds(int qt, int mt, int ns, int nw) {
-  return (rows_red_kib(mt, ns, nw) > nw * mt * 4 ? rows_red_kib(mt, ns, nw) : nw * mt * 4) * 1024 + (mt == 1 ? nw * mt * 64 : 0) + (qt == Q_NF4 ? 2048 : 0);
+constexpr int rows_lds(int mt, int ns, int nw) {
+  return (rows_red_kib(mt, ns, nw) > nw * mt * 4 ? rows_red_kib(mt, ns, nw) : nw * mt * 4) * 1024 + (mt == 1 ? nw * mt * 64 : 0);
 }
 
 // halves of an x tile on their way in registers
@@ -99,7 +99,7 @@ struct RowsPlanes {
 // How a lane's share of a weight tile becomes MFMA operands.  T16 formats: fragment s holds k = 32 s + 8 g + j, one 32-element
 // scale block per fragment.
 template <int QT>
-__device__ __forceinline__ half8 rows_fragment(const Tile<QT>& t, int s, const _Float16* lut, int) { return decode_step<QT>(t, s, lut); }
+__device__ __forceinline__ half8 rows_fragment(const Tile<QT>& t, int s, int) { return decode_step<QT>(t, s); }
 template <int QT>
 __device__ __forceinline__ float rows_scale(const Tile<QT>& t, int s) { return (float)t.d[s] * post_scale<QT>(); }
 template <int QT>
@@ -161,7 +161,7 @@ struct RowsPlanes<Q_Q6_K> {
   }
 };
 template <>
-__device__ __forceinline__ half8 rows_fragment<Q_Q6_K>(const Tile<Q_Q6_K>& t, int s, const _Float16*, int g) {
+__device__ __forceinline__ half8 rows_fragment<Q_Q6_K>(const Tile<Q_Q6_K>& t, int s, int g) {
   H8 r;
   const half2v off = {(_Float16)1056.0f, (_Float16)1056.0f};       // 1024 + 32
   const _Float16 sc = (_Float16)(float)(int8_t)(t.sc[s >> 1] >> (8 * g));
@@ -193,8 +193,7 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(RowsAr
   constexpr int NR = TWO ? NW / 2 : NW;              // wavefronts whose partial sums are in LDS at once
   extern __shared__ __attribute__((aligned(16))) char smem[];
   float* red = (float*)smem;                         // [NR][MT * NS][64][4], once the x tiles [NW][2][XB] have been read
-  float* ssq_sh = (float*)(smem + rows_lds(0, MT, NS, NW) - (NORM ? NW * MT * 64 : 0));     // [NW][MT * 16] (NORM)
-  _Float16* nf4_lut = (_Float16*)(ssq_sh + (NORM ? NW * MT * 16 : 0));
+  float* ssq_sh = (float*)(smem + rows_lds(MT, NS, NW) - (NORM ? NW * MT * 64 : 0));     // [NW][MT * 16] (NORM)
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -206,7 +205,6 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(RowsAr
   const int kt0 = sp * a.kt_per_split, kt1 = min(KT, kt0 + a.kt_per_split);
   const int row0 = blockIdx.y * (MT * 16), rows = min(MT * 16, a.M - row0);
 
-  const _Float16* lut = nullptr;
   RowsPlanes<QT> pl, pl2;
   constexpr bool RAW = QT == Q_Q6_K;
   static_assert(!RAW || !PAIR, "q6_k: single products");
@@ -280,11 +278,6 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(RowsAr
     fetch_w(tt[d], d);
     rows_issued();
   }
-  if constexpr (QT == Q_NF4) {
-    fill_nf4_banked((uint32_t*)nf4_lut, threadIdx.x, NW * 64);
-    lut = (const _Float16*)((const uint32_t*)nf4_lut + (lane & 31));
-    __syncthreads();
-  }
 
   float4v acc[NS][MT];
 #pragma unroll
@@ -307,7 +300,7 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(RowsAr
       }
 #pragma unroll
       for (int n = 0; n < NS; ++n) {
-        const half8 code = rows_fragment<QT>(t[n], s, lut, g);
+        const half8 code = rows_fragment<QT>(t[n], s, g);
         if constexpr (POST) {
           const float d = rows_scale<QT>(t[n], s);
 #pragma unroll
@@ -456,7 +449,7 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(RowsAr
 
 template <int QT, int MT, int NT, bool PAIR>
 static int gemm_rows_launch_t(const RowsArgs& a, hipStream_t st) {
-  constexpr int lds = rows_lds(QT, MT, PAIR ? 2 * NT : NT, ROWS_NW);
+  constexpr int lds = rows_lds(MT, PAIR ? 2 * NT : NT, ROWS_NW);
   static_assert(lds <= 160 * 1024, "LDS of a CU");
   auto k = gemm_rows_kernel<QT, MT, NT, PAIR>;
   if (!gemv_allow_lds((const void*)k, lds)) return -101;

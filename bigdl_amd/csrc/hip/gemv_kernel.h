@@ -212,11 +212,11 @@ __device__ __forceinline__ half8 dec_int4_fast(uint32_t w, float bias) {
 }
 
 template <int QT>
-__device__ __forceinline__ half8 decode_step(const Tile<QT>& t, int s, const _Float16* lut) {
+__device__ __forceinline__ half8 decode_step(const Tile<QT>& t, int s) {
   if constexpr (QT == Q_SYM_INT4) return dec_int4_fast(t.lo0[s], 8.0f);
   else if constexpr (QT == Q_ASYM_INT4 || QT == Q_WOQ_INT4) return dec_int4_fast(t.lo0[s], 0.0f);
   else if constexpr (QT == Q_FP4) return dec_fp4(t.lo0[s]);
-  else if constexpr (QT == Q_NF4) return dec_nf4_banked(t.lo0[s], (const uint32_t*)lut);
+  else if constexpr (QT == Q_NF4) return dec_nf4(t.lo0[s]);
   else if constexpr (QT == Q_SYM_INT5) return dec_int5(t.lo0[s], (t.hi0 >> (8 * s)) & 0xffu, 16.0f);
   else if constexpr (QT == Q_ASYM_INT5) return dec_int5(t.lo0[s], (t.hi0 >> (8 * s)) & 0xffu, 0.0f);
   else if constexpr (QT == Q_FP6) return dec_fp6(t.lo0[s], ((s < 2 ? t.hi0 : t.hi1) >> (16 * (s & 1))) & 0xffffu);
@@ -307,7 +307,7 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
   constexpr int U = 2;
 #endif
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  // carve: red | ssq | sum | lut | xsum | x
+  // carve: red | ssq | sum | xsum | x
   float* red = (float*)smem;                                  // [NW][NACC*MT][64][4]; CU: [ntc][NW][NACC][rows_g * 16][4]
   const int rows_g = (a.M + 3) >> 2;                          // CU: lane groups (4 rows each) that hold valid rows
   const int red_floats = CU ? a.cu_ntc * GEMV_NW * NACC * rows_g * 64 : GEMV_NW * NACC * MT * 256;
@@ -315,10 +315,9 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
   // its own slice, so the staging needs neither atomics nor a barrier between zeroing and accumulation
   float* ssq_sh = red + red_floats;                           // [NW][MT*16]
   float* sum_sh = ssq_sh + GEMV_NW * MT * 16;                 // [NW][MT*16]
-  _Float16* nf4_lut = (_Float16*)(sum_sh + GEMV_NW * MT * 16);   // [64*16] (nf4 only)
   // formats with a block minimum: sum of (scaled) x over every 32-block, [Kp/32 + XTAIL/32][MT*16 rows], so that the
   // "+ min * sum(x)" term is one 16-byte LDS read per MFMA step instead of a cross-lane reduction of the fragment
-  float* xsum = (float*)(nf4_lut + (QT == Q_NF4 ? 64 * 16 : 0));
+  float* xsum = sum_sh + GEMV_NW * MT * 16;
   constexpr bool XSUM = XLDS && has_min<QT>();
   const int xsum_floats = XSUM ? (((a.K + 127) >> 7) * 4 + XTAIL / 32) * MT * 16 : 0;
   // tile-per-workgroup form: the block scales (and minima) of the workgroup's whole tile row are staged in LDS by a
@@ -533,11 +532,6 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
 
   GEMV_STAMP_AT(1);
   // ---- 3. stage x (optionally scaled by the norm's gamma) in LDS, all wavefronts together ----
-  const _Float16* lut = nullptr;
-  if constexpr (QT == Q_NF4) {
-    fill_nf4_banked((uint32_t*)nf4_lut, threadIdx.x, GEMV_NW * 64);
-    lut = (const _Float16*)((const uint32_t*)nf4_lut + (lane & 31));
-  }
   if constexpr (SCLDS) {
 #pragma unroll
     for (int e = 0; e < ESC; ++e) {
@@ -744,7 +738,7 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
 #pragma unroll
         for (int st = 0; st < NSTREAM; ++st) {
           const Tile<QT>& t = tt[st][u];
-          const half8 bf = decode_step<QT>(t, s, lut);
+          const half8 bf = decode_step<QT>(t, s);
           const float d = (float)dd[st][s] * post_scale<QT>();
           const float2v d2 = {d, d};
 #pragma unroll
@@ -1004,7 +998,7 @@ static int launch_x(const GemvArgs& a_in, hipStream_t st) {
   const size_t xbytes = (size_t)a.M * (Kp + XTAIL + XPAD) * 2;
   constexpr int NACC = GATE_UP ? 2 : 1;
   auto misc = [&](int nw, bool xlds = true) {
-    return (size_t)2 * nw * MT * 16 * 4 + (QT == Q_NF4 ? 64 * 16 * 2 : 0) +
+    return (size_t)2 * nw * MT * 16 * 4 +
            (has_min_of(QT) && xlds ? (size_t)(Kp / 32 + XTAIL / 32) * MT * 16 * 4 : 0);
   };
   // tile-per-workgroup kernels: partial-sum slots, staged scales (and minima) of the tile row

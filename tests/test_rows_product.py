@@ -135,3 +135,27 @@ def test_q6k_linear_takes_the_blocks_for_few_rows(hip):
     # strides and an offset that the kernel's 16-byte loads do not take
     x = torch.randn(3, k + 3, generator=torch.Generator().manual_seed(11)).half()[:, 3:]
     torch.testing.assert_close(lowbit_matmul(x.cuda(), p, n).cpu().double(), x.double() @ w.t(), rtol=2e-3, atol=8e-3)
+
+
+@pytest.mark.parametrize("m", [1, 3, 40, 256, 300])
+def test_nf4_table_is_exact_in_every_position(hip, m):
+    """Every nf4 code in every position of a fragment, block scale 1 and one-hot rows: the products are the table, in fp16."""
+    n, k, qt = 32, 512, Q.ggml_tensor_qtype["nf4"]
+    grid = torch.linspace(-1, 1, 4096).reshape(64, 64).clone()
+    grid[:, 0] = 1                                        # every block's scale
+    table = host.dequantize(host.quantize(grid, qt), qt, (64, 64)).unique()
+    assert len(table) == 16
+    codes = torch.randint(0, 16, (n, k), generator=torch.Generator().manual_seed(7))
+    codes[:, ::64] = 15                                   # 1.0: the block's largest value
+    w = table[codes]
+    dev = host.relayout_to_device(host.quantize(w, qt).view(torch.uint8), qt, n, k).cuda()
+    want = w.half()
+    assert torch.equal(hip.dequant_t16(dev, qt, n, k).cpu(), want)
+    for first in range(0, k, m):
+        x = torch.zeros(m, k, dtype=torch.float16)
+        rows = min(m, k - first)
+        x[torch.arange(rows), first + torch.arange(rows)] = 1
+        product = hip.gemv_lowbit if m <= 16 else hip.gemm_lowbit
+        if m <= 3 and first > 24:                         # (the other rows of a fragment come with the larger m)
+            break
+        assert torch.equal(product(x.cuda(), dev, qt, n, k).cpu()[:rows], want[:, first:first + rows].t())

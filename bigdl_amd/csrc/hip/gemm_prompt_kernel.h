@@ -22,8 +22,7 @@
 //  * the weight fragment is the MFMA's A operand, so a lane holds 4 consecutive output columns of one row; the epilogue
 //    stages the wavefront's tile through LDS and stores whole 128-byte row segments; the gate / up pair form combines the
 //    two products of a column there (act(g) * u), so neither reaches memory.
-//  * the block index is remapped so that the row blocks that share a weight column panel run on one XCD (one HBM read
-//    of the panel per L2).
+//  * the block index is remapped so that the workgroups of one XCD share x and weight panels in its L2.
 // Measured and dropped: stream-K over 256 x 256 tiles (every CU the same number of k tiles whatever the tile count; the
 // 256 KiB fp32 slab per shared tile costs more than the idle CUs it removes: 130 instead of 98 us on the qkv shape),
 // x requests or the expansion moved into the MFMA segment (no change / slower), wavefront priorities (no change).
@@ -98,21 +97,27 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_prompt_kernel(GemmArgs a
   const int BNO = pair ? BN / 2 : BN;
   const int nmb = (a.M + BM - 1) / BM, nnb = (a.N + BNO - 1) / BNO;
 
-  // XCD-aware tile order: blocks b and b + 8 share an L2; consecutive tile ids (row blocks of one column panel first)
-  // go to one XCD (bijective also when the grid is not a multiple of 8)
+  // XCD-aware tile order: blocks b and b + 8 share an L2; consecutive tile ids go to one XCD (bijective also when the grid
+  // is not a multiple of 8).  Tile ids run through bands of BAND row blocks, column by column: the 32 workgroups of an XCD
+  // then share 4 x panels (16 bits an element) and 8 weight panels (4 - 8 bits) instead of reading 32 x panels each for
+  // itself.  7700 rows: 14336 x 4096 pair 1697 -> 1655 us, 6144 x 4096 351 -> 342 us; bands of 2 and 8 within 1 %.
+  constexpr int BAND = 4;
   int tid;
   {
     const int nblk = gridDim.x, b = blockIdx.x, q = nblk >> 3, rr = nblk & 7, xcd = b & 7;
     tid = (xcd < rr ? xcd * (q + 1) : rr * (q + 1) + (xcd - rr) * q) + (b >> 3);
   }
-  const int mb = tid % nmb, nb = (tid / nmb) % nnb, sp = tid / (nmb * nnb);
+  const int sp = tid / (nmb * nnb), in_split = tid - sp * (nmb * nnb);
+  const int band = in_split / (BAND * nnb), band_rows = min(BAND, nmb - band * BAND);
+  const int in_band = in_split - band * (BAND * nnb);
+  const int mb = band * BAND + in_band % band_rows, nb = in_band / band_rows;
   const int row0 = mb * BM, rows = min(BM, a.M - row0);
   const int kt0 = sp * a.kt_per_split, kt1 = min(KT, kt0 + a.kt_per_split);
   const int nkt = kt1 - kt0, T = 2 * nkt;            // T16 k tiles / 64-deep tiles of this workgroup
   const T16Planes pl = t16_planes(a.w, QT, a.N, a.K);
   const T16Planes pl2 = t16_planes(pair ? a.w2 : a.w, QT, a.N, a.K);
 
-  // ---- x tile: every wavefront stages rows of its own row half (the half it reads fragments from, so that the two
+  // ---- x tile (32-bit byte offsets from one scalar base: M * ldx < 2^31).  Every wavefront stages rows of its own row half (the half it reads fragments from, so that the two
   // halves of the workgroup may run out of step); instruction p fills rows 8 (p WN + wn) .. + 7 of the half; lane i
   // brings the 16 bytes that belong in slot i % 8 of row i / 8, i.e. k slot (i % 8) ^ (i / 8) of that row (rows past the
   // block re-read its last row: never stored)
@@ -120,10 +125,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_prompt_kernel(GemmArgs a
 #pragma unroll
   for (int p = 0; p < NA; ++p) {
     const int row = wm * (BM / WM) + (p * WN + wn) * 8 + (lane >> 3);
-    xoff[p] = (uint32_t)((int64_t)(row0 + min(row, rows - 1)) * a.ldx) + (uint32_t)((((lane & 7) ^ (lane >> 3)) & 7) << 3);
+    xoff[p] = ((uint32_t)(row0 + min(row, rows - 1)) * (uint32_t)a.ldx + (uint32_t)((((lane & 7) ^ (lane >> 3)) & 7) << 3)) * 2u;
   }
   auto stage_a = [&](int t, int buf) {
-    const _Float16* src = a.x + (int64_t)(2 * kt0 + t) * 64;
+    const char* src = (const char*)(a.x + (int64_t)(2 * kt0 + t) * 64);
     char* dst = As + buf * ABYTES + (wm * (BM / WM) + wn * 8) * 128;     // wave-uniform; the instruction adds lane * 16
 #pragma unroll
     for (int p = 0; p < NA; ++p)
@@ -464,13 +469,20 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_prompt_kernel(GemmArgs a
   constexpr int CH = 2 * NTW;                        // 16-byte chunks per row
   static_assert((MTW * 16 * CH) % 64 == 0, "row chunks do not divide over the lanes");
   const bool plain = a.act == ACT_NONE && a.residual == nullptr && !pair;
-  const char* stg2 = stg + (WN / 2) * (MTW * 16 * RB);     // pair form: the partner wavefront's tile (same rows)
+  constexpr int ITS = MTW * 16 * CH / 64;
+  int it0 = 0, it1 = ITS;
+  const char* stg2 = stg;
   if (pair) {
+    // the two wavefronts that hold a tile's first and second products take half of its rows each: wavefronts w and w + 4
+    // share a SIMD, so with the first-product wavefronts alone two of the four SIMDs did all exponentials and divisions
+    // (14336 x 4096 pair, 7700 rows: 1655 -> 1610 us)
     __builtin_amdgcn_s_barrier();                    // the partner's tile is complete in LDS
-    if (second_half) return;
+    if (second_half) { it0 = ITS / 2; stg -= (WN / 2) * (MTW * 16 * RB); }
+    else it1 = ITS / 2;
+    stg2 = stg + (WN / 2) * (MTW * 16 * RB);
   }
 #pragma unroll 1
-  for (int it = 0; it < MTW * 16 * CH / 64; ++it) {
+  for (int it = it0; it < it1; ++it) {
     const int idx = it * 64 + lane, row = idx / CH, ch = idx % CH;
     const int col = ocol0 + ch * 8;
     if (orow0 + row >= row0 + rows || col >= a.N) continue;

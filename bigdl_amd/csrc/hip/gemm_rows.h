@@ -16,4 +16,7 @@ static inline bool rows_ok(const void* x, int ldx) {
   return (ldx & 7) == 0 && ((uintptr_t)x & 15) == 0 && ldx > 0 && (int64_t)ldx * 128 < 0x40000000;
 }
 int rows_launch(const RowsArgs& a, const RowsPlan& p, int qtype, hipStream_t st);
+// gemv_q6k.hip: q6_k blocks, 1 - 4 rows
+bool gemv_q6k_takes(const RowsArgs& a);
+int gemv_q6k_launch(const RowsArgs& a, hipStream_t st);
 }  // namespace bigdl

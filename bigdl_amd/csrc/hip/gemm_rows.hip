@@ -77,5 +77,6 @@ extern "C" int bigdl_gemm_rows(const void* x, const void* w, const void* w2, voi
   a.residual = residual; a.gamma = (const _Float16*)gamma; a.gamma_offset = gamma_offset; a.eps = eps;
   a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldo = ldo; a.act = act; a.out_type = out_type;
   a.splitk = p.splitk; a.kt_per_split = p.kt_per_split;
+  if (raw && nt <= 0 && gemv_q6k_takes(a)) return gemv_q6k_launch(a, stream);
   return rows_launch(a, p, qtype, stream);
 }

@@ -33,8 +33,8 @@ TORCH_LINEAR_THRESHOLD = int(os.getenv("BIGDL_LLM_LINEAR_THRESHOLD", "512"))
 GEMV_MAX_ROWS = int(os.getenv("BIGDL_GEMV_MAX_ROWS", "16"))
 GEMM_MAX_ROWS = 256
 # q6_k weights stay in their checkpoint blocks on the GPU.  Up to this many fp16 rows are multiplied from the blocks (csrc/hip/
-# gemm_rows_kernel.h); above, and for bf16 activations, whose range fp16 does not have, the weight is expanded for a dense
-# product.  4096 x 11008, one MI355X, expanded -> from the blocks: 1 row 100 -> 25 us, 64 rows 108 -> 35, 128 rows 128 -> 58.
+# gemm_rows_kernel.h, up to four gemv_q6k.hip); above, and for bf16 activations, whose range fp16 does not have, the weight is expanded for a dense
+# product.  4096 x 11008, one MI355X, expanded -> from the blocks: 1 row 100 -> 17 us, 64 rows 108 -> 35, 128 rows 128 -> 58.
 Q6K_MAX_ROWS = 128
 # forward of frozen low-bit linears inside a training step on the fused prompt GEMM (fp16 copy of the activations)
 # instead of dequantize + dense product

@@ -118,6 +118,29 @@ def test_q6k_blocks_without_expansion(hip, m, n, k):
         assert ((out.double().cpu() - ref).abs() <= bound).all()
 
 
+# fewer rows than wavefronts, more than the grid holds at once, one block, a quad of blocks and one more, a full request
+# group and one more, an LDS image of x that is too large (the last: the tile kernel)
+@pytest.mark.parametrize("n,k", [(5, 256), (16, 1024), (9000, 1280), (33, 4096), (40, 4352), (64, 11008), (24, 28672)])
+@pytest.mark.parametrize("m", [1, 2, 3, 4])
+def test_q6k_one_wavefront_a_row(hip, m, n, k):
+    w0 = torch.randn(n, k, generator=torch.Generator().manual_seed(12)) * 0.05
+    w0[0, :256] = 0                                                      # a block of scale 0
+    raw = host.quantize(w0, Q.Q6_K)
+    w = host.dequantize(raw, Q.Q6_K, w0.shape).double()
+    x, xd = _x(m, k, 13)
+    bias, res = torch.randn(n).half(), torch.randn(m, n).half()
+    ref = torch.relu(xd @ w.t() + bias.double()) + res.double()
+    # codes, scales and x exact in fp32: products and sums round (a lane's chain is k / 64 long).  Through the tile kernel
+    # code * sub-scale rounds to 2^-11.
+    bound = (2.0 ** -11 if m * k > 40960 else 2.0 ** -17) * (xd.abs() @ w.abs().t()) + 1e-5
+    out = hip.gemm_rows(x, raw.cuda(), Q.Q6_K, n, k, out_dtype=torch.float32, bias=bias.cuda(), act="relu", residual=res.float().cuda())
+    assert ((out.double().cpu() - ref).abs() <= bound).all()
+    for dt, eps in ((torch.float16, 2.0 ** -10), (torch.bfloat16, 2.0 ** -7)):
+        out = hip.gemm_rows(x, raw.cuda(), Q.Q6_K, n, k, out_dtype=dt)
+        ref2 = xd @ w.t()
+        assert ((out.double().cpu() - ref2).abs() <= bound + eps * ref2.abs() + 1e-7).all()
+
+
 def test_q6k_linear_takes_the_blocks_for_few_rows(hip):
     from bigdl_amd.transformers.low_bit_linear import FP4Params, Q6K_MAX_ROWS, lowbit_matmul
     n, k = 96, 1024

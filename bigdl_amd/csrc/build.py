@@ -35,9 +35,11 @@ HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-Wall", "-W
 # per-file additions.  attn_prefill: MFMA accumulators in ordinary VGPRs -- the online softmax rescales them with VALU
 # multiplies, and accumulators kept in AGPRs are copied out and back around every such pass (64 moves per key tile).
 HIP_FILE_FLAGS = {"attn_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
-# the decode kernels' leading arguments arrive in scalar registers with the wavefront (gemv_kernel.h, attn_decode.hip)
+# the short kernels' leading arguments arrive in scalar registers with the wavefront (gemv_kernel.h, attn_decode.hip,
+# gemm_rows_kernel.h)
 PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=14"]
-HIP_FILE_FLAGS.update({p.name: PRELOAD for p in HIP_SOURCES if p.name.startswith("gemv_inst_") or p.name == "attn_decode.hip"})
+HIP_FILE_FLAGS.update({p.name: PRELOAD for p in HIP_SOURCES
+                       if p.name.startswith(("gemv_inst_", "gemm_rows_inst_")) or p.name == "attn_decode.hip"})
 
 
 def _newer(src: Path, dst: Path, extra=()) -> bool:

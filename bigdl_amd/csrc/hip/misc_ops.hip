@@ -499,7 +499,10 @@ extern "C" int bigdl_quant_rows_e4m3(const void* x, void* q, float* scale, int64
 }
 
 // bf16 -> fp16, 8 values per thread (the row-wise fp8 GEMM of hipBLASLt only writes bf16; PyTorch's own conversion
-// kernel for this pair of types is not vectorized and took longer than the GEMM it followed)
+// kernel for this pair of types is not vectorized and took longer than the GEMM it followed).  SAT: values beyond the fp16
+// range saturate; NaN stays NaN.
+// A linear on bf16 input: int8 203 x 4544, N = 4672 43.8 -> 41.7 us; nf4 3000 x 4096, N = 14336 390 -> 369 us.
+template <bool SAT>
 __global__ __launch_bounds__(256) void bf16_to_f16_kernel(const uint4v* __restrict__ src, uint4v* __restrict__ dst, int64_t nvec) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= nvec) return;
@@ -508,17 +511,20 @@ __global__ __launch_bounds__(256) void bf16_to_f16_kernel(const uint4v* __restri
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const float lo = __uint_as_float(v[e] << 16), hi = __uint_as_float(v[e] & 0xffff0000u);
-    const half2v h = {(_Float16)fminf(fmaxf(lo, -65504.0f), 65504.0f), (_Float16)fminf(fmaxf(hi, -65504.0f), 65504.0f)};
+    auto lim = [](float f) { return !SAT ? f : f > 65504.0f ? 65504.0f : f < -65504.0f ? -65504.0f : f; };
+    const half2v h = {(_Float16)lim(lo), (_Float16)lim(hi)};
     o[e] = __builtin_bit_cast(uint32_t, h);
   }
   dst[i] = o;
 }
 
 // n values (n % 8 == 0), both buffers 16-byte aligned and contiguous
-extern "C" int bigdl_bf16_to_f16(const void* src, void* dst, int64_t n, hipStream_t st) {
+extern "C" int bigdl_bf16_to_f16(const void* src, void* dst, int64_t n, int saturate, hipStream_t st) {
   if (n <= 0 || (n & 7) || ((uintptr_t)src & 15) || ((uintptr_t)dst & 15)) return -1;
   const int64_t nvec = n >> 3;
-  hipLaunchKernelGGL(bf16_to_f16_kernel, dim3((unsigned)((nvec + 255) / 256)), dim3(256), 0, st, (const uint4v*)src, (uint4v*)dst, nvec);
+  const dim3 grid((unsigned)((nvec + 255) / 256));
+  if (saturate) hipLaunchKernelGGL(bf16_to_f16_kernel<true>, grid, dim3(256), 0, st, (const uint4v*)src, (uint4v*)dst, nvec);
+  else hipLaunchKernelGGL(bf16_to_f16_kernel<false>, grid, dim3(256), 0, st, (const uint4v*)src, (uint4v*)dst, nvec);
   return HIP_CHECK_LAUNCH();
 }
 

@@ -306,6 +306,16 @@ def lowbit_rows(xh, w, qtype, n, k, bias=None, out_dtype=None):
     return y
 
 
+def _half(x):
+    """x on the GPU in fp16.  bf16 in one vectorized pass from 64 Ki values on; below, a conversion by PyTorch takes as long on
+    the GPU and less on the host.  (A clamp to +-65504 before it changed nothing and cost a pass: in bf16 that limit is 65536.)"""
+    if (x.dtype == torch.bfloat16 and x.numel() >= 65536 and x.is_contiguous() and x.numel() % 8 == 0
+            and x.data_ptr() % 16 == 0):
+        from ..ops import hip
+        return hip.bf16_to_f16(x, saturate=False)
+    return x.to(torch.float16)
+
+
 def lowbit_matmul(x_2d: torch.Tensor, weight: FP4Params, out_features: int, for_training: bool = False) -> torch.Tensor:
     """``x_2d @ dequant(weight)^T`` -> dtype of x_2d (reference op ``xe_linear.forward_new``).  ``for_training``: the
     forward of an autograd node whose backward will expand the weight anyway (bf16 activations): prompt-sized row
@@ -316,7 +326,7 @@ def lowbit_matmul(x_2d: torch.Tensor, weight: FP4Params, out_features: int, for_
         m, dt = x_2d.shape[0], x_2d.dtype
         t16 = weight.qlayout == "t16"
         if t16 and m <= GEMM_MAX_ROWS:
-            xh = x_2d if dt == torch.float16 else x_2d.to(torch.float16)
+            xh = x_2d if dt == torch.float16 else _half(x_2d)
             if xh.stride(1) != 1 or xh.stride(0) % 8 or xh.data_ptr() % 16:
                 xh = xh.contiguous()
             if m <= GEMV_MAX_ROWS:
@@ -328,12 +338,7 @@ def lowbit_matmul(x_2d: torch.Tensor, weight: FP4Params, out_features: int, for_
             # the dense product below: its backward needs the expanded weight anyway, and its activations are bf16 --
             # measured 0.106 against 0.154 s per QLoRA step on Llama-2-7B.  Inside an autograd node's forward grad mode is
             # off, so the caller says so explicitly.)
-            if x_2d.dtype == torch.float16:
-                xh = x_2d
-            elif x_2d.dtype == torch.bfloat16:
-                xh = x_2d.clamp(-65504.0, 65504.0).to(torch.float16)      # (bf16 reaches further than fp16)
-            else:
-                xh = x_2d.to(torch.float16)
+            xh = _half(x_2d)
             if xh.stride(1) != 1 or xh.stride(0) % 8 or xh.data_ptr() % 16:
                 xh = xh.contiguous()
             return lowbit_rows(xh, weight.data, weight.qtype, n, k, out_dtype=x_2d.dtype)

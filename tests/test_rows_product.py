@@ -182,3 +182,19 @@ def test_nf4_table_is_exact_in_every_position(hip, m):
         if m <= 3 and first > 24:                         # (the other rows of a fragment come with the larger m)
             break
         assert torch.equal(product(x.cuda(), dev, qt, n, k).cpu()[:rows], want[:, first:first + rows].t())
+
+
+@pytest.mark.parametrize("shape", [(16, 4096), (17, 4544), (300, 256), (1024, 64), (1024, 72), (511, 137)])
+def test_half_of_bf16_matches_torch(hip, shape):
+    """both sides of the 64 Ki line, an odd size; values beyond fp16's range, infinities, NaN and denormal results"""
+    from bigdl_amd.transformers.low_bit_linear import _half
+    x = torch.randn(shape, generator=torch.Generator().manual_seed(14)) * 10.0 ** torch.randint(-7, 6, shape, generator=torch.Generator().manual_seed(15))
+    x.view(-1)[:6] = torch.tensor([float("inf"), -float("inf"), float("nan"), 65504.0, 65520.0, -1e30])
+    x = x.bfloat16().cuda()
+    # (with and without limits that bf16 rounds to 65536, which is infinite in fp16)
+    for want in (x.to(torch.float16), x.clamp(-65504.0, 65504.0).to(torch.float16)):
+        torch.testing.assert_close(_half(x), want, rtol=0, atol=0, equal_nan=True)
+    sat = hip.bf16_to_f16(x)
+    torch.testing.assert_close(sat, x.float().clamp(-65504.0, 65504.0).half() if x.numel() % 8 == 0 else x.half(), rtol=0, atol=0, equal_nan=True)
+    xs = x[:, 1:]                                        # not contiguous
+    torch.testing.assert_close(_half(xs), xs.to(torch.float16), rtol=0, atol=0, equal_nan=True)

@@ -1,4 +1,5 @@
-// Dequant-fused MFMA GEMM for mid-size row counts on gfx950:  y[M,N] = f(x[M,K] . dequant(W)[N,K]^T), 64 < M <= ~512,
+// Dequant-fused MFMA GEMM for mid-size row counts on gfx950:  y[M,N] = f(x[M,K] . dequant(W)[N,K]^T) beyond the
+// few-row kernel's limits (256 rows, 192 where K > 8192) or where the prompt kernel does not take K,
 // and its grouped (mixture-of-experts) form where every 64/128-row block of x belongs to one expert.
 //
 // Takes the place of the reference's closed xe_linear.forward_new for prefill-sized inputs / xe_batch.batch_forward

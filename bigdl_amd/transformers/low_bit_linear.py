@@ -26,15 +26,14 @@ from ..ops import host
 from ..utils.common import invalidInputError
 
 TORCH_LINEAR_THRESHOLD = int(os.getenv("BIGDL_LLM_LINEAR_THRESHOLD", "512"))
-# rows above which the device path dequantizes + calls the dense GEMM instead of the fused GEMV
-# row-count policy of the fused kernels on the GPU (measured on the Llama-2-7B projection shapes, sym_int4): the skinny
-# GEMV wins up to 16 rows (one row tile), the fused MFMA GEMM from 17 to 256 rows (in isolation the two-tile GEMV ties it
-# up to 32 rows, inside the batched decode step the GEMM path is 20 % ahead at 32 rows), dequantize + hipBLASLt above
+# row-count policy of the products of tiled weights on the GPU: up to GEMV_MAX_ROWS rows ``gemv_lowbit`` (one or two rows on
+# the skinny kernel, more on the few-row kernel), up to GEMM_MAX_ROWS ``gemm_lowbit`` (few-row kernel, beyond its limits the
+# tile kernel), above the prompt kernel
 GEMV_MAX_ROWS = int(os.getenv("BIGDL_GEMV_MAX_ROWS", "16"))
 GEMM_MAX_ROWS = 256
 # q6_k weights stay in their checkpoint blocks on the GPU.  Up to this many fp16 rows are multiplied from the blocks (csrc/hip/
-# gemm_rows_kernel.h, up to four gemv_q6k.hip); above, and for bf16 activations, whose range fp16 does not have, the weight is expanded for a dense
-# product.  4096 x 11008, one MI355X, expanded -> from the blocks: 1 row 100 -> 17 us, 64 rows 108 -> 35, 128 rows 128 -> 58.
+# gemm_rows_kernel.h, up to four gemv_q6k.hip); above, and for bf16 activations, whose range fp16 does not have, the weight
+# is expanded for a dense product.  4096 x 11008, one MI355X, expanded -> from the blocks: 1 row 100 -> 17 us, 64 rows 108 -> 35, 128 rows 128 -> 58.
 Q6K_MAX_ROWS = 128
 # forward of frozen low-bit linears inside a training step on the fused prompt GEMM (fp16 copy of the activations)
 # instead of dequantize + dense product

@@ -1,0 +1,80 @@
+"""The scratch memory of products whose partial sums pass through memory."""
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from bigdl_amd import qtypes as Q
+from bigdl_amd.ops import hip, host
+
+QT = Q.ggml_tensor_qtype["sym_int4"]
+
+
+class _Allocations(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.ptrs = set()
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        out = func(*args, **(kwargs or {}))
+        if "empty" in str(func):
+            self.ptrs.add(out.data_ptr())
+        return out
+
+
+class _Library:
+    """stands for the kernels' library: two K splits, one slab, and the workspace address that each launch is given"""
+    at = {"bigdl_gemm_lowbit": 5, "bigdl_gemm_prompt": 5, "bigdl_gemm_lowbit_ex": 12}
+
+    def __init__(self):
+        self.got = []
+
+    def __getattr__(self, name):
+        if name in self.at:
+            return lambda *a: self.got.append(a[self.at[name]]) or 0
+        return lambda *a: 2
+
+
+@pytest.mark.parametrize("call", ["gemm_lowbit", "gemm_lowbit_ex", "gemm_prompt"])
+def test_every_call_allocates_its_own_scratch(monkeypatch, call):
+    """A buffer kept between calls is freed when a larger one takes its place, while captured graphs go on writing to it:
+    what a launch gets must have been allocated by that call (under capture: from the graph's pool)."""
+    lib = _Library()
+    monkeypatch.setattr(hip, "lib", lambda: lib)
+    monkeypatch.setattr(hip, "_need_cuda", lambda *t: None)
+    monkeypatch.setattr(hip, "_stream", lambda: 0)
+    n, k = 32, 256
+    w = torch.zeros(host.device_nbytes(QT, n, k), dtype=torch.uint8)
+    keep = []
+    for m in (20, 20, 40, 20):
+        x = torch.zeros(m, k, dtype=torch.float16)
+        with _Allocations() as made:
+            keep.append(getattr(hip, call)(x, w, QT, n, k))
+        assert lib.got[-1] in made.ptrs
+    assert len(lib.got) == 4
+
+
+@pytest.mark.gpu
+def test_a_captured_split_product_outlives_larger_calls():
+    """capture, a call that needs more scratch, new allocations, replay: the replays write to none of them"""
+    g = torch.Generator().manual_seed(1)
+    n, k, m = 4096, 11008, 64                                     # K split over workgroups
+    w = (torch.randint(0, 256, (host.device_nbytes(QT, n, k),), dtype=torch.uint8, generator=g) & 0xBF).cuda()
+    wide = (torch.randint(0, 256, (host.device_nbytes(QT, 8192, 256),), dtype=torch.uint8, generator=g) & 0xBF).cuda()
+    x = torch.randn(m, k, generator=g).half().cuda()
+    want = hip.gemm_lowbit(x, w, QT, n, k)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = hip.gemm_lowbit(x, w, QT, n, k)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+    for rows in (600, 1500):
+        hip.gemm_prompt(torch.ones(rows, 256, dtype=torch.float16, device="cuda"), wide, QT, 8192, 256, out_dtype=torch.float32)
+        fresh = [torch.full((1 << 20,), float(i), device="cuda") for i in range(48)]
+        x.copy_(torch.randn(m, k, generator=g).half())
+        graph.replay()
+        want = hip.gemm_lowbit(x, w, QT, n, k)
+        assert torch.equal(out, want)
+        assert all(bool((t == i).all()) for i, t in enumerate(fresh))
+        del fresh

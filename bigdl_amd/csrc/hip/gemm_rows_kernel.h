@@ -115,8 +115,9 @@ __device__ __forceinline__ int rows_chunk(int s, int g) { return 4 * (s & 1) + g
 // q6_k as the file's blocks hold it (210 bytes for 256 elements of a row: 128 of low nibbles, 64 of high bit pairs, 16 int8
 // sub-scales, fp16 d): a k-tile is half a block.  Lane group g takes bytes 16 g .. of the half's low nibbles -- 64 contiguous
 // bytes a row and request -- so that fragment s holds k = 32 ((g >> 1) + 2 (s >> 1)) + 16 (g & 1) + 8 (s & 1) + j, all of it
-// in sub-block g + 4 (s >> 1).  Code times sub-scale is exact in fp16 up to 2048 and within 2^-12 above; d multiplies the fp32
-// product (up to 16 rows).
+// in sub-block g + 4 (s >> 1).  Code times sub-scale is exact in fp16 up to 2048 and within 2^-11 above (12 % of a normal
+// matrix's weights); d multiplies the fp32 product, once for the two steps of a half k-tile.  Error of a weight, rms: 1.6e-4,
+// where the expansion to fp16 has 2.1e-4.
 // Blocks start at even bytes, every other one between two dwords.  16-byte loads from there are split by the address unit
 // (4096 x 11008, 1 row: 34 us, 25 this way); so the dwords around them are loaded and shifted into place.  The last dword's address steps
 // back where it is not needed: nothing outside the block is touched.
@@ -176,10 +177,6 @@ __device__ __forceinline__ half8 rows_fragment<Q_Q6_K>(const Tile<Q_Q6_K>& t, in
   return r.v;
 }
 template <>
-__device__ __forceinline__ float rows_scale<Q_Q6_K>(const Tile<Q_Q6_K>& t, int) { return (float)t.d; }
-template <>
-__device__ __forceinline__ half8 rows_scaled<Q_Q6_K>(const Tile<Q_Q6_K>& t, half8 code, int) { return code * t.d; }
-template <>
 __device__ __forceinline__ int rows_chunk<Q_Q6_K>(int s, int g) { return 2 * g + (s & 1); }
 
 // MT = 16-row tiles of x, NT = 16-column tiles of a weight per workgroup, WD = k-tiles of weights requested ahead.  What the
@@ -192,7 +189,7 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(const 
   a.x = p_x; a.w = p_w; a.w2 = p_w2; a.gamma = p_gamma; a.M = p_M; a.N = p_N; a.K = p_K; a.ldx = p_ldx;
   a.kt_per_split = p_kt_per_split; a.gamma_offset = p_goff;
   constexpr int NS = PAIR ? 2 * NT : NT;             // weight tiles per k-tile
-  constexpr bool POST = MT == 1;                     // block scale on the fp32 product instead of the fp16 code
+  constexpr bool POST = MT == 1;                     // block scale on the fp32 product instead of the fp16 code (q6_k: always)
   constexpr bool NORM = MT == 1;                     // the folded RMSNorm exists for up to 16 rows
   constexpr int XB = MT * 2048;                      // bytes of half a staged x tile: MT * 16 rows of 64 halves
   constexpr bool TWO = rows_two_phase(MT, NS, NW);
@@ -290,39 +287,61 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(const 
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[n][j] = float4v{0, 0, 0, 0};
 
+  auto x_fragment = [&](int h, int s, int j) {
+    return *(const half8*)(xt + h * XB + (16 * j + r) * 128 + ((rows_chunk<QT>(s, g) ^ (r & 7)) << 4));
+  };
   auto half_step = [&](Tile<QT> (&t)[NS], int h) {
+    if constexpr (RAW) {
+      half8 xa[2][MT];
 #pragma unroll
-    for (int s = 2 * h; s < 2 * h + 2; ++s) {
-      half8 xa[MT];
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < MT; ++j) xa[j] = *(const half8*)(xt + h * XB + (16 * j + r) * 128 + ((rows_chunk<QT>(s, g) ^ (r & 7)) << 4));
-      float4v sx[POST ? MT : 1];
-      if constexpr (POST && has_min<QT>()) {
-        // block sums of x in the layout of the product: a fragment of ones
-        const half8 one8 = {1, 1, 1, 1, 1, 1, 1, 1};
-#pragma unroll
-        for (int j = 0; j < MT; ++j) sx[j] = mfma16(xa[j], one8, float4v{0, 0, 0, 0});
-      }
+        for (int j = 0; j < MT; ++j) xa[i][j] = x_fragment(h, 2 * h + i, j);
 #pragma unroll
       for (int n = 0; n < NS; ++n) {
-        const half8 code = rows_fragment<QT>(t[n], s, g);
-        if constexpr (POST) {
-          const float d = rows_scale<QT>(t[n], s);
+        const half8 c0 = rows_fragment<QT>(t[n], 2 * h, g), c1 = rows_fragment<QT>(t[n], 2 * h + 1, g);
+        const float d = (float)t[n].d;
 #pragma unroll
-          for (int j = 0; j < MT; ++j) {
-            const float4v c = mfma16(xa[j], code, float4v{0, 0, 0, 0});
+        for (int j = 0; j < MT; ++j) {
+          const float4v c = mfma16(xa[1][j], c1, mfma16(xa[0][j], c0, float4v{0, 0, 0, 0}));
 #pragma unroll
-            for (int q = 0; q < 4; ++q) acc[n][j][q] = fmaf(c[q], d, acc[n][j][q]);
-            if constexpr (has_min<QT>()) {
-              const float mn = (float)t[n].m[s];
+          for (int q = 0; q < 4; ++q) acc[n][j][q] = fmaf(c[q], d, acc[n][j][q]);
+        }
+      }
+    } else {
 #pragma unroll
-              for (int q = 0; q < 4; ++q) acc[n][j][q] = fmaf(sx[j][q], mn, acc[n][j][q]);
+      for (int s = 2 * h; s < 2 * h + 2; ++s) {
+        half8 xa[MT];
+#pragma unroll
+        for (int j = 0; j < MT; ++j) xa[j] = x_fragment(h, s, j);
+        float4v sx[POST ? MT : 1];
+        if constexpr (POST && has_min<QT>()) {
+          // block sums of x in the layout of the product: a fragment of ones
+          const half8 one8 = {1, 1, 1, 1, 1, 1, 1, 1};
+#pragma unroll
+          for (int j = 0; j < MT; ++j) sx[j] = mfma16(xa[j], one8, float4v{0, 0, 0, 0});
+        }
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+          const half8 code = rows_fragment<QT>(t[n], s, g);
+          if constexpr (POST) {
+            const float d = rows_scale<QT>(t[n], s);
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+              const float4v c = mfma16(xa[j], code, float4v{0, 0, 0, 0});
+#pragma unroll
+              for (int q = 0; q < 4; ++q) acc[n][j][q] = fmaf(c[q], d, acc[n][j][q]);
+              if constexpr (has_min<QT>()) {
+                const float mn = (float)t[n].m[s];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc[n][j][q] = fmaf(sx[j][q], mn, acc[n][j][q]);
+              }
             }
-          }
-        } else {
-          const half8 bf = rows_scaled<QT>(t[n], code, s);
+          } else {
+            const half8 bf = rows_scaled<QT>(t[n], code, s);
 #pragma unroll
-          for (int j = 0; j < MT; ++j) acc[n][j] = mfma16(xa[j], bf, acc[n][j]);
+            for (int j = 0; j < MT; ++j) acc[n][j] = mfma16(xa[j], bf, acc[n][j]);
+          }
         }
       }
     }

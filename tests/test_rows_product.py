@@ -111,11 +111,33 @@ def test_q6k_blocks_without_expansion(hip, m, n, k):
     w = host.dequantize(raw, Q.Q6_K, w0.shape).double()
     x, xd = _x(m, k, 9)
     ref = xd @ w.t()
-    # code * sub-scale reaches 32 * 128: above 2048 it is rounded to 2^-11; more than 16 rows round the weight to fp16 once
+    # code * sub-scale reaches 32 * 128: above 2048 it is rounded to 2^-11
     for nt in (0, 1, 2, 3):
         out = hip.gemm_rows(x, raw.cuda(), Q.Q6_K, n, k, out_dtype=torch.float32, nt=nt)
-        bound = (2.0 ** -11 if m <= 16 else 2.0 ** -10) * (xd.abs() @ w.abs().t()) + 1e-5
+        bound = 2.0 ** -11 * (xd.abs() @ w.abs().t()) + 1e-5
         assert ((out.double().cpu() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("m", [4, 16, 17, 32, 33, 64, 100, 128])
+def test_q6k_weights_are_no_coarser_than_expanded_ones(hip, m):
+    """One-hot rows read the weights as the product uses them: d * code * sub-scale with nothing rounded while code * sub-scale is
+    at most 2048 (exact in fp16), rounded once to fp16 above; in the mean closer than weights expanded to fp16."""
+    n, k = 64, 256
+    raw = host.quantize(torch.randn(n, k, generator=torch.Generator().manual_seed(16)) * 0.05, Q.Q6_K)
+    w = host.dequantize(raw, Q.Q6_K, (n, k)).double()                     # (exact: fp32 holds d * code * sub-scale)
+    d = raw.view(torch.uint8).reshape(n, 210)[:, 208:].contiguous().view(torch.float16).double()
+    exact = (w / d).abs() <= 2048
+    assert 0.5 < exact.double().mean() < 0.99
+    used = torch.zeros(n, k, dtype=torch.float64)
+    for first in range(0, k, m):
+        rows = min(m, k - first)
+        x = torch.zeros(m, k, dtype=torch.float16)
+        x[torch.arange(rows), first + torch.arange(rows)] = 1
+        out = hip.gemm_q6k(x.cuda(), raw.view(torch.uint8).cuda(), n, k, out_dtype=torch.float32)
+        used[:, first:first + rows] = out[:rows].t().cpu().double()
+    off = (used - w).abs()
+    assert (off <= torch.where(exact, 2.0 ** -22, 2.0 ** -11) * w.abs()).all()
+    assert off.pow(2).mean() <= (w.half().double() - w).pow(2).mean()
 
 
 # fewer rows than wavefronts, more than the grid holds at once, one block, a quad of blocks and one more, a full request

@@ -18,6 +18,7 @@ from functools import reduce
 from operator import mul
 
 import torch
+import torch.autograd.forward_ad as fwad
 import torch.nn.functional as F
 from torch import nn
 
@@ -31,9 +32,10 @@ TORCH_LINEAR_THRESHOLD = int(os.getenv("BIGDL_LLM_LINEAR_THRESHOLD", "512"))
 # tile kernel), above the prompt kernel
 GEMV_MAX_ROWS = int(os.getenv("BIGDL_GEMV_MAX_ROWS", "16"))
 GEMM_MAX_ROWS = 256
-# q6_k weights stay in their checkpoint blocks on the GPU.  Up to this many fp16 rows are multiplied from the blocks (csrc/hip/
-# gemm_rows_kernel.h, up to four gemv_q6k.hip); above, and for bf16 activations, whose range fp16 does not have, the weight
-# is expanded for a dense product.  4096 x 11008, one MI355X, expanded -> from the blocks: 1 row 100 -> 17 us, 64 rows 108 -> 35, 128 rows 128 -> 58.
+# q6_k weights stay in their checkpoint blocks on the GPU.  Up to this many fp16 (or fp32) rows are multiplied from the blocks
+# (csrc/hip/gemm_rows_kernel.h, up to four gemv_q6k.hip).  The weight is expanded for a dense product above, for bf16
+# activations, whose range fp16 does not have, and where autograd, a transform or a trace looks on.  Kernel time of 4096 x 11008,
+# one MI355X, expanded -> from the blocks: 1 row 100 -> 17 us, 64 rows 107 -> 34, 128 rows 127 -> 47.
 Q6K_MAX_ROWS = 128
 # forward of frozen low-bit linears inside a training step on the fused prompt GEMM (fp16 copy of the activations)
 # instead of dequantize + dense product
@@ -315,6 +317,15 @@ def _half(x):
     return x.to(torch.float16)
 
 
+def _observed(x):
+    """Whether anything but the caller looks at what is done to x: autograd in either direction, a function transform, a trace,
+    a dispatch mode.  Those see PyTorch operations, not launches of this package."""
+    return (type(x) not in (torch.Tensor, torch.nn.Parameter) or (x.requires_grad and torch.is_grad_enabled())
+            or torch._C._functorch.is_functorch_wrapped_tensor(x) or torch._C._get_tracing_state() is not None
+            or torch._C._len_torch_dispatch_stack() > 0
+            or (fwad._current_level >= 0 and fwad.unpack_dual(x).tangent is not None))
+
+
 def lowbit_matmul(x_2d: torch.Tensor, weight: FP4Params, out_features: int, for_training: bool = False) -> torch.Tensor:
     """``x_2d @ dequant(weight)^T`` -> dtype of x_2d (reference op ``xe_linear.forward_new``).  ``for_training``: the
     forward of an autograd node whose backward will expand the weight anyway (bf16 activations): prompt-sized row
@@ -341,7 +352,8 @@ def lowbit_matmul(x_2d: torch.Tensor, weight: FP4Params, out_features: int, for_
             if xh.stride(1) != 1 or xh.stride(0) % 8 or xh.data_ptr() % 16:
                 xh = xh.contiguous()
             return lowbit_rows(xh, weight.data, weight.qtype, n, k, out_dtype=x_2d.dtype)
-        if weight.qtype == Q.Q6_K and m <= Q6K_MAX_ROWS and x_2d.dtype != torch.bfloat16 and not for_training and weight.data.data_ptr() % 4 == 0:
+        if (weight.qtype == Q.Q6_K and 0 < m <= Q6K_MAX_ROWS and dt in (torch.float16, torch.float32) and not for_training
+                and weight.data.data_ptr() % 4 == 0 and not _observed(x_2d)):
             xh = x_2d.to(torch.float16)
             if xh.stride(1) != 1 or xh.stride(0) % 8 or xh.data_ptr() % 16:
                 xh = xh.contiguous()

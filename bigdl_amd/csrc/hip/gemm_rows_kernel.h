@@ -68,7 +68,9 @@ __device__ __forceinline__ rows_rsrc rows_buffer(const void* p, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, bytes, 0x00027000);
 }
 constexpr int ROWS_NT = 2;            // cache policy of a buffer load: non-temporal
-constexpr int ROWS_OUT = 0x40000000;  // a lane offset past the end of every buffer here: the load returns zeros, no memory access
+// a lane offset past the end of every buffer here (a gigabyte at most): the load returns zeros, no memory access
+constexpr uint32_t ROWS_OUT = 0x40000000;
+static_assert(ROWS_OUT + ROWS_OUT == 0x80000000u, "a row and a column that are both outside: no overflow (the type is unsigned)");
 
 // one weight tile through buffer loads: every address is a scalar offset plus a lane constant
 template <int QT>
@@ -81,7 +83,7 @@ struct RowsPlanes {
     if constexpr (has_min_of(QT)) mn = rows_buffer(p.mn + tile0 * 64, tiles * 128);
   }
   // out: 0, or ROWS_OUT for a tile that does not exist (zeros, no memory access)
-  __device__ __forceinline__ void load(Tile<QT>& t, int tile, int lane, int out) const {
+  __device__ __forceinline__ void load(Tile<QT>& t, int tile, int lane, uint32_t out) const {
     t.lo0 = __builtin_amdgcn_raw_buffer_load_b128(lo, lane * 16 + out, tile * (lo_bits_of(QT) * 256), ROWS_NT);
     if constexpr (lo_bits_of(QT) == 8) t.lo1 = __builtin_amdgcn_raw_buffer_load_b128(lo, lane * 16 + 1024 + out, tile * 2048, ROWS_NT);
     if constexpr (hi_bits_of(QT) == 1) t.hi0 = __builtin_amdgcn_raw_buffer_load_b32(hi, lane * 4 + out, tile * 256, ROWS_NT);
@@ -90,7 +92,7 @@ struct RowsPlanes {
       t.hi0 = h.x;
       t.hi1 = h.y;
     }
-    const int r8 = (lane & 15) * 8 + out;
+    const uint32_t r8 = (lane & 15) * 8 + out;
     t.d = __builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(sc, r8, tile * 128, ROWS_NT));
     if constexpr (has_min_of(QT)) t.m = __builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(mn, r8, tile * 128, ROWS_NT));
   }
@@ -222,11 +224,12 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(const 
   // and every wait a fixed count of younger loads
   const int nk = kt1 - kt0 > wave ? (kt1 - kt0 - wave + NW - 1) / NW : 0;
   auto kmap = [&](int i) { return min(kt0 + wave + i * NW, KT - 1); };
-  auto past = [&](int i) { return i < nk ? 0 : ROWS_OUT; };
+  auto past = [&](int i) { return i < nk ? 0u : ROWS_OUT; };
 
   Tile<QT> tt[WD][NS];
   auto fetch_w = [&](Tile<QT> (&t)[NS], int i) {
-    const int kt = kmap(i), out = past(i);
+    const int kt = kmap(i);
+    const uint32_t out = past(i);
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
       if constexpr (RAW) pl.load(t[n], n, kt, lane);        // (past the end: the last tile again, never multiplied)
@@ -242,15 +245,15 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(const 
   const bool norm = NORM && a.gamma != nullptr;
   const rows_rsrc gb = rows_buffer(norm ? a.gamma : a.x, norm ? a.K * 2 : 0);
   const _Float16 goff = (_Float16)(norm ? a.gamma_offset : 1.0f);
-  int xoff[NP];
+  uint32_t xoff[NP];
 #pragma unroll
-  for (int p = 0; p < NP; ++p) xoff[p] = 8 * p + srow < rows ? (8 * p + srow) * a.ldx * 2 + slot * 16 : ROWS_OUT;
+  for (int p = 0; p < NP; ++p) xoff[p] = 8 * p + srow < rows ? (uint32_t)((8 * p + srow) * a.ldx * 2 + slot * 16) : ROWS_OUT;
   constexpr int XH = rows_x_halves(MT, NS);
   uint4v xr[XH][NP];
   uint4v gr[2];
   auto fetch_x = [&](int i, int h) {
     const int k = kmap(i) * 128 + h * 64;
-    const int out = i < nk && k + slot * 8 < a.K ? 0 : ROWS_OUT;
+    const uint32_t out = i < nk && k + slot * 8 < a.K ? 0u : ROWS_OUT;
 #pragma unroll
     for (int p = 0; p < NP; ++p) xr[h % XH][p] = __builtin_amdgcn_raw_buffer_load_b128(xb, xoff[p] + out, k * 2, 0);
     if constexpr (NORM) gr[h] = __builtin_amdgcn_raw_buffer_load_b128(gb, slot * 16 + out, k * 2, 0);

@@ -1060,9 +1060,20 @@ static int launch_x(const GemvArgs& a_in, hipStream_t st) {
       }
     }
   }
+  // 16 wavefronts when the grid is small (about one workgroup per CU) and every wavefront still gets
+  // at least two k-tiles: halves the per-wavefront instruction stream of the latency-bound small GEMVs
+  const bool wide = MT == 1 && !GATE_UP && xbytes <= GEMV_XLDS_LIMIT && grid.x <= 256 && grid.y == 1 && Kp / 128 >= 32;
   if (a.slot_expert != nullptr) {
-    // routed slots: one row each, the lean or the general 8-wavefront kernel
+    // routed slots: one row each; a single one (one token, one expert) has the wide form too.  Without it, with it, us: 4096 x 4096
+    // sym_int4 5.6, 5.1, asym_int4 6.3, 6.0; 4096 x 8192 sym_int4 7.6, 7.0
     if constexpr (MT == 1) {
+      if constexpr (!GATE_UP) {
+        if (wide) {
+          hipLaunchKernelGGL((gemv_t16_kernel<QT, 1, false, true, 16, false, false, false, false, true>), grid, dim3(1024), fixed(16) + xbytes,
+                             st, GEMV_ARGS(a));
+          return HIP_CHECK_LAUNCH();
+        }
+      }
       if (!GATE_UP && ((a.K + 511) / 512 + 7) / 8 <= 2 && xbytes <= GEMV_XLDS_LIMIT) {
         hipLaunchKernelGGL((gemv_t16_kernel<QT, 1, GATE_UP, true, 8, false, false, true, false, true>), grid, dim3(512), fixed(8) + xbytes,
                            st, GEMV_ARGS(a));
@@ -1080,9 +1091,6 @@ static int launch_x(const GemvArgs& a_in, hipStream_t st) {
       return -7;
     }
   }
-  // 16 wavefronts when the grid is small (about one workgroup per CU) and every wavefront still gets
-  // at least two k-tiles: halves the per-wavefront instruction stream of the latency-bound small GEMVs
-  const bool wide = MT == 1 && !GATE_UP && xbytes <= GEMV_XLDS_LIMIT && grid.x <= 256 && grid.y == 1 && Kp / 128 >= 32;
   if (a.att_ws != nullptr) {
     // split-KV attention partials combined in the staging prologue (host entry: x fits GEMV_XLDS_LIMIT, at most 16 rows)
     if constexpr (MT == 1 && !GATE_UP) {

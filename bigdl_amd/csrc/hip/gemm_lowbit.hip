@@ -205,9 +205,8 @@ static int pick_bn(int M) {
 // 20.5 -> 13.8, gate / up 78 -> 70, down 38.7 -> 35.7; 192 rows 45.9 -> 30.3, 35.3 -> 25.1, 116 -> 93, 82.7 -> 68.7; 256 rows
 // 39.3 -> 31.0, 27.5 -> 25.0, 150 -> 117, and down 62.6 -> 69.5: every block reads all of x and of the weight, so four blocks
 // of a long K are the tile kernel's.
-static bool takes_rows_kernel(const void* x, int ldx, int M, int N, int K, int qtype, bool pair, RowsPlan* plan) {
-  if (M > 256 || (M > 192 && K > 8192) || !is_t16(qtype)) return false;
-  if (x != nullptr && !rows_ok(x, ldx)) return false;
+static bool takes_rows_kernel(int ldx, int M, int N, int K, int qtype, bool pair, RowsPlan* plan) {
+  if (M > 256 || (M > 192 && K > 8192) || !is_t16(qtype) || !rows_ok(nullptr, ldx)) return false;
   *plan = rows_plan(M, N, K, qtype, pair, !pair && M <= 64);
   return true;
 }
@@ -220,17 +219,6 @@ static int launch_rows(const GemmArgs& a, int qtype, const RowsPlan& p, hipStrea
   return rc != 0 || p.splitk == 1 ? rc : launch_reduce(a, stream);
 }
 
-// qtype: the format as the caller knows it
-extern "C" int bigdl_gemm_lowbit_splitk(int M, int N, int K, int qtype) {
-  int sk, per;
-  RowsPlan p;
-  // (the workspace has to do for whichever kernel the alignment of x allows)
-  const int rows_sk = takes_rows_kernel(nullptr, 0, M, N, K, t16_kernel_qtype(qtype), false, &p) ? p.splitk : 1;
-  const int bm = bigdl_gemm_lowbit_bm(M);
-  plan((M + bm - 1) / bm, pick_bn(M), N, K, &sk, &per);
-  return sk > rows_sk ? sk : rows_sk;
-}
-
 extern "C" int bigdl_gemm_lowbit_bm(int M) {
   (void)M;
   static const int forced = getenv("BIGDL_GEMM_BM") ? atoi(getenv("BIGDL_GEMM_BM")) : 0;
@@ -240,7 +228,50 @@ extern "C" int bigdl_gemm_lowbit_bm(int M) {
   return 64;
 }
 
-// Dense form.  x fp16 [M, ldx] (ldx % 8 == 0, 16-byte aligned), K % 32 == 0.  workspace: fp32, >= splitk*M*N.
+// The kernel a call runs on and the fp32 scratch it needs: one place for the launches and for the size that callers ask for
+struct DensePlan {
+  bool rows;                // few-row kernel; otherwise the tile kernel
+  RowsPlan r;
+  int bm, mblocks, splitk, kt_per_split;
+  bool partial;             // the results pass through scratch and the reduce kernel
+  int64_t floats;
+};
+// fold_norm, ssq_out: the tile kernel's forms of gemm_lowbit_ex
+static DensePlan dense_plan(int M, int N, int K, int ldx, int qtype, bool pair, bool fold_norm, bool ssq_out) {
+  DensePlan p = {};
+  p.rows = !fold_norm && !ssq_out && takes_rows_kernel(ldx, M, N, K, qtype, pair, &p.r);
+  if (p.rows) {
+    p.splitk = p.r.splitk;
+    p.kt_per_split = p.r.kt_per_split;
+    p.partial = p.splitk > 1;
+  } else {
+    p.bm = bigdl_gemm_lowbit_bm(M);
+    p.mblocks = (M + p.bm - 1) / p.bm;
+    plan(p.mblocks * (pair ? 2 : 1), pick_bn(M), N, K, &p.splitk, &p.kt_per_split);
+    p.partial = p.splitk > 1 || pair || ssq_out;
+  }
+  p.floats = p.partial ? (pair ? 2 : 1) * (int64_t)p.splitk * M * N : 0;
+  return p;
+}
+static int launch_dense(GemmArgs& a, const DensePlan& p, int qtype, int64_t workspace_floats, hipStream_t stream) {
+  if (p.floats > 0 && (a.partial == nullptr || workspace_floats < p.floats)) return -5;
+  a.splitk = p.splitk;
+  a.kt_per_split = p.kt_per_split;
+  if (p.rows) return launch_rows(a, qtype, p.r, stream);
+  a.force_partial = p.partial && p.splitk == 1 ? 1 : 0;
+  a.pair_stride = (int64_t)a.splitk * a.M * a.N;
+  const int rc = dispatch(a, qtype, p.bm, pick_bn(a.M), p.mblocks, stream);
+  return rc != 0 || !p.partial ? rc : launch_reduce(a, stream);
+}
+
+// fp32 scratch, in floats, that bigdl_gemm_lowbit (pair, fold_norm, ssq_out = 0) and bigdl_gemm_lowbit_ex need for this call;
+// 0: none.  qtype: the format as the caller knows it.
+extern "C" int64_t bigdl_gemm_lowbit_workspace(int M, int N, int K, int ldx, int qtype, int pair, int fold_norm, int ssq_out) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  return dense_plan(M, N, K, ldx, t16_kernel_qtype(qtype), pair != 0, fold_norm != 0, ssq_out != 0).floats;
+}
+
+// Dense form.  x fp16 [M, ldx] (ldx % 8 == 0, 16-byte aligned), K % 32 == 0.  workspace: see bigdl_gemm_lowbit_workspace.
 extern "C" int bigdl_gemm_lowbit(const void* x, const void* w, void* out, const void* bias, const void* residual,
                                  float* workspace, int64_t workspace_floats, int M, int N, int K, int ldx, int ldo,
                                  int qtype, int act, int out_type, hipStream_t stream) {
@@ -251,25 +282,12 @@ extern "C" int bigdl_gemm_lowbit(const void* x, const void* w, void* out, const 
   GemmArgs a = {};
   a.x = (const _Float16*)x; a.w = w; a.out = out; a.bias = bias; a.residual = residual; a.partial = workspace;
   a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldo = ldo; a.act = act; a.out_type = out_type;
-  RowsPlan p;
-  if (takes_rows_kernel(x, ldx, M, N, K, qtype, false, &p)) {
-    a.splitk = p.splitk;
-    if (p.splitk > 1 && (workspace == nullptr || workspace_floats < (int64_t)p.splitk * M * N)) return -5;
-    return launch_rows(a, qtype, p, stream);
-  }
-  const int bm = bigdl_gemm_lowbit_bm(M);
-  const int bn = pick_bn(M);
-  const int mblocks = (M + bm - 1) / bm;
-  plan(mblocks, bn, N, K, &a.splitk, &a.kt_per_split);
-  if (a.splitk > 1 && (workspace == nullptr || workspace_floats < (int64_t)a.splitk * M * N)) return -5;
-  const int rc = dispatch(a, qtype, bm, bn, mblocks, stream);
-  if (rc != 0 || a.splitk == 1) return rc;
-  return launch_reduce(a, stream);
+  return launch_dense(a, dense_plan(M, N, K, ldx, qtype, false, false, false), qtype, workspace_floats, stream);
 }
 
 // Extended dense form for batched decode: RMSNorm folded in (gamma + row_ssq of x, see GemmArgs), gate / up pair in one
 // launch (w2: out = act(x W^T + bias) * (x W2^T + bias2)), and the sums of squares of the output rows (ssq_out, after
-// the residual add) for the norm folded into the next product.  workspace: fp32, >= (w2 ? 2 : 1) * splitk * M * N.
+// the residual add) for the norm folded into the next product.  workspace: see bigdl_gemm_lowbit_workspace.
 extern "C" int bigdl_gemm_lowbit_ex(const void* x, const void* w, const void* w2, void* out, const void* bias, const void* bias2,
                                     const void* residual, const void* gamma, float gamma_offset, float eps,
                                     const float* row_ssq, float* ssq_out, float* workspace, int64_t workspace_floats, int M,
@@ -285,33 +303,8 @@ extern "C" int bigdl_gemm_lowbit_ex(const void* x, const void* w, const void* w2
   a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldo = ldo; a.act = act; a.out_type = out_type;
   a.gamma = (const _Float16*)gamma; a.gamma_offset = gamma_offset; a.eps = eps; a.row_ssq = gamma != nullptr ? row_ssq : nullptr;
   a.ssq_out = ssq_out; a.w2 = w2; a.bias2 = bias2;
-  RowsPlan p;
-  if (gamma == nullptr && ssq_out == nullptr && takes_rows_kernel(x, ldx, M, N, K, qtype, w2 != nullptr, &p)) {
-    a.splitk = p.splitk;
-    if (p.splitk > 1 && (workspace == nullptr || workspace_floats < (int64_t)p.splitk * M * N)) return -5;
-    return launch_rows(a, qtype, p, stream);
-  }
-  const int bm = gamma != nullptr ? (bigdl_gemm_lowbit_bm(M) < 64 ? 64 : bigdl_gemm_lowbit_bm(M)) : bigdl_gemm_lowbit_bm(M);
-  const int bn = pick_bn(M);
-  const int mblocks = (M + bm - 1) / bm;
-  plan(mblocks * (w2 != nullptr ? 2 : 1), bn, N, K, &a.splitk, &a.kt_per_split);
-  a.force_partial = (w2 != nullptr || ssq_out != nullptr) ? 1 : 0;
-  a.pair_stride = (int64_t)a.splitk * M * N;
-  const bool partial_out = a.splitk > 1 || a.force_partial;
-  if (partial_out && (workspace == nullptr || workspace_floats < (w2 != nullptr ? 2 : 1) * (int64_t)a.splitk * M * N)) return -5;
-  const int rc = dispatch(a, qtype, bm, bn, mblocks, stream);
-  if (rc != 0 || !partial_out) return rc;
-  return launch_reduce(a, stream);
-}
-
-// splits the extended form will use (workspace sizing): pair = 1 when w2 is given
-extern "C" int bigdl_gemm_lowbit_ex_splitk(int M, int N, int K, int pair, int qtype) {
-  int sk, per;
-  RowsPlan p;
-  const int rows_sk = takes_rows_kernel(nullptr, 0, M, N, K, t16_kernel_qtype(qtype), pair != 0, &p) ? p.splitk : 1;
-  const int bm = bigdl_gemm_lowbit_bm(M);
-  plan(((M + bm - 1) / bm) * (pair ? 2 : 1), pick_bn(M), N, K, &sk, &per);
-  return sk > rows_sk ? sk : rows_sk;
+  return launch_dense(a, dense_plan(M, N, K, ldx, qtype, w2 != nullptr, gamma != nullptr, ssq_out != nullptr), qtype, workspace_floats,
+                      stream);
 }
 
 // Grouped form: `rows` sorted rows in total; row i uses the weights of the expert that the block table assigns

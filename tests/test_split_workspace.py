@@ -31,7 +31,7 @@ class _Library:
     def __getattr__(self, name):
         if name in self.at:
             return lambda *a: self.got.append(a[self.at[name]]) or 0
-        return lambda *a: 2
+        return lambda *a: 4096 if name.endswith("workspace") else 2
 
 
 @pytest.mark.parametrize("call", ["gemm_lowbit", "gemm_lowbit_ex", "gemm_prompt"])
@@ -51,6 +51,17 @@ def test_every_call_allocates_its_own_scratch(monkeypatch, call):
             keep.append(getattr(hip, call)(x, w, QT, n, k))
         assert lib.got[-1] in made.ptrs
     assert len(lib.got) == 4
+
+
+@pytest.mark.parametrize("m,n,k,pair,norms,floats", [
+    (200, 14336, 4096, 1, 0, 0),                       # a pair on the few-row kernel is combined in registers
+    (150, 11008, 4096, 1, 0, 0), (64, 11008, 4096, 1, 0, 0), (64, 4096, 4096, 0, 0, 0),
+    (64, 4096, 11008, 0, 0, 2 * 64 * 4096),            # the few-row kernel's two K splits
+    (64, 11008, 4096, 1, 1, 2 * 2 * 64 * 11008),       # a folded norm: tile kernel, both products of two K splits through scratch
+    (64, 12288, 4096, 0, 1, 3 * 64 * 12288),
+    (300, 14336, 4096, 0, 0, 0)])
+def test_scratch_is_that_of_the_kernel_that_runs(m, n, k, pair, norms, floats):
+    assert hip.lib().bigdl_gemm_lowbit_workspace(m, n, k, k, QT, pair, norms, 0) == floats
 
 
 @pytest.mark.gpu

@@ -4,6 +4,7 @@
 #include "gemm_kernel.h"
 #include "gemm_rows_kernel.h"
 #include "gemm_rows.h"
+#include <math.h>
 #include <stdlib.h>
 
 namespace bigdl {
@@ -177,6 +178,7 @@ static int dispatch(const GemmArgs& a, int qtype, int bm, int bn, int mblocks, h
   }
 }
 
+// K splits of the tile kernel.  mblocks: number of row blocks (dense: ceil(M / bm))
 static void plan(int mblocks, int bn, int N, int K, int* splitk, int* kt_per_split) {
   const int KT = (K + 127) / 128;
   const int blocks = ((N + bn - 1) / bn) * mblocks;
@@ -190,33 +192,9 @@ static void plan(int mblocks, int bn, int N, int K, int* splitk, int* kt_per_spl
   *splitk = (KT + per - 1) / per;
 }
 
-// Number of K splits the launch below will use for this shape (the caller provides splitk * M * N floats of
-// workspace when it is > 1).  mblocks: number of row blocks (dense: ceil(M / bm)).
-extern "C" int bigdl_gemm_lowbit_bm(int M);
 static int pick_bn(int M) {
   (void)M;
   return 128;
-}
-
-// Which products the few-row kernel (gemm_rows_kernel.h) takes from the tile kernel, one MI355X, tile kernel with its reduce
-// launch -> few-row kernel, us.  Llama-2-7B shapes, sym_int4: 64 rows qkv 25.3 -> 16.9, o 16.6 -> 12.4, gate / up 32.8 -> 23.7,
-// down 22.2 -> 23 (the one equal: K = 11008 makes x the larger stream, it runs in two K splits); 32 rows 19.8 -> 12.1,
-// 12.8 -> 9.0, 26.2 -> 17.6, 17.7 -> 17.8.  Llama-3-8B shapes, asym_int4, in blocks of 64 rows: 128 rows qkv 35.4 -> 16.8, o
-// 20.5 -> 13.8, gate / up 78 -> 70, down 38.7 -> 35.7; 192 rows 45.9 -> 30.3, 35.3 -> 25.1, 116 -> 93, 82.7 -> 68.7; 256 rows
-// 39.3 -> 31.0, 27.5 -> 25.0, 150 -> 117, and down 62.6 -> 69.5: every block reads all of x and of the weight, so four blocks
-// of a long K are the tile kernel's.
-static bool takes_rows_kernel(int ldx, int M, int N, int K, int qtype, bool pair, RowsPlan* plan) {
-  if (M > 256 || (M > 192 && K > 8192) || !is_t16(qtype) || !rows_ok(nullptr, ldx)) return false;
-  *plan = rows_plan(M, N, K, qtype, pair, !pair && M <= 64);
-  return true;
-}
-static int launch_rows(const GemmArgs& a, int qtype, const RowsPlan& p, hipStream_t stream) {
-  RowsArgs b = {};
-  b.x = a.x; b.w = a.w; b.w2 = a.w2; b.out = a.out; b.partial = a.partial; b.bias = a.bias; b.bias2 = a.bias2; b.residual = a.residual;
-  b.M = a.M; b.N = a.N; b.K = a.K; b.ldx = a.ldx; b.ldo = a.ldo; b.act = a.act; b.out_type = a.out_type;
-  b.splitk = p.splitk; b.kt_per_split = p.kt_per_split;
-  const int rc = rows_launch(b, p, qtype, stream);
-  return rc != 0 || p.splitk == 1 ? rc : launch_reduce(a, stream);
 }
 
 extern "C" int bigdl_gemm_lowbit_bm(int M) {
@@ -226,6 +204,71 @@ extern "C" int bigdl_gemm_lowbit_bm(int M) {
   // 64-row blocks keep two or more wavefronts per SIMD (170 VGPRs): measured 10-40 % faster than 128-row blocks at
   // every M between 64 and 1024 on the Llama-2-7B projection shapes
   return 64;
+}
+
+// What a product of 33 to 256 rows takes on the tile kernel and on the few-row kernel (gemm_rows_kernel.h), in us: the chooser
+// below compares the two.  Both models were fitted to 3300 products on one MI355X: 11 formats, 18 shapes from 512 x 2048 to
+// 8192 x 28672 and 10 gate / up pairs, 33 to 256 rows, weights from memory.  They are exact to 8 %, worst cases 25 %.
+struct DenseCost {
+  float kt;                 // tile kernel: us per k-tile of a workgroup with a CU of its own
+  float two, three;         // ... times this with 2 / 3 workgroups a CU (asym_int4 and nearly all wider formats: one after the other)
+  float rows_kt;            // few-row kernel: us per k-tile and 16-column weight tile of a workgroup
+};
+static DenseCost dense_cost(int qtype) {
+  switch (qtype) {
+    case Q_SYM_INT4: return {0.65f, 1.36f, 2.65f, 0.067f};
+    case Q_ASYM_INT4: case Q_WOQ_INT4: return {0.90f, 2.0f, 3.3f, 0.072f};
+    case Q_FP4: return {0.77f, 1.4f, 2.5f, 0.075f};
+    case Q_NF4: return {1.21f, 1.2f, 2.1f, 0.085f};
+    case Q_SYM_INT5: return {0.97f, 1.45f, 2.4f, 0.091f};
+    case Q_ASYM_INT5: return {1.54f, 1.95f, 3.15f, 0.097f};
+    case Q_FP6: return {1.23f, 1.85f, 2.9f, 0.12f};
+    case Q_SYM_INT8: return {0.78f, 1.85f, 3.2f, 0.095f};
+    case Q_FP8_E4M3: return {0.93f, 1.85f, 3.05f, 0.103f};
+    default: return {0.73f, 1.85f, 3.3f, 0.092f};        // fp8_e5m2
+  }
+}
+static double tile_us(const DenseCost& c, int M, int N, int K, bool pair) {
+  const int bm = bigdl_gemm_lowbit_bm(M), bn = pick_bn(M), mblocks = (M + bm - 1) / bm * (pair ? 2 : 1);
+  int sk, per;
+  plan(mblocks, bn, N, K, &sk, &per);
+  const double load = (double)((N + bn - 1) / bn) * mblocks * sk / gemv_cu_count();       // workgroups a CU
+  double turns = 1.0;
+  // (a second workgroup on a few CUs only is hardly felt)
+  if (load > 3.0) turns = c.three + 0.25 + 1.13 * (load - 3.0);
+  else if (load > 2.0) turns = c.three + 0.25 * (load - 2.0);
+  else if (load > 1.0) turns = 1.0 + (c.two - 1.0) * fmin(1.0, 8.0 * (load - 1.0)) + 0.25 * (load - 1.0);
+  double us = 12.3 + per * c.kt * turns;
+  if (sk > 1 || pair) us += 3.2e-6 * sk * M * N * (pair ? 2 : 1) - 4.2;     // slabs and the reduce launch; the kernel's epilogue shrinks
+  return us;
+}
+static double rows_us(const DenseCost& c, const RowsPlan& p, int K, int qtype, bool pair) {
+  const double ktiles = (double)((K + 127) / 128) / p.splitk;
+  // (fp6: the pair's kernel spills)
+  const double tiles_us = p.nt * (pair ? 2 : 1) * c.rows_kt * (pair && qtype == Q_FP6 ? 1.15 : 1.0);
+  return (lo_bits_of(qtype) == 8 ? 5.0 : 6.2) + p.turns * ktiles * (0.112 + tiles_us) + 4.2 * (p.turns - 1) + (p.splitk > 1 ? 3.5 : 0.0);
+}
+
+// Which products the few-row kernel takes from the tile kernel: those where it is expected to be ahead by what the estimates may be
+// off in its favour.  Measured, tile -> few-row kernel, us.  Taken: 64 rows sym_int4 12288 x 4096 25.3 -> 16.9, 4096 x 4096 16.3 ->
+// 11.9, pair of 11008 x 4096 33.4 -> 23.1, 4096 x 11008 22.0 -> 20.9 (two K splits); 128 rows asym_int4 6144 x 4096 35.6 -> 16.5, pair
+// of 14336 x 4096 77.5 -> 68.2.  Left: a grid that is no whole number of turns or many of them (sym_int4 14336 x 4096: 64 rows
+// 27.0 -> 28.4, 128 rows 32.0 -> 42.7, 256 rows 45.9 -> 72.1; 32000 x 4096, 64 rows 34.6 -> 43.6), and a long K that x crosses whole in
+// every workgroup (1024 x 14336: 65 rows 16.2 -> 26.9; 4096 x 11008, 192 rows 40.4 -> 54.3).  Up to 32 rows it was never behind.
+static bool takes_rows_kernel(int ldx, int M, int N, int K, int qtype, bool pair, RowsPlan* plan) {
+  if (M > 256 || !is_t16(qtype) || !rows_ok(nullptr, ldx)) return false;
+  *plan = rows_plan(M, N, K, qtype, pair, !pair && M <= 64);
+  if (M <= 32) return true;
+  const DenseCost c = dense_cost(qtype);
+  return rows_us(c, *plan, K, qtype, pair) < tile_us(c, M, N, K, pair) * (pair ? 0.90 : 0.94);
+}
+static int launch_rows(const GemmArgs& a, int qtype, const RowsPlan& p, hipStream_t stream) {
+  RowsArgs b = {};
+  b.x = a.x; b.w = a.w; b.w2 = a.w2; b.out = a.out; b.partial = a.partial; b.bias = a.bias; b.bias2 = a.bias2; b.residual = a.residual;
+  b.M = a.M; b.N = a.N; b.K = a.K; b.ldx = a.ldx; b.ldo = a.ldo; b.act = a.act; b.out_type = a.out_type;
+  b.splitk = p.splitk; b.kt_per_split = p.kt_per_split;
+  const int rc = rows_launch(b, p, qtype, stream);
+  return rc != 0 || p.splitk == 1 ? rc : launch_reduce(a, stream);
 }
 
 // The kernel a call runs on and the fp32 scratch it needs: one place for the launches and for the size that callers ask for

@@ -8,7 +8,7 @@ struct RowsArgs;
 struct RowsPlan {
   int mt, nt;               // 16-row tiles of x and 16-column weight tiles of a workgroup
   int splitk, kt_per_split;
-  double us;                // what the planner expects
+  int turns;                // of the grid over the CUs, one workgroup each
 };
 RowsPlan rows_plan(int M, int N, int K, int qtype, bool pair, bool may_split);
 // x the kernel can address: 16-byte rows, a row block within a gigabyte (its offsets are 32 bits)

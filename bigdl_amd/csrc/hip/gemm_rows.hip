@@ -23,7 +23,8 @@ RowsPlan rows_plan(int M, int N, int K, int qtype, bool pair, bool may_split) {
   const int cus = gemv_cu_count();
   const double wrow = (double)tile_bytes(qtype) * KT * (pair ? 2 : 1);
   const double xall = (double)(M < 16 * mt ? M : 16 * mt) * K * 2;
-  RowsPlan best = {mt, 0, 1, KT, 0.0};
+  RowsPlan best = {mt, 0, 1, KT, 1};
+  double best_us = 0.0;
   for (int nt = 1; nt <= 4; ++nt) {
     if (!rows_has(mt, nt, pair)) continue;
     for (int sk = 1; sk <= (may_split ? 4 : 1); ++sk) {
@@ -31,9 +32,13 @@ RowsPlan rows_plan(int M, int N, int K, int qtype, bool pair, bool may_split) {
       const int per = (KT + sk - 1) / sk;
       if ((KT + per - 1) / per != sk) continue;
       const int blocks = (tiles + nt - 1) / nt * sk * mblocks;
-      const double turns = (double)((blocks + cus - 1) / cus);
+      const int turns = (blocks + cus - 1) / cus;
+      // (what compares the tilings with each other; the time itself is rows_us of gemm_lowbit.hip)
       const double us = turns * (xall / sk / 57e3 + nt * wrow / sk / 20e3) + (sk > 1 ? 6.0 : 0.0);
-      if (best.nt == 0 || us < best.us) best = {mt, nt, sk, per, us};
+      if (best.nt == 0 || us < best_us) {
+        best = {mt, nt, sk, per, turns};
+        best_us = us;
+      }
     }
   }
   return best;

@@ -54,14 +54,26 @@ def test_every_call_allocates_its_own_scratch(monkeypatch, call):
 
 
 @pytest.mark.parametrize("m,n,k,pair,norms,floats", [
-    (200, 14336, 4096, 1, 0, 0),                       # a pair on the few-row kernel is combined in registers
-    (150, 11008, 4096, 1, 0, 0), (64, 11008, 4096, 1, 0, 0), (64, 4096, 4096, 0, 0, 0),
+    (64, 11008, 4096, 1, 0, 0), (17, 14336, 4096, 1, 0, 0),      # a pair on the few-row kernel is combined in registers
+    (64, 4096, 4096, 0, 0, 0),
     (64, 4096, 11008, 0, 0, 2 * 64 * 4096),            # the few-row kernel's two K splits
     (64, 11008, 4096, 1, 1, 2 * 2 * 64 * 11008),       # a folded norm: tile kernel, both products of two K splits through scratch
     (64, 12288, 4096, 0, 1, 3 * 64 * 12288),
     (300, 14336, 4096, 0, 0, 0)])
 def test_scratch_is_that_of_the_kernel_that_runs(m, n, k, pair, norms, floats):
     assert hip.lib().bigdl_gemm_lowbit_workspace(m, n, k, k, QT, pair, norms, 0) == floats
+
+
+@pytest.mark.parametrize("name,m,n,k,tile", [
+    # slower on the few-row kernel by a tenth and more: narrow outputs of a long K, grids of several turns
+    ("sym_int4", 65, 1024, 14336, True), ("asym_int4", 128, 2048, 14336, True), ("sym_int8", 128, 1024, 8192, True),
+    ("sym_int4", 192, 4096, 11008, True),
+    # faster there by a tenth and more; unsplit, so without scratch, which the tile kernel would need at these sizes
+    ("sym_int4", 64, 4096, 4096, False), ("asym_int4", 128, 4096, 4096, False), ("sym_int8", 128, 2048, 2048, False),
+    ("sym_int4", 128, 1024, 4096, False), ("nf4", 192, 2048, 5632, False), ("fp6", 65, 6144, 4096, False)])
+def test_kernel_of_a_product(name, m, n, k, tile):
+    floats = hip.lib().bigdl_gemm_lowbit_workspace(m, n, k, k, Q.ggml_tensor_qtype[name], 0, 0, 0)
+    assert (floats > 0) == tile
 
 
 @pytest.mark.gpu

@@ -982,9 +982,18 @@ static inline int gemv_cu_count() {
 // the CU-resident form stages them once per CU.  Llama-2-7B decode step at 1024-token context, one MI355X, tile form ->
 // CU form: 2 rows 1.94 -> 2.23 ms, 4: 2.56 -> 2.75, 6: 3.33 -> 3.25, 7: 3.45 -> 3.52, 8: 3.25 -> 3.01, 9: 3.84 -> 3.45,
 // 10: 3.88 -> 3.59, 12: 4.03 -> 3.75, 14: 4.15 -> 4.10 (16 rows of K = 4096 no longer fit next to the partial sums).
-// Hence 8 .. 13 rows by default (bigdl_gemv_cu_rows / BIGDL_GEMV_CU_ROWS=lo,hi change it).
+// Hence 8 .. 13 rows by default (bigdl_gemv_cu_rows / BIGDL_GEMV_CU_ROWS=lo,hi change it).  Most products of those rows have
+// gone to the few-row kernel since (takes_rows_kernel in gemv_lowbit.hip); the widest single ones and the products that take
+// attention partials or a LayerNorm stay.
 inline int& gemv_cu_rows_lo() { static int v = 8; return v; }
 inline int& gemv_cu_rows_hi() { static int v = 13; return v; }
+// Products with fewer tiles than CUs stay in the tile form: nothing to share, and half-empty workgroups of 16 wavefronts
+// (TinyLlama's 2048-wide products lose 10 - 20 % of a decode step in the CU form).  So do short reductions: with K = 2048 each
+// of the 16 wavefronts gets one k-tile per output tile and nothing to overlap (same model: gate / up alone in the CU form
+// still cost 14 %)
+static inline bool gemv_cu_form(int M, int N, int K) {
+  return M >= gemv_cu_rows_lo() && M <= gemv_cu_rows_hi() && (N + 15) / 16 >= gemv_cu_count() && (K >> 7) >= 24;
+}
 
 // the leading arguments (preloaded into scalar registers, see the kernel) and the whole
 #define GEMV_ARGS(a) (a).x, (a).w, (a).w2, (a).gamma, (a).slot_expert, (a).M, (a).N, (a).K, (a).ldx, a
@@ -1024,12 +1033,7 @@ static int launch_x(const GemvArgs& a_in, hipStream_t st) {
   if constexpr (MT == 1) {
     // CU-resident form: one workgroup per CU streams all its output tiles (see the kernel's comment).  Needs x and
     // at least one tile's partial sums in LDS.
-    // (products with fewer tiles than CUs stay in the tile form: nothing to share, and half-empty workgroups of 16
-    // wavefronts: TinyLlama's 2048-wide products lose 10 - 20 % of a decode step in the CU form)
-    // ... and so do short reductions: with K = 2048 each of the 16 wavefronts gets one k-tile per output tile and nothing to
-    // overlap (same model: gate / up alone in the CU form still cost 14 %)
-    const bool cu_rows = a.M >= gemv_cu_rows_lo() && a.M <= gemv_cu_rows_hi() && (a.N + 15) / 16 >= gemv_cu_count() &&
-                         (a.K >> 7) >= 24;
+    const bool cu_rows = gemv_cu_form(a.M, a.N, a.K);
     if ((GEMV_CU_ENABLE || cu_rows) && a.slot_expert == nullptr &&
         (GEMV_CU_ENABLE == 1 || cu_rows || (a.N + 15) / 16 <= gemv_cu_count())) {
       const int n_tiles = (a.N + 15) / 16;

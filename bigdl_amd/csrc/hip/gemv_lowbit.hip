@@ -37,33 +37,48 @@ static int dispatch(const GemvArgs& a, int qtype, hipStream_t stream) {
   }
 }
 
-// Whether up to 16 rows take the few-row kernel (gemm_rows_kernel.h) instead of the skinny one.  The skinny kernel gives a
-// workgroup 16 columns, and every workgroup stages all rows of x; the few-row kernel shares x among up to 64 columns but
-// needs more registers a column, so it streams a single row slower (qkv 12288 x 4096 sym_int4, 1 row: 8.7 us against
-// 10.8).  What decides is therefore the x that a CU stages, rows x column tiles per CU, counted 1.5 times for a gate / up
-// pair, whose skinny form fits fewer workgroups on a CU.  Measured pairs (skinny / few-row, us): at 6: qkv 6144 x 4096
-// asym_int4 4 rows 11.6 / 11.7; at 8: pair 5632 x 2048 4 rows 9.6 / 9.7; at 12: 6144 x 4096 8 rows 13.5 / 11.7, 4096 x 4096
-// 12 rows 8.0 / 8.0; at 18: 12288 x 4096 6 rows 14.7 / 11.7; at 21: pair 14336 x 4096 4 rows 23.6 / 19.8; at 63: pair
-// 14336 x 4096 asym_int4 12 rows 50.6 / 23.5.  Two exceptions: x that no longer fits the LDS of the skinny kernel (4096 x 14336
-// asym_int4, 8 rows: 25.9 / 18.2) goes over at once, and the CU-resident form of 8 to 11 rows keeps the widest products (32000
-// x 4096 asym_int4, 8 rows: 25.7 / 29.7; 12 rows: 31.8 / 29.7).
-static bool takes_rows_kernel(const GemvArgs& a) {
+// Whether 3 to 16 rows take the few-row kernel (gemm_rows_kernel.h) instead of the skinny one.  The skinny kernel gives a
+// workgroup 16 columns, and every workgroup stages all rows of x; the few-row kernel shares x among up to 64 columns, but a
+// workgroup of it fills a CU, so its time hardly depends on the rows and goes up with every turn of its grid.  What decides
+// is the x that a CU stages for the skinny kernel: load = rows x column tiles per CU (a pair counts 1.5 times), and
+// fit = how many of its workgroups find room for their x in a CU's LDS.  The lines below lie where, in 4200 products of 11
+// formats and 35 shapes on one MI355X, the few-row kernel was last behind by more than 4 % (the worst is now 3 %).  Skinny /
+// few-row, us.  One turn, fit 2 and more: sym_int4 8192 x 4096 7 rows (load 28) 10.3 / 11.9, 11008 x 4096 6 rows (32) 11.3 / 10.7;
+// fit 1: 4096 x 11008 6 rows (12) 11.5 / 12.9, 7 rows (14) 14.2 / 12.9; pair of 11008 x 4096, 5 rows (40) 17.3 / 16.2.  Two turns,
+// which fewer rows do not fill: pair of 28672 x 8192 3 rows 50.8 / 75.4, 14 rows 88 / 56.  The CU-resident form (8 to 13 rows)
+// keeps the widest single products (32000 x 4096 asym_int4, 8 rows: 23.5 / 27.7) and no pair (14336 x 4096, 8 rows: 23.0 / 17.8).
+static bool takes_rows_kernel(const GemvArgs& a, int qtype, const RowsPlan& plan) {
   if (a.M > 16 || a.M < 3 || a.att_ws != nullptr || a.ln_c1 != nullptr || !rows_ok(a.x, a.ldx)) return false;
+  const bool pair = a.w2 != nullptr, bits8 = lo_bits_of(qtype) == 8, planes2 = hi_bits_of(qtype) > 0;
   const int tiles = (a.N + 15) / 16, cus = gemv_cu_count();
-  const size_t xbytes = (size_t)a.M * ((a.K + 127) / 128 * 128 + XTAIL + XPAD) * 2;
-  if (xbytes > GEMV_XLDS_LIMIT_FEW_ROWS) return true;
-  if (tiles > 4 * cus && a.M >= 8 && a.M <= 11) return false;
-  return (int64_t)a.M * tiles * (a.w2 != nullptr ? 3 : 2) >= 20ll * cus;
+  const double load = (double)a.M * tiles / cus * (pair ? 3 : 2);
+  const int fit = (int)(160 * 1024 / (((a.K + 127) / 128 * 128 + XTAIL + XPAD) * 2 * (size_t)a.M + 9 * 1024));     // 9: partial sums
+  const bool resident = gemv_cu_form(a.M, a.N, a.K);
+  if (pair && resident) return true;
+  if (plan.turns > 1)
+    return fit == 0 || a.M >= 14 || (a.M <= 7 && fit == 1 && !(pair && bits8)) || (!pair && a.M >= 8 && !resident && load >= 160);
+  if (fit == 0) return a.K > 8192 || load >= 17;
+  if (pair) return load >= (a.M >= 14 ? 49 : fit == 1 ? 13 : bits8 ? 43 : 37);
+  if (planes2) return load >= 57;                    // (a tile of two planes costs the few-row kernel more)
+  if (resident && qtype == Q_FP8_E5M2) return load >= 50;
+  return load >= (fit == 1 ? 13 : 34);
 }
 
-static int launch_rows(const GemvArgs& a, int qtype, hipStream_t stream) {
-  const RowsPlan p = rows_plan(a.M, a.N, a.K, qtype, a.w2 != nullptr, false);
+static int launch_rows(const GemvArgs& a, int qtype, const RowsPlan& p, hipStream_t stream) {
   RowsArgs b = {};
   b.x = a.x; b.w = a.w; b.w2 = a.w2; b.out = a.out; b.bias = a.bias; b.bias2 = a.bias2; b.residual = a.residual;
   b.gamma = a.gamma; b.gamma_offset = a.gamma_offset; b.eps = a.eps;
   b.M = a.M; b.N = a.N; b.K = a.K; b.ldx = a.ldx; b.ldo = a.ldo; b.act = a.act; b.out_type = a.out_type;
   b.splitk = p.splitk; b.kt_per_split = p.kt_per_split;
   return rows_launch(b, p, qtype, stream);
+}
+
+// 1: bigdl_gemv_lowbit runs a plain product of this shape (pair: with w2) on the few-row kernel, 0: on the skinny one
+extern "C" int bigdl_gemv_lowbit_few_rows(int M, int N, int K, int qtype, int pair) {
+  GemvArgs a = {};
+  a.M = M; a.N = N; a.K = K; a.ldx = (K + 7) / 8 * 8; a.w2 = pair ? &a : nullptr;
+  qtype = t16_kernel_qtype(qtype);
+  return M > 0 && N > 0 && K > 0 && is_t16(qtype) && takes_rows_kernel(a, qtype, rows_plan(M, N, K, qtype, pair != 0, false));
 }
 
 // Returns 0 on success; negative = rejected on the host before any launch.
@@ -102,7 +117,10 @@ static int gemv_lowbit_impl(const void* x, const void* w, const void* w2, void* 
   a.att_qlen = att_qlen; a.att_rows_alloc = att_rows_alloc;
   a.ln_c1 = ln_c1; a.ln_c2 = ln_c2; a.ln2_c1 = ln2_c1; a.ln2_c2 = ln2_c2;
   a.slot_expert = nullptr; a.slot_scale = nullptr; a.n_total = 0; a.slot_xdiv = 1; a.n_slots = 0; a.slot_cat = 0;
-  if (is_t16(qtype) && takes_rows_kernel(a)) return launch_rows(a, qtype, stream);
+  if (is_t16(qtype)) {
+    const RowsPlan p = rows_plan(a.M, a.N, a.K, qtype, a.w2 != nullptr, false);
+    if (takes_rows_kernel(a, qtype, p)) return launch_rows(a, qtype, p, stream);
+  }
   return dispatch(a, qtype, stream);
 }
 

@@ -98,10 +98,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_prompt_kernel(GemmArgs a
   const int nmb = (a.M + BM - 1) / BM, nnb = (a.N + BNO - 1) / BNO;
 
   // XCD-aware tile order: blocks b and b + 8 share an L2; consecutive tile ids go to one XCD (bijective also when the grid
-  // is not a multiple of 8).  Tile ids run through bands of BAND row blocks, column by column: the 32 workgroups of an XCD
-  // then share 4 x panels (16 bits an element) and 8 weight panels (4 - 8 bits) instead of reading 32 x panels each for
-  // itself.  7700 rows: 14336 x 4096 pair 1697 -> 1655 us, 6144 x 4096 351 -> 342 us; bands of 2 and 8 within 1 %.
-  constexpr int BAND = 4;
+  // is not a multiple of 8).  Where the tiles of a product outnumber the CUs, the ids run through bands of four row blocks,
+  // column by column: the 32 workgroups of an XCD then share 4 x panels (16 bits an element) and 8 weight panels (4 - 8 bits)
+  // instead of reading 32 x panels each for itself.  7700 rows: 14336 x 4096 pair 1697 -> 1655 us, 6144 x 4096 351 -> 342 us; bands
+  // of 2 and 8 within 1 %.  Fewer tiles run down the columns: in bands 1024 x 4096 at 2048 rows took 38.3 us instead of 33.8,
+  // 2048 x 2048 28.6 instead of 27.2, 4096 x 11008 183 instead of 177.
+  const int BAND = nmb * nnb > 256 ? 4 : nmb;
   int tid;
   {
     const int nblk = gridDim.x, b = blockIdx.x, q = nblk >> 3, rr = nblk & 7, xcd = b & 7;
@@ -117,10 +119,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_prompt_kernel(GemmArgs a
   const T16Planes pl = t16_planes(a.w, QT, a.N, a.K);
   const T16Planes pl2 = t16_planes(pair ? a.w2 : a.w, QT, a.N, a.K);
 
-  // ---- x tile (32-bit byte offsets from one scalar base: M * ldx < 2^31).  Every wavefront stages rows of its own row half (the half it reads fragments from, so that the two
-  // halves of the workgroup may run out of step); instruction p fills rows 8 (p WN + wn) .. + 7 of the half; lane i
-  // brings the 16 bytes that belong in slot i % 8 of row i / 8, i.e. k slot (i % 8) ^ (i / 8) of that row (rows past the
-  // block re-read its last row: never stored)
+  // ---- x tile (32-bit byte offsets from one scalar base: M * ldx < 2^31).  Every wavefront stages rows of its own row half
+  // (the half it reads fragments from, so that the two halves of the workgroup may run out of step); instruction p fills
+  // rows 8 (p WN + wn) .. + 7 of the half; lane i brings the 16 bytes that belong in slot i % 8 of row i / 8, i.e. k slot
+  // (i % 8) ^ (i / 8) of that row (rows past the block re-read its last row: never stored)
   uint32_t xoff[NA];
 #pragma unroll
   for (int p = 0; p < NA; ++p) {

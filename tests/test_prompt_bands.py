@@ -42,6 +42,26 @@ def test_every_tile_of_every_band(hip, cfg, m, splitk):
     assert ((out.double().cpu() - ref).abs() <= 2.0 ** -10 * (xd.abs() @ w.abs().t()) + 2.0 ** -10 * ref.abs()).all()
 
 
+# either side of 256 tiles, where the order changes from whole columns to bands: 4 x 64 and 4 x 65 tiles, 11 x 24 (the last band
+# three blocks high), 5 x 52 of 256 columns; as a pair 9 x 29 tiles of 64 columns
+@pytest.mark.parametrize("cfg,m,n,pair", [(2, 500, 8192, False), (2, 500, 8200, False), (2, 1400, 3072, False), (0, 1030, 13312, False),
+                                          (2, 1100, 1856, True)])
+def test_more_tiles_than_compute_units(hip, cfg, m, n, pair):
+    k, qt = 256, Q.SYM_INT4
+    dev, w = _weight(n, k, qt, 1)
+    x, xd = _x(m, k)
+    hip.gemm_prompt_force(cfg, 1)
+    ref = xd @ w.t()
+    bound = 2.0 ** -10 * (xd.abs() @ w.abs().t()) + 2.0 ** -10 * ref.abs()
+    if pair:
+        out = hip.gemm_prompt_pair(x, dev, dev, qt, n, k, act="relu")
+        # the same product twice, so f(y) = max(y, 0) * y: twice the product's error times |y|, and one more rounding
+        bound, ref = 2 * bound * (ref.abs() + bound) + 2.0 ** -10 * ref * ref, ref.relu() * ref
+    else:
+        out = hip.gemm_prompt(x, dev, qt, n, k)
+    assert ((out.double().cpu() - ref).abs() <= bound + 1e-6).all()
+
+
 @pytest.mark.parametrize("cfg,m", [(2, 130), (2, 700), (0, 1030), (1, 257)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_both_halves_of_a_pair_write_their_rows(hip, cfg, m, dtype):

@@ -118,9 +118,8 @@ constexpr float P8_SCALE = 256.0f;     // probabilities are carried as 256 p (an
 // the fp16 cache needs 258 us for twice the bytes).  The MFMA k index <-> head channel assignment is free as long as
 // Q and K agree, so lane group g takes channels [16 (g + 4 c2), +16) of a row for the k-steps 2 c2 and 2 c2 + 1.
 //
-// The leading arguments arrive in scalar registers (build flag, see gemv_kernel.h): with them q and the length are requested
-// at once, and the rest of the arguments returns along with the length.  One sequence, 4 kv heads of 64, 50 keys: 8 steps of
-// 8 layers 1692 -> 1671 us, with the rows of q requested ahead of the append.
+// The leading arguments arrive in scalar registers (build flag, see gemv_kernel.h): the length is requested at once, and the
+// rest of the arguments returns along with it.
 template <int D, bool FP8, int RT, int KW, bool I4, int NWT = ATT_NW, int MINW = 1>
 __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* p_past, _Float16* p_qkv, int p_ld, int p_q_total,
                                                                      int p_splits, int p_Hq, int p_Hkv, int p_nchunk, int p_gchunk,
@@ -139,10 +138,13 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
   constexpr bool F8M = FP8 && WIDE;
   static_assert(!WIDE || (FP8 && D % 128 == 0), "16-byte fragments: e5m2 cache, rotate-half partner in k-step c + DC/2");
   static_assert(!I4 || (!FP8 && KW == 32), "int4 caches: 32 keys per wavefront");
-  constexpr bool AHEAD = RT == 1 && D <= 128;              // registers for a second block's fragments
-  // fp16 caches: 12 sequences x 8 heads x 1900 keys 1.5 us a launch; e5m2 caches gain nothing (64 x 32 x 1000: 125 us either
-  // way), and the 32-key e5m2 form's 8-byte pieces would not make whole 64 bytes
-  constexpr bool FOLD = !I4 && !FP8;
+  // The next block in flight and the new value stored with its block: one row tile and heads of 96 and 128 channels.  fp16 caches,
+  // 12 sequences x 8 heads of 128: 6000 keys 113 -> 102 us, 1900 keys in two ranges 20.5 -> 20.0.  Heads of 256 spilled (500 keys
+  // 20.7 -> 25.0), two row tiles and heads of 64 lost a wavefront per SIMD (20 query heads a group 11.3 -> 12.0; 64: 500 keys
+  // 7.8 -> 8.2).  e5m2 caches take the block in flight up to 128 channels, in the 32-key form (heads of 64, 1900 keys in
+  // eight ranges 5.7 -> 5.3), and store a value a byte at a time: folded, its 8-byte pieces would not make whole 64 bytes.
+  constexpr bool AHEAD = RT == 1 && D <= 128 && (D > 64 || FP8);
+  constexpr bool FOLD = AHEAD && !I4 && !FP8;
   // first head channel of this lane's 8 values in k-step c.  int4: lane group g owns the D/4 contiguous channels
   // (D/4) g .. of a key, one load of D/8 bytes
   auto chan = [](int c, int g) {
@@ -218,7 +220,7 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
     if constexpr (FP8) return dec_e5m2(p.x, p.y);
     else return p;
   };
-  // A decode step's one new value row is not stored element by element (V^T: two bytes in each of D lines, which memory
+  // FOLD: a decode step's one new value row is not stored element by element (V^T: two bytes in each of D lines, which memory
   // turns into a read and a write of every line) but put into the fragments of the block that holds its key, by the
   // wavefront that multiplies that block, and stored with them: 64 whole bytes a channel.
   const bool fold_v = FOLD && a.q_total == 1 && (a.rope != nullptr || a.rot == 0) && a.q_off == 0 && past < a.Lmax;
@@ -242,15 +244,15 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
       *(uint4v*)(vc + ((int64_t)(16 * d + rr) * a.Lmax + kb) * 2 + 16 * g) = out;
     }
   };
-  // The rows of q are requested ahead of the append: they depend on nothing it does, and its barrier waits for its stores
   half8 qraw[RT][DC];
-#pragma unroll
-  for (int t = 0; t < RT; ++t) {
+  // (rows past the last one read it again: a branch around the loads took longer, one sequence of 32 heads, 40 keys 6.5 us
+  // instead of 6.1)
+  auto load_q = [&](int t) {
     const int row = min(16 * t + rr, rows - 1);
     const _Float16* qp = a.qkv + (int64_t)(b * a.q_total + a.q_off + row / Gc) * a.ld + (hkv * G + g0 + row % Gc) * D;
 #pragma unroll
     for (int c = 0; c < DC; ++c) qraw[t][c] = *(const half8*)(qp + chan(c, g));
-  }
+  };
   // ---- fused RoPE(k) + KV append for the new tokens that fall into this workgroup's key range ----
   if (a.rope != nullptr || a.rot == 0) {
     if (a.q_off == 0) {
@@ -340,6 +342,7 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
         }
       }
     }
+    __syncthreads();   // appended keys become visible to the whole workgroup (vmcnt(0) + barrier)
   }
 
   const float qscale = a.softcap > 0.0f ? a.scale : a.scale * 1.4426950408889634f;
@@ -360,6 +363,7 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
     const int tokidx = b * a.q_total + tok;
     lim[t] = valid ? past + tok : -1;
     lo_lim[t] = (a.window > 0 && valid) ? max(0, past + tok - a.window + 1) : 0;
+    load_q(t);
     float qv[DC][8];
 #pragma unroll
     for (int c = 0; c < DC; ++c)
@@ -446,8 +450,6 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
       }
     }
   }
-
-  if (a.rope != nullptr || a.rot == 0) __syncthreads();   // appended keys become visible to the whole workgroup (vmcnt(0) + barrier)
 
   float m_run[RT], l_run[RT];
   float4v o[RT][DT];
@@ -676,11 +678,6 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
   } else {
     int kb = blk0 * ATT_KEYS + wave * KW;
     const int end = min(blk1 * ATT_KEYS, kv_len);
-    auto last_words = [&](Frag& f) {
-      if constexpr (FOLD)
-        if (fold_v && past >= kb && past < kb + KW)      // (the newest key: only ever in a wavefront's last block)
-          fold_new_value(kb, [&](int d, int w) -> uint32_t& { return ((uint32_t*)&f.v[d])[w]; });
-    };
     if constexpr (AHEAD) {
       // The next block is requested before this one is worked on; the asm statement keeps the compiler from moving the
       // loads back to their use.  (The last block stands alone: a request under a condition would make every block wait
@@ -694,14 +691,15 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
           process(kb, RawK{}, RawV{}, cur);
           cur = nxt;
         }
-        last_words(cur);
+        if constexpr (FOLD)
+          if (fold_v && past >= kb && past < kb + KW)      // (the newest key: only ever in a wavefront's last block)
+            fold_new_value(kb, [&](int d, int w) -> uint32_t& { return ((uint32_t*)&cur.v[d])[w]; });
         process(kb, RawK{}, RawV{}, cur);
       }
     } else {
       for (; kb < end; kb += ATT_KEYS) {
         Frag cur;
         load_frag(kb, cur);
-        last_words(cur);
         process(kb, RawK{}, RawV{}, cur);
       }
     }

@@ -33,3 +33,12 @@ def test_a_new_value_row_lands_in_its_column_only(d, hkv, group, splits, past):
     ref = (p @ vt[..., :past + 1].double().transpose(-1, -2)).reshape(b, hq * d)
     # probabilities and outputs of 2^-11 on values up to about 4
     torch.testing.assert_close(out.cpu().double(), ref, rtol=2e-3, atol=4e-3)
+
+
+# the most query heads a kv head that one row tile holds, one more (two tiles), heads of 256, and more heads a kv head than a
+# workgroup takes (two workgroups a kv head append the same row)
+@pytest.mark.parametrize("d,hkv,group", [(128, 2, 16), (96, 1, 17), (128, 1, 32), (128, 1, 40), (256, 2, 2)])
+@pytest.mark.parametrize("splits", [1, 2])
+@pytest.mark.parametrize("past", [0, 31, 256, 511])
+def test_groups_of_many_heads_and_wide_heads(d, hkv, group, splits, past):
+    test_a_new_value_row_lands_in_its_column_only(d, hkv, group, splits, past)

@@ -59,16 +59,6 @@ struct AttnArgs {
 constexpr float NEG_BIG = -1.0e30f;
 constexpr int ATT_NW = 8;          // wavefronts per workgroup
 
-template <bool FP8>
-__device__ __forceinline__ half8 load_kv8(const void* base, int64_t elem_off) {
-  if constexpr (FP8) {
-    const uint2v w = *(const uint2v*)((const uint8_t*)base + elem_off);
-    return dec_e5m2(w.x, w.y);
-  } else {
-    return *(const half8*)((const _Float16*)base + elem_off);
-  }
-}
-
 // 8 int4 values of one cache word -> fp16 (nibble k -> element 2k, nibble k + 4 -> element 2k + 1), minus the zero
 // point 8, times `sc`.  0x6400 | n is the fp16 number 1024 + n.
 __device__ __forceinline__ half8 dq_i4(uint32_t w, _Float16 sc) {

@@ -128,12 +128,14 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
   constexpr bool F8M = FP8 && WIDE;
   static_assert(!WIDE || (FP8 && D % 128 == 0), "16-byte fragments: e5m2 cache, rotate-half partner in k-step c + DC/2");
   static_assert(!I4 || (!FP8 && KW == 32), "int4 caches: 32 keys per wavefront");
-  // The next block in flight and the new value stored with its block: one row tile and heads of 96 and 128 channels.  fp16 caches,
-  // 12 sequences x 8 heads of 128: 6000 keys 113 -> 102 us, 1900 keys in two ranges 20.5 -> 20.0.  Heads of 256 spilled (500 keys
-  // 20.7 -> 25.0), two row tiles and heads of 64 lost a wavefront per SIMD (20 query heads a group 11.3 -> 12.0; 64: 500 keys
-  // 7.8 -> 8.2).  e5m2 caches take the block in flight up to 128 channels, in the 32-key form (heads of 64, 1900 keys in
-  // eight ranges 5.7 -> 5.3), and store a value a byte at a time: folded, its 8-byte pieces would not make whole 64 bytes.
-  constexpr bool AHEAD = RT == 1 && D <= 128 && (D > 64 || FP8);
+  // The next block in flight, the new value stored with its block and q requested ahead of the append: one row tile and heads of
+  // up to 128 channels.  fp16 caches, 12 sequences x 8 heads of 128, 6000 keys: 113 -> 102 us.  In a step, where caches are cold:
+  // 8 layers of 4 kv heads of 64, 4 tokens, 45 / 1900 keys 849 -> 840 / 930 -> 922 us; 16 sequences x 32 heads of 128, 1000 keys
+  // 1168 -> 1141 (2 layers).  Heads of 256 spilled (4 layers of 8 heads, 500 keys 676 -> 753 us), two row tiles lost registers (20
+  // query heads a group, 1900 keys 11.3 -> 12.1 us a launch).  e5m2 caches take the block in flight (in the 32-key form: 4 heads of
+  // 64, 1900 keys in eight ranges 5.7 -> 5.3 us) and nothing else: their 8-byte pieces would not make whole 64 bytes of a
+  // value column, and q ahead cost 4 - 8 % with several key ranges (14.0 -> 15.1 us).
+  constexpr bool AHEAD = RT == 1 && D <= 128;
   constexpr bool FOLD = AHEAD && !I4 && !FP8;
   // first head channel of this lane's 8 values in k-step c.  int4: lane group g owns the D/4 contiguous channels
   // (D/4) g .. of a key, one load of D/8 bytes
@@ -243,6 +245,10 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
 #pragma unroll
     for (int c = 0; c < DC; ++c) qraw[t][c] = *(const half8*)(qp + chan(c, g));
   };
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int t = 0; t < RT; ++t) load_q(t);
+  }
   // ---- fused RoPE(k) + KV append for the new tokens that fall into this workgroup's key range ----
   if (a.rope != nullptr || a.rot == 0) {
     if (a.q_off == 0) {
@@ -332,7 +338,7 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
         }
       }
     }
-    __syncthreads();   // appended keys become visible to the whole workgroup (vmcnt(0) + barrier)
+    if constexpr (!FOLD) __syncthreads();   // appended keys become visible to the whole workgroup (vmcnt(0) + barrier)
   }
 
   const float qscale = a.softcap > 0.0f ? a.scale : a.scale * 1.4426950408889634f;
@@ -353,7 +359,7 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
     const int tokidx = b * a.q_total + tok;
     lim[t] = valid ? past + tok : -1;
     lo_lim[t] = (a.window > 0 && valid) ? max(0, past + tok - a.window + 1) : 0;
-    load_q(t);
+    if constexpr (!FOLD) load_q(t);
     float qv[DC][8];
 #pragma unroll
     for (int c = 0; c < DC; ++c)
@@ -441,6 +447,8 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
     }
   }
 
+  // (with q requested ahead its rotation stands between the stores and the wait for them)
+  if (FOLD && (a.rope != nullptr || a.rot == 0)) __syncthreads();
   float m_run[RT], l_run[RT];
   float4v o[RT][DT];
 #pragma unroll

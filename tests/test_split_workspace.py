@@ -76,17 +76,20 @@ def test_kernel_of_a_product(name, m, n, k, tile):
     assert (floats > 0) == tile
 
 
-@pytest.mark.parametrize("name,m,n,k,pair,few", [
+@pytest.mark.parametrize("name,m,n,k,pair,norm,few", [
     # two turns of the few-row kernel for three to seven rows (28672 x 8192, 3 rows: 50.8 -> 75.4 us), small x, narrow outputs
-    ("sym_int4", 3, 28672, 8192, 1, 0), ("sym_int8", 4, 28672, 8192, 0, 0), ("sym_int4", 3, 32000, 4096, 0, 0),
-    ("sym_int4", 4, 11008, 4096, 0, 0), ("sym_int4", 8, 5632, 2048, 0, 0), ("sym_int4", 7, 8192, 4096, 0, 0),
-    ("sym_int4", 12, 32000, 4096, 0, 0), ("fp6", 16, 4096, 4096, 0, 0), ("sym_int8", 4, 14336, 4096, 1, 0),
+    ("sym_int4", 3, 28672, 8192, 1, 0, 0), ("sym_int8", 4, 28672, 8192, 0, 0, 0), ("sym_int4", 3, 32000, 4096, 0, 0, 0),
+    ("sym_int4", 4, 11008, 4096, 0, 0, 0), ("sym_int4", 8, 5632, 2048, 0, 0, 0), ("sym_int4", 7, 8192, 4096, 0, 0, 0),
+    ("sym_int4", 12, 32000, 4096, 0, 0, 0), ("fp6", 16, 4096, 4096, 0, 0, 0), ("sym_int8", 4, 14336, 4096, 1, 0, 0),
     # and where it is ahead by a tenth and more
-    ("asym_int4", 12, 6144, 4096, 0, 1), ("asym_int4", 12, 14336, 4096, 1, 1), ("asym_int4", 12, 4096, 14336, 0, 1),
-    ("sym_int4", 16, 32000, 4096, 0, 1), ("sym_int4", 8, 11008, 4096, 1, 1), ("fp6", 16, 11008, 4096, 0, 1),
-    ("sym_int4", 7, 4096, 11008, 0, 1), ("sym_int8", 6, 8192, 8192, 0, 1), ("sym_int4", 2, 32000, 4096, 1, 0)])
-def test_kernel_of_a_few_rows(name, m, n, k, pair, few):
-    assert hip.lib().bigdl_gemv_lowbit_few_rows(m, n, k, Q.ggml_tensor_qtype[name], pair) == few
+    ("asym_int4", 12, 6144, 4096, 0, 0, 1), ("asym_int4", 12, 14336, 4096, 1, 0, 1), ("asym_int4", 12, 4096, 14336, 0, 0, 1),
+    ("sym_int4", 16, 32000, 4096, 0, 0, 1), ("sym_int4", 8, 11008, 4096, 1, 0, 1), ("fp6", 16, 11008, 4096, 0, 0, 1),
+    ("sym_int4", 7, 4096, 11008, 0, 0, 1), ("sym_int8", 6, 8192, 8192, 0, 0, 1), ("sym_int4", 2, 32000, 4096, 1, 0, 0),
+    # with a folded norm
+    ("asym_int4", 12, 32000, 4096, 0, 1, 1), ("asym_int4", 8, 128256, 4096, 0, 1, 0), ("sym_int4", 8, 5632, 2048, 0, 1, 1),
+    ("sym_int4", 5, 8192, 4096, 0, 1, 0), ("sym_int4", 5, 14336, 4096, 1, 1, 1), ("fp4", 3, 28672, 8192, 1, 1, 0)])
+def test_kernel_of_a_few_rows(name, m, n, k, pair, norm, few):
+    assert hip.lib().bigdl_gemv_lowbit_few_rows(m, n, k, Q.ggml_tensor_qtype[name], pair, norm) == few
 
 
 @pytest.mark.gpu

@@ -1,6 +1,6 @@
-// Dequant-fused MFMA GEMM for mid-size row counts on gfx950:  y[M,N] = f(x[M,K] . dequant(W)[N,K]^T) beyond the
-// few-row kernel's limits (256 rows, 192 where K > 8192) or where the prompt kernel does not take K,
-// and its grouped (mixture-of-experts) form where every 64/128-row block of x belongs to one expert.
+// Dequant-fused MFMA GEMM for mid-size row counts on gfx950:  y[M,N] = f(x[M,K] . dequant(W)[N,K]^T) for the products of
+// 33 - 256 rows where the few-row kernel is not expected to be ahead (dense_cost in gemm_lowbit.hip), for more rows where the
+// prompt kernel does not take K, and its grouped (mixture-of-experts) form where every 64/128-row block of x belongs to one expert.
 //
 // Takes the place of the reference's closed xe_linear.forward_new for prefill-sized inputs / xe_batch.batch_forward
 // (call sites python/llm/src/ipex_llm/transformers/low_bit_linear.py:657-668) and of the per-expert Python loop of
@@ -415,8 +415,8 @@ static int gemm_launch_mt(const GemmArgs& a, int mblocks, hipStream_t st) {
 }
 
 // bm: rows per block (64 / 128); bn: columns per block (128).  64-column blocks were measured too (more workgroups
-// streaming weights at few rows): slower or equal on every Llama-2-7B projection shape.  Up to 64 rows the dense products
-// run on gemm_rows_kernel.h.
+// streaming weights at few rows): slower or equal on every Llama-2-7B projection shape.  Up to 32 rows the dense products
+// run on gemm_rows_kernel.h, more where gemm_lowbit.hip expects it to be ahead.
 template <int QT>
 static int gemm_launch_qt(const GemmArgs& a, int bm, int bn, int mblocks, hipStream_t st) {
   if (bn != 128) return -4;

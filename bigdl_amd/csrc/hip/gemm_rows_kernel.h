@@ -16,8 +16,8 @@
 //  * Loads are ordered by hand (rows_issued) and go through buffer descriptors: scalar offsets instead of 64-bit vector
 //    addresses (which spilled), and what lies outside x or past the last k-tile costs no memory access.
 // Measured, one MI355X, sym_int4, us, before (skinny kernel up to 16 rows, tile kernel above) -> this kernel: qkv 12288 x 4096 at
-// 12 / 32 / 64 rows 15.3 -> 11.6, 19.8 -> 12.1, 25.3 -> 16.9; gate / up 11008 x 4096 28.1 -> 17.7, 26.2 -> 17.6, 32.8 -> 23.7; o
-// 4096 x 4096 8.0 -> 8.0, 12.8 -> 9.0, 16.6 -> 12.4; down 4096 x 11008 16.5 -> 13.5, 17.7 -> 17.8, 22.2 -> 23 (two K splits).
+// 12 / 32 / 64 rows 15.3 -> 11.6, 19.8 -> 12.1, 25.3 -> 16.9; gate / up 11008 x 4096 28.1 -> 17.7, 26.2 -> 17.6, 33.4 -> 23.1; o
+// 4096 x 4096 8.0 -> 8.0, 12.8 -> 9.0, 16.3 -> 11.9; down 4096 x 11008 16.5 -> 13.5, 17.7 -> 17.8, 22.0 -> 20.9 (two K splits).
 // A decode step of 12 sequences of a Llama-3-8B-shaped q4_k model with 1900 keys each: 156 -> 108 us a layer.
 #pragma once
 #include "gemv_kernel.h"

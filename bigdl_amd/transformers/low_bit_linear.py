@@ -28,14 +28,14 @@ from ..utils.common import invalidInputError
 
 TORCH_LINEAR_THRESHOLD = int(os.getenv("BIGDL_LLM_LINEAR_THRESHOLD", "512"))
 # row-count policy of the products of tiled weights on the GPU: up to GEMV_MAX_ROWS rows ``gemv_lowbit`` (one or two rows on
-# the skinny kernel, more on the few-row kernel), up to GEMM_MAX_ROWS ``gemm_lowbit`` (few-row kernel, beyond its limits the
-# tile kernel), above the prompt kernel
+# the skinny kernel, more there or on the few-row kernel), up to GEMM_MAX_ROWS ``gemm_lowbit`` (few-row or tile kernel, whichever
+# is expected to be faster), above the prompt kernel
 GEMV_MAX_ROWS = int(os.getenv("BIGDL_GEMV_MAX_ROWS", "16"))
 GEMM_MAX_ROWS = 256
 # q6_k weights stay in their checkpoint blocks on the GPU.  Up to this many fp16 (or fp32) rows are multiplied from the blocks
 # (csrc/hip/gemm_rows_kernel.h, up to four gemv_q6k.hip).  The weight is expanded for a dense product above, for bf16
-# activations, whose range fp16 does not have, and where autograd, a transform or a trace looks on.  Kernel time of 4096 x 11008,
-# one MI355X, expanded -> from the blocks: 1 row 100 -> 17 us, 64 rows 107 -> 34, 128 rows 127 -> 47.
+# activations (that product keeps their range; the fp16 copies that the tiled formats multiply do not), and where autograd, a
+# transform or a trace looks on.  Kernel time of 4096 x 11008, one MI355X, expanded -> from the blocks: 1 row 100 -> 17 us, 64 rows 107 -> 34, 128 rows 127 -> 47.
 Q6K_MAX_ROWS = 128
 # forward of frozen low-bit linears inside a training step on the fused prompt GEMM (fp16 copy of the activations)
 # instead of dequantize + dense product

@@ -317,13 +317,15 @@ def _half(x):
     return x.to(torch.float16)
 
 
+_wrapped, _tracing = torch._C._functorch.is_functorch_wrapped_tensor, torch._C._get_tracing_state
+_dispatch_modes, _PLAIN = torch._C._len_torch_dispatch_stack, (torch.Tensor, torch.nn.Parameter)
+
+
 def _observed(x):
     """Whether anything but the caller looks at what is done to x: autograd in either direction, a function transform, a trace,
     a dispatch mode.  Those see PyTorch operations, not launches of this package."""
-    return (type(x) not in (torch.Tensor, torch.nn.Parameter) or (x.requires_grad and torch.is_grad_enabled())
-            or torch._C._functorch.is_functorch_wrapped_tensor(x) or torch._C._get_tracing_state() is not None
-            or torch._C._len_torch_dispatch_stack() > 0
-            or (fwad._current_level >= 0 and fwad.unpack_dual(x).tangent is not None))
+    return ((x.requires_grad and torch.is_grad_enabled()) or _wrapped(x) or _tracing() is not None or _dispatch_modes() > 0
+            or type(x) not in _PLAIN or (fwad._current_level >= 0 and fwad.unpack_dual(x).tangent is not None))
 
 
 def lowbit_matmul(x_2d: torch.Tensor, weight: FP4Params, out_features: int, for_training: bool = False) -> torch.Tensor:
@@ -353,12 +355,12 @@ def lowbit_matmul(x_2d: torch.Tensor, weight: FP4Params, out_features: int, for_
                 xh = xh.contiguous()
             return lowbit_rows(xh, weight.data, weight.qtype, n, k, out_dtype=x_2d.dtype)
         if (weight.qtype == Q.Q6_K and 0 < m <= Q6K_MAX_ROWS and dt in (torch.float16, torch.float32) and not for_training
-                and weight.data.data_ptr() % 4 == 0 and not _observed(x_2d)):
-            xh = x_2d.to(torch.float16)
+                and weight.data_ptr() % 4 == 0 and not _observed(x_2d)):
+            xh = x_2d if dt == torch.float16 else x_2d.to(torch.float16)
             if xh.stride(1) != 1 or xh.stride(0) % 8 or xh.data_ptr() % 16:
                 xh = xh.contiguous()
-            raw = weight.data.view(torch.uint8) if weight.data.dtype != torch.uint8 else weight.data
-            return hip.gemm_q6k(xh, raw, n, k, out_dtype=x_2d.dtype)
+            raw = weight.data
+            return hip.gemm_q6k(xh, raw if raw.dtype == torch.uint8 else raw.view(torch.uint8), n, k, out_dtype=dt)
         cdt = x_2d.dtype if x_2d.dtype in (torch.float16, torch.bfloat16) else torch.float16
         w = dequant_weight(weight, cdt)
         xc = x_2d.to(cdt)

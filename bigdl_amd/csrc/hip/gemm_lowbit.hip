@@ -249,16 +249,20 @@ static double rows_us(const DenseCost& c, const RowsPlan& p, int K, int qtype, b
   return (lo_bits_of(qtype) == 8 ? 5.0 : 6.2) + p.turns * ktiles * (0.112 + tiles_us) + 4.2 * (p.turns - 1) + (p.splitk > 1 ? 3.5 : 0.0);
 }
 
-// Which products the few-row kernel takes from the tile kernel: those where it is expected to be ahead by what the estimates may be
-// off in its favour.  Measured, tile -> few-row kernel, us.  Taken: 64 rows sym_int4 12288 x 4096 25.3 -> 16.9, 4096 x 4096 16.3 ->
-// 11.9, pair of 11008 x 4096 33.4 -> 23.1, 4096 x 11008 22.0 -> 20.9 (two K splits); 128 rows asym_int4 6144 x 4096 35.6 -> 16.5, pair
-// of 14336 x 4096 77.5 -> 68.2.  Left: a grid that is no whole number of turns or many of them (sym_int4 14336 x 4096: 64 rows
-// 27.0 -> 28.4, 128 rows 32.0 -> 42.7, 256 rows 45.9 -> 72.1; 32000 x 4096, 64 rows 34.6 -> 43.6), and a long K that x crosses whole in
-// every workgroup (1024 x 14336: 65 rows 16.2 -> 26.9; 4096 x 11008, 192 rows 40.4 -> 54.3).  Up to 32 rows it was never behind.
+// Which products the few-row kernel takes from the tile kernel: above 64 rows those where it is expected to be ahead by what the
+// estimates may be off in its favour.  Measured alone, tile -> few-row kernel, us.  Taken: 64 rows sym_int4
+// 12288 x 4096 25.3 -> 16.9, 4096 x 4096 16.3 -> 11.9, pair of 11008 x 4096 33.4 -> 23.1, 4096 x 11008 22.0 -> 20.9 (two K splits);
+// 128 rows asym_int4 6144 x 4096 35.6 -> 16.5, pair of 14336 x 4096 77.5 -> 68.2.  Left: a grid of many turns (sym_int4 14336 x 4096:
+// 128 rows 32.0 -> 42.7, 256 rows 45.9 -> 72.1; 152064 x 3584, 64 rows 106 -> 172), and a long K that x crosses whole in every
+// workgroup (1024 x 14336: 65 rows 16.2 -> 26.9; 4096 x 11008, 192 rows 40.4 -> 54.3).
+// Up to 64 rows a pass runs nearly all of its products on the few-row kernel, and a lone product on the tile kernel between them is
+// slower than alone (its code is out of the caches by then): in decode steps of 64 sequences the head of 32000 x 4096 (three
+// turns) took 38 us alone on the tile kernel, 42 among other tile products and 47 among few-row products, where the few-row
+// kernel takes 43; 4 steps of 3 layers 2802 and 2783 us.  So up to three turns stay there.  Up to 32 rows it was never behind.
 static bool takes_rows_kernel(int ldx, int M, int N, int K, int qtype, bool pair, RowsPlan* plan) {
   if (M > 256 || !is_t16(qtype) || !rows_ok(nullptr, ldx)) return false;
   *plan = rows_plan(M, N, K, qtype, pair, !pair && M <= 64);
-  if (M <= 32) return true;
+  if (M <= 32 || (M <= 64 && plan->turns <= 3)) return true;
   const DenseCost c = dense_cost(qtype);
   return rows_us(c, *plan, K, qtype, pair) < tile_us(c, M, N, K, pair) * (pair ? 0.90 : 0.94);
 }

@@ -70,7 +70,9 @@ def test_scratch_is_that_of_the_kernel_that_runs(m, n, k, pair, norms, floats):
     ("sym_int4", 192, 4096, 11008, True),
     # faster there by a tenth and more; unsplit, so without scratch, which the tile kernel would need at these sizes
     ("sym_int4", 64, 4096, 4096, False), ("asym_int4", 128, 4096, 4096, False), ("sym_int8", 128, 2048, 2048, False),
-    ("sym_int4", 128, 1024, 4096, False), ("nf4", 192, 2048, 5632, False), ("fp6", 65, 6144, 4096, False)])
+    ("sym_int4", 128, 1024, 4096, False), ("nf4", 192, 2048, 5632, False), ("fp6", 65, 6144, 4096, False),
+    # up to 64 rows and three turns, whatever the estimates say
+    ("sym_int4", 33, 14336, 4096, False), ("sym_int4", 64, 14336, 4096, False), ("sym_int8", 64, 12288, 4096, False)])
 def test_kernel_of_a_product(name, m, n, k, tile):
     floats = hip.lib().bigdl_gemm_lowbit_workspace(m, n, k, k, Q.ggml_tensor_qtype[name], 0, 0, 0)
     assert (floats > 0) == tile

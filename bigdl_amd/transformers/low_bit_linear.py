@@ -35,7 +35,8 @@ GEMM_MAX_ROWS = 256
 # q6_k weights stay in their checkpoint blocks on the GPU.  Up to this many fp16 (or fp32) rows are multiplied from the blocks
 # (csrc/hip/gemm_rows_kernel.h, up to four gemv_q6k.hip).  The weight is expanded for a dense product above, for bf16
 # activations (that product keeps their range; the fp16 copies that the tiled formats multiply do not), and where autograd, a
-# transform or a trace looks on.  Kernel time of 4096 x 11008, one MI355X, expanded -> from the blocks: 1 row 100 -> 17 us, 64 rows 107 -> 34, 128 rows 127 -> 47.
+# transform or a trace looks on.  4096 x 11008, one MI355X, expanded -> from the blocks: a call with 1 row 85 -> 13 us; kernel time
+# with 64 rows 107 -> 34, with 128 rows 127 -> 47.
 Q6K_MAX_ROWS = 128
 # forward of frozen low-bit linears inside a training step on the fused prompt GEMM (fp16 copy of the activations)
 # instead of dequantize + dense product

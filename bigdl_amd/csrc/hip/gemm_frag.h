@@ -1,0 +1,19 @@
+// Interface of the product on x in fragment order (gemm_frag.hip) for the entry points that share it.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace bigdl {
+struct FragArgs;
+struct FragPlan {
+  int mt, ns;               // 16-row tiles of x and 16-column weight tiles of a workgroup (pair form: ns / 2 of each weight); ns 0: none
+  int splitk, kt_per_split;
+  double us;                // what it is expected to take with its reduce launch, without the pass that orders x
+};
+static inline double frag_pack_us(int M, int K) { return 3.4 + 1e-6 * M * K; }
+FragPlan frag_plan(int M, int N, int K, int qtype, bool pair, bool may_split);
+// halves of x in fragment order
+static inline int64_t frag_halves(int M, int K) { return (int64_t)((K + 127) / 128) * 4 * ((M + 15) / 16) * 512; }
+int frag_pack(const void* x, void* xp, int M, int K, int ldx, bool bf16, hipStream_t st);
+int frag_launch(const FragArgs& a, const FragPlan& p, int qtype, hipStream_t st);
+}  // namespace bigdl

@@ -1,0 +1,128 @@
+// Planner and entry points of the low-bit product on x in fragment order (kernel: gemm_frag_kernel.h; one instantiation unit per
+// weight format: gemm_frag_inst_*.hip), and the pass that puts x into that order.
+#include "gemm_frag_kernel.h"
+#include "gemm_frag.h"
+
+namespace bigdl {
+#define FRAG_FORMATS(X)                                                                                                     \
+  X(Q_SYM_INT4, sym_int4) X(Q_ASYM_INT4, asym_int4) X(Q_WOQ_INT4, woq_int4) X(Q_FP4, fp4) X(Q_NF4, nf4)                     \
+  X(Q_SYM_INT5, sym_int5) X(Q_ASYM_INT5, asym_int5) X(Q_FP6, fp6) X(Q_SYM_INT8, sym_int8) X(Q_FP8_E4M3, fp8_e4m3)           \
+  X(Q_FP8_E5M2, fp8_e5m2)
+#define FRAG_DECLARE(id, name) int gemm_frag_launch_##name(const FragArgs& a, int mt, int ns, hipStream_t st);
+FRAG_FORMATS(FRAG_DECLARE)
+
+// x [M, K] (fp16, or bf16: rounded to fp16) -> fragments of 16 rows x 32 columns, [k / 32][row / 16][lane][8 halves]: lane (g, r)
+// of a fragment holds row r, columns 8 g .. 8 g + 7.  Rows past M and columns past K are zero.  One wavefront a fragment: 16
+// pieces of 64 bytes in, 1 KiB out.
+__global__ __launch_bounds__(256) void frag_pack_kernel(const void* x, _Float16* xp, int M, int K, int ldx, int mt_all, int frags, int bf16) {
+  const int f = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (f >= frags) return;
+  const int k = f / mt_all * 32 + (lane >> 4) * 8, m = f % mt_all * 16 + (lane & 15);
+  half8 v = {0, 0, 0, 0, 0, 0, 0, 0};
+  if (m < M && k < K) {
+    const uint4v raw = *(const uint4v*)((const uint16_t*)x + (int64_t)m * ldx + k);
+    v = __builtin_bit_cast(half8, raw);
+    if (bf16) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[2 * i] = (_Float16)__uint_as_float(raw[i] << 16);
+        v[2 * i + 1] = (_Float16)__uint_as_float(raw[i] & 0xffff0000u);
+      }
+    }
+  }
+  *(half8*)(xp + ((int64_t)f * 64 + lane) * 8) = v;
+}
+int frag_pack(const void* x, void* xp, int M, int K, int ldx, bool bf16, hipStream_t st) {
+  const int mt = (M + 15) / 16, frags = (K + 127) / 128 * 4 * mt;
+  hipLaunchKernelGGL(frag_pack_kernel, dim3((frags + 3) / 4), dim3(256), 0, st, x, (_Float16*)xp, M, K, ldx, mt, frags, (int)bf16);
+  return HIP_CHECK_LAUNCH();
+}
+
+// Time of a tiling in us: a + turns * (turn + k-tiles * (x * mt + w * ns + xw * mt * ns)) + part * (million partial sums written),
+// turns of a grid with one workgroup a CU.  Fitted per format to 45000 launches on one MI355X: 15 shapes from 1024 x 2048 to
+// 32000 x 4096 and pairs, 33 to 512 rows, every tiling, 1 / 2 / 4 splits of K, weights from memory.  Exact to 12 %, worst cases
+// 25 %; the tiling chosen by it was on average 1 % slower than the fastest, at worst 26 %.
+struct FragCost { float a, turn, x, w, xw, part; };
+static FragCost frag_cost(int qtype) {
+  switch (qtype) {
+    case Q_SYM_INT4: return {3.71f, 2.80f, 0.0090f, 0.0084f, 0.0134f, 2.5f};
+    case Q_ASYM_INT4: case Q_WOQ_INT4: return {3.86f, 3.00f, 0.0099f, 0.0193f, 0.0125f, 2.3f};
+    case Q_FP4: return {3.84f, 2.63f, 0.0026f, 0.0213f, 0.0145f, 2.6f};
+    case Q_NF4: return {3.98f, 2.40f, 0.0f, 0.0341f, 0.0151f, 2.7f};
+    case Q_SYM_INT5: return {4.15f, 2.43f, 0.0f, 0.0419f, 0.0154f, 2.6f};
+    case Q_ASYM_INT5: return {4.24f, 2.83f, 0.0f, 0.0451f, 0.0153f, 2.5f};
+    case Q_FP6: return {3.72f, 2.71f, 0.0f, 0.0746f, 0.0146f, 2.9f};
+    case Q_SYM_INT8: return {3.69f, 3.19f, 0.0125f, 0.0267f, 0.0118f, 2.3f};
+    case Q_FP8_E4M3: return {3.71f, 3.27f, 0.0064f, 0.0336f, 0.0136f, 2.4f};
+    default: return {3.71f, 3.10f, 0.0171f, 0.0258f, 0.0098f, 2.2f};        // fp8_e5m2
+  }
+}
+
+FragPlan frag_plan(int M, int N, int K, int qtype, bool pair, bool may_split) {
+  const int KT = (K + 127) / 128, tiles = (N + 15) / 16, mt_all = (M + 15) / 16;
+  FragPlan best = {0, 0, 1, KT, 1e30};
+  if (frag_halves(M, K) * 2 >= ROWS_OUT) return best;
+  const FragCost c = frag_cost(qtype);
+  const int cus = gemv_cu_count();
+  for (int mt = 3; mt <= 8; ++mt) {
+    const int mblocks = (mt_all + mt - 1) / mt;
+    for (int ns = 2; ns <= 8; ++ns) {
+      if (!frag_has(mt, ns) || (pair && (ns & 1))) continue;
+      const int64_t blocks = (int64_t)((tiles + (pair ? ns / 2 : ns) - 1) / (pair ? ns / 2 : ns)) * mblocks;
+      for (int sk = 1; sk <= (may_split ? 4 : 1); sk *= 2) {
+        const int per = (KT + sk - 1) / sk;
+        if (sk > 1 && (KT < 8 * sk || (KT + per - 1) / per != sk)) break;
+        const double turns = (double)((blocks * sk + cus - 1) / cus);
+        double us = c.a + turns * (c.turn + per * (c.x * mt + c.w * ns + c.xw * mt * ns));
+        if (sk > 1) us += 4.0 + 1e-6 * sk * M * N * (c.part + 1.0);     // partial sums, and the launch that adds them up
+        if (us < best.us) best = {mt, ns, sk, per, us};
+      }
+    }
+  }
+  return best;
+}
+
+int frag_launch(const FragArgs& a_in, const FragPlan& p, int qtype, hipStream_t st) {
+  FragArgs a = a_in;
+  const uintptr_t at = (uintptr_t)a.out | (uintptr_t)a.residual;
+  a.vec = (a.N & 3) == 0 && (a.ldo & 3) == 0 && (at & (a.out_type == OUT_F32 ? 15 : 7)) == 0;
+  switch (qtype) {
+#define FRAG_CASE(id, name) case id: return gemm_frag_launch_##name(a, p.mt, p.ns, st);
+    FRAG_FORMATS(FRAG_CASE)
+    default: return -2;
+  }
+}
+}  // namespace bigdl
+
+using namespace bigdl;
+
+extern "C" int64_t bigdl_frag_halves(int M, int K) { return frag_halves(M, K); }
+
+// K % 8 == 0, rows of x 16-byte aligned; x_type: OUT_F16 or OUT_BF16; xp: bigdl_frag_halves halves, 16-byte aligned
+extern "C" int bigdl_frag_pack(const void* x, void* xp, int64_t halves, int M, int K, int ldx, int x_type, hipStream_t stream) {
+  if (M <= 0 || K <= 0 || (K & 7) || (ldx & 7) || ((uintptr_t)x & 15) || ((uintptr_t)xp & 15) || halves < frag_halves(M, K)) return -1;
+  if (x_type != OUT_F16 && x_type != OUT_BF16) return -3;
+  return frag_pack(x, xp, M, K, ldx, x_type == OUT_BF16, stream);
+}
+
+// y = act(x W^T + bias) [* (x W2^T + bias2)] [+ residual] of x in fragment order, on an explicit tiling.  workspace: fp32,
+// splitk * M * N (twice that with w2) when split: the partial sums stay there, nothing is written to out.  For tests and
+// measurements; the public products choose by themselves.
+extern "C" int bigdl_gemm_frag(const void* xp, int64_t halves, const void* w, const void* w2, void* out, const void* bias, const void* bias2,
+                               const void* residual, float* workspace, int64_t workspace_floats, int M, int N, int K, int ldo,
+                               int qtype, int act, int out_type, int mt, int ns, int splitk, hipStream_t stream) {
+  qtype = t16_kernel_qtype(qtype);
+  if (M <= 0 || N <= 0 || K <= 0 || (K & 31) || ((uintptr_t)xp & 15) || ((uintptr_t)w & 15) || (w2 && ((uintptr_t)w2 & 15)) || splitk < 1 ||
+      halves < frag_halves(M, K) || frag_halves(M, K) * 2 >= ROWS_OUT)
+    return -1;
+  if (out_type < 0 || out_type > 2) return -3;
+  const int KT = (K + 127) / 128;
+  FragPlan p = {mt, ns, splitk, (KT + splitk - 1) / splitk, 0.0};
+  p.splitk = (KT + p.kt_per_split - 1) / p.kt_per_split;
+  if (p.splitk > 1 && (workspace == nullptr || workspace_floats < (w2 ? 2 : 1) * (int64_t)p.splitk * M * N)) return -5;
+  FragArgs a = {};
+  a.xp = (const _Float16*)xp; a.w = w; a.w2 = w2; a.out = out; a.partial = workspace; a.bias = bias; a.bias2 = bias2; a.residual = residual;
+  a.M = M; a.N = N; a.K = K; a.mt_all = (M + 15) / 16; a.ldo = ldo; a.act = act; a.out_type = out_type;
+  a.splitk = p.splitk; a.kt_per_split = p.kt_per_split;
+  return frag_launch(a, p, qtype, stream);
+}

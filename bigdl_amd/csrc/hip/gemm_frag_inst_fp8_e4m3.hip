@@ -1,0 +1,5 @@
+// Instantiation unit of the product on x in fragment order for one weight format.
+#include "gemm_frag_kernel.h"
+namespace bigdl {
+int gemm_frag_launch_fp8_e4m3(const FragArgs& a, int mt, int ns, hipStream_t st) { return gemm_frag_launch_qt<Q_FP8_E4M3>(a, mt, ns, st); }
+}  // namespace bigdl

@@ -1,0 +1,5 @@
+// Instantiation unit of the product on x in fragment order for one weight format.
+#include "gemm_frag_kernel.h"
+namespace bigdl {
+int gemm_frag_launch_woq_int4(const FragArgs& a, int mt, int ns, hipStream_t st) { return gemm_frag_launch_qt<Q_WOQ_INT4>(a, mt, ns, st); }
+}  // namespace bigdl

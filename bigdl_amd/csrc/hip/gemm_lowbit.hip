@@ -4,6 +4,8 @@
 #include "gemm_kernel.h"
 #include "gemm_rows_kernel.h"
 #include "gemm_rows.h"
+#include "gemm_frag_kernel.h"
+#include "gemm_frag.h"
 #include <math.h>
 #include <stdlib.h>
 
@@ -19,6 +21,7 @@ int gemm_launch_fp6(const GemmArgs& a, int bm, int bn, int mblocks, hipStream_t 
 int gemm_launch_sym_int8(const GemmArgs& a, int bm, int bn, int mblocks, hipStream_t st);
 int gemm_launch_fp8_e4m3(const GemmArgs& a, int bm, int bn, int mblocks, hipStream_t st);
 int gemm_launch_fp8_e5m2(const GemmArgs& a, int bm, int bn, int mblocks, hipStream_t st);
+double prompt_us(int M, int N, int K, int qtype, bool pair);        // gemm_prompt.hip
 
 // out[m][n] = epilogue(sum_s partial[s][m][n]); pair form: act(first) * second; optional folded RMSNorm factor of the
 // row (row_ssq) and sum of squares of the rows written (ssq_out, for the norm folded into the next product).
@@ -275,19 +278,52 @@ static int launch_rows(const GemmArgs& a, int qtype, const RowsPlan& p, hipStrea
   return rc != 0 || p.splitk == 1 ? rc : launch_reduce(a, stream);
 }
 
+// Which products the kernel on x in fragment order takes: those where it and the pass that orders x are expected to be ahead of
+// the faster of the others, by 3 % for what the estimates may be off.  Measured, us, before -> it + that pass: sym_int4
+// 4096 x 4096 at 77 / 256 rows 15.2 -> 9.6 + 3.7, 23.1 -> 14.3 + 4.5; asym_int4 pair of 14336 x 4096 at 77 rows 67.6 -> 32.1 + 3.7; sym_int8
+// 4672 x 4544 at 203 rows 38.7 -> 22 + 4.3.  Left: up to 64 rows most products (12288 x 4096, 64 rows 17.2 -> 15.1 + 3.7), large grids
+// of many rows (14336 x 4096, 256 rows 43.0 -> 47.0 + 4.5).  x in bf16 needs that pass anyway (in place of its conversion).
+enum XKind { X_ROWS = 0, X_ROWS_BF16 = 1, X_FRAGMENTS = 2 };
+static bool takes_frag_kernel(int ldx, int M, int N, int K, int qtype, bool pair, int x_kind, FragPlan* plan) {
+  if (M <= 32 || !is_t16(qtype)) return false;
+  *plan = frag_plan(M, N, K, qtype, pair, !pair);
+  if (plan->ns == 0) return false;
+  if (x_kind == X_FRAGMENTS) return true;
+  double other;
+  if (M > 256 && K >= 256 && (K & 127) == 0) {
+    if (M > 512) return false;                         // (what the estimates cover)
+    other = prompt_us(M, N, K, qtype, pair);
+  } else {
+    const DenseCost c = dense_cost(qtype);
+    const int rows = M < 256 ? M : 256;                // (callers pass more rows 256 at a time)
+    RowsPlan r;
+    other = takes_rows_kernel(ldx, rows, N, K, qtype, pair, &r) ? rows_us(c, r, K, qtype, pair) : tile_us(c, rows, N, K, pair);
+    other *= (M + 255) / 256;
+  }
+  return plan->us + (x_kind == X_ROWS ? frag_pack_us(M, K) : 0.0) < 0.97 * other;
+}
+
 // The kernel a call runs on and the fp32 scratch it needs: one place for the launches and for the size that callers ask for
 struct DensePlan {
+  bool frag;                // kernel on x in fragment order (scratch: x in that order, partial sums)
+  FragPlan f;
   bool rows;                // few-row kernel; otherwise the tile kernel
   RowsPlan r;
   int bm, mblocks, splitk, kt_per_split;
   bool partial;             // the results pass through scratch and the reduce kernel
-  int64_t floats;
+  int64_t xfloats, floats;  // scratch of x / in all
 };
 // fold_norm, ssq_out: the tile kernel's forms of gemm_lowbit_ex
-static DensePlan dense_plan(int M, int N, int K, int ldx, int qtype, bool pair, bool fold_norm, bool ssq_out) {
+static DensePlan dense_plan(int M, int N, int K, int ldx, int qtype, bool pair, bool fold_norm, bool ssq_out, int x_kind) {
   DensePlan p = {};
-  p.rows = !fold_norm && !ssq_out && takes_rows_kernel(ldx, M, N, K, qtype, pair, &p.r);
-  if (p.rows) {
+  p.frag = !fold_norm && !ssq_out && takes_frag_kernel(ldx, M, N, K, qtype, pair, x_kind, &p.f);
+  p.rows = !p.frag && !fold_norm && !ssq_out && takes_rows_kernel(ldx, M, N, K, qtype, pair, &p.r);
+  if (p.frag) {
+    p.splitk = p.f.splitk;
+    p.kt_per_split = p.f.kt_per_split;
+    p.partial = p.splitk > 1;
+    p.xfloats = x_kind == X_FRAGMENTS ? 0 : frag_halves(M, K) / 2;
+  } else if (p.rows) {
     p.splitk = p.r.splitk;
     p.kt_per_split = p.r.kt_per_split;
     p.partial = p.splitk > 1;
@@ -297,13 +333,31 @@ static DensePlan dense_plan(int M, int N, int K, int ldx, int qtype, bool pair, 
     plan(p.mblocks * (pair ? 2 : 1), pick_bn(M), N, K, &p.splitk, &p.kt_per_split);
     p.partial = p.splitk > 1 || pair || ssq_out;
   }
-  p.floats = p.partial ? (pair ? 2 : 1) * (int64_t)p.splitk * M * N : 0;
+  p.floats = p.xfloats + (p.partial ? (pair ? 2 : 1) * (int64_t)p.splitk * M * N : 0);
   return p;
 }
-static int launch_dense(GemmArgs& a, const DensePlan& p, int qtype, int64_t workspace_floats, hipStream_t stream) {
+static int launch_frag(GemmArgs& a, const DensePlan& p, int qtype, int x_kind, hipStream_t stream) {
+  FragArgs b = {};
+  b.xp = a.x;
+  if (x_kind != X_FRAGMENTS) {
+    const int rc = frag_pack(a.x, a.partial, a.M, a.K, a.ldx, x_kind == X_ROWS_BF16, stream);
+    if (rc != 0) return rc;
+    b.xp = (const _Float16*)a.partial;
+    a.partial += p.xfloats;
+  }
+  b.w = a.w; b.w2 = a.w2; b.out = a.out; b.partial = a.partial; b.bias = a.bias; b.bias2 = a.bias2; b.residual = a.residual;
+  b.M = a.M; b.N = a.N; b.K = a.K; b.mt_all = (a.M + 15) / 16; b.ldo = a.ldo; b.act = a.act; b.out_type = a.out_type;
+  b.splitk = p.splitk; b.kt_per_split = p.kt_per_split;
+  const int rc = frag_launch(b, p.f, qtype, stream);
+  return rc != 0 || p.splitk == 1 ? rc : launch_reduce(a, stream);
+}
+static int launch_dense(GemmArgs& a, const DensePlan& p, int qtype, int x_kind, int64_t workspace_floats, hipStream_t stream) {
   if (p.floats > 0 && (a.partial == nullptr || workspace_floats < p.floats)) return -5;
+  if (x_kind != X_ROWS && !p.frag) return -8;
+  if (p.xfloats > 0 && ((uintptr_t)a.partial & 15)) return -1;
   a.splitk = p.splitk;
   a.kt_per_split = p.kt_per_split;
+  if (p.frag) return launch_frag(a, p, qtype, x_kind, stream);
   if (p.rows) return launch_rows(a, qtype, p.r, stream);
   a.force_partial = p.partial && p.splitk == 1 ? 1 : 0;
   a.pair_stride = (int64_t)a.splitk * a.M * a.N;
@@ -312,24 +366,32 @@ static int launch_dense(GemmArgs& a, const DensePlan& p, int qtype, int64_t work
 }
 
 // fp32 scratch, in floats, that bigdl_gemm_lowbit (pair, fold_norm, ssq_out = 0) and bigdl_gemm_lowbit_ex need for this call;
-// 0: none.  qtype: the format as the caller knows it.
-extern "C" int64_t bigdl_gemm_lowbit_workspace(int M, int N, int K, int ldx, int qtype, int pair, int fold_norm, int ssq_out) {
+// 0: none.  qtype: the format as the caller knows it.  x_kind: as in those calls.
+extern "C" int64_t bigdl_gemm_lowbit_workspace(int M, int N, int K, int ldx, int qtype, int pair, int fold_norm, int ssq_out, int x_kind) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return dense_plan(M, N, K, ldx, t16_kernel_qtype(qtype), pair != 0, fold_norm != 0, ssq_out != 0).floats;
+  return dense_plan(M, N, K, ldx, t16_kernel_qtype(qtype), pair != 0, fold_norm != 0, ssq_out != 0, x_kind).floats;
 }
 
-// Dense form.  x fp16 [M, ldx] (ldx % 8 == 0, 16-byte aligned), K % 32 == 0.  workspace: see bigdl_gemm_lowbit_workspace.
+// whether a call with x of this kind runs on the kernel that takes x in fragment order (for X_ROWS_BF16: whether it takes such rows)
+extern "C" int bigdl_gemm_lowbit_frag(int M, int N, int K, int ldx, int qtype, int pair, int x_kind) {
+  if (M <= 0 || N <= 0 || K <= 0 || (K & 31)) return 0;
+  FragPlan p;
+  return takes_frag_kernel(ldx, M, N, K, t16_kernel_qtype(qtype), pair != 0, x_kind, &p);
+}
+
+// Dense form.  x_kind 0: x fp16 [M, ldx] (ldx % 8 == 0, 16-byte aligned); 1: bf16 rows, rounded to fp16 (where bigdl_gemm_lowbit_frag
+// says so); 2: fp16 in fragment order (bigdl_frag_pack; ldx is not looked at).  K % 32 == 0.  workspace: see bigdl_gemm_lowbit_workspace.
 extern "C" int bigdl_gemm_lowbit(const void* x, const void* w, void* out, const void* bias, const void* residual,
                                  float* workspace, int64_t workspace_floats, int M, int N, int K, int ldx, int ldo,
-                                 int qtype, int act, int out_type, hipStream_t stream) {
+                                 int qtype, int act, int out_type, int x_kind, hipStream_t stream) {
   qtype = t16_kernel_qtype(qtype);
   if (M <= 0 || N <= 0 || K <= 0 || (K & 31) || (ldx & 7) || ((uintptr_t)x & 15) || ((uintptr_t)w & 15)) return -1;
-  if (out_type < 0 || out_type > 2) return -3;
+  if (out_type < 0 || out_type > 2 || x_kind < 0 || x_kind > 2) return -3;
   if ((int64_t)M * ldx >= (1ll << 31)) return -6;
   GemmArgs a = {};
   a.x = (const _Float16*)x; a.w = w; a.out = out; a.bias = bias; a.residual = residual; a.partial = workspace;
   a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldo = ldo; a.act = act; a.out_type = out_type;
-  return launch_dense(a, dense_plan(M, N, K, ldx, qtype, false, false, false), qtype, workspace_floats, stream);
+  return launch_dense(a, dense_plan(M, N, K, ldx, qtype, false, false, false, x_kind), qtype, x_kind, workspace_floats, stream);
 }
 
 // Extended dense form for batched decode: RMSNorm folded in (gamma + row_ssq of x, see GemmArgs), gate / up pair in one
@@ -338,20 +400,20 @@ extern "C" int bigdl_gemm_lowbit(const void* x, const void* w, void* out, const 
 extern "C" int bigdl_gemm_lowbit_ex(const void* x, const void* w, const void* w2, void* out, const void* bias, const void* bias2,
                                     const void* residual, const void* gamma, float gamma_offset, float eps,
                                     const float* row_ssq, float* ssq_out, float* workspace, int64_t workspace_floats, int M,
-                                    int N, int K, int ldx, int ldo, int qtype, int act, int out_type, hipStream_t stream) {
+                                    int N, int K, int ldx, int ldo, int qtype, int act, int out_type, int x_kind, hipStream_t stream) {
   qtype = t16_kernel_qtype(qtype);
   if (M <= 0 || N <= 0 || K <= 0 || (K & 31) || (ldx & 7) || ((uintptr_t)x & 15) || ((uintptr_t)w & 15)) return -1;
   if (w2 != nullptr && ((uintptr_t)w2 & 15)) return -1;
   if (gamma != nullptr && (((uintptr_t)gamma & 15) || row_ssq == nullptr)) return -1;
-  if (out_type < 0 || out_type > 2) return -3;
+  if (out_type < 0 || out_type > 2 || x_kind < 0 || x_kind > 2) return -3;
   if ((int64_t)M * ldx >= (1ll << 31)) return -6;
   GemmArgs a = {};
   a.x = (const _Float16*)x; a.w = w; a.out = out; a.bias = bias; a.residual = residual; a.partial = workspace;
   a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldo = ldo; a.act = act; a.out_type = out_type;
   a.gamma = (const _Float16*)gamma; a.gamma_offset = gamma_offset; a.eps = eps; a.row_ssq = gamma != nullptr ? row_ssq : nullptr;
   a.ssq_out = ssq_out; a.w2 = w2; a.bias2 = bias2;
-  return launch_dense(a, dense_plan(M, N, K, ldx, qtype, w2 != nullptr, gamma != nullptr, ssq_out != nullptr), qtype, workspace_floats,
-                      stream);
+  return launch_dense(a, dense_plan(M, N, K, ldx, qtype, w2 != nullptr, gamma != nullptr, ssq_out != nullptr, x_kind), qtype, x_kind,
+                      workspace_floats, stream);
 }
 
 // Grouped form: `rows` sorted rows in total; row i uses the weights of the expert that the block table assigns

@@ -34,7 +34,7 @@ static int prompt_dispatch(const GemmArgs& a, int qtype, int cfg, hipStream_t st
 struct PromptCfg { int bm, bn; double eff; };
 static const PromptCfg kPromptCfgs[PROMPT_NCFG] = {{256, 256, 1.0}, {256, 192, 0.79}, {128, 128, 0.65}};
 
-struct PromptPlan { int cfg, splitk, kt_per_split; };
+struct PromptPlan { int cfg, splitk, kt_per_split; double cost; };
 static int g_force_cfg = -1, g_force_sk = 0;         // bigdl_gemm_prompt_force (tests / sweeps)
 
 // Cost of a launch in units of (output element x 128-deep k tile) per CU: rounds of 256 concurrent tiles, every tile
@@ -45,8 +45,7 @@ static PromptPlan prompt_plan(int M, int N, int K, bool pair = false) {
   static const int env_cfg = getenv("BIGDL_PROMPT_CFG") ? atoi(getenv("BIGDL_PROMPT_CFG")) : -1;
   static const int env_sk = getenv("BIGDL_PROMPT_SPLITK") ? atoi(getenv("BIGDL_PROMPT_SPLITK")) : 0;
   const int forced_cfg = g_force_cfg >= 0 ? g_force_cfg : env_cfg, forced_sk = g_force_sk > 0 ? g_force_sk : env_sk;
-  PromptPlan best = {0, 1, KT};
-  double best_cost = 1e300;
+  PromptPlan best = {0, 1, KT, 1e300};
   for (int c = 0; c < PROMPT_NCFG; ++c) {
     if (forced_cfg >= 0 && c != forced_cfg) continue;
     const PromptCfg& pc = kPromptCfgs[c];
@@ -59,10 +58,29 @@ static PromptPlan prompt_plan(int M, int N, int K, bool pair = false) {
       const int64_t rounds = (tiles * rsk + 255) / 256;
       double cost = (double)rounds * pc.bm * pc.bn / pc.eff * (per + 1.5);
       if (rsk > 1) cost += 0.035 * rsk * (double)M * N + 6e4;
-      if (cost < best_cost) { best_cost = cost; best = {c, rsk, per}; }
+      if (cost < best.cost) best = {c, rsk, per, cost};
     }
   }
   return best;
+}
+
+// The plan's cost in us, for the choice between this kernel and others at 257 - 512 rows: fitted per format to 55 products each
+// (the shapes of gemm_frag.hip's fit); exact to 14 %, worst cases 20 %.
+double prompt_us(int M, int N, int K, int qtype, bool pair) {
+  float per = 40.9f;                                   // fp8_e5m2
+  switch (qtype) {
+    case Q_SYM_INT4: per = 38.8f; break;
+    case Q_ASYM_INT4: case Q_WOQ_INT4: per = 40.7f; break;
+    case Q_FP4: per = 41.7f; break;
+    case Q_NF4: per = 44.8f; break;
+    case Q_SYM_INT5: per = 47.5f; break;
+    case Q_ASYM_INT5: per = 54.2f; break;
+    case Q_FP6: per = 55.0f; break;
+    case Q_SYM_INT8: per = 42.7f; break;
+    case Q_FP8_E4M3: per = 45.6f; break;
+    default: break;
+  }
+  return 5.5 + 1e-6 * per * prompt_plan(M, N, K, pair).cost;
 }
 
 // the staged 16-bit epilogue covers this output; otherwise one fp32 slab + the reduce kernel

@@ -83,18 +83,19 @@ struct RowsPlanes {
     if constexpr (has_min_of(QT)) mn = rows_buffer(p.mn + tile0 * 64, tiles * 128);
   }
   // out: 0, or ROWS_OUT for a tile that does not exist (zeros, no memory access)
+  template <int AUX = ROWS_NT>
   __device__ __forceinline__ void load(Tile<QT>& t, int tile, int lane, uint32_t out) const {
-    t.lo0 = __builtin_amdgcn_raw_buffer_load_b128(lo, lane * 16 + out, tile * (lo_bits_of(QT) * 256), ROWS_NT);
-    if constexpr (lo_bits_of(QT) == 8) t.lo1 = __builtin_amdgcn_raw_buffer_load_b128(lo, lane * 16 + 1024 + out, tile * 2048, ROWS_NT);
-    if constexpr (hi_bits_of(QT) == 1) t.hi0 = __builtin_amdgcn_raw_buffer_load_b32(hi, lane * 4 + out, tile * 256, ROWS_NT);
+    t.lo0 = __builtin_amdgcn_raw_buffer_load_b128(lo, lane * 16 + out, tile * (lo_bits_of(QT) * 256), AUX);
+    if constexpr (lo_bits_of(QT) == 8) t.lo1 = __builtin_amdgcn_raw_buffer_load_b128(lo, lane * 16 + 1024 + out, tile * 2048, AUX);
+    if constexpr (hi_bits_of(QT) == 1) t.hi0 = __builtin_amdgcn_raw_buffer_load_b32(hi, lane * 4 + out, tile * 256, AUX);
     if constexpr (hi_bits_of(QT) == 2) {
-      const uint2v h = __builtin_amdgcn_raw_buffer_load_b64(hi, lane * 8 + out, tile * 512, ROWS_NT);
+      const uint2v h = __builtin_amdgcn_raw_buffer_load_b64(hi, lane * 8 + out, tile * 512, AUX);
       t.hi0 = h.x;
       t.hi1 = h.y;
     }
     const uint32_t r8 = (lane & 15) * 8 + out;
-    t.d = __builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(sc, r8, tile * 128, ROWS_NT));
-    if constexpr (has_min_of(QT)) t.m = __builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(mn, r8, tile * 128, ROWS_NT));
+    t.d = __builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(sc, r8, tile * 128, AUX));
+    if constexpr (has_min_of(QT)) t.m = __builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(mn, r8, tile * 128, AUX));
   }
 };
 

@@ -665,14 +665,16 @@ class NativeDecoder:
         cfg = self.cfg
         if cfg.gated_mlp:
             gt, up = lw.gate, lw.up
-            if (gt.fused and up.fused and gt.qtype == up.qtype and gt.n == up.n and gt.n % 16 == 0 and self.prefill_fused
+            two = gt.fused and up.fused and gt.qtype == up.qtype and gt.n == up.n and gt.k == up.k and x.dtype == torch.float16
+            frag = (two and x.shape[0] > GEMM_MAX_ROWS and self.prefill_fused and not Lin.cache_dense and not self.prefill_fp8
+                    and hip.gemm_lowbit_frag(x.shape[0], gt.n, gt.k, gt.qtype, pair=True))
+            if (not frag and gt.fused and up.fused and gt.qtype == up.qtype and gt.n == up.n and gt.n % 16 == 0 and self.prefill_fused
                     and x.shape[0] > GEMM_MAX_ROWS and x.dtype == torch.float16 and not Lin.cache_dense and not self.prefill_fp8
                     and hip.gemm_prompt_supported(gt.qtype, gt.k)):
                 # both input projections and act(g) * u in one launch: g and u never reach memory
                 g = hip.gemm_prompt_pair(x.contiguous(), gt.w, up.w, gt.qtype, gt.n, gt.k, bias=gt.bias, bias2=up.bias,
                                          act=cfg.act)
-            elif (gt.fused and up.fused and gt.qtype == up.qtype and gt.n == up.n and gt.k == up.k and x.dtype == torch.float16
-                    and GEMV_MAX_ROWS < x.shape[0] <= GEMM_MAX_ROWS):
+            elif two and (frag or GEMV_MAX_ROWS < x.shape[0] <= GEMM_MAX_ROWS):
                 g = hip.gemm_lowbit_ex(x.contiguous(), gt.w, gt.qtype, gt.n, gt.k, w2=up.w, bias=gt.bias, bias2=up.bias, act=cfg.act)
             else:
                 g = self._linear_dense(x, gt)

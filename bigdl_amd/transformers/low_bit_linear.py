@@ -296,12 +296,15 @@ def dequant_weight_rows(weight: FP4Params, row0: int, nrows: int, dtype=torch.fl
 
 
 def lowbit_rows(xh, w, qtype, n, k, bias=None, out_dtype=None):
-    """More than GEMM_MAX_ROWS fp16 rows times a T16 weight on this repository's own kernels: the prompt-sized fused GEMM
-    where it applies (K a multiple of 128), otherwise the mid-size fused GEMM GEMM_MAX_ROWS rows at a time."""
+    """More than GEMM_MAX_ROWS fp16 rows times a T16 weight on this repository's own kernels: the one that takes x in fragment
+    order where it is expected to be ahead, the prompt-sized fused GEMM where that applies (K a multiple of 128), otherwise the
+    mid-size fused GEMM GEMM_MAX_ROWS rows at a time."""
     from ..ops import hip
+    m = xh.shape[0]
+    if hip.gemm_lowbit_frag(m, n, k, qtype, ldx=xh.stride(0)):
+        return hip.gemm_lowbit(xh, w, qtype, n, k, bias=bias, out_dtype=out_dtype)
     if hip.gemm_prompt_supported(qtype, k):
         return hip.gemm_prompt(xh, w, qtype, n, k, bias=bias, out_dtype=out_dtype)
-    m = xh.shape[0]
     y = torch.empty(m, n, dtype=out_dtype or torch.float16, device=xh.device)
     for r0 in range(0, m, GEMM_MAX_ROWS):
         hip.gemm_lowbit(xh[r0:r0 + GEMM_MAX_ROWS], w, qtype, n, k, bias=bias, out=y[r0:r0 + GEMM_MAX_ROWS])
@@ -338,6 +341,10 @@ def lowbit_matmul(x_2d: torch.Tensor, weight: FP4Params, out_features: int, for_
         from ..ops import hip
         m, dt = x_2d.shape[0], x_2d.dtype
         t16 = weight.qlayout == "t16"
+        if (t16 and dt == torch.bfloat16 and m > GEMV_MAX_ROWS and (m <= GEMM_MAX_ROWS or not for_training) and x_2d.stride(1) == 1
+                and x_2d.stride(0) % 8 == 0 and x_2d.data_ptr() % 16 == 0 and getattr(weight, "_dense_cache", None) is None
+                and hip.gemm_lowbit_frag(m, n, k, weight.qtype, ldx=x_2d.stride(0), bf16=True)):
+            return hip.gemm_lowbit(x_2d, weight, weight.qtype, n, k, out_dtype=dt)       # (rounded to fp16 while it is ordered)
         if t16 and m <= GEMM_MAX_ROWS:
             xh = x_2d if dt == torch.float16 else _half(x_2d)
             if xh.stride(1) != 1 or xh.stride(0) % 8 or xh.data_ptr() % 16:

@@ -1,0 +1,90 @@
+"""The low-bit product on x in fragment order (csrc/hip/gemm_frag_kernel.h) against a float64 product of the dequantized weight."""
+import pytest
+import torch
+
+from bigdl_amd import qtypes as Q
+from bigdl_amd.ops import host
+
+pytestmark = pytest.mark.gpu
+FORMATS = ["sym_int4", "asym_int4", "woq_int4", "fp4", "nf4", "sym_int5", "asym_int5", "fp6", "sym_int8", "fp8_e4m3", "fp8_e5m2"]
+TILINGS = [(3, 2), (3, 3), (3, 4), (3, 6), (4, 2), (4, 3), (4, 4), (4, 6), (4, 8), (5, 3), (5, 4), (5, 6), (5, 8), (6, 2), (6, 4), (6, 6),
+           (7, 3), (7, 4), (8, 3), (8, 4)]
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from bigdl_amd.ops import hip as h
+    h.lib()
+    return h
+
+
+def _weight(n, k, qt, seed):
+    w = torch.randn(n, k, generator=torch.Generator().manual_seed(seed)) * 0.05
+    raw = host.quantize(w, qt)
+    raw = raw.view(torch.uint8) if raw.dtype != torch.uint8 else raw
+    return host.relayout_to_device(raw, qt, n, k).cuda(), host.dequantize(raw, qt, w.shape).double()
+
+
+def _x(m, k, seed, dtype=torch.float16):
+    """[m, k] rows inside a buffer of NaN: what lies behind a row or below the last one must not be read as data"""
+    buf = torch.full((m + 2, k + 24), float("nan"), dtype=dtype)
+    buf[:m, :k] = torch.randn(m, k, generator=torch.Generator().manual_seed(seed)).to(dtype)
+    return buf.cuda()[:m, :k], buf[:m, :k].half().double()
+
+
+def _close(out, x, w, ref):
+    # code * scale (+ min) is rounded to fp16: 2^-11 of a weight's larger term, on top of the table's of nf4, times two
+    bound = 2.0 ** -9 * (x.abs() @ w.abs().t()) + 1e-5
+    assert torch.isfinite(out).all()
+    assert ((out.double().cpu() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("m,k", [(1, 32), (16, 128), (77, 2080), (130, 1184)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_fragment_order(hip, m, k, dtype):
+    x, xd = _x(m, k, 1, dtype)
+    kt, mt = (k + 127) // 128, (m + 15) // 16
+    want = torch.zeros(mt * 16, kt * 128, dtype=torch.float64)
+    want[:m, :k] = xd
+    # [k step][row tile][k group][row][8]
+    want = want.view(mt, 16, kt * 4, 4, 8).permute(2, 0, 3, 1, 4).reshape(-1)
+    assert torch.equal(hip.frag_pack(x).cpu().double(), want)
+
+
+# (rows, N, K): cut row and column tiles, a cut last k-tile, fewer k-tiles than wavefronts, one more than those in flight
+@pytest.mark.parametrize("name", FORMATS)
+@pytest.mark.parametrize("m,n,k", [(1, 16, 32), (33, 130, 3232), (77, 37, 2080), (113, 200, 1024), (203, 80, 1184)])
+def test_every_tiling_matches_float64(hip, name, m, n, k):
+    k = k if name not in ("nf4", "woq_int4") else (k + 127) // 128 * 128
+    qt = Q.ggml_tensor_qtype[name]
+    dev, w = _weight(n, k, qt, 1)
+    x, xd = _x(m, k, 2)
+    xp = hip.frag_pack(x)
+    ref = xd @ w.t()
+    for mt, ns in TILINGS:
+        _close(hip.gemm_frag(xp, m, dev, qt, n, k, out_dtype=torch.float32, mt=mt, ns=ns), xd, w, ref)
+    parts = hip.gemm_frag(xp, m, dev, qt, n, k, out_dtype=torch.float32, mt=4, ns=3, splitk=3)
+    if parts.dim() == 3:
+        _close(parts.sum(0), xd, w, ref)
+
+
+@pytest.mark.parametrize("name", ["sym_int4", "asym_int5", "nf4", "sym_int8"])
+@pytest.mark.parametrize("m,n", [(24, 104), (77, 70), (130, 33)])
+def test_pairs_bias_residual(hip, name, m, n):
+    k = 1280
+    qt = Q.ggml_tensor_qtype[name]
+    (dg, wg), (du, wu) = _weight(n, k, qt, 3), _weight(n, k, qt, 4)
+    x, xd = _x(m, k, 5)
+    xp = hip.frag_pack(x)
+    b1, b2 = torch.randn(n).half(), torch.randn(n).half()
+    silu = torch.nn.functional.silu
+    for mt, ns in [t for t in TILINGS if t[1] % 2 == 0]:
+        got = hip.gemm_frag(xp, m, dg, qt, n, k, w2=du, bias=b1.cuda(), bias2=b2.cuda(), act="silu", out_dtype=torch.float32, mt=mt, ns=ns)
+        ref = silu(xd @ wg.t() + b1.double()) * (xd @ wu.t() + b2.double())
+        torch.testing.assert_close(got.cpu().double(), ref, rtol=4e-3, atol=8e-3)      # two products of 2^-9 and 2^-10 each, silu's slope 1.1
+    for dtype in (torch.float16, torch.bfloat16, torch.float32):
+        res = torch.randn(m, n).to(dtype)
+        out = res.cuda()
+        hip.gemm_frag(xp, m, dg, qt, n, k, bias=b1.cuda(), residual=out, out=out, mt=5, ns=3)    # in place, as on the residual stream
+        tol = dict(rtol=8e-3, atol=2e-2) if dtype == torch.bfloat16 else dict(rtol=2e-3, atol=8e-3)
+        torch.testing.assert_close(out.cpu().double(), xd @ wg.t() + b1.double() + res.double(), **tol)

@@ -24,6 +24,13 @@
 
 namespace bigdl {
 
+// out_type of an output in fragment order, fp16: x of the next product
+constexpr int OUT_FRAG = 3;
+// place, in halves, of (row m, column k) in fragment order
+__device__ __forceinline__ int64_t frag_at(int m, int k, int mt_all) {
+  return (((int64_t)(k >> 5) * mt_all + (m >> 4)) * 64 + ((k & 31) >> 3) * 16 + (m & 15)) * 8 + (k & 7);
+}
+
 struct FragArgs {
   const _Float16* xp;     // [KT * 4][mt_all][64 lanes][8]: see frag_pack_kernel
   const void* w;          // T16 [N, K]
@@ -210,6 +217,10 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void gemm_frag_kernel(FragArgs a) 
       if (a.bias != nullptr) y[q] += (float)((const _Float16*)a.bias)[c];
       y[q] = act_apply(a.act, y[q]);
       if (pair) y[q] *= u[q] + (a.bias2 != nullptr ? (float)((const _Float16*)a.bias2)[c] : 0.0f);
+    }
+    if (a.out_type == OUT_FRAG) {
+      *(half4*)((_Float16*)a.out + frag_at(m, col, a.mt_all)) = half4{(_Float16)y[0], (_Float16)y[1], (_Float16)y[2], (_Float16)y[3]};
+      continue;
     }
     const int64_t oi = (int64_t)m * a.ldo + col;
     if (a.vec && a.out_type != OUT_F32) {

@@ -278,6 +278,63 @@ static int launch_rows(const GemmArgs& a, int qtype, const RowsPlan& p, hipStrea
   return rc != 0 || p.splitk == 1 ? rc : launch_reduce(a, stream);
 }
 
+// The kernel a call runs on and the fp32 scratch it needs: one place for the launches and for the size that callers ask for
+struct DensePlan {
+  bool rows;                // few-row kernel; otherwise the tile kernel
+  RowsPlan r;
+  int bm, mblocks, splitk, kt_per_split;
+  bool partial;             // the results pass through scratch and the reduce kernel
+  int64_t floats;
+};
+// fold_norm, ssq_out: the tile kernel's forms of gemm_lowbit_ex
+static DensePlan dense_plan(int M, int N, int K, int ldx, int qtype, bool pair, bool fold_norm, bool ssq_out) {
+  DensePlan p = {};
+  p.rows = !fold_norm && !ssq_out && takes_rows_kernel(ldx, M, N, K, qtype, pair, &p.r);
+  if (p.rows) {
+    p.splitk = p.r.splitk;
+    p.kt_per_split = p.r.kt_per_split;
+    p.partial = p.splitk > 1;
+  } else {
+    p.bm = bigdl_gemm_lowbit_bm(M);
+    p.mblocks = (M + p.bm - 1) / p.bm;
+    plan(p.mblocks * (pair ? 2 : 1), pick_bn(M), N, K, &p.splitk, &p.kt_per_split);
+    p.partial = p.splitk > 1 || pair || ssq_out;
+  }
+  p.floats = p.partial ? (pair ? 2 : 1) * (int64_t)p.splitk * M * N : 0;
+  return p;
+}
+static int launch_dense(GemmArgs& a, const DensePlan& p, int qtype, int64_t workspace_floats, hipStream_t stream) {
+  if (p.floats > 0 && (a.partial == nullptr || workspace_floats < p.floats)) return -5;
+  a.splitk = p.splitk;
+  a.kt_per_split = p.kt_per_split;
+  if (p.rows) return launch_rows(a, qtype, p.r, stream);
+  a.force_partial = p.partial && p.splitk == 1 ? 1 : 0;
+  a.pair_stride = (int64_t)a.splitk * a.M * a.N;
+  const int rc = dispatch(a, qtype, p.bm, pick_bn(a.M), p.mblocks, stream);
+  return rc != 0 || !p.partial ? rc : launch_reduce(a, stream);
+}
+
+// fp32 scratch, in floats, that bigdl_gemm_lowbit (pair, fold_norm, ssq_out = 0) and bigdl_gemm_lowbit_ex need for this call;
+// 0: none.  qtype: the format as the caller knows it.
+extern "C" int64_t bigdl_gemm_lowbit_workspace(int M, int N, int K, int ldx, int qtype, int pair, int fold_norm, int ssq_out) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  return dense_plan(M, N, K, ldx, t16_kernel_qtype(qtype), pair != 0, fold_norm != 0, ssq_out != 0).floats;
+}
+
+// Dense form.  x fp16 [M, ldx] (ldx % 8 == 0, 16-byte aligned), K % 32 == 0.  workspace: see bigdl_gemm_lowbit_workspace.
+extern "C" int bigdl_gemm_lowbit(const void* x, const void* w, void* out, const void* bias, const void* residual,
+                                 float* workspace, int64_t workspace_floats, int M, int N, int K, int ldx, int ldo,
+                                 int qtype, int act, int out_type, hipStream_t stream) {
+  qtype = t16_kernel_qtype(qtype);
+  if (M <= 0 || N <= 0 || K <= 0 || (K & 31) || (ldx & 7) || ((uintptr_t)x & 15) || ((uintptr_t)w & 15)) return -1;
+  if (out_type < 0 || out_type > 2) return -3;
+  if ((int64_t)M * ldx >= (1ll << 31)) return -6;
+  GemmArgs a = {};
+  a.x = (const _Float16*)x; a.w = w; a.out = out; a.bias = bias; a.residual = residual; a.partial = workspace;
+  a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldo = ldo; a.act = act; a.out_type = out_type;
+  return launch_dense(a, dense_plan(M, N, K, ldx, qtype, false, false, false), qtype, workspace_floats, stream);
+}
+
 // Which products the kernel on x in fragment order takes: those where it and the pass that orders x are expected to be ahead of
 // the faster of the others, by 3 % for what the estimates may be off.  Measured, us, before -> it + that pass: sym_int4
 // 4096 x 4096 at 77 / 256 rows 15.2 -> 9.6 + 3.7, 23.1 -> 14.3 + 4.5; asym_int4 pair of 14336 x 4096 at 77 rows 67.6 -> 32.1 + 3.7; sym_int8
@@ -303,95 +360,56 @@ static bool takes_frag_kernel(int ldx, int M, int N, int K, int qtype, bool pair
   return plan->us + (x_kind == X_ROWS ? frag_pack_us(M, K) : 0.0) < 0.97 * other;
 }
 
-// The kernel a call runs on and the fp32 scratch it needs: one place for the launches and for the size that callers ask for
-struct DensePlan {
-  bool frag;                // kernel on x in fragment order (scratch: x in that order, partial sums)
-  FragPlan f;
-  bool rows;                // few-row kernel; otherwise the tile kernel
-  RowsPlan r;
-  int bm, mblocks, splitk, kt_per_split;
-  bool partial;             // the results pass through scratch and the reduce kernel
-  int64_t xfloats, floats;  // scratch of x / in all
-};
-// fold_norm, ssq_out: the tile kernel's forms of gemm_lowbit_ex
-static DensePlan dense_plan(int M, int N, int K, int ldx, int qtype, bool pair, bool fold_norm, bool ssq_out, int x_kind) {
-  DensePlan p = {};
-  p.frag = !fold_norm && !ssq_out && takes_frag_kernel(ldx, M, N, K, qtype, pair, x_kind, &p.f);
-  p.rows = !p.frag && !fold_norm && !ssq_out && takes_rows_kernel(ldx, M, N, K, qtype, pair, &p.r);
-  if (p.frag) {
-    p.splitk = p.f.splitk;
-    p.kt_per_split = p.f.kt_per_split;
-    p.partial = p.splitk > 1;
-    p.xfloats = x_kind == X_FRAGMENTS ? 0 : frag_halves(M, K) / 2;
-  } else if (p.rows) {
-    p.splitk = p.r.splitk;
-    p.kt_per_split = p.r.kt_per_split;
-    p.partial = p.splitk > 1;
-  } else {
-    p.bm = bigdl_gemm_lowbit_bm(M);
-    p.mblocks = (M + p.bm - 1) / p.bm;
-    plan(p.mblocks * (pair ? 2 : 1), pick_bn(M), N, K, &p.splitk, &p.kt_per_split);
-    p.partial = p.splitk > 1 || pair || ssq_out;
-  }
-  p.floats = p.xfloats + (p.partial ? (pair ? 2 : 1) * (int64_t)p.splitk * M * N : 0);
-  return p;
-}
-static int launch_frag(GemmArgs& a, const DensePlan& p, int qtype, int x_kind, hipStream_t stream) {
-  FragArgs b = {};
-  b.xp = a.x;
-  if (x_kind != X_FRAGMENTS) {
-    const int rc = frag_pack(a.x, a.partial, a.M, a.K, a.ldx, x_kind == X_ROWS_BF16, stream);
-    if (rc != 0) return rc;
-    b.xp = (const _Float16*)a.partial;
-    a.partial += p.xfloats;
-  }
-  b.w = a.w; b.w2 = a.w2; b.out = a.out; b.partial = a.partial; b.bias = a.bias; b.bias2 = a.bias2; b.residual = a.residual;
-  b.M = a.M; b.N = a.N; b.K = a.K; b.mt_all = (a.M + 15) / 16; b.ldo = a.ldo; b.act = a.act; b.out_type = a.out_type;
-  b.splitk = p.splitk; b.kt_per_split = p.kt_per_split;
-  const int rc = frag_launch(b, p.f, qtype, stream);
-  return rc != 0 || p.splitk == 1 ? rc : launch_reduce(a, stream);
-}
-static int launch_dense(GemmArgs& a, const DensePlan& p, int qtype, int x_kind, int64_t workspace_floats, hipStream_t stream) {
-  if (p.floats > 0 && (a.partial == nullptr || workspace_floats < p.floats)) return -5;
-  if (x_kind != X_ROWS && !p.frag) return -8;
-  if (p.xfloats > 0 && ((uintptr_t)a.partial & 15)) return -1;
-  a.splitk = p.splitk;
-  a.kt_per_split = p.kt_per_split;
-  if (p.frag) return launch_frag(a, p, qtype, x_kind, stream);
-  if (p.rows) return launch_rows(a, qtype, p.r, stream);
-  a.force_partial = p.partial && p.splitk == 1 ? 1 : 0;
-  a.pair_stride = (int64_t)a.splitk * a.M * a.N;
-  const int rc = dispatch(a, qtype, p.bm, pick_bn(a.M), p.mblocks, stream);
-  return rc != 0 || !p.partial ? rc : launch_reduce(a, stream);
-}
-
-// fp32 scratch, in floats, that bigdl_gemm_lowbit (pair, fold_norm, ssq_out = 0) and bigdl_gemm_lowbit_ex need for this call;
-// 0: none.  qtype: the format as the caller knows it.  x_kind: as in those calls.
-extern "C" int64_t bigdl_gemm_lowbit_workspace(int M, int N, int K, int ldx, int qtype, int pair, int fold_norm, int ssq_out, int x_kind) {
-  if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return dense_plan(M, N, K, ldx, t16_kernel_qtype(qtype), pair != 0, fold_norm != 0, ssq_out != 0, x_kind).floats;
-}
-
-// whether a call with x of this kind runs on the kernel that takes x in fragment order (for X_ROWS_BF16: whether it takes such rows)
+// Whether the kernel on x in fragment order is the one for this product.  x_kind 0: fp16 rows; 1: bf16 rows, or x that its producer
+// writes in that order (no pass of its own over x); 2: x in that order already (whether it can be multiplied at all).
 extern "C" int bigdl_gemm_lowbit_frag(int M, int N, int K, int ldx, int qtype, int pair, int x_kind) {
-  if (M <= 0 || N <= 0 || K <= 0 || (K & 31)) return 0;
+  if (M <= 0 || N <= 0 || K <= 0 || (K & 31) || x_kind < 0 || x_kind > X_FRAGMENTS) return 0;
   FragPlan p;
-  return takes_frag_kernel(ldx, M, N, K, t16_kernel_qtype(qtype), pair != 0, x_kind, &p);
+  return takes_frag_kernel(ldx, M, N, K, t16_kernel_qtype(qtype), pair != 0, x_kind, &p) ? 1 : 0;
 }
 
-// Dense form.  x_kind 0: x fp16 [M, ldx] (ldx % 8 == 0, 16-byte aligned); 1: bf16 rows, rounded to fp16 (where bigdl_gemm_lowbit_frag
-// says so); 2: fp16 in fragment order (bigdl_frag_pack; ldx is not looked at).  K % 32 == 0.  workspace: see bigdl_gemm_lowbit_workspace.
-extern "C" int bigdl_gemm_lowbit(const void* x, const void* w, void* out, const void* bias, const void* residual,
-                                 float* workspace, int64_t workspace_floats, int M, int N, int K, int ldx, int ldo,
-                                 int qtype, int act, int out_type, int x_kind, hipStream_t stream) {
+// fp32 scratch, in floats, of the call below: x in fragment order (unless it comes so) and the partial sums of a split K
+extern "C" int64_t bigdl_gemm_frag_workspace(int M, int N, int K, int qtype, int pair, int x_kind) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const FragPlan p = frag_plan(M, N, K, t16_kernel_qtype(qtype), pair != 0, !pair);
+  return (x_kind == X_FRAGMENTS ? 0 : frag_halves(M, K) / 2) + (p.splitk > 1 ? (int64_t)p.splitk * M * N : 0);
+}
+
+// y = act(x W^T + bias) [* (x W2^T + bias2)] [+ residual] on the kernel on x in fragment order.  x_kind 0: x fp16 [M, ldx] (ldx % 8 == 0,
+// 16-byte aligned); 1: bf16 rows, rounded to fp16; 2: fp16 in fragment order (ldx is not looked at).  K % 32 == 0.  out_type 3 (pairs,
+// N % 128 == 0, no residual): fp16 in fragment order; rows past M of its last row tile are left as they are, they reach only rows of
+// a product that are not stored.
+extern "C" int bigdl_gemm_frag_dense(const void* x, const void* w, const void* w2, void* out, const void* bias, const void* bias2,
+                                     const void* residual, float* workspace, int64_t workspace_floats, int M, int N, int K, int ldx,
+                                     int ldo, int qtype, int act, int out_type, int x_kind, hipStream_t stream) {
   qtype = t16_kernel_qtype(qtype);
-  if (M <= 0 || N <= 0 || K <= 0 || (K & 31) || (ldx & 7) || ((uintptr_t)x & 15) || ((uintptr_t)w & 15)) return -1;
-  if (out_type < 0 || out_type > 2 || x_kind < 0 || x_kind > 2) return -3;
-  if ((int64_t)M * ldx >= (1ll << 31)) return -6;
+  if (M <= 0 || N <= 0 || K <= 0 || (K & 31) || ((uintptr_t)x & 15) || ((uintptr_t)w & 15) || !is_t16(qtype)) return -1;
+  if (x_kind != X_FRAGMENTS && ((ldx & 7) || ldx < K)) return -1;
+  if (w2 != nullptr && ((uintptr_t)w2 & 15)) return -1;
+  if (out_type == OUT_FRAG && (w2 == nullptr || residual != nullptr || (N & 127) || ((uintptr_t)out & 15))) return -1;
+  if (out_type < 0 || out_type > OUT_FRAG || x_kind < 0 || x_kind > X_FRAGMENTS) return -3;
+  const FragPlan p = frag_plan(M, N, K, qtype, w2 != nullptr, w2 == nullptr);
+  if (p.ns == 0) return -6;
+  const int64_t xfloats = x_kind == X_FRAGMENTS ? 0 : frag_halves(M, K) / 2;
+  const int64_t floats = xfloats + (p.splitk > 1 ? (int64_t)p.splitk * M * N : 0);
+  if (floats > 0 && (workspace == nullptr || workspace_floats < floats)) return -5;
+  if ((uintptr_t)workspace & 15) return -1;
+  FragArgs b = {};
+  b.xp = (const _Float16*)x;
+  if (xfloats > 0) {
+    const int rc = frag_pack(x, workspace, M, K, ldx, x_kind == X_ROWS_BF16, stream);
+    if (rc != 0) return rc;
+    b.xp = (const _Float16*)workspace;
+  }
+  b.w = w; b.w2 = w2; b.out = out; b.partial = workspace + xfloats; b.bias = bias; b.bias2 = bias2; b.residual = residual;
+  b.M = M; b.N = N; b.K = K; b.mt_all = (M + 15) / 16; b.ldo = ldo; b.act = act; b.out_type = out_type;
+  b.splitk = p.splitk; b.kt_per_split = p.kt_per_split;
+  const int rc = frag_launch(b, p, qtype, stream);
+  if (rc != 0 || p.splitk == 1) return rc;
   GemmArgs a = {};
-  a.x = (const _Float16*)x; a.w = w; a.out = out; a.bias = bias; a.residual = residual; a.partial = workspace;
-  a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldo = ldo; a.act = act; a.out_type = out_type;
-  return launch_dense(a, dense_plan(M, N, K, ldx, qtype, false, false, false, x_kind), qtype, x_kind, workspace_floats, stream);
+  a.out = out; a.bias = bias; a.residual = residual; a.partial = workspace + xfloats;
+  a.M = M; a.N = N; a.K = K; a.ldo = ldo; a.act = act; a.out_type = out_type; a.splitk = p.splitk;
+  return launch_reduce(a, stream);
 }
 
 // Extended dense form for batched decode: RMSNorm folded in (gamma + row_ssq of x, see GemmArgs), gate / up pair in one
@@ -400,20 +418,20 @@ extern "C" int bigdl_gemm_lowbit(const void* x, const void* w, void* out, const 
 extern "C" int bigdl_gemm_lowbit_ex(const void* x, const void* w, const void* w2, void* out, const void* bias, const void* bias2,
                                     const void* residual, const void* gamma, float gamma_offset, float eps,
                                     const float* row_ssq, float* ssq_out, float* workspace, int64_t workspace_floats, int M,
-                                    int N, int K, int ldx, int ldo, int qtype, int act, int out_type, int x_kind, hipStream_t stream) {
+                                    int N, int K, int ldx, int ldo, int qtype, int act, int out_type, hipStream_t stream) {
   qtype = t16_kernel_qtype(qtype);
   if (M <= 0 || N <= 0 || K <= 0 || (K & 31) || (ldx & 7) || ((uintptr_t)x & 15) || ((uintptr_t)w & 15)) return -1;
   if (w2 != nullptr && ((uintptr_t)w2 & 15)) return -1;
   if (gamma != nullptr && (((uintptr_t)gamma & 15) || row_ssq == nullptr)) return -1;
-  if (out_type < 0 || out_type > 2 || x_kind < 0 || x_kind > 2) return -3;
+  if (out_type < 0 || out_type > 2) return -3;
   if ((int64_t)M * ldx >= (1ll << 31)) return -6;
   GemmArgs a = {};
   a.x = (const _Float16*)x; a.w = w; a.out = out; a.bias = bias; a.residual = residual; a.partial = workspace;
   a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldo = ldo; a.act = act; a.out_type = out_type;
   a.gamma = (const _Float16*)gamma; a.gamma_offset = gamma_offset; a.eps = eps; a.row_ssq = gamma != nullptr ? row_ssq : nullptr;
   a.ssq_out = ssq_out; a.w2 = w2; a.bias2 = bias2;
-  return launch_dense(a, dense_plan(M, N, K, ldx, qtype, w2 != nullptr, gamma != nullptr, ssq_out != nullptr, x_kind), qtype, x_kind,
-                      workspace_floats, stream);
+  return launch_dense(a, dense_plan(M, N, K, ldx, qtype, w2 != nullptr, gamma != nullptr, ssq_out != nullptr), qtype, workspace_floats,
+                      stream);
 }
 
 // Grouped form: `rows` sorted rows in total; row i uses the weights of the expert that the block table assigns

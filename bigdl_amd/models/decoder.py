@@ -521,8 +521,25 @@ class NativeDecoder:
                     kernel_size=ck.get("kernel_size", 7), pooling=ck.get("pooling", "maxpool"))
 
     # ------------------------------------------------------------------ prefill (eager)
+    def _takes_frags(self, rows, lin: Optional[Lin], w2: Optional[Lin] = None, prompt=True):
+        """whether the product of so many rows (with w2: the gate / up pair) takes x in fragment order from its producer: the norm
+        in front of it, or the pair in front of a down projection"""
+        from ..ops import hip
+        if lin is None or not lin.fused or rows <= GEMV_MAX_ROWS or lin.k % 128:
+            return False
+        if w2 is not None and not (w2.fused and w2.qtype == lin.qtype and w2.n == lin.n and w2.k == lin.k):
+            return False
+        if rows > GEMM_MAX_ROWS and not (prompt and self.prefill_fused and not Lin.cache_dense and not self.prefill_fp8):
+            return False
+        return hip.gemm_lowbit_frag(rows, lin.n, lin.k, lin.qtype, pair=w2 is not None, bf16=True)
+
+    def _mlp_takes_frags(self, rows, lw):
+        return self.cfg.gated_mlp and lw.moe is None and lw.gate is not None and self._takes_frags(rows, lw.gate, lw.up)
+
     def _linear_dense(self, x, lin: Lin):
         from ..ops import hip
+        if type(x) is hip.Frags:
+            return hip.gemm_lowbit(x, lin.w, lin.qtype, lin.n, lin.k, bias=lin.bias)
         if lin.fused and x.shape[0] <= GEMV_MAX_ROWS:
             return hip.gemv_lowbit(x.contiguous(), lin.w, lin.qtype, lin.n, lin.k, bias=lin.bias)
         if lin.fused and x.shape[0] <= GEMM_MAX_ROWS:
@@ -638,17 +655,21 @@ class NativeDecoder:
             return hip.layer_norm(x, w, b, self.cfg.rms_eps)
         return hip.rms_norm(x, w, self.cfg.rms_eps, offset=self.cfg.norm_offset, residual=residual, res_out=res_out)
 
-    def _add_norm(self, h, add, w, b=None):
+    def _add_norm(self, h, add, w, b=None, frags=False):
         """(norm(h + add), h + add): the residual add rides in the RMSNorm launch (the prompt pass otherwise spends one
-        elementwise launch per add: 64 of them, 0.37 ms, on a 1024-token Llama-2-7B prompt).  ``add`` None: (norm(h), h)."""
+        elementwise launch per add: 64 of them, 0.37 ms, on a 1024-token Llama-2-7B prompt).  ``add`` None: (norm(h), h).
+        ``frags``: an RMSNorm's result in fragment order, for the product that reads it."""
         from ..ops import hip
+        frags = frags and self.cfg.norm != "layer" and h.dtype == torch.float16
         if add is None:
+            if frags:
+                return hip.rms_norm(h, w, self.cfg.rms_eps, offset=self.cfg.norm_offset, frags=True), h
             return self._norm(h, w, b), h
         if self.cfg.norm == "layer" or add.dtype != h.dtype or not (h.is_contiguous() and add.is_contiguous()):
             h = h + add
             return self._norm(h, w, b), h
         hn = torch.empty_like(h)
-        x = hip.rms_norm(add, w, self.cfg.rms_eps, offset=self.cfg.norm_offset, residual=h, res_out=hn)
+        x = hip.rms_norm(add, w, self.cfg.rms_eps, offset=self.cfg.norm_offset, residual=h, res_out=hn, frags=frags)
         return x, hn
 
     def _embed_extras(self, h, pos):
@@ -663,7 +684,11 @@ class NativeDecoder:
     def _mlp_dense(self, x, lw):
         from ..ops import hip
         cfg = self.cfg
-        if cfg.gated_mlp:
+        if type(x) is hip.Frags:
+            gt, up = lw.gate, lw.up
+            g = hip.gemm_lowbit_ex(x, gt.w, gt.qtype, gt.n, gt.k, w2=up.w, bias=gt.bias, bias2=up.bias, act=cfg.act,
+                                   out_frags=self._takes_frags(x.shape[0], lw.down))
+        elif cfg.gated_mlp:
             gt, up = lw.gate, lw.up
             two = gt.fused and up.fused and gt.qtype == up.qtype and gt.n == up.n and gt.k == up.k and x.dtype == torch.float16
             frag = (two and x.shape[0] > GEMM_MAX_ROWS and self.prefill_fused and not Lin.cache_dense and not self.prefill_fp8
@@ -763,7 +788,9 @@ class NativeDecoder:
             mrope_delta = int(top[0]) + 1 - s
         pend = None                          # MLP output of the previous layer, added to h by the next norm launch
         for li, lw in enumerate(self.layers):
-            x, h = self._add_norm(h, pend, lw.input_norm, lw.input_norm_b)
+            plain = not cfg.parallel_residual
+            x, h = self._add_norm(h, pend, lw.input_norm, lw.input_norm_b,
+                                  frags=plain and lw.mla is None and self._takes_frags(h.shape[0], lw.qkv))
             pend = None
             qkv = self._linear_dense(x, lw.qkv) if lw.mla is None else self._mla_qkv_dense(x, lw.mla)
             if nd:
@@ -826,7 +853,8 @@ class NativeDecoder:
                 x2 = x if lw.post_norm is None else self._norm(h, lw.post_norm, lw.post_norm_b)
                 h = h + o + self._mlp_dense(x2, lw)
                 continue
-            x, h = self._add_norm(h, o, lw.pre_ffn_norm if lw.pre_ffn_norm is not None else lw.post_norm, lw.post_norm_b)
+            x, h = self._add_norm(h, o, lw.pre_ffn_norm if lw.pre_ffn_norm is not None else lw.post_norm, lw.post_norm_b,
+                                  frags=self._mlp_takes_frags(h.shape[0], lw))
             if lw.moe is not None:
                 m = lw.moe.forward_dense(x, self)
             else:
@@ -1189,9 +1217,10 @@ class NativeDecoder:
         return st
 
     def _gemv(self, x, lin: Lin, out, *, gamma=None, residual=None, w2: Lin = None, act=None, att_partials=None,
-              beta=False):
+              beta=False, then: Lin = None):
         """out = epilogue(norm?(x) @ W^T): fused kernel for T16 weights, unfused torch ops otherwise.  ``beta``
-        (a tensor or None, instead of the default False) selects LayerNorm(gamma, beta) as the norm."""
+        (a tensor or None, instead of the default False) selects LayerNorm(gamma, beta) as the norm.  ``then``: the product that alone
+        reads a pair's result; where it takes x in fragment order the result comes back so, and not in ``out``."""
         from ..ops import hip
         cfg = self.cfg
         m = x.shape[0]
@@ -1206,7 +1235,10 @@ class NativeDecoder:
                 and w2.qtype == lin.qtype and w2.n == lin.n and not os.environ.get("BIGDL_NO_PAIR_GEMM")):
             # batched decode (17 .. 256 rows): gate and up in one launch, act(g) * u in the few-row kernel's epilogue or, where
             # the tile kernel runs, in its reduce kernel (at 64 rows of 11008 x 4096: 23 and 33 us)
-            xin = x if gamma is None else hip.rms_norm(x, gamma, cfg.rms_eps, offset=cfg.norm_offset)
+            frags = gamma is not None and self._takes_frags(m, lin, w2, prompt=False)
+            xin = x if gamma is None else hip.rms_norm(x, gamma, cfg.rms_eps, offset=cfg.norm_offset, frags=frags)
+            if frags and then is not None and self._takes_frags(m, then, prompt=False):
+                return hip.gemm_lowbit_ex(xin, lin.w, lin.qtype, lin.n, lin.k, w2=w2.w, bias=lin.bias, bias2=w2.bias, act=act, out_frags=True)
             return hip.gemm_lowbit_ex(xin, lin.w, lin.qtype, lin.n, lin.k, w2=w2.w, bias=lin.bias, bias2=w2.bias, act=act, out=out)
         if (lin.fused and (w2 is None or w2.fused) and m > GEMV_MAX_ROWS and att_partials is None and self.fold_batched_norm
                 and (w2 is None or (w2.qtype == lin.qtype and w2.n == lin.n))):
@@ -1222,7 +1254,8 @@ class NativeDecoder:
                                       act=act, out=out)
         if lin.fused and (w2 is None or w2.fused) and m > GEMV_MAX_ROWS and att_partials is None:
             # batched decode (17 .. 64 rows): RMSNorm kernel + MFMA GEMM with the epilogue fused
-            xin = x if gamma is None else hip.rms_norm(x, gamma, cfg.rms_eps, offset=cfg.norm_offset)
+            xin = x if gamma is None else hip.rms_norm(x, gamma, cfg.rms_eps, offset=cfg.norm_offset,
+                                                       frags=w2 is None and self._takes_frags(m, lin, prompt=False))
             if w2 is None:
                 return hip.gemm_lowbit(xin, lin.w, lin.qtype, lin.n, lin.k, bias=lin.bias, residual=residual, act=act, out=out)
             g = hip.gemm_lowbit(xin, lin.w, lin.qtype, lin.n, lin.k, bias=lin.bias, out=out)
@@ -1287,12 +1320,11 @@ class NativeDecoder:
         return slot
 
     def _mlp_in(self, h, lw, a, gamma, beta):
-        """a = act(gate(norm(h))) * up(norm(h))  or  act(up(norm(h)))"""
+        """act(gate(norm(h))) * up(norm(h))  or  act(up(norm(h))): in a, or as the down projection takes it (see ``_gemv``)"""
         cfg = self.cfg
         if cfg.gated_mlp:
-            self._gemv(h, lw.gate, a, gamma=gamma, beta=beta, w2=lw.up, act=cfg.act)
-        else:
-            self._gemv(h, lw.up, a, gamma=gamma, beta=beta, act=cfg.act)
+            return self._gemv(h, lw.gate, a, gamma=gamma, beta=beta, w2=lw.up, act=cfg.act, then=lw.down)
+        return self._gemv(h, lw.up, a, gamma=gamma, beta=beta, act=cfg.act)
 
     def _decode_body(self, st, batch: int, q_len: int, chain: bool):
         from ..ops import hip
@@ -1339,9 +1371,9 @@ class NativeDecoder:
                 # the MLP reads the layer input: its first GEMV runs before o_proj adds the attention output to h
                 a = act[:, : lw.up.n]
                 if lw.post_norm is None:
-                    self._mlp_in(h, lw, a, lw.input_norm, lw.input_norm_b)
+                    a = self._mlp_in(h, lw, a, lw.input_norm, lw.input_norm_b)
                 else:
-                    self._mlp_in(h, lw, a, lw.post_norm, lw.post_norm_b)
+                    a = self._mlp_in(h, lw, a, lw.post_norm, lw.post_norm_b)
             if lw.post_attn_out_norm is None and self.tp_group is None:
                 self._gemv(attn, lw.o, h, residual=h, att_partials=att_partials)
             else:
@@ -1355,9 +1387,9 @@ class NativeDecoder:
                 lw.moe.forward_decode(self, h, ffn_norm)
                 self._ssq_owner = None
                 continue
-            a = act[:, : lw.up.n]
             if not (layer_norm and cfg.parallel_residual):
-                self._mlp_in(h, lw, a, ffn_norm, lw.post_norm_b if layer_norm else False)
+                a = act[:, : lw.up.n]
+                a = self._mlp_in(h, lw, a, ffn_norm, lw.post_norm_b if layer_norm else False)
             if lw.post_ffn_out_norm is None and self.tp_group is None:
                 self._gemv(a, lw.down, h, residual=h)
             else:

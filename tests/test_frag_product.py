@@ -88,3 +88,36 @@ def test_pairs_bias_residual(hip, name, m, n):
         hip.gemm_frag(xp, m, dg, qt, n, k, bias=b1.cuda(), residual=out, out=out, mt=5, ns=3)    # in place, as on the residual stream
         tol = dict(rtol=8e-3, atol=2e-2) if dtype == torch.bfloat16 else dict(rtol=2e-3, atol=8e-3)
         torch.testing.assert_close(out.cpu().double(), xd @ wg.t() + b1.double() + res.double(), **tol)
+
+
+@pytest.mark.parametrize("rows,width", [(33, 128), (77, 2048), (130, 4096 + 128), (64, 9216)])
+def test_norm_in_fragment_order(hip, rows, width):
+    g = torch.Generator().manual_seed(7)
+    x, res = torch.randn(rows, width, generator=g).half().cuda(), torch.randn(rows, width, generator=g).half().cuda()
+    w = (1 + 0.1 * torch.randn(width, generator=g)).half().cuda()
+    h0, h1 = torch.empty_like(x), torch.empty_like(x)
+    want = hip.frag_pack(hip.rms_norm(x, w, 1e-5, residual=res, res_out=h0))
+    got = hip.rms_norm(x, w, 1e-5, residual=res, res_out=h1, frags=True)
+    assert got.shape == (rows, width) and torch.equal(h0, h1)
+    tiles = (rows + 15) // 16
+    live = (torch.arange(tiles * 16, device="cuda") < rows).view(tiles, 1, 16, 1)        # rows past the last one are not written
+    view = (width // 32, tiles, 4, 16, 8)
+    assert torch.equal(torch.where(live, got.data.view(view), 0), torch.where(live, want.view(view), 0))
+
+
+@pytest.mark.parametrize("name", ["sym_int4", "q4_k"])
+@pytest.mark.parametrize("m", [64, 77, 203, 400])
+def test_norm_pair_down_without_rows_in_between(hip, name, m):
+    """norm -> gate / up -> down with x in fragment order all along, against the same products on rows"""
+    n, k = 1536, 1024
+    qt = Q.ggml_tensor_qtype[name]
+    (dg, _), (du, _), (dd, _) = _weight(n, k, qt, 3), _weight(n, k, qt, 4), _weight(k, n, qt, 5)
+    x = _x(m, k, 6)[0].contiguous()
+    w = torch.ones(k, dtype=torch.float16, device="cuda")
+    y = hip.rms_norm(x, w, 1e-5)
+    ref = hip.gemm_lowbit(hip.gemm_lowbit_ex(y, dg, qt, n, k, w2=du, act="silu"), dd, qt, k, n, out_dtype=torch.float32)
+    f = hip.rms_norm(x, w, 1e-5, frags=True)
+    f = hip.gemm_lowbit_ex(f, dg, qt, n, k, w2=du, act="silu", out_frags=True)
+    got = hip.gemm_lowbit(f, dd, qt, k, n, out_dtype=torch.float32)
+    # the same fp16 operands; sums in another order move the pair's results by a rounding to fp16 (2^-11) here and there
+    assert ((got - ref).norm() / ref.norm()).item() < 2.0 ** -11

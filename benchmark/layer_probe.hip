@@ -132,7 +132,7 @@ int main(int argc, char** argv) {
   };
   auto k_attn = [&](int l) {
     const int rc = bigdl_attn_decode(qkv, kc[l], vc[l], attn, ws, counters, past, nullptr, 0, nullptr, rope, nullptr, max_pos, D, 0,
-                                     0.088388f, 0.0f, 1, Hq, Hkv, 1, 0, 1, QKV, Lmax, D, splits, 0, 1, 0, 1, nullptr, nullptr, st);
+                                     0.088388f, 0.0f, 1, Hq, Hkv, 1, 0, 1, QKV, Lmax, D, splits, 0, 1, 0, 1, nullptr, nullptr, 0, st);
     if (rc != 0) { printf("attn launch failed %d\n", rc); exit(1); }
   };
   auto k_o = [&](int l) {

@@ -54,7 +54,12 @@ struct AttnArgs {
   int defer_combine;     // 1: stop after writing the per-split partials (the consumer GEMV combines them)
   int nchunk, gchunk;    // query-head chunks per kv head and heads per chunk (1, Hq/Hkv unless Hq/Hkv > 32)
   int ablate;            // measurement builds only (bigdl_attn_set_ablation): 1 = K / V loads without the products
+  int frag_mt;             // out in fragment order of so many 16-row tiles (0: rows), for the product that reads it
 };
+// place of (row m, column c) of the output
+__device__ __forceinline__ int64_t out_at(int m, int c, int width, int frag_mt) {
+  return frag_mt > 0 ? frag_at(m, c, frag_mt) : (int64_t)m * width + c;
+}
 
 constexpr float NEG_BIG = -1.0e30f;
 constexpr int ATT_NW = 8;          // wavefronts per workgroup
@@ -741,7 +746,7 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
     if (single) {
       const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
       const int tok = a.q_off + row / Gc, gq = g0 + row % Gc;
-      _Float16* dst = a.out + (int64_t)(b * a.q_total + tok) * (a.Hq * D) + (hkv * G + gq) * D + d4;
+      _Float16* dst = a.out + out_at(b * a.q_total + tok, (hkv * G + gq) * D + d4, a.Hq * D, a.frag_mt);
       half4 hv = {(_Float16)(acc[0] * inv), (_Float16)(acc[1] * inv), (_Float16)(acc[2] * inv), (_Float16)(acc[3] * inv)};
       *(half4*)dst = hv;
     } else {
@@ -785,7 +790,7 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
     }
     const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
     const int tok = a.q_off + row / Gc, gq = g0 + row % Gc;
-    _Float16* dst = a.out + (int64_t)(b * a.q_total + tok) * (a.Hq * D) + (hkv * G + gq) * D + d4;
+    _Float16* dst = a.out + out_at(b * a.q_total + tok, (hkv * G + gq) * D + d4, a.Hq * D, a.frag_mt);
     half4 hv = {(_Float16)(acc[0] * inv), (_Float16)(acc[1] * inv), (_Float16)(acc[2] * inv), (_Float16)(acc[3] * inv)};
     *(half4*)dst = hv;
   }
@@ -939,7 +944,7 @@ extern "C" int bigdl_attn_decode(void* qkv, void* kc, void* vc, void* out, float
                                  const float* rope, const int* position_ids, int rope_max_pos, int rot, int interleaved, float scale,
                                  float softcap, int B, int Hq, int Hkv, int q_total, int q_off, int q_cnt, int ld,
                                  int Lmax, int D, int splits, int window, int fp8, int append, int defer_combine,
-                                 void* k_scale, void* v_scale, hipStream_t stream) {
+                                 void* k_scale, void* v_scale, int frag, hipStream_t stream) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || q_cnt <= 0 || q_off < 0 || q_off + q_cnt > q_total || splits <= 0 ||
       (Lmax & 255) || (ld & 7)) return -1;
   if (((uintptr_t)qkv | (uintptr_t)kc | (uintptr_t)vc | (uintptr_t)ws | (uintptr_t)out) & 15) return -1;
@@ -960,6 +965,8 @@ extern "C" int bigdl_attn_decode(void* qkv, void* kc, void* vc, void* out, float
   a.q_total = q_total; a.q_off = q_off; a.q_cnt = q_cnt; a.defer_combine = defer_combine;
   a.nchunk = nchunk; a.gchunk = gchunk; a.ablate = g_attn_ablate;
   a.ks = (_Float16*)k_scale; a.vs = (_Float16*)v_scale;
+  if (frag && ((Hq * D) & 127)) return -1;
+  a.frag_mt = frag ? (B * q_total + 15) / 16 : 0;
   if (k_scale != nullptr || v_scale != nullptr) {
     // int4 caches: the kernel appends itself (quantization needs the whole rotated key), full rotary only
     if (k_scale == nullptr || v_scale == nullptr || fp8 || a.rot < 0 || (((uintptr_t)k_scale | (uintptr_t)v_scale) & 15)) return -1;

@@ -39,6 +39,7 @@ struct PrefillArgs {
   int causal, window;
   int v_transposed;                  // v is [B, Hkv, D, Lk] (v_ss = stride of d, keys contiguous)
   int kv_e5m2;                       // k / v hold e5m2 bytes (strides in bytes); needs v_transposed
+  int frag_mt;                       // out in fragment order of so many 16-row tiles, rows [B * Sq] (0: rows, o_sb and o_ss)
 };
 
 constexpr int PF_BN = 64;
@@ -395,7 +396,8 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(PrefillArgs a) {
         half4 h;
 #pragma unroll
         for (int e = 0; e < 4; ++e) h[e] = (_Float16)(o[u][db][e] * inv);
-        *(half4*)(op + 16 * db + 4 * g) = h;
+        if (a.frag_mt > 0) *(half4*)(a.out + frag_at(b * a.Sq + qi[u], hq * DR + 16 * db + 4 * g, a.frag_mt)) = h;
+        else *(half4*)(op + 16 * db + 4 * g) = h;
       }
     }
 }
@@ -670,13 +672,15 @@ extern "C" int bigdl_attn_prefill(const void* q, const void* k, const void* v, v
                                   int Hkv, int Sq, int Lk, int D, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb,
                                   int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t o_sb,
                                   int64_t o_ss, int64_t m_sb, int64_t m_sq, int64_t m_sh, const float* alibi, float scale,
-                                  float softcap, int causal, int window, int v_transposed, int kv_e5m2, hipStream_t st) {
+                                  float softcap, int causal, int window, int v_transposed, int kv_e5m2, int frag, hipStream_t st) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || Sq <= 0 || Lk <= 0 || B > 65535 || Hq > 65535) return -1;
   if (causal && Lk < Sq) return -1;
   if (((uintptr_t)q & 15) || ((uintptr_t)k & 15) || ((uintptr_t)v & 15) || ((uintptr_t)out & 7)) return -1;
   if ((q_sb | q_sh | q_ss | k_sb | k_sh | k_ss | v_sb | v_sh | v_ss) & 7) return -1;    // 16-byte (8-byte: e5m2) row starts
   if ((o_sb | o_ss) & 3) return -1;
   PrefillArgs a;
+  if (frag && ((Hq * D) & 127)) return -1;
+  a.frag_mt = frag ? (B * Sq + 15) / 16 : 0;
   a.q = (const _Float16*)q; a.k = (const _Float16*)k; a.v = (const _Float16*)v; a.out = (_Float16*)out;
   a.mask = (const _Float16*)mask; a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.Sq = Sq; a.Lk = Lk;
   a.q_sb = q_sb; a.q_sh = q_sh; a.q_ss = q_ss; a.k_sb = k_sb; a.k_sh = k_sh; a.k_ss = k_ss;

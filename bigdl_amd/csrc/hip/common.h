@@ -30,6 +30,12 @@ __device__ __forceinline__ float4v mfma16(half8 a, half8 b, float4v c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
+// Fragment order of fp16 activations, [k / 32][row / 16][lane][8]: lane 16 g + r of a fragment holds row r, columns 8 g .. 8 g + 7
+// (gemm_frag_kernel.h).  Place, in halves, of (row m, column k), mt_all row tiles:
+__device__ __forceinline__ int64_t frag_at(int m, int k, int mt_all) {
+  return (((int64_t)(k >> 5) * mt_all + (m >> 4)) * 64 + ((k & 31) >> 3) * 16 + (m & 15)) * 8 + (k & 7);
+}
+
 __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t mask, uint32_t orv) { return (a & mask) | orv; }
 
 union H8 {

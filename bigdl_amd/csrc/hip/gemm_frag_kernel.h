@@ -26,10 +26,6 @@ namespace bigdl {
 
 // out_type of an output in fragment order, fp16: x of the next product
 constexpr int OUT_FRAG = 3;
-// place, in halves, of (row m, column k) in fragment order
-__device__ __forceinline__ int64_t frag_at(int m, int k, int mt_all) {
-  return (((int64_t)(k >> 5) * mt_all + (m >> 4)) * 64 + ((k & 31) >> 3) * 16 + (m & 15)) * 8 + (k & 7);
-}
 
 struct FragArgs {
   const _Float16* xp;     // [KT * 4][mt_all][64 lanes][8]: see frag_pack_kernel

@@ -125,8 +125,7 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const void* x, const void
       load8<DT>(w, c, g);
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[i][j] = v[i][j] * rs * (g[j] + offset);
-      const int64_t in_order = (((int64_t)(c >> 5) * frag_mt + (row >> 4)) * 64 + ((c & 31) >> 3) * 16 + (row & 15)) * 8;
-      store8<DT>(out, frag_mt > 0 ? in_order : row * (int64_t)H + c, v[i]);
+      store8<DT>(out, frag_mt > 0 ? frag_at((int)row, c, frag_mt) : row * (int64_t)H + c, v[i]);
     }
   }
 }

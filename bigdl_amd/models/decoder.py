@@ -833,7 +833,9 @@ class NativeDecoder:
                 kk, vt, kv8 = cache.k[li][rows_, :, :past + s], cache.v[li][rows_, :, :, :past + s], True
             else:
                 kk, vt = self._read_cache(li, past + s, slot)
-            attn = self._sdpa(q, kk, vt, past, lw.window, kv_e5m2=kv8).reshape(b * s, hq * d)
+            attn = self._sdpa(q, kk, vt, past, lw.window, kv_e5m2=kv8, frags=nd == 0 and self._takes_frags(b * s, lw.o))
+            if type(attn) is not hip.Frags:
+                attn = attn.reshape(b * s, hq * d)
             if snap is not None:
                 # the prompt has attended to all of its keys; what later tokens will see is the voted subset + the window
                 from ..transformers.kv import snapkv_indices
@@ -1143,14 +1145,14 @@ class NativeDecoder:
             return kf, vf
         return k, vt
 
-    def _sdpa(self, q, k, vt, past, window, kv_e5m2=False):
+    def _sdpa(self, q, k, vt, past, window, kv_e5m2=False, frags=False):
         """q [B,Hq,S,D], k [B,Hkv,past+S,D], vt = V^T [B,Hkv,D,past+S] -> [B, S, Hq*D]; with ``kv_e5m2`` k / vt are
-        views of the fp8 cache (bytes)"""
+        views of the fp8 cache (bytes).  ``frags``: in fragment order where the kernel of this package runs"""
         cfg = self.cfg
         if cfg.head_dim in (64, 96, 128, 256) and vt.stride(2) % 8 == 0 and vt.data_ptr() % 16 == 0:
             from ..ops import hip
             return hip.attn_prefill(q, k, vt, scale=self.attn_scale, causal=True, softcap=cfg.attn_softcap, window=window,
-                                    v_transposed=True, alibi=self.alibi, kv_e5m2=kv_e5m2)
+                                    v_transposed=True, alibi=self.alibi, kv_e5m2=kv_e5m2, frags=frags)
         assert not kv_e5m2
         if self.alibi is not None:
             raise NotImplementedError("ALiBi attention needs head_dim 64, 96 or 128")
@@ -1205,6 +1207,10 @@ class NativeDecoder:
                                     device=dev),
             "splits": splits,
         }
+        st["attn_frags"] = None              # for output projections that take x in fragment order
+        if m > 32 and cfg.q_size % 128 == 0:
+            st["attn_frags"] = hip.Frags(torch.zeros(hip.lib().bigdl_frag_halves(m, cfg.q_size), dtype=torch.float16, device=dev), m,
+                                         cfg.q_size)
         if cfg.mla_kv_lora:
             st["mla_lat"] = torch.zeros(m, cfg.mla_q_lora + cfg.mla_kv_lora + cfg.rot_dim, dtype=torch.float16, device=dev)
         # with several KV splits the cross-split combine is folded into the o_proj GEMV's x staging
@@ -1359,6 +1365,9 @@ class NativeDecoder:
                                 n_kv_heads=cfg.num_kv_heads, head_dim=cfg.head_dim, q_len=q_len, batch=batch,
                                 rot_dim=cfg.rot_dim or cfg.head_dim, interleaved=cfg.rope_interleaved,
                                 attn_scaling=self.rope_scaling_factor)
+            if st["attn_frags"] is not None:
+                to_frags = not self.fold_batched_norm and self._takes_frags(batch * q_len, lw.o, prompt=False)
+                attn = st["attn_frags"] if to_frags else st["attn"]
             hip.attn_decode(qkv, cache.k[li], cache.v[li], cache.past_len, attn, st["ws"], st["counters"],
                             n_heads=cfg.num_heads, n_kv_heads=cfg.num_kv_heads, head_dim=cfg.head_dim, q_len=q_len,
                             batch=batch, scale=self.attn_scale, splits=st["splits"], softcap=cfg.attn_softcap,

@@ -121,3 +121,44 @@ def test_norm_pair_down_without_rows_in_between(hip, name, m):
     got = hip.gemm_lowbit(f, dd, qt, k, n, out_dtype=torch.float32)
     # the same fp16 operands; sums in another order move the pair's results by a rounding to fp16 (2^-11) here and there
     assert ((got - ref).norm() / ref.norm()).item() < 2.0 ** -11
+
+
+@pytest.mark.parametrize("b,sq,hq,d", [(1, 77, 4, 128), (3, 20, 6, 64), (1, 130, 4, 96)])
+def test_prompt_attention_in_fragment_order(hip, b, sq, hq, d):
+    q, k, v = (torch.randn(b, hq, sq, d, device="cuda").half() for _ in range(3))
+    want = hip.frag_pack(hip.attn_prefill(q, k, v, scale=d ** -0.5).view(b * sq, hq * d))
+    got = hip.attn_prefill(q, k, v, scale=d ** -0.5, frags=True)
+    tiles = (b * sq + 15) // 16
+    live = (torch.arange(tiles * 16, device="cuda") < b * sq).view(tiles, 1, 16, 1)
+    view = (hq * d // 32, tiles, 4, 16, 8)
+    assert torch.equal(torch.where(live, got.data.view(view), 0), torch.where(live, want.view(view), 0))
+
+
+@pytest.mark.parametrize("batch,past,fp8", [(33, 40, False), (50, 300, True), (1, 90, False)])
+def test_engine_with_and_without_fragment_order(hip, monkeypatch, batch, past, fp8):
+    """prompt pass and decode steps: every product that takes x in fragment order against the same engine on rows"""
+    from bigdl_amd.models import decoder as D
+    cfg = D.DecoderConfig(vocab_size=2048, hidden_size=1024, intermediate_size=2048, num_layers=2, num_heads=8, num_kv_heads=4,
+                          head_dim=128, max_position=512)
+    ids = torch.randint(0, 2048, (batch, past + 2), generator=torch.Generator().manual_seed(3)).cuda()
+    taken = []
+
+    def run(frags):
+        if not frags:
+            monkeypatch.setattr(hip, "gemm_lowbit_frag", lambda *a, **k: False)
+        else:
+            real = hip._gemm_frag_dense
+            monkeypatch.setattr(hip, "_gemm_frag_dense", lambda x, kind, *a, **k: (taken.append(kind), real(x, kind, *a, **k))[1])
+        eng = D.build_random_decoder(cfg, Q.SYM_INT4, device="cuda", seed=0)
+        eng.ensure_cache(batch, past + 16, fp8=fp8)
+        out = [eng.prefill(ids[:, :past]).view(batch, -1)]
+        for j in range(2):
+            out.append(eng.decode(ids[:, past + j:past + j + 1].contiguous(), 1)[0].clone())
+        monkeypatch.undo()
+        return out
+
+    with_frags, on_rows = run(True), run(False)
+    assert 2 in taken
+    for a, b in zip(with_frags, on_rows):
+        # the same fp16 operands and fp32 sums in another order: single roundings to fp16 (2^-11) differ and pass through two layers
+        assert ((a - b).norm() / b.norm()).item() < 4e-3

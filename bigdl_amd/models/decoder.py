@@ -524,14 +524,15 @@ class NativeDecoder:
     def _takes_frags(self, rows, lin: Optional[Lin], w2: Optional[Lin] = None, prompt=True):
         """whether the product of so many rows (with w2: the gate / up pair) takes x in fragment order from its producer: the norm
         in front of it, or the pair in front of a down projection"""
-        from ..ops import hip
-        if lin is None or not lin.fused or rows <= GEMV_MAX_ROWS or lin.k % 128:
+        # (513 rows and more of such a K are the prompt kernel's; asked four times a layer, so the cheapest question first)
+        if not 32 < rows <= 512 or lin is None or not lin.fused or lin.k & 127:
             return False
         if w2 is not None and not (w2.fused and w2.qtype == lin.qtype and w2.n == lin.n and w2.k == lin.k):
             return False
         if rows > GEMM_MAX_ROWS and not (prompt and self.prefill_fused and not Lin.cache_dense and not self.prefill_fp8):
             return False
-        return hip.gemm_lowbit_frag(rows, lin.n, lin.k, lin.qtype, pair=w2 is not None, bf16=True)
+        from ..ops import hip
+        return hip.gemm_lowbit_frag(rows, lin.n, lin.k, lin.qtype, None, w2 is not None, True)
 
     def _mlp_takes_frags(self, rows, lw):
         return self.cfg.gated_mlp and lw.moe is None and lw.gate is not None and self._takes_frags(rows, lw.gate, lw.up)
@@ -691,7 +692,7 @@ class NativeDecoder:
         elif cfg.gated_mlp:
             gt, up = lw.gate, lw.up
             two = gt.fused and up.fused and gt.qtype == up.qtype and gt.n == up.n and gt.k == up.k and x.dtype == torch.float16
-            frag = (two and x.shape[0] > GEMM_MAX_ROWS and self.prefill_fused and not Lin.cache_dense and not self.prefill_fp8
+            frag = (two and GEMM_MAX_ROWS < x.shape[0] and self.prefill_fused and not Lin.cache_dense and not self.prefill_fp8
                     and hip.gemm_lowbit_frag(x.shape[0], gt.n, gt.k, gt.qtype, pair=True))
             if (not frag and gt.fused and up.fused and gt.qtype == up.qtype and gt.n == up.n and gt.n % 16 == 0 and self.prefill_fused
                     and x.shape[0] > GEMM_MAX_ROWS and x.dtype == torch.float16 and not Lin.cache_dense and not self.prefill_fp8
@@ -1209,7 +1210,7 @@ class NativeDecoder:
         }
         st["attn_frags"] = None              # for output projections that take x in fragment order
         if m > 32 and cfg.q_size % 128 == 0:
-            st["attn_frags"] = hip.Frags(torch.zeros(hip.lib().bigdl_frag_halves(m, cfg.q_size), dtype=torch.float16, device=dev), m,
+            st["attn_frags"] = hip.Frags(torch.zeros(hip.frag_halves(m, cfg.q_size), dtype=torch.float16, device=dev), m,
                                          cfg.q_size)
         if cfg.mla_kv_lora:
             st["mla_lat"] = torch.zeros(m, cfg.mla_q_lora + cfg.mla_kv_lora + cfg.rot_dim, dtype=torch.float16, device=dev)

@@ -384,7 +384,8 @@ extern "C" int bigdl_gemm_frag_dense(const void* x, const void* w, const void* w
                                      int ldo, int qtype, int act, int out_type, int x_kind, hipStream_t stream) {
   qtype = t16_kernel_qtype(qtype);
   if (M <= 0 || N <= 0 || K <= 0 || (K & 31) || ((uintptr_t)x & 15) || ((uintptr_t)w & 15) || !is_t16(qtype)) return -1;
-  if (x_kind != X_FRAGMENTS && ((ldx & 7) || ldx < K)) return -1;
+  if (x_kind != X_FRAGMENTS && (ldx & 7)) return -1;
+  if (x_kind != X_FRAGMENTS && (int64_t)M * ldx >= (1ll << 31)) return -6;
   if (w2 != nullptr && ((uintptr_t)w2 & 15)) return -1;
   if (out_type == OUT_FRAG && (w2 == nullptr || residual != nullptr || (N & 127) || ((uintptr_t)out & 15))) return -1;
   if (out_type < 0 || out_type > OUT_FRAG || x_kind < 0 || x_kind > X_FRAGMENTS) return -3;

@@ -1,5 +1,6 @@
 // Dequant-fused product for a few rows of x on gfx950:  y[M,N] = f(x[M,K] . dequant(W)[N,K]^T), up to 64 rows (blocks of
-// 16 * MT rows above that).  Batched decode, short prompts and speculative verification run on it; up to 16 rows it folds
+// 16 * MT rows above that).  Batched decode, short prompts and speculative verification run on it, as far as they do not on the product
+// on x in fragment order (gemm_frag_kernel.h: most products of more than 64 rows); up to 16 rows it folds
 // the RMSNorm of x in, and a gate / up pair is one launch with act(g) * u in its epilogue.
 //
 // What bounds it: the weights (28 MB for Llama-2-7B's qkv, 5.6 us at the 5 TB/s that 256 CUs draw) and, from about 32 rows on, x,

@@ -162,3 +162,13 @@ def test_engine_with_and_without_fragment_order(hip, monkeypatch, batch, past, f
     for a, b in zip(with_frags, on_rows):
         # the same fp16 operands and fp32 sums in another order: single roundings to fp16 (2^-11) differ and pass through two layers
         assert ((a - b).norm() / b.norm()).item() < 4e-3
+
+
+def test_rows_of_stride_zero(hip):
+    """one row seen 77 times: accepted by the other kernels, so by the pass that orders x too"""
+    n, k = 4096, 4096
+    qt = Q.SYM_INT4
+    w = (torch.randint(0, 256, (host.device_nbytes(qt, n, k),), dtype=torch.uint8) & 0xBF).cuda()
+    x = torch.randn(1, k).half().cuda().expand(77, k)
+    out = hip.gemm_lowbit(x, w, qt, n, k)
+    assert torch.equal(out, hip.gemm_lowbit(x.contiguous(), w, qt, n, k)) and torch.equal(out, out[:1].expand(77, n))

@@ -524,8 +524,9 @@ class NativeDecoder:
     def _takes_frags(self, rows, lin: Optional[Lin], w2: Optional[Lin] = None, prompt=True):
         """whether the product of so many rows (with w2: the gate / up pair) takes x in fragment order from its producer: the norm
         in front of it, or the pair in front of a down projection"""
-        # (513 rows and more of such a K are the prompt kernel's; asked four times a layer, so the cheapest question first)
-        if not 32 < rows <= 512 or lin is None or not lin.fused or lin.k & 127:
+        # (513 rows and more of such a K are the prompt kernel's, up to GEMV_MAX_ROWS gemv_lowbit's; asked four times a layer, so the
+        # cheapest question first)
+        if not 32 < rows <= 512 or rows <= GEMV_MAX_ROWS or lin is None or not lin.fused or lin.k & 127:
             return False
         if w2 is not None and not (w2.fused and w2.qtype == lin.qtype and w2.n == lin.n and w2.k == lin.k):
             return False

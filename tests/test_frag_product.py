@@ -164,6 +164,40 @@ def test_engine_with_and_without_fragment_order(hip, monkeypatch, batch, past, f
         assert ((a - b).norm() / b.norm()).item() < 4e-3
 
 
+def test_only_known_entries_take_fragment_order(hip):
+    m, k, n = 48, 256, 128
+    w = _weight(n, k, Q.SYM_INT4, 1)[0]
+    x = hip.rms_norm(torch.randn(m, k).half().cuda(), torch.ones(k, dtype=torch.float16, device="cuda"), 1e-5, frags=True)
+    rows = torch.zeros(m, k, dtype=torch.float16, device="cuda")
+    for call in (lambda: hip.gemv_lowbit(x, w, Q.SYM_INT4, n, k), lambda: hip.gemm_prompt(x, w, Q.SYM_INT4, n, k),
+                 lambda: hip.gemm_rows(x, w, Q.SYM_INT4, n, k), lambda: hip.frag_pack(x), lambda: hip.bf16_to_f16(x),
+                 lambda: hip.gemm_lowbit(rows, w, Q.SYM_INT4, n, k, out=hip.Frags(rows.new_empty(hip.frag_halves(m, n)), m, n))):
+        with pytest.raises(ValueError):
+            call()
+
+
+@pytest.mark.parametrize("gemv_max", [16, 64])
+def test_engine_with_products_on_gemv(hip, monkeypatch, gemv_max):
+    """40 rows: the products run on gemv_lowbit where BIGDL_GEMV_MAX_ROWS says so, and get rows from whatever is in front of them"""
+    from bigdl_amd.models import decoder as D
+    cfg = D.DecoderConfig(vocab_size=1024, hidden_size=1024, intermediate_size=2048, num_layers=2, num_heads=16, num_kv_heads=4,
+                          head_dim=128, max_position=512, norm="layer", gated_mlp=False, act="gelu")     # (a pair is 32 rows at most there)
+    assert hip.gemm_lowbit_frag(40, 1024, 2048, Q.SYM_INT4, None, False, True)
+    ids = torch.randint(0, 1024, (40, 9), generator=torch.Generator().manual_seed(3)).cuda()
+
+    def run():
+        eng = D.build_random_decoder(cfg, Q.SYM_INT4, device="cuda", seed=0)
+        eng.ensure_cache(40, 64, fp8=False)
+        return eng.prefill(ids[:, :8]).view(40, -1), eng.decode(ids[:, 8:].contiguous(), 1)[0].clone()
+
+    monkeypatch.setattr(D, "GEMV_MAX_ROWS", gemv_max)
+    got = run()
+    monkeypatch.setattr(hip, "gemm_lowbit_frag", lambda *a, **k: False)
+    for a, b in zip(got, run()):
+        # the same fp16 operands and fp32 sums in another order, as above
+        assert ((a - b).norm() / b.norm()).item() < 4e-3
+
+
 def test_rows_of_stride_zero(hip):
     """one row seen 77 times: accepted by the other kernels, so by the pass that orders x too"""
     n, k = 4096, 4096

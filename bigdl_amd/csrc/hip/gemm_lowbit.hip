@@ -343,6 +343,8 @@ extern "C" int bigdl_gemm_lowbit(const void* x, const void* w, void* out, const 
 enum XKind { X_ROWS = 0, X_ROWS_BF16 = 1, X_FRAGMENTS = 2 };
 static bool takes_frag_kernel(int ldx, int M, int N, int K, int qtype, bool pair, int x_kind, FragPlan* plan) {
   if (M <= 32 || !is_t16(qtype)) return false;
+  // (rows that bigdl_gemm_frag_dense refuses: the callers' other ways take them as they are, or 256 at a time)
+  if (x_kind != X_FRAGMENTS && ((ldx & 7) || (int64_t)M * ldx >= (1ll << 31))) return false;
   *plan = frag_plan(M, N, K, qtype, pair, !pair);
   if (plan->ns == 0) return false;
   if (x_kind == X_FRAGMENTS) return true;

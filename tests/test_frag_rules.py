@@ -26,3 +26,14 @@ def test_engine_gives_gemv_rows(monkeypatch, gemv_max, taken):
     eng = SimpleNamespace(prefill_fused=True, prefill_fp8=False)
     for prompt in (False, True):
         assert D.NativeDecoder._takes_frags(eng, 64, lin, prompt=prompt) == taken
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_rows_far_apart_stay_with_the_other_kernels(bf16):
+    """a call that the rule takes is one that the launcher accepts: rows 16 bytes aligned, the last one within 2^31 elements.  300 last
+    positions of sequences of 2048 tokens are 600 K row widths."""
+    m, k = 300, 4544
+    assert hip.gemm_lowbit_frag(m, 4544, k, QT, k, False, bf16)
+    assert hip.gemm_lowbit_frag(m, 4544, k, QT, 1 << 22, False, bf16)
+    assert not hip.gemm_lowbit_frag(m, 4544, k, QT, 2048 * k, False, bf16)
+    assert not hip.gemm_lowbit_frag(m, 4544, k, QT, k + 4, False, bf16)

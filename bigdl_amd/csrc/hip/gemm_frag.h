@@ -4,6 +4,12 @@
 #include <stdint.h>
 
 namespace bigdl {
+// Rows of a call that the rule (gemm_lowbit.hip) gives to this product: above 512 only where K is no multiple of 128 and the
+// alternative is the tile kernel, 256 rows at a time.  Measured at 200 such products of 513 to 2500 rows, 10 formats, pairs among them:
+// 1.06 to 3.4 times the former speed (4672 x 4544, 1024 rows, sym_int4 141 -> 75 us, sym_int8 153 -> 80; 14336 x 4128, 1500 rows,
+// sym_int4 310 -> 293).  One call of 4096 rows of 14336 x 4128 lost (asym_int4 926 -> 1143 us, sym_int8 999 -> 1155), so more rows go in
+// pieces, which also bounds the copy of x.
+constexpr int FRAG_MAX_ROWS = 2048;
 struct FragArgs;
 struct FragPlan {
   int mt, ns;               // 16-row tiles of x and 16-column weight tiles of a workgroup (pair form: ns / 2 of each weight); ns 0: none

@@ -1,5 +1,5 @@
-// Dequant-fused product on x in fragment order for gfx950:  y[M,N] = f(x[M,K] . dequant(W)[N,K]^T), 33 rows to a few hundred: short
-// prompts, wide decode batches, module calls.
+// Dequant-fused product on x in fragment order for gfx950:  y[M,N] = f(x[M,K] . dequant(W)[N,K]^T), 33 to 512 rows, and up to
+// FRAG_MAX_ROWS where K is no multiple of 128: short prompts, wide decode batches, module calls.
 //
 // What bounds products of so many rows is neither the weights (28 MB for Llama-2-7B's qkv, 6 us) nor the matrix cores (64 rows:
 // 5 us) but x, which every workgroup pulls through its CU's L1.  Measured rates per CU, x in L2: 70 GB/s for requests of 8 rows x

@@ -348,6 +348,7 @@ static bool takes_frag_kernel(int ldx, int M, int N, int K, int qtype, bool pair
   *plan = frag_plan(M, N, K, qtype, pair, !pair);
   if (plan->ns == 0) return false;
   if (x_kind == X_FRAGMENTS) return true;
+  if (M > FRAG_MAX_ROWS) return false;
   double other;
   if (M > 256 && K >= 256 && (K & 127) == 0) {
     if (M > 512) return false;                         // (what the estimates cover)

@@ -297,17 +297,22 @@ def dequant_weight_rows(weight: FP4Params, row0: int, nrows: int, dtype=torch.fl
 
 def lowbit_rows(xh, w, qtype, n, k, bias=None, out_dtype=None):
     """More than GEMM_MAX_ROWS fp16 rows times a T16 weight on this repository's own kernels: the one that takes x in fragment
-    order where it is expected to be ahead, the prompt-sized fused GEMM where that applies (K a multiple of 128), otherwise the
-    mid-size fused GEMM GEMM_MAX_ROWS rows at a time."""
+    order where it is expected to be ahead, the prompt-sized fused GEMM where that applies (K a multiple of 128), otherwise
+    FRAG_MAX_ROWS rows at a time on the former, or GEMM_MAX_ROWS on the mid-size fused GEMM."""
     from ..ops import hip
     m = xh.shape[0]
-    if hip.gemm_lowbit_frag(m, n, k, qtype, ldx=xh.stride(0)):
+    if hip.gemm_lowbit_frag(m, n, k, qtype, xh.stride(0)):
         return hip.gemm_lowbit(xh, w, qtype, n, k, bias=bias, out_dtype=out_dtype)
     if hip.gemm_prompt_supported(qtype, k):
         return hip.gemm_prompt(xh, w, qtype, n, k, bias=bias, out_dtype=out_dtype)
     y = torch.empty(m, n, dtype=out_dtype or torch.float16, device=xh.device)
-    for r0 in range(0, m, GEMM_MAX_ROWS):
-        hip.gemm_lowbit(xh[r0:r0 + GEMM_MAX_ROWS], w, qtype, n, k, bias=bias, out=y[r0:r0 + GEMM_MAX_ROWS])
+    r0 = 0
+    while r0 < m:
+        rows = min(m - r0, hip.FRAG_MAX_ROWS)
+        if rows > GEMM_MAX_ROWS and not hip.gemm_lowbit_frag(rows, n, k, qtype, xh.stride(0)):
+            rows = GEMM_MAX_ROWS
+        hip.gemm_lowbit(xh[r0:r0 + rows], w, qtype, n, k, bias=bias, out=y[r0:r0 + rows])
+        r0 += rows
     return y
 
 

@@ -90,6 +90,20 @@ def test_pairs_bias_residual(hip, name, m, n):
         torch.testing.assert_close(out.cpu().double(), xd @ wg.t() + b1.double() + res.double(), **tol)
 
 
+@pytest.mark.parametrize("name", ["sym_int4", "fp6"])
+@pytest.mark.parametrize("m", [700, 2048, 2100])
+def test_many_rows_of_a_ragged_k(hip, name, m):
+    """a K that the prompt kernel does not take: one call of up to FRAG_MAX_ROWS rows, more in pieces"""
+    from bigdl_amd.transformers.low_bit_linear import lowbit_rows
+    n, k = 328, 1184
+    qt = Q.ggml_tensor_qtype[name]
+    dev, w = _weight(n, k, qt, 1)
+    x, xd = _x(m, k, 2)
+    bias = torch.randn(n, generator=torch.Generator().manual_seed(3)).half()
+    assert hip.gemm_lowbit_frag(min(m, hip.FRAG_MAX_ROWS), n, k, qt, x.stride(0))
+    _close(lowbit_rows(x, dev, qt, n, k, bias=bias.cuda(), out_dtype=torch.float32), xd, w, xd @ w.t() + bias.double())
+
+
 @pytest.mark.parametrize("rows,width", [(33, 128), (77, 2048), (130, 4096 + 128), (64, 9216)])
 def test_norm_in_fragment_order(hip, rows, width):
     g = torch.Generator().manual_seed(7)

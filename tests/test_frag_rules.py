@@ -7,6 +7,7 @@ import torch
 from bigdl_amd import qtypes as Q
 from bigdl_amd.models import decoder as D
 from bigdl_amd.ops import hip
+from bigdl_amd.transformers.low_bit_linear import lowbit_rows
 
 QT = Q.ggml_tensor_qtype["sym_int4"]
 
@@ -37,3 +38,16 @@ def test_rows_far_apart_stay_with_the_other_kernels(bf16):
     assert hip.gemm_lowbit_frag(m, 4544, k, QT, 1 << 22, False, bf16)
     assert not hip.gemm_lowbit_frag(m, 4544, k, QT, 2048 * k, False, bf16)
     assert not hip.gemm_lowbit_frag(m, 4544, k, QT, k + 4, False, bf16)
+
+
+@pytest.mark.parametrize("name,n,k", [("asym_int4", 14336, 4128), ("sym_int8", 14336, 4128), ("sym_int4", 4672, 4544)])
+def test_many_rows_go_in_pieces(monkeypatch, name, n, k):
+    """no multiple of 128 columns: calls of up to FRAG_MAX_ROWS rows, as measured; of 4096 rows the first two were slower than before"""
+    qt = Q.ggml_tensor_qtype[name]
+    assert hip.gemm_lowbit_frag(hip.FRAG_MAX_ROWS, n, k, qt) and not hip.gemm_lowbit_frag(hip.FRAG_MAX_ROWS + 1, n, k, qt)
+    got = []
+    monkeypatch.setattr(hip, "gemm_lowbit", lambda x, *a, out, **kw: got.append((x[0, 0].item(), x.shape[0], out[0, 0].item(), out.shape[0])))
+    rows = torch.arange(4196).half()[:, None].repeat(1, 8)[:, :1]
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: rows.expand(4196, n))
+    lowbit_rows(rows.expand(4196, k), None, qt, n, k)
+    assert got == [(0, 2048, 0, 2048), (2048, 2048, 2048, 2048), (4096, 100, 4096, 100)]

@@ -7,7 +7,7 @@ import torch
 from bigdl_amd import qtypes as Q
 from bigdl_amd.models import decoder as D
 from bigdl_amd.ops import hip
-from bigdl_amd.transformers.low_bit_linear import lowbit_rows
+from bigdl_amd.transformers.low_bit_linear import lowbit_matmul, lowbit_rows
 
 QT = Q.ggml_tensor_qtype["sym_int4"]
 
@@ -51,3 +51,27 @@ def test_many_rows_go_in_pieces(monkeypatch, name, n, k):
     monkeypatch.setattr(torch, "empty", lambda *a, **kw: rows.expand(4196, n))
     lowbit_rows(rows.expand(4196, k), None, qt, n, k)
     assert got == [(0, 2048, 0, 2048), (2048, 2048, 2048, 2048), (4096, 100, 4096, 100)]
+
+
+@pytest.mark.parametrize("rows,asked", [(17, 0), (32, 0), (33, 1)])
+def test_few_bf16_rows_ask_nothing(monkeypatch, rows, asked):
+    """a call of 17 to 32 bf16 rows is bound by the host and the rule never takes it"""
+    w = SimpleNamespace(is_cuda=True, _shape=(256, 256), qlayout="t16", qtype=QT)
+    calls = []
+    monkeypatch.setattr(hip, "gemm_lowbit_frag", lambda *a: calls.append(a) or False)
+    monkeypatch.setattr(hip, "gemm_lowbit", lambda x, *a, **kw: x)
+    y = lowbit_matmul(torch.ones(rows, 256, dtype=torch.bfloat16), w, 256)
+    assert y.dtype == torch.float16 and len(calls) == asked
+
+
+def test_scratch_sizes_are_the_librarys():
+    """remembered per library: what one answers is not taken for another's"""
+    lib = hip.lib()
+    args = (64, 4096, 11008, 11008, QT, 0, 0, 0)
+    assert hip._gemm_floats(lib, *args) == lib.bigdl_gemm_lowbit_workspace(*args) > 0
+
+    class Other:
+        def bigdl_gemm_lowbit_workspace(self, *a):
+            return 7
+
+    assert hip._gemm_floats(Other(), *args) == 7

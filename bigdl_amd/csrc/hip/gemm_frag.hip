@@ -74,7 +74,10 @@ FragPlan frag_plan(int M, int N, int K, int qtype, bool pair, bool may_split) {
         if (sk > 1 && (KT < 8 * sk || (KT + per - 1) / per != sk)) break;
         const double turns = (double)((blocks * sk + cus - 1) / cus);
         double us = c.a + turns * (c.turn + per * (c.x * mt + c.w * ns + c.xw * mt * ns));
-        if (sk > 1) us += 4.0 + 1e-6 * sk * M * N * (c.part + 1.0);     // partial sums, and the launch that adds them up
+        // partial sums, and the launch that adds them up: 4 us on the GPU.  Where the host is behind it costs 3.5 us there, so a split has
+        // to be ahead by more than 1.5 us, which is what the estimates may be off (prompt of 34 tokens, two layers of 2048 x 5632, nf4:
+        // 0.2 us ahead by the estimate, 282 us a pass where it is 273 without)
+        if (sk > 1) us += 5.5 + 1e-6 * sk * M * N * (c.part + 1.0);
         if (us < best.us) best = {mt, ns, sk, per, us};
       }
     }

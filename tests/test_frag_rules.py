@@ -75,3 +75,12 @@ def test_scratch_sizes_are_the_librarys():
             return 7
 
     assert hip._gemm_floats(Other(), *args) == 7
+
+
+@pytest.mark.parametrize("name,m,n,k,split", [("nf4", 34, 2048, 5632, False), ("fp4", 98, 1792, 14336, False),
+                                              ("nf4", 70, 1280, 11776, True), ("sym_int4", 36, 1856, 11136, True)])
+def test_a_split_is_worth_its_launch(name, m, n, k, split):
+    """split K: a second launch, so only where the estimate is ahead by more than it may be off"""
+    qt = Q.ggml_tensor_qtype[name]
+    floats = hip.lib().bigdl_gemm_frag_workspace(m, n, k, qt, 0, 2)
+    assert (floats > 0) == split and floats % (m * n) == 0

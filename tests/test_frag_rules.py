@@ -84,3 +84,19 @@ def test_a_split_is_worth_its_launch(name, m, n, k, split):
     qt = Q.ggml_tensor_qtype[name]
     floats = hip.lib().bigdl_gemm_frag_workspace(m, n, k, qt, 0, 2)
     assert (floats > 0) == split and floats % (m * n) == 0
+
+
+def test_out_and_fragment_order_exclude_each_other(monkeypatch):
+    monkeypatch.setattr(hip, "_need_cuda", lambda *t: None)
+    monkeypatch.setattr(hip, "_stream", lambda: 0)
+    monkeypatch.setattr(hip, "lib", lambda: SimpleNamespace(bigdl_rms_norm=lambda *a: 0, bigdl_attn_prefill=lambda *a: 0))
+    monkeypatch.setattr(hip, "_gemm_frag_dense", lambda *a, out, **kw: out)
+    monkeypatch.setattr(hip, "gemm_lowbit_frag", lambda *a: True)
+    x, w = torch.zeros(48, 128, dtype=torch.float16), torch.zeros(hip._t16_nbytes(QT, 128, 128), dtype=torch.uint8)
+    q = x.view(1, 48, 1, 128).transpose(1, 2)
+    for call in (lambda **kw: hip.rms_norm(x, x[0], 1e-5, frags=True, **kw),
+                 lambda **kw: hip.gemm_lowbit_ex(x, w, QT, 128, 128, w2=w, out_frags=True, **kw),
+                 lambda **kw: hip.attn_prefill(q, q, q, scale=1.0, frags=True, **kw)):
+        assert type(call()) is hip.Frags
+        with pytest.raises(ValueError, match="no out"):
+            call(out=torch.empty_like(x))

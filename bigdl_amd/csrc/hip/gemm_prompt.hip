@@ -40,11 +40,9 @@ static int g_force_cfg = -1, g_force_sk = 0;         // bigdl_gemm_prompt_force 
 // Cost of a launch in units of (output element x 128-deep k tile) per CU: rounds of 256 concurrent tiles, every tile
 // paying its k tiles + a fixed prologue / epilogue; K splits add the fp32 slab traffic and the reduce launch.
 // pair: the gate / up form (two products per output column: blocks cover bn / 2 output columns, no K split)
-static PromptPlan prompt_plan(int M, int N, int K, bool pair = false) {
+// forced_cfg >= 0, forced_sk > 0: only plans of these
+static PromptPlan prompt_plan_of(int M, int N, int K, bool pair, int forced_cfg, int forced_sk) {
   const int KT = K >> 7;
-  static const int env_cfg = getenv("BIGDL_PROMPT_CFG") ? atoi(getenv("BIGDL_PROMPT_CFG")) : -1;
-  static const int env_sk = getenv("BIGDL_PROMPT_SPLITK") ? atoi(getenv("BIGDL_PROMPT_SPLITK")) : 0;
-  const int forced_cfg = g_force_cfg >= 0 ? g_force_cfg : env_cfg, forced_sk = g_force_sk > 0 ? g_force_sk : env_sk;
   PromptPlan best = {0, 1, KT, 1e300};
   for (int c = 0; c < PROMPT_NCFG; ++c) {
     if (forced_cfg >= 0 && c != forced_cfg) continue;
@@ -63,9 +61,15 @@ static PromptPlan prompt_plan(int M, int N, int K, bool pair = false) {
   }
   return best;
 }
+static PromptPlan prompt_plan(int M, int N, int K, bool pair = false) {
+  static const int env_cfg = getenv("BIGDL_PROMPT_CFG") ? atoi(getenv("BIGDL_PROMPT_CFG")) : -1;
+  static const int env_sk = getenv("BIGDL_PROMPT_SPLITK") ? atoi(getenv("BIGDL_PROMPT_SPLITK")) : 0;
+  return prompt_plan_of(M, N, K, pair, g_force_cfg >= 0 ? g_force_cfg : env_cfg, g_force_sk > 0 ? g_force_sk : env_sk);
+}
 
-// The plan's cost in us, for the choice between this kernel and others at 257 - 512 rows: fitted per format to 55 products each
-// (the shapes of gemm_frag.hip's fit); exact to 14 %, worst cases 20 %.
+// The cost in us of the plan that nothing forces (callers remember the choice by the product's sizes), for the choice between this
+// kernel and others at 257 - 512 rows: fitted per format to 55 products each (the shapes of gemm_frag.hip's fit); exact to 14 %, worst
+// cases 20 %.
 double prompt_us(int M, int N, int K, int qtype, bool pair) {
   float per = 40.9f;                                   // fp8_e5m2
   switch (qtype) {
@@ -80,7 +84,7 @@ double prompt_us(int M, int N, int K, int qtype, bool pair) {
     case Q_FP8_E4M3: per = 45.6f; break;
     default: break;
   }
-  return 5.5 + 1e-6 * per * prompt_plan(M, N, K, pair).cost;
+  return 5.5 + 1e-6 * per * prompt_plan_of(M, N, K, pair, -1, 0).cost;
 }
 
 // the staged 16-bit epilogue covers this output; otherwise one fp32 slab + the reduce kernel

@@ -100,3 +100,16 @@ def test_out_and_fragment_order_exclude_each_other(monkeypatch):
         assert type(call()) is hip.Frags
         with pytest.raises(ValueError, match="no out"):
             call(out=torch.empty_like(x))
+
+
+def test_a_forced_prompt_plan_does_not_choose_the_kernel():
+    """the choice is remembered by the product's sizes, so it may not depend on what a sweep forces for its own calls"""
+    lib = hip.lib()
+    for m, n, k in ((400, 4096, 11008), (512, 4096, 11008), (512, 12288, 4096), (512, 14336, 4096)):
+        free = lib.bigdl_gemm_lowbit_frag(m, n, k, k, QT, 0, 0)
+        try:
+            for cfg, splitk in ((0, 1), (2, 1), (2, 8)):
+                hip.gemm_prompt_force(cfg, splitk)
+                assert lib.bigdl_gemm_lowbit_frag(m, n, k, k, QT, 0, 0) == free
+        finally:
+            hip.gemm_prompt_force()

@@ -41,11 +41,17 @@ struct FragArgs {
   int vec;                // rows of out / residual take 4-column accesses
 };
 
-// registers of a wavefront: accumulators, XD steps of x, two k-tiles of weights, addresses and the decoding
+// registers of a wavefront: accumulators, XD steps of x, WD k-tiles of weights, and addresses and the decoding (for the formats with
+// high bits measured from the compiler's allocation).  256 with eight wavefronts; with four 512, of which 448 are planned for: not
+// every value can sit in the accumulation half.  A tiling that spills costs: 6 x 4 tiles of fp6, 16384 x 4096, on eight wavefronts
+// with 52 registers in scratch 40.2 us, on four 30.1; 3 x 6 and 5 x 8 of fp6 37.8 -> 35.8 and 60.4 -> 50.8; 4 x 6 of sym_int5 32.8 -> 30.9.
 constexpr int frag_tile_vgprs(int qt) { return lo_bits_of(qt) + hi_bits_of(qt) + 2 + (has_min_of(qt) ? 2 : 0); }
-constexpr int frag_need(int qt, int mt, int ns, int xd, int wd) { return 4 * mt * ns + 4 * mt * xd + wd * ns * frag_tile_vgprs(qt) + 40; }
+constexpr int frag_decode_vgprs(int qt, int ns) { return qt == Q_FP6 ? 16 + 10 * ns : qt == Q_SYM_INT5 ? 10 + 6 * ns : 40; }
+constexpr int frag_need(int qt, int mt, int ns, int xd, int wd) {
+  return 4 * mt * ns + 4 * mt * xd + wd * ns * frag_tile_vgprs(qt) + frag_decode_vgprs(qt, ns);
+}
 constexpr int frag_nw(int qt, int mt, int ns) { return frag_need(qt, mt, ns, 2, 2) <= 256 ? 8 : 4; }
-constexpr int frag_xd(int qt, int mt, int ns) { return frag_need(qt, mt, ns, 4, 2) <= (frag_nw(qt, mt, ns) == 8 ? 256 : 512) ? 4 : 2; }
+constexpr int frag_xd(int qt, int mt, int ns) { return frag_need(qt, mt, ns, 4, 2) <= (frag_nw(qt, mt, ns) == 8 ? 256 : 448) ? 4 : 2; }
 // partial sums of a wavefront are mt * ns KiB; as many wavefronts park theirs at once as fit
 constexpr int frag_red(int mt, int ns, int nw) { return mt * ns * nw <= 144 ? nw : nw / 2; }
 constexpr int frag_lds(int mt, int ns, int nw) { return frag_red(mt, ns, nw) * mt * ns * 1024; }

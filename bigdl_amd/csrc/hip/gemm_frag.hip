@@ -2,6 +2,7 @@
 // weight format: gemm_frag_inst_*.hip), and the pass that puts x into that order.
 #include "gemm_frag_kernel.h"
 #include "gemm_frag.h"
+#include <math.h>
 
 namespace bigdl {
 #define FRAG_FORMATS(X)                                                                                                     \
@@ -38,23 +39,25 @@ int frag_pack(const void* x, void* xp, int M, int K, int ldx, bool bf16, hipStre
   return HIP_CHECK_LAUNCH();
 }
 
-// Time of a tiling in us: a + turns * (turn + k-tiles * (x * mt + w * ns + xw * mt * ns)) + part * (million partial sums written),
-// turns of a grid with one workgroup a CU.  Fitted per format to 45000 launches on one MI355X: 15 shapes from 1024 x 2048 to
-// 32000 x 4096 and pairs, 33 to 512 rows, every tiling, 1 / 2 / 4 splits of K, weights from memory.  Exact to 12 %, worst cases
-// 25 %; the tiling chosen by it was on average 1 % slower than the fastest, at worst 26 %.
-struct FragCost { float a, turn, x, w, xw, part; };
+// Time of a tiling in us: a + turns * (turn + tile * mt * ns + k-tiles * (x * mt + w * ns + xw * mt * ns)) + load * k-tiles * mem * ns +
+// part * (million partial sums written); load: workgroups a CU, turns: that number rounded up.  tile is the exchange of the sums and the
+// stores, which a short K does not hide; mem is the memory's share of the weights, all workgroups' together.  Fitted per format to 20000
+// launches on one MI355X: random shapes from 512 x 256 to 30000 x 14000 and pairs, 33 to 2048 rows, every tiling, 1 / 2 / 4 splits of
+// K, caches flushed of the weights.  Off by 6 % on average, by more than 12 % for one launch in ten.  Without those two terms K below 1536
+// came out up to half too fast: 437 rows of 11616 x 640 nf4 20 us, measured 37.
+struct FragCost { float a, turn, tile, x, w, xw, mem, part; };
 static FragCost frag_cost(int qtype) {
   switch (qtype) {
-    case Q_SYM_INT4: return {3.71f, 2.80f, 0.0090f, 0.0084f, 0.0134f, 2.5f};
-    case Q_ASYM_INT4: case Q_WOQ_INT4: return {3.86f, 3.00f, 0.0099f, 0.0193f, 0.0125f, 2.3f};
-    case Q_FP4: return {3.84f, 2.63f, 0.0026f, 0.0213f, 0.0145f, 2.6f};
-    case Q_NF4: return {3.98f, 2.40f, 0.0f, 0.0341f, 0.0151f, 2.7f};
-    case Q_SYM_INT5: return {4.15f, 2.43f, 0.0f, 0.0419f, 0.0154f, 2.6f};
-    case Q_ASYM_INT5: return {4.24f, 2.83f, 0.0f, 0.0451f, 0.0153f, 2.5f};
-    case Q_FP6: return {3.72f, 2.71f, 0.0f, 0.0746f, 0.0146f, 2.9f};
-    case Q_SYM_INT8: return {3.69f, 3.19f, 0.0125f, 0.0267f, 0.0118f, 2.3f};
-    case Q_FP8_E4M3: return {3.71f, 3.27f, 0.0064f, 0.0336f, 0.0136f, 2.4f};
-    default: return {3.71f, 3.10f, 0.0171f, 0.0258f, 0.0098f, 2.2f};        // fp8_e5m2
+    case Q_SYM_INT4: return {3.01f, 1.26f, 0.219f, 0.0251f, 0.0192f, 0.0041f, 0.0184f, 0.72f};
+    case Q_ASYM_INT4: case Q_WOQ_INT4: return {2.97f, 1.66f, 0.231f, 0.0270f, 0.0273f, 0.0033f, 0.0168f, 0.71f};
+    case Q_FP4: return {2.98f, 1.27f, 0.226f, 0.0193f, 0.0254f, 0.0059f, 0.0184f, 0.67f};
+    case Q_NF4: return {2.84f, 1.40f, 0.219f, 0.0146f, 0.0383f, 0.0069f, 0.0195f, 0.80f};
+    case Q_SYM_INT5: return {2.76f, 1.43f, 0.240f, 0.0165f, 0.0490f, 0.0056f, 0.0194f, 0.64f};
+    case Q_ASYM_INT5: return {3.08f, 1.29f, 0.257f, 0.0182f, 0.0547f, 0.0044f, 0.0221f, 0.94f};
+    case Q_FP6: return {2.58f, 1.77f, 0.244f, 0.0098f, 0.0759f, 0.0064f, 0.0204f, 0.52f};
+    case Q_SYM_INT8: return {2.77f, 1.76f, 0.227f, 0.0307f, 0.0344f, 0.0023f, 0.0208f, 0.42f};
+    case Q_FP8_E4M3: return {2.93f, 1.52f, 0.240f, 0.0253f, 0.0419f, 0.0039f, 0.0199f, 0.37f};
+    default: return {2.70f, 1.92f, 0.217f, 0.0337f, 0.0299f, 0.0016f, 0.0198f, 0.43f};        // fp8_e5m2
   }
 }
 
@@ -72,12 +75,11 @@ FragPlan frag_plan(int M, int N, int K, int qtype, bool pair, bool may_split) {
       for (int sk = 1; sk <= (may_split ? 4 : 1); sk *= 2) {
         const int per = (KT + sk - 1) / sk;
         if (sk > 1 && (KT < 8 * sk || (KT + per - 1) / per != sk)) break;
-        const double turns = (double)((blocks * sk + cus - 1) / cus);
-        double us = c.a + turns * (c.turn + per * (c.x * mt + c.w * ns + c.xw * mt * ns));
+        const double load = (double)(blocks * sk) / cus;
+        double us = c.a + ceil(load) * (c.turn + c.tile * mt * ns + per * (c.x * mt + c.w * ns + c.xw * mt * ns)) + load * per * c.mem * ns;
         // partial sums, and the launch that adds them up: 4 us on the GPU.  Where the host is behind it costs 3.5 us there, so a split has
-        // to be ahead by more than 1.5 us, which is what the estimates may be off (prompt of 34 tokens, two layers of 2048 x 5632, nf4:
-        // 0.2 us ahead by the estimate, 282 us a pass where it is 273 without)
-        if (sk > 1) us += 5.5 + 1e-6 * sk * M * N * (c.part + 1.0);
+        // to be ahead by that much (34 rows of 2048 x 5632 nf4 in a prompt of two layers: 282 us a pass, without the split 273)
+        if (sk > 1) us += 7.5 + 1e-6 * sk * M * N * (c.part + 1.0);
         if (us < best.us) best = {mt, ns, sk, per, us};
       }
     }

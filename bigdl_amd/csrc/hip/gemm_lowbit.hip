@@ -335,22 +335,31 @@ extern "C" int bigdl_gemm_lowbit(const void* x, const void* w, void* out, const 
   return launch_dense(a, dense_plan(M, N, K, ldx, qtype, false, false, false), qtype, workspace_floats, stream);
 }
 
-// Which products the kernel on x in fragment order takes: those where it and the pass that orders x are expected to be ahead of
-// the faster of the others, by 3 % for what the estimates may be off.  Measured, us, before -> it + that pass: sym_int4
-// 4096 x 4096 at 77 / 256 rows 15.2 -> 9.6 + 3.7, 23.1 -> 14.3 + 4.5; asym_int4 pair of 14336 x 4096 at 77 rows 67.6 -> 32.1 + 3.7; sym_int8
-// 4672 x 4544 at 203 rows 38.7 -> 22 + 4.3.  Left: up to 64 rows most products (12288 x 4096, 64 rows 17.2 -> 15.1 + 3.7), large grids
-// of many rows (14336 x 4096, 256 rows 43.0 -> 47.0 + 4.5).  x in bf16 needs that pass anyway (in place of its conversion).
-enum XKind { X_ROWS = 0, X_ROWS_BF16 = 1, X_FRAGMENTS = 2 };
-static bool takes_frag_kernel(int ldx, int M, int N, int K, int qtype, bool pair, int x_kind, FragPlan* plan) {
+// Which products the kernel on x in fragment order takes: those where it is expected to be ahead of the faster of the others.
+//  * Rows: with the pass that orders them, by 5 % for what the estimates may be off.  Up to 64 rows, where little is gained, and below
+//    16 us by 3 us more: a call takes the host 13 us, and the second launch up to 3.  Of 6000 random products of 33 to 512 rows, pairs
+//    among them, it takes 37 %, and 0.6 % of all are slower by more than 2 % for it (5.6 % by estimates without their tile and mem
+//    terms); the mean speed is 1.15 times the former.  Measured, us, before -> with the pass -> x in fragment order already: sym_int4
+//    4096 x 4096 at 160 / 256 rows 22.7 -> 16.6 -> 12.7, 23.7 -> 19.1 -> 14.6; sym_int8 4672 x 4544 at 203 rows 37.6 -> 24.1 -> 20.7.  Left:
+//    sym_int4 4096 x 4096 at 77 rows 14.6 -> 12.2 -> 9.1, 12288 x 4096 at 64 rows 16.5 -> 18.3 -> 15.4, 14336 x 4096 at 256 rows 45.6 -> 55.1 -> 50.5.
+//  * Rows in bf16 need a pass in any case, their conversion: by 5 %.
+//  * x whose producer writes it in that order: in a whole step, against the others with x in rows, it is ahead where both are
+//    alike alone (their split sums take a launch more, and they come back to cold code), so up to 256 rows unless it is expected
+//    to be 15 % behind.  Steps of 8 layers, us, without it / with 3 % ahead asked for / as here: llama3-8b nf4 33 rows 988 / 896 / 857,
+//    q4_k 64 rows 970 / 915 / 871, llama2-7b sym_int4 64 rows 1157 / 1121 / 1074.  Against the prompt kernel by 5 %: prompts of 8 layers,
+//    without it / always / as here: llama2-7b sym_int4 300 tokens 2159 / 1822 / 1826, 512 tokens 2355 / 2589 / 2254.
+enum XKind { X_ROWS = 0, X_ROWS_BF16 = 1, X_FRAGMENTS = 2, X_PRODUCED = 3 };
+static bool takes_frag_kernel(int ldx, int M, int N, int K, int qtype, bool pair, int x_kind, bool out_frags, FragPlan* plan) {
   if (M <= 32 || !is_t16(qtype)) return false;
   // (rows that bigdl_gemm_frag_dense refuses: the callers' other ways take them as they are, or 256 at a time)
-  if (x_kind != X_FRAGMENTS && ((ldx & 7) || (int64_t)M * ldx >= (1ll << 31))) return false;
+  if (x_kind < X_FRAGMENTS && ((ldx & 7) || (int64_t)M * ldx >= (1ll << 31))) return false;
   *plan = frag_plan(M, N, K, qtype, pair, !pair);
   if (plan->ns == 0) return false;
   if (x_kind == X_FRAGMENTS) return true;
   if (M > FRAG_MAX_ROWS) return false;
   double other;
-  if (M > 256 && K >= 256 && (K & 127) == 0) {
+  const bool prompt = M > 256 && K >= 256 && (K & 127) == 0;
+  if (prompt) {
     if (M > 512) return false;                         // (what the estimates cover)
     other = prompt_us(M, N, K, qtype, pair);
   } else {
@@ -360,15 +369,18 @@ static bool takes_frag_kernel(int ldx, int M, int N, int K, int qtype, bool pair
     other = takes_rows_kernel(ldx, rows, N, K, qtype, pair, &r) ? rows_us(c, r, K, qtype, pair) : tile_us(c, rows, N, K, pair);
     other *= (M + 255) / 256;
   }
-  return plan->us + (x_kind == X_ROWS ? frag_pack_us(M, K) : 0.0) < 0.97 * other;
+  if (x_kind == X_ROWS) return plan->us + frag_pack_us(M, K) + (M <= 64 || other < 16.0 ? 3.0 : 0.0) < 0.95 * other;
+  if (x_kind == X_ROWS_BF16) return plan->us < 0.95 * other;
+  return plan->us - (out_frags ? frag_pack_us(M, N) : 0.0) < other * (prompt ? 0.95 : 1.15);
 }
 
-// Whether the kernel on x in fragment order is the one for this product.  x_kind 0: fp16 rows; 1: bf16 rows, or x that its producer
-// writes in that order (no pass of its own over x); 2: x in that order already (whether it can be multiplied at all).
-extern "C" int bigdl_gemm_lowbit_frag(int M, int N, int K, int ldx, int qtype, int pair, int x_kind) {
-  if (M <= 0 || N <= 0 || K <= 0 || (K & 31) || x_kind < 0 || x_kind > X_FRAGMENTS) return 0;
+// Whether the kernel on x in fragment order is the one for this product.  x_kind 0: fp16 rows; 1: bf16 rows; 2: x in that order already
+// (whether it can be multiplied at all); 3: x that its producer writes in that order if so.  out_frags (with 3): the result of a pair
+// goes out in that order too, to a product that saves its pass.
+extern "C" int bigdl_gemm_lowbit_frag(int M, int N, int K, int ldx, int qtype, int pair, int x_kind, int out_frags) {
+  if (M <= 0 || N <= 0 || K <= 0 || (K & 31) || x_kind < 0 || x_kind > X_PRODUCED) return 0;
   FragPlan p;
-  return takes_frag_kernel(ldx, M, N, K, t16_kernel_qtype(qtype), pair != 0, x_kind, &p) ? 1 : 0;
+  return takes_frag_kernel(ldx, M, N, K, t16_kernel_qtype(qtype), pair != 0, x_kind, out_frags != 0, &p) ? 1 : 0;
 }
 
 // fp32 scratch, in floats, of the call below: x in fragment order (unless it comes so) and the partial sums of a split K

@@ -521,9 +521,9 @@ class NativeDecoder:
                     kernel_size=ck.get("kernel_size", 7), pooling=ck.get("pooling", "maxpool"))
 
     # ------------------------------------------------------------------ prefill (eager)
-    def _takes_frags(self, rows, lin: Optional[Lin], w2: Optional[Lin] = None, prompt=True):
-        """whether the product of so many rows (with w2: the gate / up pair) takes x in fragment order from its producer: the norm
-        in front of it, or the pair in front of a down projection"""
+    def _takes_frags(self, rows, lin: Optional[Lin], w2: Optional[Lin] = None, prompt=True, then: Optional[Lin] = None):
+        """whether the product of so many rows (with w2: the gate / up pair, in front of ``then``) takes x in fragment order from its
+        producer: the norm in front of it, or the pair in front of a down projection"""
         # (513 rows and more of such a K are the prompt kernel's, up to GEMV_MAX_ROWS gemv_lowbit's; asked four times a layer, so the
         # cheapest question first)
         if not 32 < rows <= 512 or rows <= GEMV_MAX_ROWS or lin is None or not lin.fused or lin.k & 127:
@@ -533,10 +533,12 @@ class NativeDecoder:
         if rows > GEMM_MAX_ROWS and not (prompt and self.prefill_fused and not Lin.cache_dense and not self.prefill_fp8):
             return False
         from ..ops import hip
-        return hip.gemm_lowbit_frag(rows, lin.n, lin.k, lin.qtype, None, w2 is not None, True)
+        return hip.gemm_lowbit_frag(rows, lin.n, lin.k, lin.qtype, None, w2 is not None, 3,
+                                    then is not None and self._takes_frags(rows, then, None, prompt))
 
     def _mlp_takes_frags(self, rows, lw):
-        return self.cfg.gated_mlp and lw.moe is None and lw.gate is not None and self._takes_frags(rows, lw.gate, lw.up)
+        return (self.cfg.gated_mlp and lw.moe is None and lw.gate is not None
+                and self._takes_frags(rows, lw.gate, lw.up, True, lw.down))
 
     def _linear_dense(self, x, lin: Lin):
         from ..ops import hip
@@ -1243,7 +1245,7 @@ class NativeDecoder:
                 and w2.qtype == lin.qtype and w2.n == lin.n and not os.environ.get("BIGDL_NO_PAIR_GEMM")):
             # batched decode (17 .. 256 rows): gate and up in one launch, act(g) * u in the few-row kernel's epilogue or, where
             # the tile kernel runs, in its reduce kernel (at 64 rows of 11008 x 4096: 23 and 33 us)
-            frags = gamma is not None and self._takes_frags(m, lin, w2, prompt=False)
+            frags = gamma is not None and self._takes_frags(m, lin, w2, False, then)
             xin = x if gamma is None else hip.rms_norm(x, gamma, cfg.rms_eps, offset=cfg.norm_offset, frags=frags)
             if frags and then is not None and self._takes_frags(m, then, prompt=False):
                 return hip.gemm_lowbit_ex(xin, lin.w, lin.qtype, lin.n, lin.k, w2=w2.w, bias=lin.bias, bias2=w2.bias, act=act, out_frags=True)

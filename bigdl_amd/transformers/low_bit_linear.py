@@ -348,7 +348,7 @@ def lowbit_matmul(x_2d: torch.Tensor, weight: FP4Params, out_features: int, for_
         t16 = weight.qlayout == "t16"
         # (32 rows and fewer are never that kernel's: nothing more is asked for them, their calls are bound by the host)
         if (m > 32 and dt == torch.bfloat16 and t16 and m > GEMV_MAX_ROWS and (m <= GEMM_MAX_ROWS or not for_training)
-                and hip.gemm_lowbit_frag(m, n, k, weight.qtype, x_2d.stride(0), False, True) and x_2d.stride(1) == 1
+                and hip.gemm_lowbit_frag(m, n, k, weight.qtype, x_2d.stride(0), False, 1) and x_2d.stride(1) == 1
                 and x_2d.data_ptr() % 16 == 0 and getattr(weight, "_dense_cache", None) is None):
             return hip.gemm_lowbit(x_2d, weight, weight.qtype, n, k, out_dtype=dt)       # (rounded to fp16 while it is ordered)
         if t16 and m <= GEMM_MAX_ROWS:

@@ -202,7 +202,7 @@ def test_engine_with_products_on_gemv(hip, monkeypatch, gemv_max):
     from bigdl_amd.models import decoder as D
     cfg = D.DecoderConfig(vocab_size=1024, hidden_size=1024, intermediate_size=2048, num_layers=2, num_heads=16, num_kv_heads=4,
                           head_dim=128, max_position=512, norm="layer", gated_mlp=False, act="gelu")     # (a pair is 32 rows at most there)
-    assert hip.gemm_lowbit_frag(40, 1024, 2048, Q.SYM_INT4, None, False, True)
+    assert hip.gemm_lowbit_frag(40, 1024, 2048, Q.SYM_INT4, None, False, 3)
     ids = torch.randint(0, 1024, (40, 9), generator=torch.Generator().manual_seed(3)).cuda()
 
     def run():

@@ -29,15 +29,15 @@ def test_engine_gives_gemv_rows(monkeypatch, gemv_max, taken):
         assert D.NativeDecoder._takes_frags(eng, 64, lin, prompt=prompt) == taken
 
 
-@pytest.mark.parametrize("bf16", [False, True])
-def test_rows_far_apart_stay_with_the_other_kernels(bf16):
+@pytest.mark.parametrize("kind", [0, 1])
+def test_rows_far_apart_stay_with_the_other_kernels(kind):
     """a call that the rule takes is one that the launcher accepts: rows 16 bytes aligned, the last one within 2^31 elements.  300 last
     positions of sequences of 2048 tokens are 600 K row widths."""
     m, k = 300, 4544
-    assert hip.gemm_lowbit_frag(m, 4544, k, QT, k, False, bf16)
-    assert hip.gemm_lowbit_frag(m, 4544, k, QT, 1 << 22, False, bf16)
-    assert not hip.gemm_lowbit_frag(m, 4544, k, QT, 2048 * k, False, bf16)
-    assert not hip.gemm_lowbit_frag(m, 4544, k, QT, k + 4, False, bf16)
+    assert hip.gemm_lowbit_frag(m, 4544, k, QT, k, False, kind)
+    assert hip.gemm_lowbit_frag(m, 4544, k, QT, 1 << 22, False, kind)
+    assert not hip.gemm_lowbit_frag(m, 4544, k, QT, 2048 * k, False, kind)
+    assert not hip.gemm_lowbit_frag(m, 4544, k, QT, k + 4, False, kind)
 
 
 @pytest.mark.parametrize("name,n,k", [("asym_int4", 14336, 4128), ("sym_int8", 14336, 4128), ("sym_int4", 4672, 4544)])
@@ -106,10 +106,36 @@ def test_a_forced_prompt_plan_does_not_choose_the_kernel():
     """the choice is remembered by the product's sizes, so it may not depend on what a sweep forces for its own calls"""
     lib = hip.lib()
     for m, n, k in ((400, 4096, 11008), (512, 4096, 11008), (512, 12288, 4096), (512, 14336, 4096)):
-        free = lib.bigdl_gemm_lowbit_frag(m, n, k, k, QT, 0, 0)
+        free = lib.bigdl_gemm_lowbit_frag(m, n, k, k, QT, 0, 0, 0)
         try:
             for cfg, splitk in ((0, 1), (2, 1), (2, 8)):
                 hip.gemm_prompt_force(cfg, splitk)
-                assert lib.bigdl_gemm_lowbit_frag(m, n, k, k, QT, 0, 0) == free
+                assert lib.bigdl_gemm_lowbit_frag(m, n, k, k, QT, 0, 0, 0) == free
         finally:
             hip.gemm_prompt_force()
+
+
+@pytest.mark.parametrize("name,m,n,k,pair,kind,taken", [
+    # rows, with the pass that orders them: measured ahead by a tenth and more
+    ("sym_int8", 203, 4672, 4544, 0, 0, True), ("sym_int4", 256, 4096, 4096, 0, 0, True), ("sym_int4", 160, 4096, 4096, 0, 0, True),
+    ("asym_int4", 300, 4096, 14336, 0, 0, True),
+    # behind: a short K, which does not hide the exchange of the sums (nf4 18 -> 37 us), grids of several turns, a single row block
+    ("nf4", 437, 11616, 640, 0, 0, False), ("fp8_e5m2", 341, 11504, 1536, 0, 0, False), ("sym_int4", 256, 14336, 4096, 0, 0, False),
+    ("sym_int4", 64, 12288, 4096, 0, 0, False), ("fp8_e5m2", 35, 4160, 10880, 0, 0, False), ("sym_int4", 59, 2368, 9152, 1, 0, False),
+    # alike on the GPU, a launch more for the host
+    ("sym_int8", 90, 4096, 4544, 0, 0, False),
+    # bf16 rows need a pass in any case
+    ("sym_int4", 77, 4096, 4096, 0, 1, True), ("sym_int4", 32, 4096, 4096, 0, 1, False),
+    # x that its producer writes in that order: a decode batch of 33 and 64, a prompt of 300 tokens; of 512 the pair is the prompt kernel's
+    ("nf4", 33, 4096, 14336, 0, 3, True), ("sym_int4", 64, 4096, 11008, 0, 3, True), ("sym_int4", 64, 11008, 4096, 1, 3, True),
+    ("sym_int4", 300, 12288, 4096, 0, 3, True), ("sym_int4", 512, 11008, 4096, 1, 3, False), ("nf4", 512, 14336, 4096, 1, 3, False),
+    ("nf4", 513, 4096, 4096, 0, 3, False)])
+def test_kernel_of_a_product(name, m, n, k, pair, kind, taken):
+    assert hip.lib().bigdl_gemm_lowbit_frag(m, n, k, k, Q.ggml_tensor_qtype[name], pair, kind, 0) == taken
+
+
+def test_a_pair_in_front_of_such_a_product():
+    """the next product's pass, 4 us, is saved where the pair's result goes out in that order"""
+    qt = Q.ggml_tensor_qtype["nf4"]
+    taken = [[hip.gemm_lowbit_frag(m, 5632, 2048, qt, None, True, 3, out) for m in range(257, 513)] for out in (False, True)]
+    assert sum(taken[0]) < sum(taken[1]) and all(b or not a for a, b in zip(*taken))

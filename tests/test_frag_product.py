@@ -96,6 +96,77 @@ def test_pairs_bias_residual(hip, name, m, n):
         torch.testing.assert_close(out.cpu().double(), xd @ wg.t() + b1.double() + res.double(), **tol)
 
 
+# N odd, a multiple of 4 and of 16; K with and without a cut last k-tile
+@pytest.mark.parametrize("name,m,n,k,kind", [("asym_int4", 258, 261, 9440, 0), ("sym_int4", 276, 212, 10784, 0), ("nf4", 283, 208, 8832, 1),
+                                             ("nf4", 283, 208, 8832, 2), ("sym_int8", 283, 229, 10560, 1), ("fp6", 266, 210, 6400, 2)])
+def test_split_of_k_in_the_public_call(hip, name, m, n, k, kind):
+    """partial sums behind the ordered x, added up by the launch that applies bias, activation and the residual: in place, rows apart"""
+    qt = Q.ggml_tensor_qtype[name]
+    assert hip.lib().bigdl_gemm_frag_workspace(m, n, k, qt, 0, 2) >= 2 * m * n
+    dev, w = _weight(n, k, qt, 1)
+    x, xd = _x(m, k, 2, torch.bfloat16 if kind == 1 else torch.float16)
+    assert kind == 2 or hip.gemm_lowbit_frag(m, n, k, qt, x.stride(0), False, kind)
+    g = torch.Generator().manual_seed(3)
+    bias, res = torch.randn(n, generator=g).half(), torch.randn(m, n, generator=g).half()
+    for dtype, step in ((torch.float32, 0.0), (torch.float16, 2.0 ** -11)):
+        buf = torch.full((m, n + 8), 7.0, dtype=dtype, device="cuda")
+        out = buf[:, :n]
+        out.copy_(res)
+        hip.gemm_lowbit(hip.Frags(hip.frag_pack(x), m, k) if kind == 2 else x, dev, qt, n, k, bias=bias.cuda(), act="silu", residual=out, out=out)
+        first = xd @ w.t() + bias.double()
+        ref = torch.nn.functional.silu(first) + res.double()
+        off = (out.double().cpu() - ref).abs()
+        # _close's bound through silu, 1.1 steep at most, and the result's rounding; all together as for the pairs below
+        assert (off <= 1.1 * (2.0 ** -9 * (xd.abs() @ w.abs().t()) + 1e-5) + step * ref.abs()).all()
+        assert (off.norm() / ref.norm()).item() < 1.1 * 2.0 ** -10.5 + step and (buf[:, n:] == 7).all()
+
+
+@pytest.mark.parametrize("name,m,n,k", [("sym_int4", 77, 2048, 2048), ("sym_int8", 203, 1536, 4096), ("asym_int4", 300, 520, 1056)])
+def test_bf16_rows_of_a_linear(hip, monkeypatch, name, m, n, k):
+    """rounded to fp16 by the pass that orders them; up to fp16's largest and past it, as the conversion of the other kernels does"""
+    from bigdl_amd.transformers.low_bit_linear import FP4Params, lowbit_matmul
+    qt = Q.ggml_tensor_qtype[name]
+    w = torch.randn(n, k, generator=torch.Generator().manual_seed(1)) * 0.05
+    raw = host.quantize(w, qt)
+    raw = raw.view(torch.uint8) if raw.dtype != torch.uint8 else raw
+    par = FP4Params(raw.flatten(), quantized=True, _shape=(n, k), qtype=qt).to("cuda")
+    x, xd = _x(m, k, 2, torch.bfloat16)
+    kinds = []
+    real = hip._gemm_frag_dense
+    monkeypatch.setattr(hip, "_gemm_frag_dense", lambda x, kind, *a, **kw: (kinds.append(kind), real(x, kind, *a, **kw))[1])
+    out = lowbit_matmul(x, par, n)
+    assert kinds == [1] and out.dtype == torch.bfloat16
+    wd = host.dequantize(raw, qt, (n, k)).double()
+    ref = xd @ wd.t()
+    bound = 2.0 ** -9 * (xd.abs() @ wd.abs().t()) + 2.0 ** -8 * ref.abs() + 1e-5
+    assert ((out.double().cpu() - ref).abs() <= bound).all()
+    big = torch.zeros(m, k, dtype=torch.bfloat16, device="cuda")
+    big[0, 0], big[1, 1], big[2, 2] = 3e38, -3e38, float("nan")
+    monkeypatch.setattr(hip, "gemm_lowbit_frag", lambda *a, **kw: False)
+    other = lowbit_matmul(big, par, n)
+    monkeypatch.undo()
+    assert torch.equal(lowbit_matmul(big, par, n).isfinite(), other.isfinite()) and not other[:3].isfinite().any()
+
+
+@pytest.mark.parametrize("splits", [1, 2, 5])
+@pytest.mark.parametrize("b,q_len,hq,hkv,d", [(40, 1, 8, 2, 64), (17, 3, 4, 4, 128), (33, 1, 40, 1, 96)])
+def test_decode_attention_in_fragment_order(hip, splits, b, q_len, hq, hkv, d):
+    """one key range, and several that the last workgroup combines"""
+    g = torch.Generator().manual_seed(5)
+    cap, past = 512, 300
+    qkv = torch.randn(b * q_len, (hq + 2 * hkv) * d, generator=g).half().cuda()
+    k, vt = torch.randn(b, hkv, cap, d, generator=g).half().cuda(), torch.randn(b, hkv, d, cap, generator=g).half().cuda()
+    lens = torch.full((b,), past, dtype=torch.int32, device="cuda")
+    ws = torch.empty(hip.attn_decode_ws_floats(b, hq, hkv, q_len, d, splits) + 16, device="cuda")
+    cnt = torch.zeros(hip.attn_decode_counters(b, hq, hkv), dtype=torch.int32, device="cuda")
+    rows = torch.empty(b * q_len, hq * d, dtype=torch.float16, device="cuda")
+    frags = hip.Frags(torch.zeros(hip.frag_halves(b * q_len, hq * d), dtype=torch.float16, device="cuda"), b * q_len, hq * d)
+    for out in (rows, frags):
+        hip.attn_decode(qkv, k, vt, lens, out, ws, cnt, n_heads=hq, n_kv_heads=hkv, head_dim=d, q_len=q_len, batch=b, scale=d ** -0.5,
+                        splits=splits, append=True)
+    assert rows.isfinite().all() and torch.equal(frags.data, hip.frag_pack(rows))
+
+
 @pytest.mark.parametrize("name", ["sym_int4", "fp6"])
 @pytest.mark.parametrize("m", [700, 2048, 2100])
 def test_many_rows_of_a_ragged_k(hip, name, m):
@@ -218,11 +289,15 @@ def test_engine_with_products_on_gemv(hip, monkeypatch, gemv_max):
         assert ((a - b).norm() / b.norm()).item() < 4e-3
 
 
-def test_rows_of_stride_zero(hip):
-    """one row seen 77 times: accepted by the other kernels, so by the pass that orders x too"""
-    n, k = 4096, 4096
-    qt = Q.SYM_INT4
-    w = (torch.randint(0, 256, (host.device_nbytes(qt, n, k),), dtype=torch.uint8) & 0xBF).cuda()
-    x = torch.randn(1, k).half().cuda().expand(77, k)
-    out = hip.gemm_lowbit(x, w, qt, n, k)
-    assert torch.equal(out, hip.gemm_lowbit(x.contiguous(), w, qt, n, k)) and torch.equal(out, out[:1].expand(77, n))
+@pytest.mark.parametrize("name,n,k", [("sym_int4", 2048, 2048), ("nf4", 1536, 4096)])
+def test_rows_of_stride_zero(hip, name, n, k):
+    """one row seen 203 times: accepted by the other kernels, so by the pass that orders x too"""
+    qt = Q.ggml_tensor_qtype[name]
+    dev, w = _weight(n, k, qt, 1)
+    row = torch.randn(1, k, generator=torch.Generator().manual_seed(2)).half()
+    x = row.cuda().expand(203, k)
+    assert torch.equal(hip.frag_pack(x), hip.frag_pack(x.contiguous())) and hip.gemm_lowbit_frag(203, n, k, qt, 0)
+    out = hip.gemm_lowbit(x, dev, qt, n, k, out_dtype=torch.float32)
+    xd = row.double().expand(203, k)
+    _close(out, xd, w, xd @ w.t())
+    assert torch.equal(out, out[:1].expand(203, n))

@@ -23,22 +23,32 @@ class _Allocations(TorchDispatchMode):
 
 class _Library:
     """stands for the kernels' library: two K splits, one slab, and the workspace address that each launch is given"""
-    at = {"bigdl_gemm_lowbit": 5, "bigdl_gemm_prompt": 5, "bigdl_gemm_lowbit_ex": 12}
+    at = {"bigdl_gemm_lowbit": 5, "bigdl_gemm_prompt": 5, "bigdl_gemm_lowbit_ex": 12, "bigdl_gemm_frag_dense": 7}
 
     def __init__(self):
-        self.got = []
+        self.got, self.names = [], []
 
     def __getattr__(self, name):
         if name in self.at:
-            return lambda *a: self.got.append(a[self.at[name]]) or 0
+            return lambda *a: self.names.append(name) or self.got.append(a[self.at[name]]) or 0
         return lambda *a: 4096 if name.endswith("workspace") else 2
 
 
-@pytest.mark.parametrize("call", ["gemm_lowbit", "gemm_lowbit_ex", "gemm_prompt"])
-def test_every_call_allocates_its_own_scratch(monkeypatch, call):
+@pytest.fixture(autouse=True)
+def _choices_of_the_real_library():
+    """what the stand-in below answers is not remembered"""
+    yield
+    hip.gemm_lowbit_frag.cache_clear()
+
+
+@pytest.mark.parametrize("call,frag", [("gemm_lowbit", False), ("gemm_lowbit_ex", False), ("gemm_prompt", False), ("gemm_lowbit", True),
+                                       ("gemm_lowbit_ex", True)])
+def test_every_call_allocates_its_own_scratch(monkeypatch, call, frag):
     """A buffer kept between calls is freed when a larger one takes its place, while captured graphs go on writing to it:
     what a launch gets must have been allocated by that call (under capture: from the graph's pool)."""
     lib = _Library()
+    lib.bigdl_gemm_lowbit_frag = lambda *a: int(frag)          # (asked for more than 32 rows)
+    hip.gemm_lowbit_frag.cache_clear()
     monkeypatch.setattr(hip, "lib", lambda: lib)
     monkeypatch.setattr(hip, "_need_cuda", lambda *t: None)
     monkeypatch.setattr(hip, "_stream", lambda: 0)
@@ -50,7 +60,7 @@ def test_every_call_allocates_its_own_scratch(monkeypatch, call):
         with _Allocations() as made:
             keep.append(getattr(hip, call)(x, w, QT, n, k))
         assert lib.got[-1] in made.ptrs
-    assert len(lib.got) == 4
+    assert len(lib.got) == 4 and lib.names.count("bigdl_gemm_frag_dense") == int(frag)
 
 
 @pytest.mark.parametrize("m,n,k,pair,norms,floats", [

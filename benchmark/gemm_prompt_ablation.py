@@ -1,7 +1,6 @@
 """A/B timing of builds of the prompt GEMM in ONE process, rounds interleaved (separate processes differ by more than the
 builds do: clocks, caches).  Every `libbigdl_hip_<name>.so` under bigdl_amd/lib/abl/ is loaded next to the production
-library and called through its own handle; measurement builds (PROMPT_ABL, see csrc/hip/gemm_prompt_kernel.h) give
-wrong results by construction, only their time matters.
+library and called through its own handle.
     PYTHONPATH=. python benchmark/gemm_prompt_ablation.py [--shape qkv] [--cfg 1] [--libs abl1,abl2] [--rounds 12]"""
 import argparse
 import ctypes

@@ -5,51 +5,42 @@
 // and are expanded on the way to the matrix cores, so a prompt pass neither writes nor re-reads an fp16 copy of the
 // model and calls no library GEMM.
 //
-// Structure (one workgroup = WM x WN wavefronts = one BM x BN output tile, K walked in 64-deep tiles):
-//  * x tile [BM][64 k] goes global -> LDS directly (global_load_lds, 16 bytes per lane), one tile ahead, two buffers.
+// Structure (one workgroup = 2 x 4 wavefronts = one BM x BN output tile, K walked in 64-deep tiles):
+//  * x tile [BM][64 k] goes global -> LDS directly (buffer_load .. lds, 16 bytes per lane), up to two tiles ahead, three buffers.
 //    The LDS image is lane-linear as the instruction requires; the bank swizzle (16-byte slot ^= row & 7) is applied
 //    to the per-lane SOURCE address and again on the fragment reads.
 //  * the weight tile [BN][64 k] is expanded ONCE per workgroup: every wavefront owns a share of the block's 16-row weight
 //    tile rows, loads their raw T16 tiles (codes + block scales, 16-byte loads, one whole 128-deep tile per two k tiles)
 //    two tiles ahead, expands them with the register bit tricks of the skinny kernels, folds the block scale in as a
 //    packed fp16 multiply and writes the fp16 fragments to the other LDS buffer with one 16-byte store per unit.
-//    (The earlier form expanded weights per wavefront in registers: every weight was decoded by both row halves of the
-//    workgroup and the decode stood in the MFMA's issue slots.)
+//  * one instruction stream per wavefront (comments at the loop): behind the MFMAs on an x fragment the next k step's
+//    fragment is read into its place, and a share of the expansion and at most one memory request ride between two groups
+//    of MFMAs.  Two wavefronts a SIMD fill each other's gaps; one barrier per 64-deep tile.
 //  * fragments: both operands are read with ds_read_b128 from 128-byte rows; slot ^= row & 7 makes the four 16-lane
 //    groups of the read and the eight 8-lane groups of the expansion's ds_write_b128 conflict free.
-//  * 8-wavefront tiles run their two row halves as a ping-pong pair, one segment apart: while one wavefront of a SIMD
-//    issues MFMAs its partner reads fragments, expands weights and requests the next tiles (comments at the loop).
 //  * the weight fragment is the MFMA's A operand, so a lane holds 4 consecutive output columns of one row; the epilogue
 //    stages the wavefront's tile through LDS and stores whole 128-byte row segments; the gate / up pair form combines the
 //    two products of a column there (act(g) * u), so neither reaches memory.
 //  * the block index is remapped so that the workgroups of one XCD share x and weight panels in its L2.
+// What bounds it: power.  8192 x 8192 x 8192 in fp16 runs the library's product at 1.42 GHz (87 % of the MFMA cycles, 1300 - 1350
+// TFLOP/s; 2110 with zeros), this kernel at 1.5 - 1.6; the cycles of the 256 x 256 loop are 15 % over the MFMAs'.
+// The earlier form ran the two row halves as a ping-pong pair, load and MFMA segments in turn with a barrier behind each (4 a tile) and
+// a tile's requests in one burst, behind which every wavefront stood still.  Old -> new, us, weights of 4 layers in turn: sym_int4
+// 7680 rows x 14336 x 4096 827 -> 715, 1024 x 4096 x 4096 48.5 -> 43.6, nf4 924 -> 777 and 55.5 -> 50.4, fp6 1041 -> 900 and 63 -> 54.7.
 // Measured and dropped: stream-K over 256 x 256 tiles (every CU the same number of k tiles whatever the tile count; the
-// 256 KiB fp32 slab per shared tile costs more than the idle CUs it removes: 130 instead of 98 us on the qkv shape),
-// x requests or the expansion moved into the MFMA segment (no change / slower), wavefront priorities (no change).
+// 256 KiB fp32 slab per shared tile costs more than the idle CUs it removes: 130 instead of 98 us on the qkv shape), wavefront
+// priorities (none / slower), weights expanded by both row halves in registers (no LDS for them, but twice the vector work: int4 3 - 6 %
+// ahead of the ping-pong form, nf4 14 - 18 % behind), 32 x 32 x 16 MFMAs (alone 1650 TFLOP/s on normal data, 16 x 16 x 32 1870).
 #pragma once
 #include "gemm_kernel.h"
-
-// PROMPT_ABL (measurement builds, results wrong): 1 = no weight loads in the loop, 2 = no x tile loads in the loop,
-// 4 = no expansion (codes written as they are), 8 = no barrier in the loop, 16 = no MFMA, 32 = no LDS fragment reads
-#ifndef PROMPT_ABL
-#define PROMPT_ABL 0
-#endif
-// phases per 64-deep tile of the 256 x 256 / 256 x 192 configurations (1 or 2)
-#ifndef PROMPT_PH0
-#define PROMPT_PH0 2
-#endif
-#ifndef PROMPT_PH1
-#define PROMPT_PH1 1
-#endif
 
 namespace bigdl {
 
 typedef __attribute__((address_space(3))) void lds_void_t;
-typedef __attribute__((address_space(1))) const void glb_cvoid_t;
 
-// LDS bytes of the tile buffers: two x + two weight buffers, or the epilogue's staging area (rows padded by 16 bytes)
+// LDS bytes of the tile buffers: three x + two weight buffers, or the epilogue's staging area (rows padded by 16 bytes)
 constexpr int prompt_lds_tiles(int BM, int BN, int NW, int MTW, int NTW) {
-  const int a = 2 * (BM + BN) * 128, b = NW * MTW * 16 * (32 * NTW + 16);
+  const int a = (3 * BM + 2 * BN) * 128, b = NW * MTW * 16 * (32 * NTW + 16);
   return a > b ? a : b;
 }
 
@@ -68,23 +59,63 @@ __device__ __forceinline__ half8 unit_expand(const Tile<QT>& t) {
   return code * d;
 }
 
+// (buffer operations: a scalar offset plus a lane constant is the whole address, and their arrival is counted, while a global load to
+// LDS makes the compiler wait for everything in flight at the next use of a loaded register)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_of(const void* p) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0xffffffff, 0x00027000);
+}
+// 16 bytes per lane from a buffer (lane offset + wavefront offset) to consecutive LDS
+__device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t b, char* lds, uint32_t lane_off, uint32_t off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(b, (lds_void_t*)lds, 16, lane_off, off, 0, 0);
+}
+// the planes of one row of T16 tiles
+struct RowPlanes { __amdgpu_buffer_rsrc_t lo, hi, sc, mn; };
+template <int QT>
+__device__ __forceinline__ RowPlanes row_planes(const T16Planes& p, int64_t tile) {
+  RowPlanes b;
+  b.lo = buf_of(p.lo + tile * (lo_bits_of(QT) * 256));
+  if constexpr (hi_bits_of(QT) > 0) b.hi = buf_of(p.hi + tile * (hi_bits_of(QT) * 256));
+  b.sc = buf_of(p.sc + tile * 64);
+  if constexpr (has_min<QT>()) b.mn = buf_of(p.mn + tile * 64);
+  return b;
+}
+// requests of load_raw (vmcnt is counted by them below)
+template <int QT>
+constexpr int raw_loads() { return lo_bits_of(QT) / 4 + (hi_bits_of(QT) > 0) + 1 + has_min<QT>(); }
+template <int QT>
+__device__ __forceinline__ void load_raw(Tile<QT>& t, const RowPlanes& p, int tile, int lane) {
+  t.lo0 = __builtin_amdgcn_raw_buffer_load_b128(p.lo, lane * 16, tile * (lo_bits_of(QT) * 256), 0);
+  if constexpr (lo_bits_of(QT) == 8) t.lo1 = __builtin_amdgcn_raw_buffer_load_b128(p.lo, lane * 16, tile * 2048 + 1024, 0);
+  if constexpr (hi_bits_of(QT) == 1) t.hi0 = __builtin_amdgcn_raw_buffer_load_b32(p.hi, lane * 4, tile * 256, 0);
+  if constexpr (hi_bits_of(QT) == 2) {
+    const uint2v h = __builtin_amdgcn_raw_buffer_load_b64(p.hi, lane * 8, tile * 512, 0);
+    t.hi0 = h.x;
+    t.hi1 = h.y;
+  }
+  t.d = __builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(p.sc, (lane & 15) * 8, tile * 128, 0));
+  if constexpr (has_min<QT>()) t.m = __builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(p.mn, (lane & 15) * 8, tile * 128, 0));
+}
+
 // WM x WN wavefronts; a wavefront owns MTW x NTW 16 x 16 output tiles
-template <int QT, int WM, int WN, int MTW, int NTW, int PH>
+template <int QT, int WM, int WN, int MTW, int NTW>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_prompt_kernel(GemmArgs a) {
   constexpr int NW = WM * WN;
   constexpr int BM = WM * MTW * 16, BN = WN * NTW * 16;
-  constexpr int NA = BM / (8 * NW);                 // global_load_lds per lane and x tile
-  constexpr bool PP = NW == 8;                      // two wavefronts per SIMD: the row halves run as a ping-pong pair
+  constexpr int NA = BM / (8 * NW);                 // requests per wavefront and x tile
   // weight tile rows (16 rows each) of the block over the wavefronts: FULL whole rows per wavefront, and with 1.5 rows per
   // wavefront (BN = 192 on 8 wavefronts) a pair of wavefronts shares a third row, one k half of the T16 tile each
   constexpr int RT = BN / 16;
   constexpr int FULL = RT / NW, HALF = (RT % NW) ? 1 : 0;
-  static_assert(BM % (8 * NW) == 0 && (RT % NW == 0 || (2 * RT == 3 * NW && NW % 2 == 0)), "tile does not divide over the wavefronts");
-  constexpr int SLOTS = FULL + HALF, NUW = 2 * SLOTS;  // expansion units per wavefront and 64-deep tile (at most)
+  constexpr int SLOTS = FULL + HALF;
+  constexpr int RL = SLOTS * raw_loads<QT>();        // weight requests per wavefront and T16 tile
+  // (large tiles of formats that need more registers: the fragment reads stay behind the MFMAs they replace, or the loop spills: fp6
+  // 256 x 256 2x slower, int8 and int5 6 - 10 %; where they fit, reads in between are up to 3 % faster)
+  constexpr bool TIGHT = MTW * NTW >= 24 && (lo_bits_of(QT) == 8 || hi_bits_of(QT) > 0);
+  static_assert(NW == 8 && BM % (8 * NW) == 0 && RT % 2 == 0 && (RT % NW == 0 || 2 * RT == 3 * NW), "tile does not divide over the wavefronts");
   constexpr int ABYTES = BM * 128, BBYTES = BN * 128;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  char* const As = smem;                            // [2][BM][128 B]
-  char* const Bs = smem + 2 * ABYTES;               // [2][BN][128 B]
+  char* const As = smem;                            // [3][BM][128 B]
+  char* const Bs = smem + 3 * ABYTES;               // [2][BN][128 B]
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -116,71 +147,52 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_prompt_kernel(GemmArgs a
   const int row0 = mb * BM, rows = min(BM, a.M - row0);
   const int kt0 = sp * a.kt_per_split, kt1 = min(KT, kt0 + a.kt_per_split);
   const int nkt = kt1 - kt0, T = 2 * nkt;            // T16 k tiles / 64-deep tiles of this workgroup
-  const T16Planes pl = t16_planes(a.w, QT, a.N, a.K);
-  const T16Planes pl2 = t16_planes(pair ? a.w2 : a.w, QT, a.N, a.K);
 
-  // ---- x tile (32-bit byte offsets from one scalar base: M * ldx < 2^31).  Every wavefront stages rows of its own row half
-  // (the half it reads fragments from, so that the two halves of the workgroup may run out of step); instruction p fills
-  // rows 8 (p WN + wn) .. + 7 of the half; lane i brings the 16 bytes that belong in slot i % 8 of row i / 8, i.e. k slot
+  // ---- x tile (32-bit byte offsets from the block's first row: M * ldx < 2^31); instruction p of wavefront (wm, wn) fills rows
+  // 8 (p WN + wn) .. + 7 of its half; lane i brings the 16 bytes that belong in slot i % 8 of row i / 8, i.e. k slot
   // (i % 8) ^ (i / 8) of that row (rows past the block re-read its last row: never stored)
   uint32_t xoff[NA];
 #pragma unroll
   for (int p = 0; p < NA; ++p) {
     const int row = wm * (BM / WM) + (p * WN + wn) * 8 + (lane >> 3);
-    xoff[p] = ((uint32_t)(row0 + min(row, rows - 1)) * (uint32_t)a.ldx + (uint32_t)((((lane & 7) ^ (lane >> 3)) & 7) << 3)) * 2u;
+    xoff[p] = ((uint32_t)min(row, rows - 1) * (uint32_t)a.ldx + (uint32_t)((((lane & 7) ^ (lane >> 3)) & 7) << 3)) * 2u;
   }
-  auto stage_a = [&](int t, int buf) {
-    const char* src = (const char*)(a.x + (int64_t)(2 * kt0 + t) * 64);
+  const auto xb = buf_of(a.x + (int64_t)row0 * a.ldx + kt0 * 128);
+  auto stage_a = [&](int t, int buf, int p) {
     char* dst = As + buf * ABYTES + (wm * (BM / WM) + wn * 8) * 128;     // wave-uniform; the instruction adds lane * 16
-#pragma unroll
-    for (int p = 0; p < NA; ++p)
-      __builtin_amdgcn_global_load_lds((glb_cvoid_t*)(src + xoff[p]), (lds_void_t*)(dst + p * WN * 1024), 16, 0, 0);
+    lds_dma16(xb, dst + p * WN * 1024, xoff[p], t * 128);
   };
 
-  // ---- weight tile rows of this wavefront (block-relative index; clamped in the buffer: a row past N is loaded from the
-  // last valid one and never stored) and their raw data: one whole T16 tile (128 k = two 64-deep tiles) per slot, loaded
-  // once per pair of tiles with full 16-byte code loads
+  // ---- weight tile rows of this wavefront (block-relative index; a row past N is loaded from the last valid one and never
+  // stored) and their raw data: one whole T16 tile (128 k = two 64-deep tiles) per slot
   const int ntiles = (a.N + 15) >> 4;
-  static_assert(RT % 2 == 0, "the pair form splits the block's tile rows in two");
-  int slot_rt[SLOTS], slot_second[SLOTS];
-  int64_t slot_tile[SLOTS];
+  int slot_rt[SLOTS];
+  RowPlanes wp[SLOTS];
 #pragma unroll
   for (int i = 0; i < SLOTS; ++i) {
     if constexpr (HALF) slot_rt[i] = (wave >> 1) * 3 + (i < FULL ? (wave & 1) : 2);
     else slot_rt[i] = wave * FULL + i;
-    const int second = pair && slot_rt[i] >= RT / 2;
+    const bool second = pair && slot_rt[i] >= RT / 2;
     const int trow = pair ? nb * (RT / 2) + slot_rt[i] - second * (RT / 2) : nb * RT + slot_rt[i];
-    slot_tile[i] = (int64_t)min(trow, ntiles - 1) * KT + kt0;
-    slot_second[i] = second;
+    wp[i] = row_planes<QT>(t16_planes(second ? a.w2 : a.w, QT, a.N, a.K), (int64_t)min(trow, ntiles - 1) * KT + kt0);
   }
   const int half_sel = wave & 1;                     // which k half of the shared row this wavefront expands
   Tile<QT> rawC[SLOTS], rawN[SLOTS];                 // T16 tile being expanded / the next one (in flight)
-  auto fetch_raw = [&](Tile<QT> (&raw)[SLOTS], int kt) {
-#pragma unroll
-    for (int i = 0; i < SLOTS; ++i) load_tile<QT>(raw[i], slot_second[i] ? pl2 : pl, slot_tile[i] + kt, lane);
-  };
 
   // fragment slot of k step s for this lane: (4 s + g) ^ (r & 7); s = 1 flips bit 2
   const int fsw0 = ((g ^ (r & 7)) & 7) << 4;
   const int frag_off[2] = {r * 128 + fsw0, r * 128 + (fsw0 ^ 64)};
 
-  // expansion of units [u0, u1) of the 64-deep tile with parity h (= its LDS buffer) from the current raw set: unit u is
-  // k step u % 2 of slot u / 2; the shared row's units exist only in the wavefront that owns that k half
-  auto expand = [&](auto hc, auto u0c, auto u1c) {
-    constexpr int h = decltype(hc)::value, u0 = decltype(u0c)::value, u1 = decltype(u1c)::value;
-    char* base = Bs + h * BBYTES;
-#pragma unroll
-    for (int u = u0; u < u1; ++u) {
-      const int i = u >> 1;
-      if (i >= FULL && half_sel != h) continue;        // wave-uniform
-      half8 v0, v1;
-      // (both steps of the parity are instantiated, the static one is kept: decode_step wants a constant step)
-      if (u & 1) v0 = unit_expand<QT, 2 * h + 1>(rawC[i]);
-      else v0 = unit_expand<QT, 2 * h>(rawC[i]);
-      if constexpr (PROMPT_ABL & 4) v0 = __builtin_bit_cast(half8, uint4v{rawC[i].lo0[0], rawC[i].lo0[1], 0x3c003c00u, 0x3c003c00u});
-      (void)v1;
-      *(half8*)(base + slot_rt[i] * 2048 + frag_off[u & 1]) = v0;
-    }
+  // unit u (k step u % 2 of slot u / 2) of a 64-deep tile of parity h, from rawC to the weight buffer h; the shared row's units
+  // exist only in the wavefront that owns that k half
+  auto expand = [&](auto hc, int u) {
+    constexpr int h = decltype(hc)::value;
+    const int i = u >> 1;
+    if (i >= FULL && half_sel != h) return;          // wave-uniform
+    half8 v;
+    if (u & 1) v = unit_expand<QT, 2 * h + 1>(rawC[i]);
+    else v = unit_expand<QT, 2 * h>(rawC[i]);
+    *(half8*)(Bs + h * BBYTES + slot_rt[i] * 2048 + frag_off[u & 1]) = v;
   };
 
   float4v acc[MTW][NTW];
@@ -191,221 +203,99 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_prompt_kernel(GemmArgs a
 
   typedef std::integral_constant<int, 0> I0;
   typedef std::integral_constant<int, 1> I1;
+  typedef std::integral_constant<int, 2> I2;
+  typedef std::integral_constant<int, 3> I3;
   auto lds_w = [&](int buf, int s) { return Bs + buf * BBYTES + wn * (NTW * 2048) + frag_off[s]; };
   auto lds_x = [&](int buf, int s) { return As + buf * ABYTES + wm * (MTW * 2048) + frag_off[s]; };
-  auto frag = [&](const char* p, int i) {
-    if constexpr (PROMPT_ABL & 32) return __builtin_bit_cast(half8, uint4v{(uint32_t)(uintptr_t)p + i, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u});
-    else return *(const half8*)(p + i * 2048);
-  };
-  auto mfma_or_not = [&](float4v& c, const half8& w, const half8& x) {
-    if constexpr (PROMPT_ABL & 16) {
-      const uint4v v = __builtin_bit_cast(uint4v, x) ^ __builtin_bit_cast(uint4v, w);
-      c[0] += __uint_as_float((v[0] ^ v[1] ^ v[2] ^ v[3]) & 0x3f800000u);
-    } else {
-      c = mfma16(w, x, c);                             // D[n = 4 g + q][m = r]
-    }
-  };
+  auto frag = [&](const char* p, int i) { return *(const half8*)(p + i * 2048); };
 
-  if constexpr (PP) {
-    // ---- ping-pong pipeline (8 wavefronts = two per SIMD).  A 64-deep tile runs as PH phases (PH = 1: both k steps at
-    // once, PH = 2: one k step each); a phase is a LOAD segment (the phase's fragment reads, its share of the expansion
-    // of tile t + 1 into the other weight buffer, the tile's global requests) and a COMPUTE segment (the phase's MFMAs,
-    // nothing else), with a workgroup barrier after every segment.  The wavefronts of row half 1 (waves 4 - 7: the SIMD
-    // partners of waves 0 - 3) pass one extra barrier before the loop, so they are always one segment behind: while one
-    // wavefront of a SIMD holds the matrix pipe its partner reads LDS, expands weights and issues loads, and neither
-    // sits in the other's issue slots.  What makes the skew safe:
-    //  * x rows are staged by the row half that reads them, and a half is in step with itself;
-    //  * a weight buffer is last read in the last load segment of its tile and first rewritten in the first load
-    //    segment of the next tile, when the trailing half is already in the compute segment behind that last read; its
-    //    expansion ends in the last load segment of the tile before, one segment before the leading half's first read;
-    //  * LDS stores and fragment reads are waited for (lgkmcnt(0)) before the barrier that ends their segment, global
-    //    requests (x tile t + 1, issued in the first segment of tile t; raw weight tiles, issued two tiles ahead)
-    //    before the last barrier of the tile.
-    constexpr int SP = 2 / PH;                       // k steps per phase
-    half8 wf[SP][NTW], xf[SP][MTW];
-    auto seg_end = [&]() {
-      __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(63));
+  // ---- the loop.  Tile t (x buffer t % 3, weight buffer t % 2) runs as two k steps of MTW groups of NTW MFMAs.  Fragments: x in one
+  // register set that rolls (group j's is replaced behind its last use), weights in two.  At the turn between the two steps of
+  // tile t every read of tile t is done and every store of tile t + 1, hence:
+  //  * second step of t, first of t + 1: tile t + 2 is expanded into weight buffer t % 2; second step: x tile t + 3 is requested
+  //    into x buffer t % 3.  Both are last read in the first step of t, before the turn (lgkmcnt(0), barrier);
+  //  * what the second step of t reads of tile t + 1: its expansion ended in the first step of t, its x was requested a tile and a
+  //    half ago (vmcnt: what is younger may still be under way).
+  half8 wf[2][NTW], xf[MTW];
+  // k step S (0 .. 3 of the T16 tile) of tile t = 2 kt + S / 2
+  auto step = [&](auto sc, int t, int xcur, int xnext, int xfree) {
+    constexpr int S = decltype(sc)::value;
+    constexpr bool first = (S & 1) == 0;               // first k step of a tile
+    // what is read for the next k step, and the weight tile under expansion: t + 1 in the first k step (its second half of
+    // units), t + 2 in the second
+    const char* px = first ? lds_x(xcur, 1) : lds_x(xnext, 0);
+    const char* pw = first ? lds_w(S >> 1, 1) : lds_w((S >> 1) ^ 1, 0);
+    typedef std::integral_constant<int, first ? (S >> 1) ^ 1 : (S >> 1)> H;
+#pragma unroll
+    for (int j = 0; j < MTW; ++j) {
+#pragma unroll
+      for (int n = 0; n < NTW; ++n) acc[j][n] = mfma16(wf[S & 1][n], xf[j], acc[j][n]);     // D[n = 4 g + q][m = r]
+      if constexpr (TIGHT) __builtin_amdgcn_sched_barrier(0);
+      xf[j] = frag(px, j);
+#pragma unroll
+      for (int n = 0; n < NTW; ++n)
+        if (n * MTW / NTW == j) wf[~S & 1][n] = frag(pw, n);
+#pragma unroll
+      for (int u = 0; u < SLOTS; ++u)
+        if ((2 * u + 1) * MTW / (2 * SLOTS) == j) expand(H{}, first ? SLOTS + u : u);
+      if constexpr (!first) {
+#pragma unroll
+        for (int p = 0; p < NA; ++p)
+          if (p * MTW / NA == j) stage_a(min(t + 3, T - 1), xfree, p);
+      }
+      if constexpr (S == 2) {
+#pragma unroll
+        for (int i = 0; i < SLOTS; ++i)
+          if (i * MTW / SLOTS == j) load_raw<QT>(rawN[i], wp[i], min((t >> 1) + 2, nkt - 1), lane);
+      }
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (!(PROMPT_ABL & 8)) __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    auto load_seg = [&](auto curc, auto phc, int t) {
-      constexpr int cur = decltype(curc)::value, nxt = cur ^ 1, ph = decltype(phc)::value;
-#pragma unroll
-      for (int s = 0; s < SP; ++s) {
-        const char* pw = lds_w(cur, ph * SP + s);
-        const char* px = lds_x(cur, ph * SP + s);
-#pragma unroll
-        for (int n = 0; n < NTW; ++n) wf[s][n] = frag(pw, n);
-        // (one phase per tile: the x fragments of the second k step are read under the first step's MFMAs: x rows belong
-        // to this row half alone, while a weight buffer may be rewritten by the other half during the compute segment)
-        if (PH == 1 && s == 1) continue;
-#pragma unroll
-        for (int j = 0; j < MTW; ++j) xf[s][j] = frag(px, j);
-      }
-      if constexpr (ph == 0) {
-        if constexpr (!(PROMPT_ABL & 2)) stage_a(min(t + 1, T - 1), nxt);
-        // odd tile 2 j + 1: the raw T16 tile j + 2 (first expanded two tiles later) goes into the set copied out after
-        // the previous tile
-        if constexpr (cur == 1 && !(PROMPT_ABL & 1)) fetch_raw(rawN, min((t >> 1) + 2, nkt - 1));
-      }
-      expand(std::integral_constant<int, nxt>{}, std::integral_constant<int, ph * NUW / PH>{},
-             std::integral_constant<int, (ph + 1) * NUW / PH>{});
-      seg_end();
-    };
-    auto comp_seg = [&](auto curc, auto phc) {
-      constexpr int cur = decltype(curc)::value, ph = decltype(phc)::value;
-      __builtin_amdgcn_s_setprio(1);
-      if constexpr (PH == 1) {
-        const char* px = lds_x(cur, 1);
-#pragma unroll
-        for (int j = 0; j < MTW; ++j) xf[1][j] = frag(px, j);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int s = 0; s < SP; ++s) {
-#pragma unroll
-        for (int j = 0; j < MTW; ++j)
-#pragma unroll
-          for (int n = 0; n < NTW; ++n) mfma_or_not(acc[j][n], wf[s][n], xf[s][j]);
-        if constexpr (PH == 1) __builtin_amdgcn_sched_barrier(0);
-      }
-      __builtin_amdgcn_s_setprio(0);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (ph == PH - 1) {
-        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-        if constexpr (cur == 0) {                      // even tile done: its T16 tile is used up, the next one has landed
-#pragma unroll
-          for (int i = 0; i < SLOTS; ++i) rawC[i] = rawN[i];
-        }
-      }
-      if constexpr (!(PROMPT_ABL & 8)) __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    fetch_raw(rawC, 0);
-    stage_a(0, 0);
-    fetch_raw(rawN, min(1, nkt - 1));
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-    expand(I0{}, I0{}, std::integral_constant<int, NUW>{});
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(63));
-    __builtin_amdgcn_s_barrier();
-    if (wm == 1) __builtin_amdgcn_s_barrier();
-    for (int t = 0; t < T; t += 2) {
-      load_seg(I0{}, I0{}, t);
-      comp_seg(I0{}, I0{});
-      if constexpr (PH == 2) {
-        load_seg(I0{}, I1{}, t);
-        comp_seg(I0{}, I1{});
-      }
-      load_seg(I1{}, I0{}, t + 1);
-      comp_seg(I1{}, I0{});
-      if constexpr (PH == 2) {
-        load_seg(I1{}, I1{}, t + 1);
-        comp_seg(I1{}, I1{});
-      }
     }
-    if (wm == 0) __builtin_amdgcn_s_barrier();
-  } else {
-    // ---- software-pipelined form (4 wavefronts, one per SIMD: no partner to alternate with; none of the configurations
-    // in gemm_prompt_launch uses it since the 128 x 128 tile went to 8 wavefronts).  Tile t (LDS buffers t % 2)
-    // runs as four phases of HM x NTW MFMAs: (k step 0, row half 0), (0, 1), (1, 0), (1, 1); fragments live in two named
-    // register sets per operand (the set of the phase in flight and the set being filled for the next one; static
-    // indices: a run-time set index would put them in scratch).  Phases 0 - 2 also expand tile t + 1 into the other weight
-    // buffer and read the next phase's fragments; the scheduler is asked to put one MFMA, then a few vector instructions,
-    // then an LDS read, and so on, so that expansion and reads ride in the issue slots between the MFMAs.  Phase 3 opens
-    // with the tile's only barrier: behind it every wavefront has its last fragments of tile t in registers and tile
-    // t + 1 is complete in LDS (own stores: lgkmcnt(0); x tile t + 1 and the raw weights, requested a tile or more
-    // earlier: vmcnt(0)), so the phase requests x tile t + 2 into the buffer just released, reads the first fragments of
-    // tile t + 1 and runs its MFMAs under those reads.
-    constexpr int HM = MTW / 2;
-    static_assert(MTW % 2 == 0 && HALF == 0, "a phase covers half of the wavefront's row tiles");
-    half8 wfA[NTW], wfB[NTW], xfA[HM], xfB[HM];
-    auto read_w = [&](half8 (&wf)[NTW], int buf, int s) {
-      const char* p = lds_w(buf, s);
-#pragma unroll
-      for (int n = 0; n < NTW; ++n) wf[n] = frag(p, n);
-    };
-    auto read_x = [&](half8 (&xf)[HM], int buf, int s, int half) {
-      const char* p = lds_x(buf, s) + half * (HM * 2048);
-#pragma unroll
-      for (int j = 0; j < HM; ++j) xf[j] = frag(p, j);
-    };
-    auto mma = [&](const half8 (&wf)[NTW], const half8 (&xf)[HM], auto halfc) {
-      constexpr int half = decltype(halfc)::value;
-#pragma unroll
-      for (int j = 0; j < HM; ++j)
-#pragma unroll
-        for (int n = 0; n < NTW; ++n) mfma_or_not(acc[half * HM + j][n], wf[n], xf[j]);
-    };
-    auto interleave = [&](auto nmc, auto nvc, auto nrc, auto nwc) {
-      constexpr int nm = decltype(nmc)::value, nv = decltype(nvc)::value, nr = decltype(nrc)::value, nw = decltype(nwc)::value;
-#pragma unroll
-      for (int k = 0; k < nm; ++k) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (k < nr) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        if (nv > 0) __builtin_amdgcn_sched_group_barrier(0x002, nv, 0);
-        if (k >= nm - nw) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-      }
-    };
-    constexpr int PM = HM * NTW;                      // MFMAs per phase
-    constexpr int U0 = NUW - 2 * (NUW / 3), U1 = U0 + NUW / 3, U2 = NUW;     // units per phase: 4 -> 2, 1, 1
-    constexpr int VPU = 16;                           // vector instructions of one unit's expansion (scheduling hint)
-    typedef std::integral_constant<int, PM> CPM;
-    auto tile_body = [&](auto curc, int t) {
-      constexpr int cur = decltype(curc)::value, nxt = cur ^ 1;
-      typedef std::integral_constant<int, nxt> HN;
-      // phase 0
-      read_x(xfB, cur, 0, 1);
-      expand(HN{}, std::integral_constant<int, 0>{}, std::integral_constant<int, U0>{});
-      mma(wfA, xfA, I0{});
-      interleave(CPM{}, std::integral_constant<int, (U0 * VPU + PM - 1) / PM>{}, std::integral_constant<int, HM>{}, std::integral_constant<int, U0>{});
-      __builtin_amdgcn_sched_barrier(0);
-      // phase 1
-      read_w(wfB, cur, 1);
-      read_x(xfA, cur, 1, 0);
-      expand(HN{}, std::integral_constant<int, U0>{}, std::integral_constant<int, U1>{});
-      mma(wfA, xfB, I1{});
-      interleave(CPM{}, std::integral_constant<int, ((U1 - U0) * VPU + PM - 1) / PM>{}, std::integral_constant<int, HM + NTW>{}, std::integral_constant<int, U1 - U0>{});
-      __builtin_amdgcn_sched_barrier(0);
-      // phase 2
-      read_x(xfB, cur, 1, 1);
-      expand(HN{}, std::integral_constant<int, U1>{}, std::integral_constant<int, U2>{});
-      mma(wfB, xfA, I0{});
-      interleave(CPM{}, std::integral_constant<int, ((U2 - U1) * VPU + PM - 1) / PM>{}, std::integral_constant<int, HM>{}, std::integral_constant<int, U2 - U1>{});
-      __builtin_amdgcn_sched_barrier(0);
-      // phase 3
-      __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
-      if constexpr (!(PROMPT_ABL & 8)) __builtin_amdgcn_s_barrier();
-      if constexpr (cur == 0) {
-#pragma unroll
-        for (int i = 0; i < SLOTS; ++i) rawC[i] = rawN[i];
-      }
-      if constexpr (!(PROMPT_ABL & 2)) stage_a(min(t + 2, T - 1), cur);
-      if constexpr (cur == 1 && !(PROMPT_ABL & 1)) fetch_raw(rawN, min((t >> 1) + 2, nkt - 1));
-      read_w(wfA, nxt, 0);
-      read_x(xfA, nxt, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      mma(wfB, xfB, I1{});
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    fetch_raw(rawC, 0);
-    stage_a(0, 0);
-    fetch_raw(rawN, min(1, nkt - 1));
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-    expand(I0{}, I0{}, std::integral_constant<int, NUW>{});
-    __builtin_amdgcn_sched_barrier(0);
-    stage_a(1, 1);
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(63));    // own LDS stores
+  };
+  auto turn = [&](auto nc) {
+    // own reads and stores done, the next x tile landed
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(decltype(nc)::value));
     __builtin_amdgcn_s_barrier();
-    read_w(wfA, 0, 0);
-    read_x(xfA, 0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
-    for (int t = 0; t < T; t += 2) {
-      tile_body(I0{}, t);
-      tile_body(I1{}, t + 1);
-    }
+  };
+#pragma unroll
+  for (int i = 0; i < SLOTS; ++i) load_raw<QT>(rawC[i], wp[i], 0, lane);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int p = 0; p < NA; ++p) stage_a(0, 0, p);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int p = 0; p < NA; ++p) stage_a(1, 1, p);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < SLOTS; ++i) load_raw<QT>(rawN[i], wp[i], min(1, nkt - 1), lane);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int p = 0; p < NA; ++p) stage_a(min(2, T - 1), 2, p);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < 2 * SLOTS; ++u) expand(I0{}, u);
+#pragma unroll
+  for (int u = 0; u < SLOTS; ++u) expand(I1{}, u);
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(2 * NA + RL));
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int j = 0; j < MTW; ++j) xf[j] = frag(lds_x(0, 0), j);
+#pragma unroll
+  for (int n = 0; n < NTW; ++n) wf[0][n] = frag(lds_w(0, 0), n);
+  int b0 = 0;
+  for (int t = 0; t < T; t += 2) {
+    const int b1 = b0 == 2 ? 0 : b0 + 1, b2 = b1 == 2 ? 0 : b1 + 1;
+    step(I0{}, t, b0, b1, b2);
+    turn(std::integral_constant<int, NA>{});           // younger than x tile t + 1: x tile t + 2 (and raw weights that rawC takes now)
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) rawC[i] = rawN[i];
+    step(I1{}, t, b0, b1, b0);
+    step(I2{}, t + 1, b1, b2, b0);
+    turn(std::integral_constant<int, NA + RL>{});      // younger than x tile t + 2: x tile t + 3, raw weights
+    step(I3{}, t + 1, b1, b2, b1);
+    b0 = b2;
   }
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));         // the clamped look-ahead loads of the last tile
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));   // the look-ahead of the last tile: requests (clamped), reads and expansion
 
   // ---- epilogue.  A lane holds 4 consecutive output columns (n = 16 tile + 4 g + q) of row m = 16 j + r.
   // Two forms: fp32 partial slabs (K splits, or an output the staged form does not cover: the reduce kernel of
@@ -483,81 +373,75 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_prompt_kernel(GemmArgs a
     else it1 = ITS / 2;
     stg2 = stg + (WN / 2) * (MTW * 16 * RB);
   }
-#pragma unroll 1
-  for (int it = it0; it < it1; ++it) {
-    const int idx = it * 64 + lane, row = idx / CH, ch = idx % CH;
-    const int col = ocol0 + ch * 8;
-    if (orow0 + row >= row0 + rows || col >= a.N) continue;
-    uint4v pk = *(const uint4v*)(stg + row * RB + ch * 16);
-    const int64_t oi = (int64_t)(orow0 + row) * a.ldo + col;
-    if (pair) {
-      // act(first) * second on the rounded 16-bit values (what a separate activation kernel would read)
-      const uint4v pu = *(const uint4v*)(stg2 + row * RB + ch * 16);
+  // the 16-bit pairs of a 16-byte chunk, f(first, second) each
+  auto chunk = [&](uint4v p, uint4v q, auto f) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float lo, hi, ulo, uhi;
-        if (a.out_type == OUT_F16) {
-          const half2v h = u2h(pk[e]), hu = u2h(pu[e]);
-          lo = (float)h[0]; hi = (float)h[1]; ulo = (float)hu[0]; uhi = (float)hu[1];
-        } else {
-          lo = bf16_bits_to_f32((uint16_t)(pk[e] & 0xffffu)); hi = bf16_bits_to_f32((uint16_t)(pk[e] >> 16));
-          ulo = bf16_bits_to_f32((uint16_t)(pu[e] & 0xffffu)); uhi = bf16_bits_to_f32((uint16_t)(pu[e] >> 16));
-        }
-        lo = act_apply(a.act, lo) * ulo;
-        hi = act_apply(a.act, hi) * uhi;
-        if (a.out_type == OUT_F16) pk[e] = h2u(half2v{(_Float16)lo, (_Float16)hi});
-        else pk[e] = (uint32_t)f32_to_bf16_bits(lo) | ((uint32_t)f32_to_bf16_bits(hi) << 16);
+    for (int e = 0; e < 4; ++e) {
+      float lo, hi, qlo, qhi;
+      if (a.out_type == OUT_F16) {
+        const half2v h = u2h(p[e]), hq = u2h(q[e]);
+        lo = (float)h[0]; hi = (float)h[1]; qlo = (float)hq[0]; qhi = (float)hq[1];
+      } else {
+        lo = bf16_bits_to_f32((uint16_t)(p[e] & 0xffffu)); hi = bf16_bits_to_f32((uint16_t)(p[e] >> 16));
+        qlo = bf16_bits_to_f32((uint16_t)(q[e] & 0xffffu)); qhi = bf16_bits_to_f32((uint16_t)(q[e] >> 16));
       }
-    } else if (!plain) {
-      uint4v rr = uint4v{0, 0, 0, 0};
-      if (a.residual != nullptr) rr = *(const uint4v*)((const uint16_t*)a.residual + oi);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float lo, hi, rlo, rhi;
-        if (a.out_type == OUT_F16) {
-          const half2v h = u2h(pk[e]), hr = u2h(rr[e]);
-          lo = (float)h[0]; hi = (float)h[1]; rlo = (float)hr[0]; rhi = (float)hr[1];
-        } else {
-          lo = bf16_bits_to_f32((uint16_t)(pk[e] & 0xffffu)); hi = bf16_bits_to_f32((uint16_t)(pk[e] >> 16));
-          rlo = bf16_bits_to_f32((uint16_t)(rr[e] & 0xffffu)); rhi = bf16_bits_to_f32((uint16_t)(rr[e] >> 16));
-        }
-        lo = act_apply(a.act, lo) + rlo;
-        hi = act_apply(a.act, hi) + rhi;
-        if (a.out_type == OUT_F16) pk[e] = h2u(half2v{(_Float16)lo, (_Float16)hi});
-        else pk[e] = (uint32_t)f32_to_bf16_bits(lo) | ((uint32_t)f32_to_bf16_bits(hi) << 16);
-      }
+      lo = f(lo, qlo);
+      hi = f(hi, qhi);
+      if (a.out_type == OUT_F16) p[e] = h2u(half2v{(_Float16)lo, (_Float16)hi});
+      else p[e] = (uint32_t)f32_to_bf16_bits(lo) | ((uint32_t)f32_to_bf16_bits(hi) << 16);
     }
-    *(uint4v*)((uint16_t*)a.out + oi) = pk;
-  }
+    return p;
+  };
+  // fn(own chunk, the same chunk of the partner's tile or the residual) -> what is stored
+  auto rows_out = [&](auto fn) {
+#pragma unroll 2
+    for (int it = it0; it < it1; ++it) {
+      const int idx = it * 64 + lane, row = idx / CH, ch = idx % CH;
+      const int col = ocol0 + ch * 8;
+      if (orow0 + row >= row0 + rows || col >= a.N) continue;
+      const uint4v p = *(const uint4v*)(stg + row * RB + ch * 16);
+      const int64_t oi = (int64_t)(orow0 + row) * a.ldo + col;
+      uint4v q = uint4v{0, 0, 0, 0};
+      if (pair) q = *(const uint4v*)(stg2 + row * RB + ch * 16);
+      else if (a.residual != nullptr) q = *(const uint4v*)((const uint16_t*)a.residual + oi);
+      *(uint4v*)((uint16_t*)a.out + oi) = fn(p, q);
+    }
+  };
+  // act(first) * second on the rounded 16-bit values (what a separate activation kernel would read).  The usual gate has a loop of
+  // its own: with the choice of the activation inside, an element took twice the instructions
+  if (pair && a.act == ACT_SILU) rows_out([&](uint4v p, uint4v q) { return chunk(p, q, [](float x, float u) { return act_apply(ACT_SILU, x) * u; }); });
+  else if (pair) rows_out([&](uint4v p, uint4v q) { return chunk(p, q, [&](float x, float u) { return act_apply(a.act, x) * u; }); });
+  else if (plain) rows_out([](uint4v p, uint4v) { return p; });
+  else rows_out([&](uint4v p, uint4v q) { return chunk(p, q, [&](float x, float u) { return act_apply(a.act, x) + u; }); });
 }
 
-template <int QT, int WM, int WN, int MTW, int NTW, int PH>
+template <int QT, int WM, int WN, int MTW, int NTW>
 static int gemm_prompt_launch_cfg(const GemmArgs& a, hipStream_t st) {
   constexpr int NW = WM * WN, BM = WM * MTW * 16, BN = WN * NTW * 16;
   const size_t lds = prompt_lds_tiles(BM, BN, NW, MTW, NTW);
   static bool attr_set = false;
   if (!attr_set) {
-    if (hipFuncSetAttribute((const void*)gemm_prompt_kernel<QT, WM, WN, MTW, NTW, PH>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    if (hipFuncSetAttribute((const void*)gemm_prompt_kernel<QT, WM, WN, MTW, NTW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return -101;
     attr_set = true;
   }
   const int bno = a.w2 != nullptr ? BN / 2 : BN;
   const int tiles = ((a.M + BM - 1) / BM) * ((a.N + bno - 1) / bno);
-  hipLaunchKernelGGL((gemm_prompt_kernel<QT, WM, WN, MTW, NTW, PH>), dim3(tiles * a.splitk), dim3(64 * NW), lds, st, a);
+  hipLaunchKernelGGL((gemm_prompt_kernel<QT, WM, WN, MTW, NTW>), dim3(tiles * a.splitk), dim3(64 * NW), lds, st, a);
   return HIP_CHECK_LAUNCH();
 }
 
-// configurations in the order of gemm_prompt.hip's table: 256 x 256, 256 x 192, 128 x 128 (8 wavefronts each)
-#define PROMPT_NCFG 3
+// configurations in the order of gemm_prompt.hip's table: 256 x 256, 256 x 192, 128 x 128, 256 x 128, 192 x 256, 192 x 128
+#define PROMPT_NCFG 6
 template <int QT>
 static int gemm_prompt_launch(const GemmArgs& a, int cfg, hipStream_t st) {
   switch (cfg) {
-    case 0: return gemm_prompt_launch_cfg<QT, 2, 4, 8, 4, PROMPT_PH0>(a, st);
-    case 1: return gemm_prompt_launch_cfg<QT, 2, 4, 8, 3, PROMPT_PH1>(a, st);
-    // 128 x 128 also runs on 8 wavefronts as a ping-pong pair of row halves (one phase per 64-deep tile): 43.8 us on
-    // the 1024 x 4096 x 4096 product against 54.4 us with 4 wavefronts of 64 x 64 each (and ahead on every other shape).
-    // 128 x 256 and 256 x 128 tiles on 8 wavefronts were measured too: within 4 % of the planned choice at best.
-    case 2: return gemm_prompt_launch_cfg<QT, 2, 4, 4, 2, 1>(a, st);
+    case 0: return gemm_prompt_launch_cfg<QT, 2, 4, 8, 4>(a, st);
+    case 1: return gemm_prompt_launch_cfg<QT, 2, 4, 8, 3>(a, st);
+    case 2: return gemm_prompt_launch_cfg<QT, 2, 4, 4, 2>(a, st);
+    case 3: return gemm_prompt_launch_cfg<QT, 2, 4, 8, 2>(a, st);
+    case 4: return gemm_prompt_launch_cfg<QT, 2, 4, 6, 4>(a, st);
+    case 5: return gemm_prompt_launch_cfg<QT, 2, 4, 6, 2>(a, st);
     default: return -4;
   }
 }

@@ -26,6 +26,7 @@
 //    group of wavefronts taking alternate key tiles (51 / 588 us on the earlier kernel), tiles requested two phases
 //    ahead through a second register set (29 / 295 us), the normaliser as an extra MFMA row block (no change).
 #include "common.h"
+#include <type_traits>
 
 namespace bigdl {
 
@@ -62,6 +63,27 @@ __device__ __forceinline__ float pf_sum4(float x) {
 __device__ __forceinline__ float pf_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 // how far a tile's maximum may exceed the running one before the accumulators are rescaled: weights stay <= 2^8
 constexpr float PF_LAZY = 8.0f;
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t pf_buf(const void* p) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0xffffffff, 0x00027000);
+}
+// 16 bytes per lane to consecutive LDS
+__device__ __forceinline__ void pf_dma16(__amdgpu_buffer_rsrc_t b, char* lds, uint32_t off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(b, (__attribute__((address_space(3))) void*)lds, 16, off, 0, 0, 0);
+}
+
+// f(integral_constant) for I .. N - 1
+template <int I, int N, typename F>
+__device__ __forceinline__ void pf_for(F f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    pf_for<I + 1, N>(f);
+  }
+}
+
+__device__ __forceinline__ float16v pf_mfma32(half8 a, half8 b, float16v c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
 
 // QB = 16-query blocks per wavefront: every K / V^T fragment read from LDS feeds QB MFMAs, which is what keeps the
 // kernel off the LDS-bandwidth limit (QB = 2: 128 queries per workgroup).
@@ -403,6 +425,304 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(PrefillArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
+// The long-prompt form (V transposed, no additive mask, ALiBi or soft cap; head_dim 64 / 128): 8 wavefronts of 32 queries each, so
+// a K / V^T fragment read from LDS feeds a product of 32 queries, in two groups that run out of step.  A tile of 64 keys is two blocks of a
+// wavefront's time: the weights (exponentials: vector unit) and the products S^T of the next tile and O^T of this one (matrix unit,
+// LDS).  The groups (wavefronts w and w + 4 share a SIMD) are one block apart, a barrier
+// behind every block: while one group multiplies the other takes exponentials.
+// SPLIT: the groups take alternate tiles of the same 128 queries, each with its own tile buffers, and are added up at the end.
+// What bounds it: power and the vector unit.  7700 tokens of 32 heads, causal: 798 us of the kernel above -> 508 (960 TFLOP/s), about 4000
+// cycles for a tile of the 8 wavefronts (2230 of MFMAs) at 1.6 GHz; with 16 x 16 x 32 MFMAs 4550 cycles at 1.8 GHz, the same time.
+// 1024 tokens 28.1 -> 25.0, 2048 86.9 -> 55.4, 4096 254 -> 153.  Measured and dropped: the three parts of a tile in one instruction stream
+// (values of the tile before, softmax, scores of the next; registers for two sets of scores: 7 % slower), tiles through registers
+// instead of straight to LDS, all requests of a tile at once, 4 and 6 reads ahead (2 - 3 %).
+// ---------------------------------------------------------------------------------------------
+template <int D, bool SPLIT>
+__global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PrefillArgs a) {
+  constexpr int BM = SPLIT ? 128 : 256, SW = SPLIT ? 4 : 8;      // queries of a workgroup; wavefronts that stage a tile
+  constexpr int DB = D / 32, STEPS = D / 16, CH = D / 8;
+  constexpr int TB = PF_BN * D * 2;                   // bytes of a K or V^T tile
+  constexpr int NI = TB / 1024 / SW;                  // requests per wavefront and tile
+  constexpr int R = SPLIT ? 2 : 4;                    // tile buffers for K, and for V
+  constexpr int RK = SPLIT ? 2 : 3;                   // K tiles requested ahead of a step (V: one less)
+  extern __shared__ __attribute__((aligned(16))) _Float16 pf_smem[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 31, h = lane >> 5, grp = wave >> 2;      // query of the wavefront (fragment row); half of a fragment's depth
+  const int wq = SPLIT ? wave & 3 : wave, ws = wq;    // query group; share of the staging
+  char* const Kb = (char*)pf_smem + (SPLIT ? grp * 2 * R * TB : 0);  // [R][64 keys][D], [R][D][64 keys]
+  char* const Vb = Kb + R * TB;
+  // LDS images: chunk c (16 bytes) of a row lies at chunk c ^ swz(row).  The scores' rows are taken in an order that leaves a lane
+  // the 8 consecutive keys that it multiplies next: row 16 t + 8 c + 4 h + q of a key block is its key 16 t + 8 h + 4 c + q
+  auto kswz = [](int key) { return D == 128 ? key & 15 : (key >> 1) & 7; };
+  auto vswz = [](int d) { return (d >> 1) & 7; };
+
+  const int nqb = gridDim.x, nbh = gridDim.y * gridDim.z;
+  const int lin = blockIdx.x + nqb * (blockIdx.y + gridDim.y * blockIdx.z);
+  // One workgroup a CU, the longest first, of all the heads of an XCD (an eighth of them where they divide, whole groups of a KV head):
+  // 4096 tokens of 32 heads 195 -> 153 us against one head after the other, 2 x 2048 115 -> 90, 7700 523 -> 508
+  int bh = lin % nbh, qslot = lin / nbh;
+  if ((nbh & 7) == 0) {
+    const int idx = lin >> 3, heads = nbh >> 3;
+    bh = (lin & 7) * heads + idx % heads;
+    qslot = idx / heads;
+  }
+  const int hq = bh % (int)gridDim.y, b = bh / (int)gridDim.y;
+  const int qb = nqb - 1 - qslot;                     // the longest first
+  const int hkv = hq / (a.Hq / a.Hkv);
+  const int q0 = qb * BM;
+  const int offset = a.Lk - a.Sq;
+  const int wq0 = q0 + 32 * wq;                       // first query of the wavefront
+  const int qi = wq0 + r, pos = qi + offset;
+  half8 qf[STEPS], pf[4];
+  float16v o[DB], s[2];                               // S^T by blocks of 32 keys, O^T by blocks of 32 channels: element i is row
+  float m = -INFINITY, l = 0.0f;                      // 8 (i / 4) + 4 h + i % 4
+  const _Float16* qp = a.q + b * a.q_sb + hq * a.q_sh + (int64_t)min(qi, a.Sq - 1) * a.q_ss + 8 * h;
+#pragma unroll
+  for (int st = 0; st < STEPS; ++st) qf[st] = *(const half8*)(qp + 16 * st);
+#pragma unroll
+  for (int j = 0; j < DB; ++j)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[j][e] = 0.0f;
+  int kbeg = 0, kend = a.Lk;
+  if (a.causal) kend = min(a.Lk, q0 + BM + offset);
+  if (a.window > 0) kbeg = max(0, q0 + offset - a.window + 1) / PF_BN * PF_BN;
+  // whole tiles in the loop; the sequence's last keys, fewer than a tile, behind it
+  const int kpart = a.Lk / PF_BN * PF_BN;
+  auto tiles_to = [&](int k1) { return k1 > kbeg ? (k1 - kbeg + PF_BN - 1) / PF_BN : 0; };
+  const int ntile = tiles_to(min(kend, kpart));
+  const int n = SPLIT ? (ntile + 1) / 2 : ntile;      // steps of the loop
+  auto first_key = [&](int i) { return kbeg + PF_BN * (SPLIT ? 2 * i + grp : i); };
+  // steps of the wavefront: tiles of its group with a key that one of its queries sees
+  const int last = min(wq0 + 31, a.Sq - 1) + offset;  // last key position of its queries
+  const int nt = wq0 < a.Sq ? tiles_to(a.causal ? min(min(kend, kpart), last + 1) : kpart) : 0;
+  const int nw = SPLIT ? (nt + 1 - grp) / 2 : nt;
+
+  // ---- tiles to LDS
+  const _Float16* kbase = a.k + b * a.k_sb + hkv * a.k_sh;
+  const _Float16* vbase = a.v + b * a.v_sb + hkv * a.v_sh;
+  uint32_t koff[NI], voff[NI];
+#pragma unroll
+  for (int p = 0; p < NI; ++p) {
+    const int c = (ws * NI + p) * 64 + lane;          // chunk of the tile, in the order of the LDS image
+    const int key = c / CH, d = c / 8;
+    koff[p] = ((uint32_t)key * (uint32_t)a.k_ss + 8 * ((c % CH) ^ kswz(key))) * 2;
+    voff[p] = ((uint32_t)d * (uint32_t)a.v_ss + 8 * ((c % 8) ^ vswz(d))) * 2;
+  }
+  auto tile_at = [&](int i, bool is_k) { return pf_buf(is_k ? kbase + (int64_t)first_key(i) * a.k_ss : vbase + first_key(i)); };
+  auto dma = [&](const __amdgpu_buffer_rsrc_t& tile, int i, bool is_k, int p) {      // request p of tile i
+    pf_dma16(tile, (is_k ? Kb : Vb) + i % R * TB + (ws * NI + p) * 1024, is_k ? koff[p] : voff[p]);
+  };
+  auto stage = [&](int i, bool is_k) {
+    if (SPLIT && 2 * i + grp >= ntile) return;        // (an odd count: the other group's tile)
+#pragma unroll
+    for (int p = 0; p < NI; ++p) dma(tile_at(i, is_k), i, is_k, p);
+  };
+  // all requests but those of the last weights (so), or all
+  auto landed = [&](bool so) {
+    if (so) __builtin_amdgcn_s_waitcnt(0x0070 | 2 * NI);      // vmcnt lgkmcnt(0)
+    else __builtin_amdgcn_s_waitcnt(0x0070);
+  };
+  auto block_end = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // ---- the two blocks
+  const float sc2 = a.scale * 1.4426950408889634f;
+  // keys that a query does not see: -infinity
+  auto mask = [&](int k0) {
+    if (k0 + PF_BN <= a.Lk && (!a.causal || k0 + PF_BN - 1 <= wq0 + offset) && (a.window <= 0 || k0 > wq0 + 31 + offset - a.window)) return;
+    const int hi = a.causal ? min(pos, a.Lk - 1) : a.Lk - 1, lo = a.window > 0 ? pos - a.window : -1;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int key = k0 + 32 * kb + 16 * (e >> 3) + 8 * h + (e & 7);
+        s[kb][e] = (key <= hi) & (key > lo) ? s[kb][e] : -INFINITY;
+      }
+  };
+  // The weights of the scores in s.  The vector unit is what a tile waits for: every MFMA of the other group takes it 8 to 10 cycles
+  // (hence 32 x 32 x 16: half as many), an exponential and a conversion cost two instructions' time.  dmas: the requests of K tile
+  // i + RK and V tile i + RK - 1 among them, a few at a time: 8 wavefronts' requests in one burst hold every wavefront up for 400 to 1100
+  // cycles
+  auto weights = [&](bool dmas, int i) {
+    // (maximum, not fmaxf: that has the compiler quiet every operand first; a NaN score makes its query's result NaN either way)
+    auto top2 = [](float x, float y) { return __builtin_elementwise_maximum(x, y); };
+    float t[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {                     // four chains of eight
+      t[j] = top2(s[j >> 1][8 * (j & 1)], s[j >> 1][8 * (j & 1) + 1]);
+#pragma unroll
+      for (int e = 2; e < 8; e += 2) t[j] = top2(top2(t[j], s[j >> 1][8 * (j & 1) + e]), s[j >> 1][8 * (j & 1) + e + 1]);
+    }
+    t[0] = top2(top2(top2(t[0], t[1]), t[2]), t[3]);
+    const uint2v both = __builtin_amdgcn_permlane32_swap(__float_as_uint(t[0]), __float_as_uint(t[0]), false, false);
+    const float mnew = top2(top2(__uint_as_float(both.x), __uint_as_float(both.y)) * sc2, m);
+    // (the running maximum follows only where it is exceeded by 2^PF_LAZY, as above)
+    if (__builtin_amdgcn_ballot_w64(mnew > m + PF_LAZY) != 0) {
+      const float alpha = pf_exp2(m - (mnew == -INFINITY ? 0.0f : mnew));
+      l *= alpha;
+#pragma unroll
+      for (int j = 0; j < DB; ++j) o[j] *= alpha;
+      m = mnew;
+    }
+    const float mref = m == -INFINITY ? 0.0f : m;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float p[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        p[e] = pf_exp2(__builtin_fmaf(s[j >> 2][4 * (j & 3) + e], sc2, -mref));
+        pf[j >> 1][4 * (j & 1) + e] = (_Float16)p[e];
+      }
+      l += (p[0] + p[1]) + (p[2] + p[3]);             // (the 2 lanes of a query are added up after the loop)
+      if (dmas) {
+#pragma unroll
+        for (int p = j * 2 * NI / 8; p < (j + 1) * 2 * NI / 8; ++p) {
+          const int at = p < NI ? i + RK : i + RK - 1;
+          dma(tile_at(at, p < NI), at, p < NI, p % NI);
+        }
+      }
+    }
+    // (done here, before the block ends: the compiler takes the exponentials to their use, among the products)
+    asm volatile("" : "+v"(pf[0]), "+v"(pf[1]), "+v"(pf[2]), "+v"(pf[3]), "+v"(l));
+  };
+
+  // fragment f of a block's products: f < SF the scores' (k step f / 2, key block f % 2) of the K tile kt, then the values' (16 keys
+  // (f - SF) / DB, channel block (f - SF) % DB) of the V^T tile vt
+  constexpr int SF = 2 * STEPS, VF = 4 * DB, AHEAD = 8;
+  auto frag_of = [&](auto fc, const char* kt, const char* vt) {
+    constexpr int f = decltype(fc)::value;
+    if constexpr (f < SF) {
+      const int key = (r & 16) + 8 * (r >> 2 & 1) + 4 * (r >> 3 & 1) + (r & 3);      // (kswz does not look at the key block's bit)
+      return *(const half8*)(kt + key * (2 * D) + 16 * ((2 * (f / 2) + h) ^ kswz(key)) + 32 * (f % 2) * (2 * D));
+    } else {                                          // (nor vswz at the channel block's)
+      return *(const half8*)(vt + r * 128 + 16 * ((2 * ((f - SF) / DB) + h) ^ vswz(r)) + 32 * ((f - SF) % DB) * 128);
+    }
+  };
+  // the products of fragments F0 .. F1 - 1, AHEAD reads in flight (the order is held: left to itself the compiler waits for every
+  // read by itself)
+  auto products = [&](auto f0c, auto f1c, const char* kt, const char* vt) {
+    constexpr int F0 = decltype(f0c)::value, F1 = decltype(f1c)::value;
+    half8 fr[AHEAD];
+    float16v z;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) z[e] = 0.0f;
+    pf_for<F0, F0 + AHEAD>([&](auto fc) { fr[decltype(fc)::value % AHEAD] = frag_of(fc, kt, vt); });
+    __builtin_amdgcn_sched_barrier(0);
+    pf_for<F0, F1>([&](auto fc) {
+      constexpr int f = decltype(fc)::value;
+      if constexpr (f < SF) s[f % 2] = pf_mfma32(fr[f % AHEAD], qf[f / 2], f < 2 ? z : s[f % 2]);
+      else o[(f - SF) % DB] = pf_mfma32(fr[f % AHEAD], pf[(f - SF) / DB], o[(f - SF) % DB]);
+      if constexpr (f + AHEAD < F1) fr[f % AHEAD] = frag_of(std::integral_constant<int, f + AHEAD>{}, kt, vt);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  typedef std::integral_constant<int, 0> FS;
+  typedef std::integral_constant<int, SF> FV;
+  typedef std::integral_constant<int, SF + VF> FE;
+
+#pragma unroll
+  for (int i = 0; i < RK; ++i) {
+    if (i < n) stage(i, true);
+    if (i < n && i < RK - 1) stage(i, false);
+  }
+  landed(false);
+  block_end();
+  // Group 1 is a block behind.  Block pair i of group 0 is slots 2 i + 1 (weights) and 2 i + 2 (products), of group 1 2 i + 2 and
+  // 2 i + 3.  The products i read K tile i + 1 and V tile i; the weights i request K tile i + RK and V tile i + RK - 1.
+  //  * All stage a tile (RK = 3, 4 buffers): into the buffers of K tile i - 1 and V tile i - 2, last read by the products i - 2 (slots
+  //    2 i - 2 and 2 i - 1).  What the products i + 1 read (from slot 2 i + 4) was requested by the weights i - 1 and has landed at the
+  //    end of slot 2 i + 3 (group 0: the weights i + 1, group 1: the products i) but for the requests of the last weights.
+  //  * Each group its own (RK = 2, 2 buffers): into those of K tile i and V tile i - 1, last read by its products i - 1; requested by
+  //    the weights i, landed at the end of the products i.
+  if (grp == 1) block_end();
+  if (nw > 0) products(FS{}, FV{}, Kb, Vb);
+  block_end();
+  for (int i = 0; i < n; ++i) {
+    const bool dmas = SPLIT ? 2 * (i + RK) + grp < ntile : i + RK < n;
+    if (!dmas && i + RK - 1 < n) stage(i + RK - 1, false);
+    if (i < nw) {
+      mask(first_key(i));
+      weights(dmas, i);
+    } else if (dmas) {                                // a tile that none of the wavefront's queries sees
+      stage(i + RK, true);
+      stage(i + RK - 1, false);
+    }
+    // (split groups wait at the end of the products: these requests are for the products i + 1)
+    if (!SPLIT && grp == 0) landed(dmas);
+    block_end();
+    // (behind the last tile: scores of what lies there, not looked at)
+    if (i < nw) products(FS{}, FE{}, Kb + (i + 1) % R * TB, Vb + i % R * TB);
+    if (SPLIT) landed(false);
+    else if (grp == 1) landed(dmas);
+    block_end();
+  }
+  if (grp == 0) block_end();
+  if (kend > kpart) {                                 // (uniform) the sequence's last keys, group 0's with SPLIT; what lies behind them as zeros
+    if (!SPLIT || grp == 0) {
+#pragma unroll
+      for (int p = 0; p < NI; ++p) {
+        const int c = (ws * NI + p) * 64 + lane;
+        const int key = c / CH, d = c / 8, kc = (c % 8) ^ vswz(d);
+        half8 kv = {0, 0, 0, 0, 0, 0, 0, 0}, vv = kv;
+        if (kpart + key < a.Lk) kv = *(const half8*)(kbase + (int64_t)(kpart + key) * a.k_ss + 8 * ((c % CH) ^ kswz(key)));
+        const _Float16* vp = vbase + (int64_t)d * a.v_ss + kpart + 8 * kc;
+        if (kpart + 8 * kc + 8 <= a.Lk) vv = *(const half8*)vp;
+        else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (kpart + 8 * kc + e < a.Lk) vv[e] = vp[e];
+        }
+        *(half8*)(Kb + c * 16) = kv;
+        *(half8*)(Vb + c * 16) = vv;
+      }
+    }
+    __syncthreads();
+    if ((!SPLIT || grp == 0) && wq0 < a.Sq && !(a.causal && kpart > last)) {
+      products(FS{}, FV{}, Kb, Vb);
+      mask(kpart);
+      weights(false, 0);
+      products(FV{}, FE{}, Kb, Vb);
+    }
+    if (SPLIT) __syncthreads();
+  }
+
+  if constexpr (SPLIT) {
+    // group 1 hands its sums over in LDS (all tiles are read: the barrier above)
+    float* const os = (float*)pf_smem + wq * (16 * DB + 2) * 64 + lane;
+    if (grp == 1) {
+#pragma unroll
+      for (int j = 0; j < 16 * DB; ++j) os[j * 64] = o[j >> 4][j & 15];
+      os[16 * DB * 64] = m;
+      os[(16 * DB + 1) * 64] = l;
+    }
+    __syncthreads();
+    if (grp == 1) return;
+    const float m1 = os[16 * DB * 64], top = fmaxf(m, m1), ref = top == -INFINITY ? 0.0f : top;
+    const float wa = pf_exp2(m - ref), wb = pf_exp2(m1 - ref);      // (-inf: 0)
+    l = l * wa + os[(16 * DB + 1) * 64] * wb;
+#pragma unroll
+    for (int j = 0; j < 16 * DB; ++j) o[j >> 4][j & 15] = o[j >> 4][j & 15] * wa + os[j * 64] * wb;
+  }
+  const uint2v both = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+  const float sum = __uint_as_float(both.x) + __uint_as_float(both.y);
+  if (qi >= a.Sq) return;
+  const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
+  _Float16* op = a.out + b * a.o_sb + (int64_t)qi * a.o_ss + hq * D;
+#pragma unroll
+  for (int j = 0; j < 4 * DB; ++j) {
+    const int d = 32 * (j >> 2) + 8 * (j & 3) + 4 * h;
+    half4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (_Float16)(o[j >> 2][4 * (j & 3) + e] * inv);
+    if (a.frag_mt > 0) *(half4*)(a.out + frag_at(b * a.Sq + qi, hq * D + d, a.frag_mt)) = v;
+    else *(half4*)(op + d) = v;
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 // RoPE + KV-cache append for a whole prompt, one launch per layer:
 //   q heads : rotated in place in the fused qkv buffer
 //   k heads : rotated in place (the attention of this call reads them unquantized) and copied to the K cache
@@ -643,6 +963,45 @@ static int launch_pf_one(const PrefillArgs& a, hipStream_t st) {
   return HIP_CHECK_LAUNCH();
 }
 
+// Which form: 0 = 64 queries a workgroup, several to a CU, 1 / 2 = the long-prompt form of 256 queries / 128 in split groups.  Long prompts: from
+// 321 queries (1025 of 64 channels) and more than 256 blocks of 64 on; us, old -> new: 32 heads of 128 channels 512 tokens 14.8 -> 16.7, 700
+// 26.0 -> 20.1, 3 x 300 16.7 -> 17.8, 3 x 400 22.8 -> 19.7, of 64 channels 512 10.4 -> 12.2, 1300 25.1 -> 21.2, 3 x 700 24.1 -> 24.9.  Between them by
+// the time of the longest workgroup or of all on 256 CUs, with a workgroup's start and end, fitted to 40 shapes: us, 256 / split: 1024 35.4 /
+// 25.0, 2048 62 / 55, 2500 78 / 86, 2 x 900 34.6 / 36.0, 2 x 1500 59 / 67.
+static int prompt_form(const PrefillArgs& a, int D) {
+  const int64_t heads = (int64_t)a.Hq * a.B;
+  if (a.Sq <= (D == 64 ? 1024 : 320) || (a.Sq + 63) / 64 * heads <= 256) return 0;
+  double us[2];
+  for (int f = 0; f < 2; ++f) {
+    const int BM = f ? 128 : 256, nqb = (a.Sq + BM - 1) / BM, offset = a.Lk - a.Sq;
+    double total = 0.0, longest = 0.0;
+    for (int j = 0; j < nqb; ++j) {
+      const int kend = a.causal && (j + 1) * BM + offset < a.Lk ? (j + 1) * BM + offset : a.Lk;
+      const int first = a.window > 0 ? j * BM + offset - a.window + 1 : 0, kbeg = first > 0 ? first / PF_BN * PF_BN : 0;
+      const double steps = (kend - kbeg + PF_BN - 1) / PF_BN * (f ? 0.5 : 1.0);
+      total += steps;
+      longest = longest > steps ? longest : steps;
+    }
+    const double turns = nqb * heads > 256 ? nqb * heads / 256.0 : 1.0, shared = total * heads / 256.0;
+    us[f] = 8.5 * turns + (f ? 2.4 : 1.75) * (longest > shared ? longest : shared);
+  }
+  return us[1] < us[0] ? 2 : 1;
+}
+
+template <int D, bool SPLIT>
+static int launch_prompt(const PrefillArgs& a, hipStream_t st) {
+  constexpr int BM = SPLIT ? 128 : 256;
+  constexpr int tiles = PF_BN * D * 2 * 8, sums = SPLIT ? 4 * (D / 2 + 2) * 256 : 0;
+  constexpr int lds = tiles > sums ? tiles : sums;
+  static bool attr = false;
+  if (!attr) {
+    if (hipFuncSetAttribute((const void*)attn_prompt_kernel<D, SPLIT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return -5;
+    attr = true;
+  }
+  hipLaunchKernelGGL((attn_prompt_kernel<D, SPLIT>), dim3((a.Sq + BM - 1) / BM, a.Hq, a.B), dim3(512), lds, st, a);
+  return HIP_CHECK_LAUNCH();
+}
+
 template <int D, int QB, int DR = D>
 static int launch_pf_qb(const PrefillArgs& a, hipStream_t st) {
   if (a.kv_e5m2) {
@@ -660,7 +1019,15 @@ static int launch_pf_qb(const PrefillArgs& a, hipStream_t st) {
 template <int D, int DR = D>
 static int launch_pf(const PrefillArgs& a, hipStream_t st) {
   // QB = 2 (128 queries per workgroup) halves the LDS traffic per MFMA but needs 240 VGPRs (one wavefront per
-  // SIMD); measured slower than QB = 1 from 1K to 8K tokens on MI355X, so QB = 1 is used throughout.
+  // SIMD); measured slower than QB = 1 from 1K to 8K tokens on MI355X, so QB = 1 is used throughout in this form.
+  if constexpr (DR == D && (D == 64 || D == 128)) {
+    if (a.v_transposed && !a.kv_e5m2 && a.mask == nullptr && a.alibi == nullptr && a.softcap <= 0.0f && a.scale > 0.0f &&
+        a.k_ss >= 0 && a.k_ss < (1 << 24) && a.v_ss >= 0 && a.v_ss < (1 << 24)) {      // (a tile's offsets are 32 bits)
+      const int form = prompt_form(a, D);
+      if (form == 1) return launch_prompt<D, false>(a, st);
+      if (form == 2) return launch_prompt<D, true>(a, st);
+    }
+  }
   return launch_pf_qb<D, 1, DR>(a, st);
 }
 

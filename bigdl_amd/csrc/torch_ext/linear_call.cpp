@@ -1,0 +1,175 @@
+// The host side of a few-row product in one native call.  A call of one row lasts 4 us on the GPU and took the host 12.8: 5.8 of
+// them were checks, an output and 26 arguments in Python.  What is not an ordinary tensor, or does not fit a kernel as it lies, comes
+// back as None and takes the Python way (transformers/low_bit_linear.py), which also raises the errors.
+#include <Python.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+#include <ATen/ATen.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPStream.h>
+#include <mutex>
+#include <string>
+#include <unordered_map>
+
+namespace {
+
+// entry points of libbigdl_hip.so (csrc/hip), handed over by bind()
+typedef int (*GemvFn)(const void*, const void*, const void*, void*, const void*, const void*, const void*, const void*, float, float, int,
+                      int, int, int, int, int, int, int, const void*, int, int, int, int, int, int, hipStream_t);
+typedef int (*GemmFn)(const void*, const void*, void*, const void*, const void*, float*, int64_t, int, int, int, int, int, int, int, int,
+                      hipStream_t);
+typedef int (*FragRuleFn)(int, int, int, int, int, int, int, int);
+typedef int64_t (*FragFloatsFn)(int, int, int, int, int, int);
+typedef int64_t (*GemmFloatsFn)(int, int, int, int, int, int, int, int);
+typedef int (*FragFn)(const void*, const void*, const void*, void*, const void*, const void*, const void*, float*, int64_t, int, int, int,
+                      int, int, int, int, int, int, hipStream_t);
+typedef int (*RowsFn)(const void*, const void*, const void*, void*, const void*, const void*, const void*, const void*, float, float,
+                      float*, int64_t, int, int, int, int, int, int, int, int, int, int, hipStream_t);
+GemvFn gemv_lowbit;
+GemmFn gemm_lowbit;
+FragRuleFn frag_rule;
+FragFloatsFn frag_floats;
+GemmFloatsFn gemm_floats;
+FragFn frag_dense;
+RowsFn gemm_rows;
+bool bound = false;
+
+constexpr int Q_Q6_K = 26;
+
+// an ordinary tensor in GPU memory that nothing but the caller looks at: no subclass, wrapper, graph, tangent
+bool plain(const at::Tensor& t) {
+  const auto keys = t.key_set();
+  return t.is_cuda() && t.layout() == at::kStrided && !t.is_conj() && !t.is_neg() && !t.requires_grad() &&
+         t.unsafeGetTensorImpl()->autograd_meta() == nullptr && !keys.has_any(c10::python_ks) &&
+         !keys.has(c10::DispatchKey::FuncTorchBatched) && !keys.has(c10::DispatchKey::FuncTorchGradWrapper) &&
+         !keys.has(c10::DispatchKey::Functionalize) && !keys.has(c10::DispatchKey::BatchedNestedTensor);
+}
+
+// scratch of a dense call by its sizes (floats; frag: on the kernel that takes x in fragment order).  Asking takes a microsecond.
+struct Sizes {
+  int m, n, k, qtype, ldx;
+  bool operator==(const Sizes& o) const { return m == o.m && n == o.n && k == o.k && qtype == o.qtype && ldx == o.ldx; }
+};
+struct SizesHash {
+  size_t operator()(const Sizes& s) const {
+    size_t h = (size_t)s.m;
+    for (int v : {s.n, s.k, s.qtype, s.ldx}) h = h * 1000003u ^ (size_t)v;
+    return h;
+  }
+};
+struct Way { bool frag; int64_t floats; };
+std::mutex ways_lock;
+std::unordered_map<Sizes, Way, SizesHash> ways;
+
+Way way_of(const Sizes& s) {
+  std::lock_guard<std::mutex> hold(ways_lock);
+  const auto it = ways.find(s);
+  if (it != ways.end()) return it->second;
+  Way w;
+  w.frag = s.m > 32 && frag_rule(s.m, s.n, s.k, s.ldx, s.qtype, 0, 0, 0) == 1;
+  w.floats = w.frag ? frag_floats(s.m, s.n, s.k, s.qtype, 0, 0) : gemm_floats(s.m, s.n, s.k, s.ldx, s.qtype, 0, 0, 0);
+  if (ways.size() >= 4096) ways.clear();
+  ways.emplace(s, w);
+  return w;
+}
+
+PyObject* rejected(const char* what, int rc) {
+  PyErr_Format(PyExc_RuntimeError, "%s: native launcher rejected the call (code %d)", what, rc);
+  return nullptr;
+}
+
+// product(x, w, n, k, qtype, nbytes, gemv_rows, gemm_rows) -> y [m, n] of x's type, or None.  x fp16 [m, k] on the GPU; w: nbytes bytes,
+// tiled for the device, or q6_k blocks.  Up to gemv_rows rows on the skinny kernel, up to gemm_rows on the others.  bf16 up to 32 rows
+// of a tiled weight and 64 Ki values, converted by PyTorch's operation as the Python way does (18 rows of 2048: 18.6 -> 13 us of host time).
+PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 8 || !bound || !THPVariable_CheckExact(args[0]) || !THPVariable_Check(args[1])) Py_RETURN_NONE;
+  long v[6];
+  for (int i = 0; i < 6; ++i) {
+    v[i] = PyLong_AsLong(args[2 + i]);
+    if (v[i] == -1 && PyErr_Occurred()) return nullptr;
+  }
+  const at::Tensor& x = THPVariable_Unpack(args[0]);
+  const at::Tensor& w = THPVariable_Unpack(args[1]);
+  const int64_t n = v[0], k = v[1];
+  const int qtype = (int)v[2];
+  const bool bf16 = x.scalar_type() == at::kBFloat16, q6k = qtype == Q_Q6_K;
+  if (!plain(x) || (x.scalar_type() != at::kHalf && !bf16) || x.dim() != 2 || x.size(1) != k || x.stride(1) != 1 || x.stride(0) % 8 != 0 ||
+      !w.is_cuda() || w.device() != x.device() || w.key_set().has_any(c10::python_ks) || (int64_t)w.nbytes() != v[3] ||
+      c10::impl::TorchDispatchModeTLS::any_modes_set() || torch::jit::tracer::isTracing())
+    Py_RETURN_NONE;
+  const int64_t m = x.size(0), ldx = bf16 ? k : x.stride(0);
+  if (bf16 && (q6k || m > 32 || m * k >= 65536 || x.stride(0) != k)) Py_RETURN_NONE;
+  if (m < 1 || m > v[5] || n < 1 || n > INT32_MAX || k < 1 || k > INT32_MAX || ldx > INT32_MAX || ldx < 0) Py_RETURN_NONE;
+  at::Tensor half;
+  if (bf16) half = x.to(at::kHalf);
+  const void* xp = bf16 ? half.const_data_ptr() : x.const_data_ptr();
+  const void* wp = w.const_data_ptr();
+  if ((uintptr_t)xp % 16 != 0 || (q6k && (k % 256 != 0 || (uintptr_t)wp % 4 != 0 || !w.is_contiguous()))) Py_RETURN_NONE;
+  at::Tensor y = at::empty({m, n}, x.options());
+  void* yp = y.data_ptr();
+  at::Tensor scratch;
+  const hipStream_t stream = c10::hip::getCurrentHIPStream().stream();
+  const char* what;
+  const int out_type = bf16 ? 1 : 0;                  // (csrc/hip/common.h)
+  int rc;
+  if (q6k) {
+    what = "gemm_rows";
+    Py_BEGIN_ALLOW_THREADS
+    rc = gemm_rows(xp, wp, nullptr, yp, nullptr, nullptr, nullptr, nullptr, 0.0f, 1e-6f, nullptr, 0, (int)m, (int)n, (int)k, (int)ldx, (int)n,
+                   qtype, 0, 0, 0, 1, stream);
+    Py_END_ALLOW_THREADS
+  } else if (m <= v[4]) {
+    what = "gemv_lowbit";
+    Py_BEGIN_ALLOW_THREADS
+    rc = gemv_lowbit(xp, wp, nullptr, yp, nullptr, nullptr, nullptr, nullptr, 1e-6f, 0.0f, (int)m, (int)n, (int)k, (int)ldx, (int)n, qtype, 0,
+                     out_type, nullptr, 0, 0, 0, 0, 0, 0, stream);
+    Py_END_ALLOW_THREADS
+  } else {
+    const Way way = way_of({(int)m, (int)n, (int)k, qtype, (int)ldx});
+    // (allocated by the call, never kept: a captured call's scratch belongs to its graph, calls on different streams share none)
+    float* sp = nullptr;
+    if (way.floats > 0) {
+      scratch = at::empty({way.floats}, x.options().dtype(at::kFloat));
+      sp = (float*)scratch.data_ptr();
+    }
+    what = way.frag ? "gemm_frag_dense" : "gemm_lowbit";
+    Py_BEGIN_ALLOW_THREADS
+    rc = way.frag ? frag_dense(xp, wp, nullptr, yp, nullptr, nullptr, nullptr, sp, way.floats, (int)m, (int)n, (int)k, (int)ldx, (int)n, qtype, 0,
+                               0, 0, stream)
+                  : gemm_lowbit(xp, wp, yp, nullptr, nullptr, sp, way.floats, (int)m, (int)n, (int)k, (int)ldx, (int)n, qtype, 0, out_type, stream);
+    Py_END_ALLOW_THREADS
+  }
+  if (rc != 0) return rejected(what, rc);
+  return THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
+}
+
+// bind({name: address}) of the seven entry points above
+PyObject* bind(PyObject*, PyObject* table) {
+  struct { const char* name; void** to; } want[] = {
+      {"bigdl_gemv_lowbit", (void**)&gemv_lowbit}, {"bigdl_gemm_lowbit", (void**)&gemm_lowbit},
+      {"bigdl_gemm_lowbit_frag", (void**)&frag_rule}, {"bigdl_gemm_frag_workspace", (void**)&frag_floats},
+      {"bigdl_gemm_lowbit_workspace", (void**)&gemm_floats}, {"bigdl_gemm_frag_dense", (void**)&frag_dense},
+      {"bigdl_gemm_rows", (void**)&gemm_rows}};
+  for (auto& e : want) {
+    PyObject* at = PyDict_Check(table) ? PyDict_GetItemString(table, e.name) : nullptr;
+    void* p = at ? PyLong_AsVoidPtr(at) : nullptr;
+    if (p == nullptr) {
+      if (!PyErr_Occurred()) PyErr_Format(PyExc_ValueError, "no address for %s", e.name);
+      return nullptr;
+    }
+    *e.to = p;
+  }
+  bound = true;
+  Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {{"product", (PyCFunction)(void (*)(void))product, METH_FASTCALL, nullptr}, {"bind", bind, METH_O, nullptr},
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "bigdl_linear_call", nullptr, -1, methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_bigdl_linear_call() { return PyModule_Create(&module); }

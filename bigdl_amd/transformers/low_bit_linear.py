@@ -344,8 +344,15 @@ def lowbit_matmul(x_2d: torch.Tensor, weight: FP4Params, out_features: int, for_
     n, k = weight._shape
     if weight.is_cuda:
         from ..ops import hip
-        m, dt = x_2d.shape[0], x_2d.dtype
         t16 = weight.qlayout == "t16"
+        if t16 or (weight.qtype == Q.Q6_K and not for_training):
+            # fp16 rows that lie as the few-row kernels take them; everything else is declined (None) and takes the way below
+            qt = weight.qtype
+            y = hip.linear_call()(x_2d, weight, n, k, qt, hip._t16_nbytes(qt, n, k) if t16 else n * (k // 256) * 210, GEMV_MAX_ROWS,
+                                  GEMM_MAX_ROWS if t16 else Q6K_MAX_ROWS)
+            if y is not None:
+                return y
+        m, dt = x_2d.shape[0], x_2d.dtype
         # (32 rows and fewer are never that kernel's: nothing more is asked for them, their calls are bound by the host)
         if (m > 32 and dt == torch.bfloat16 and t16 and m > GEMV_MAX_ROWS and (m <= GEMM_MAX_ROWS or not for_training)
                 and hip.gemm_lowbit_frag(m, n, k, weight.qtype, x_2d.stride(0), False, 1) and x_2d.stride(1) == 1

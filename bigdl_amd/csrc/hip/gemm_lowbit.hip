@@ -346,8 +346,11 @@ extern "C" int bigdl_gemm_lowbit(const void* x, const void* w, void* out, const 
 //  * x whose producer writes it in that order: in a whole step, against the others with x in rows, it is ahead where both are
 //    alike alone (their split sums take a launch more, and they come back to cold code), so up to 256 rows unless it is expected
 //    to be 15 % behind.  Steps of 8 layers, us, without it / with 3 % ahead asked for / as here: llama3-8b nf4 33 rows 988 / 896 / 857,
-//    q4_k 64 rows 970 / 915 / 871, llama2-7b sym_int4 64 rows 1157 / 1121 / 1074.  Against the prompt kernel by 5 %: prompts of 8 layers,
-//    without it / always / as here: llama2-7b sym_int4 300 tokens 2159 / 1822 / 1826, 512 tokens 2355 / 2589 / 2254.
+//    q4_k 64 rows 970 / 915 / 871, llama2-7b sym_int4 64 rows 1157 / 1121 / 1074.
+//  * Against the prompt kernel (257 - 512 rows) this kernel's estimate is a tenth too high: at 1.08 of its time for rows the choice among
+//    90 random products loses 0.4 % on average, 9 % at most (at 0.95 1.6 and 22); at 1.14 for produced x prompts of 3 layers take, us, at
+//    0.95 / 1.14 / 1.3: llama2-7b sym_int4 300 tokens 699 / 699 / 733, 400 809 / 799 / 831, llama3-8b nf4 300 778 / 765 / 779, q4_k 450 887 /
+//    893 / 910, tinyllama nf4 300 399 / 370 / 376.
 enum XKind { X_ROWS = 0, X_ROWS_BF16 = 1, X_FRAGMENTS = 2, X_PRODUCED = 3 };
 static bool takes_frag_kernel(int ldx, int M, int N, int K, int qtype, bool pair, int x_kind, bool out_frags, FragPlan* plan) {
   if (M <= 32 || !is_t16(qtype)) return false;
@@ -369,9 +372,9 @@ static bool takes_frag_kernel(int ldx, int M, int N, int K, int qtype, bool pair
     other = takes_rows_kernel(ldx, rows, N, K, qtype, pair, &r) ? rows_us(c, r, K, qtype, pair) : tile_us(c, rows, N, K, pair);
     other *= (M + 255) / 256;
   }
-  if (x_kind == X_ROWS) return plan->us + frag_pack_us(M, K) + (M <= 64 || other < 16.0 ? 3.0 : 0.0) < 0.95 * other;
+  if (x_kind == X_ROWS) return plan->us + frag_pack_us(M, K) + (M <= 64 || other < 16.0 ? 3.0 : 0.0) < (prompt ? 1.08 : 0.95) * other;
   if (x_kind == X_ROWS_BF16) return plan->us < 0.95 * other;
-  return plan->us - (out_frags ? frag_pack_us(M, N) : 0.0) < other * (prompt ? 0.95 : 1.15);
+  return plan->us - (out_frags ? frag_pack_us(M, N) : 0.0) < other * (prompt ? 1.14 : 1.15);
 }
 
 // Whether the kernel on x in fragment order is the one for this product.  x_kind 0: fp16 rows; 1: bf16 rows; 2: x in that order already

@@ -92,7 +92,8 @@ double prompt_us(int M, int N, int K, int qtype, bool pair) {
     case Q_FP8_E5M2: fmt = 1.08f; break;
     default: break;
   }
-  return prompt_plan_of(M, N, K, pair, -1, 0, fmt).us;
+  const PromptPlan p = prompt_plan_of(M, N, K, pair, -1, 0, fmt);
+  return p.splitk >= 4 && p.cfg != 2 ? 1.12 * p.us : p.us;      // (large tiles of many splits: 10 - 15 % over the estimate)
 }
 
 // the staged 16-bit epilogue covers this output; otherwise one fp32 slab + the reduce kernel

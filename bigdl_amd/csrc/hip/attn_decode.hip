@@ -106,6 +106,47 @@ __device__ __forceinline__ void split_e4m3(const float (&x)[8], uint2v& hi, uint
 }
 constexpr float P8_SCALE = 256.0f;     // probabilities are carried as 256 p (and the row sums with them)
 
+// Cross-split combine by the last-arriving workgroup of a (sequence, KV head, chunk) `bh`: row r of its partials is query head
+// head0 + r % Gc of token tok0 + r / Gc.  `s_flag`: one int of LDS.
+template <int D, int RT, int NT>
+__device__ __forceinline__ void combine_splits(const AttnArgs& a, int bh, int head0, int tok0, int rows, int Gc, int* s_flag) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const int ticket = __hip_atomic_fetch_add(&a.counters[bh], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int last = ticket == a.splits - 1;
+    if (last) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __hip_atomic_store(&a.counters[bh], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    *s_flag = last;
+  }
+  __syncthreads();
+  if (!*s_flag) return;
+
+  const float* wbase = a.ws + (int64_t)bh * a.splits * (RT * 16) * (D + 4);
+  for (int idx = threadIdx.x; idx < rows * (D / 4); idx += NT) {
+    const int row = idx / (D / 4), d4 = (idx % (D / 4)) * 4;
+    float mm = NEG_BIG;
+    for (int s = 0; s < a.splits; ++s) mm = fmaxf(mm, wbase[((int64_t)s * RT * 16 + row) * (D + 4) + D]);
+    float lt = 0.0f;
+    float4v acc = {0, 0, 0, 0};
+    for (int s = 0; s < a.splits; ++s) {
+      const float* src = wbase + ((int64_t)s * RT * 16 + row) * (D + 4);
+      const float f = exp2f(src[D] - mm);
+      lt += f * src[D + 1];
+      acc += *(const float4v*)(src + d4) * f;
+    }
+    const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+    _Float16* dst = a.out + out_at(tok0 + row / Gc, (head0 + row % Gc) * D + d4, a.Hq * D, a.frag_mt);
+    half4 hv = {(_Float16)(acc[0] * inv), (_Float16)(acc[1] * inv), (_Float16)(acc[2] * inv), (_Float16)(acc[3] * inv)};
+    *(half4*)dst = hv;
+  }
+}
+
 // D = head dim (multiple of 32), RT = number of 16-row tiles, KW = keys per wavefront per iteration.
 // KW = 64 (e5m2 caches, D % 128 == 0): every lane loads 16 bytes of a key row / of a V^T channel row instead of 8, i.e.
 // half as many load instructions and 64-byte instead of 32-byte contiguous pieces per 4 lanes.  With 8-byte pieces the
@@ -757,44 +798,12 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
   }
   if (single || a.defer_combine) return;
 
-  // ---- cross-split combine by the last-arriving workgroup of this (b, hkv) ----
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    const int ticket = __hip_atomic_fetch_add(&a.counters[bh], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const int last = ticket == a.splits - 1;
-    if (last) {
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __hip_atomic_store(&a.counters[bh], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    *s_flag = last;
-  }
-  __syncthreads();
-  if (!*s_flag) return;
-
-  const float* wbase = a.ws + (int64_t)bh * a.splits * (RT * 16) * (D + 4);
-  for (int idx = threadIdx.x; idx < rows * (D / 4); idx += NW * 64) {
-    const int row = idx / (D / 4), d4 = (idx % (D / 4)) * 4;
-    float mm = NEG_BIG;
-    for (int s = 0; s < a.splits; ++s) mm = fmaxf(mm, wbase[((int64_t)s * RT * 16 + row) * (D + 4) + D]);
-    float lt = 0.0f;
-    float4v acc = {0, 0, 0, 0};
-    for (int s = 0; s < a.splits; ++s) {
-      const float* src = wbase + ((int64_t)s * RT * 16 + row) * (D + 4);
-      const float f = exp2f(src[D] - mm);
-      lt += f * src[D + 1];
-      acc += *(const float4v*)(src + d4) * f;
-    }
-    const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-    const int tok = a.q_off + row / Gc, gq = g0 + row % Gc;
-    _Float16* dst = a.out + out_at(b * a.q_total + tok, (hkv * G + gq) * D + d4, a.Hq * D, a.frag_mt);
-    half4 hv = {(_Float16)(acc[0] * inv), (_Float16)(acc[1] * inv), (_Float16)(acc[2] * inv), (_Float16)(acc[3] * inv)};
-    *(half4*)dst = hv;
-  }
+  combine_splits<D, RT, NW * 64>(a, bh, hkv * G + g0, b * a.q_total + a.q_off, rows, Gc, s_flag);
 }
+
+}  // namespace bigdl
+#include "attn_decode_stream.h"
+namespace bigdl {
 
 template <int D, bool FP8, int RT, int KW, bool I4 = false, int NWT = ATT_NW, int MINW = 1>
 static int launch_one(const AttnArgs& a, size_t, hipStream_t st) {
@@ -814,6 +823,20 @@ static int launch_one(const AttnArgs& a, size_t, hipStream_t st) {
   return HIP_CHECK_LAUNCH();
 }
 
+template <int D, bool FP8, int NW>
+static int launch_stream(const AttnArgs& a, hipStream_t st) {
+  const size_t smem = attn_stream_lds<D, FP8, NW>(a.Hq / a.Hkv);
+  static bool attr = false;
+  if (!attr && smem > 65536) {
+    if (hipFuncSetAttribute((const void*)attn_stream_kernel<D, FP8, NW>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
+      return -5;
+    attr = true;
+  }
+  hipLaunchKernelGGL((attn_stream_kernel<D, FP8, NW>), dim3(a.splits, a.Hkv, a.B), dim3(NW * 64), smem, st, a.past_len, a.qkv, a.ld, a.splits,
+                     a.Hq, a.Hkv, a.Lmax, a.kc, a.vc, a);
+  return HIP_CHECK_LAUNCH();
+}
+
 template <int D, bool FP8, bool I4 = false>
 static int launch_rt(const AttnArgs& a, hipStream_t st) {
   const int rows = a.gchunk * a.q_cnt;
@@ -825,10 +848,24 @@ static int launch_rt(const AttnArgs& a, hipStream_t st) {
     return -4;
   }
   if (rt == 1) {
+    static const char* force = getenv("BIGDL_ATTN_KEYS");      // "32" / "64": the register form, with so many keys (measurements)
+    // One new token, heads of 64 or 128: the form whose K / V^T come through LDS in whole lines (attn_decode_stream.h).  Us a launch,
+    // caches cold, register form -> two / four wavefronts a workgroup, at (sequence, KV head, range) groups x keys a range:
+    //   fp16 128:  32 x 40 7.2 -> 5.6 / 6.1     192 x 2000 50 -> 50 / 44    256 x 1100 36 -> 31 / 30    512 x 1100 68 -> 53 / 54    1024 x 1100 127 -> 101 / 106
+    //   e5m2 128:  160 x 220 8.2 -> 8.4 / 7.5   192 x 2000 32 -> 39 / 28    256 x 1100 26 -> 25 / 21    512 x 1100 43 -> 33 / 33    1024 x 1100 73 -> 57 / 62
+    //   fp16 64:   20 x 220 6.5 -> 7.6 / 6.5    160 x 1100 19 -> 23 / 17    512 x 1100 38 -> 31 / 30    640 x 1100 50 -> 37 / 38
+    //   e5m2 64:   96 x 2000 21 -> 28 / 19      160 x 4000 35 -> 54 / 37    512 x 1100 27 -> 24 / 20    640 x 1100 34 -> 25 / 26
+    // From two workgroups a CU on the two-wavefront form has as many bytes under way in smaller pieces, below it the longer block fills the
+    // CU.  What stays in the register form: e5m2 heads of 64 with few long ranges (half the bytes a wavefront: 160 x 4000 above).
+    if constexpr (D == 64 || D == 128) {
+      const int64_t groups = (int64_t)a.B * a.Hkv * a.splits;
+      const bool fits = a.q_total == 1 && a.nchunk == 1 && (int64_t)a.Lmax * D * (FP8 ? 1 : 2) < (1ll << 31) && ((uintptr_t)a.rope & 15) == 0;
+      if (!force && fits && !(FP8 && D == 64 && a.splits == 1 && groups < 512))
+        return groups >= (D == 64 ? 640 : 512) ? launch_stream<D, FP8, 2>(a, st) : launch_stream<D, FP8, 4>(a, st);
+    }
     // 64 keys per wavefront (16-byte fragments).  With one KV split and fewer than 512 (sequence, head) pairs the
     // workgroup has ATT_NW wavefronts; with several splits or 512 pairs and more it has four (below).
     if constexpr (FP8 && D % 128 == 0) {
-      static const char* force = getenv("BIGDL_ATTN_KEYS");      // "32" / "64": override for measurements
       const bool wide = force ? atoi(force) == 64 : true;
       // batched decode (512 or more (sequence, head) workgroups, one KV split): four-wavefront workgroups, so
       // that two of them share a CU and one streams keys while the other is in its softmax / merge phase.  Measured

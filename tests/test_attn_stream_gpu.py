@@ -1,0 +1,139 @@
+"""Decode attention of one new token with K / V^T through LDS in whole lines (csrc/hip/attn_decode_stream.h) against float64: lengths
+around its blocks (64 keys a wavefront in e5m2 caches, 32 in fp16; two or four wavefronts), several lengths in a batch, ranges without
+keys, groups of 1 to 16 query heads, and what changes a score.  The cache behind the last piece that holds a key is NaN: nothing of it
+may reach a result."""
+import math
+
+import pytest
+import torch
+
+from bigdl_amd.ops import hip
+
+pytestmark = pytest.mark.gpu
+
+LMAX = 1024
+
+
+def _f64(q, k, v, scale, softcap=0.0, window=0, slopes=None, mask=None):
+    """q [Hq, D], k / v [Hkv, n, D] (the newest key last), all float64"""
+    hq, n = q.shape[0], k.shape[1]
+    g = hq // k.shape[0]
+    s = torch.einsum("hd,hnd->hn", q, k.repeat_interleave(g, 0)) * scale
+    if softcap:
+        s = softcap * torch.tanh(s / softcap)
+    pos = torch.arange(n)
+    if slopes is not None:
+        s = s + slopes.double()[:, None] * (pos - (n - 1))
+    if mask is not None:
+        s = s + mask.double()[:n]
+    if window:
+        s = s.masked_fill(pos <= n - 1 - window, -math.inf)
+    return torch.einsum("hn,hnd->hd", torch.softmax(s, -1), v.repeat_interleave(g, 0))
+
+
+def _rotate(x, pos, table, interleaved):
+    """x [H, D] float64; table [max_pos, rot / 2, 2]"""
+    rot = 2 * table.shape[1]
+    c, s = table[pos, :, 0].double(), table[pos, :, 1].double()
+    y = x.clone()
+    if interleaved:
+        a, b = x[:, 0:rot:2], x[:, 1:rot:2]
+        y[:, 0:rot:2], y[:, 1:rot:2] = a * c - b * s, b * c + a * s
+    else:
+        h = rot // 2
+        a, b = x[:, :h], x[:, h:rot]
+        y[:, :h], y[:, h:rot] = a * c - b * s, b * c + a * s
+    return y
+
+
+def _case(d, fp8, hq, hkv, pasts, splits, defer=False, interleaved=False, rot=None, rope=True, **opt):
+    torch.manual_seed(hash((d, fp8, hq, hkv, len(pasts), splits)) % 1000)
+    b = len(pasts)
+    piece = 64 if fp8 else 32
+    k = torch.randn(b, hkv, LMAX, d).half()
+    v = torch.randn(b, hkv, d, LMAX).half()
+    if fp8:
+        k, v = k.to(torch.float8_e5m2), v.to(torch.float8_e5m2)
+    kf, vf = k.double(), v.double()
+    raw = torch.uint8 if fp8 else torch.int16
+    kd, vd = k.view(raw).clone(), v.view(raw).clone()
+    for i, p in enumerate(pasts):
+        end = (p + 1 + piece - 1) // piece * piece
+        kd[i, :, end:] = 0x7F if fp8 else 0x7FFF
+        vd[i, :, :, end:] = 0x7F if fp8 else 0x7FFF
+        kd[i, :, p] = 0x7F if fp8 else 0x7FFF          # the new token's place: written by the call
+        vd[i, :, :, p] = 0x7F if fp8 else 0x7FFF
+    dt = torch.uint8 if fp8 else torch.float16
+    kd, vd = kd.view(dt).cuda(), vd.view(dt).cuda()
+    before_k, before_v = kd.clone(), vd.clone()
+    qkv = torch.randn(b, (hq + 2 * hkv) * d).half()
+    half = (rot or d) // 2
+    ang = torch.arange(LMAX).float()[:, None] / (10000 ** (torch.arange(half).float() / half))
+    table = torch.stack([ang.cos(), ang.sin()], -1).contiguous()
+    out = torch.full((b, hq * d), float("nan"), dtype=torch.float16, device="cuda")
+    ws = torch.empty(hip.attn_decode_ws_floats(b, hq, hkv, 1, d, splits), dtype=torch.float32, device="cuda")
+    counters = torch.zeros(hip.attn_decode_counters(b, hq, hkv), dtype=torch.int32, device="cuda")
+    scale = 1.0 / math.sqrt(d)
+    slopes = torch.rand(hq) * 0.05 if opt.pop("alibi", False) else None
+    mask = (torch.randn(b, 1, LMAX) * 2).half() if opt.pop("mask", False) else None
+    hip.attn_decode(qkv.cuda(), kd, vd, torch.tensor(pasts, dtype=torch.int32, device="cuda"), out, ws, counters, n_heads=hq, n_kv_heads=hkv,
+                    head_dim=d, q_len=1, batch=b, scale=scale, splits=splits, rope_table=table.cuda() if rope else None, append=not rope,
+                    interleaved=interleaved, defer_combine=defer, alibi=None if slopes is None else slopes.cuda(),
+                    mask=None if mask is None else mask.cuda(), **opt)
+    torch.cuda.synchronize()
+    if defer and splits > 1:
+        # [b * hkv][splits][16][d + 4]: O row, maximum (log2), sum
+        w = ws[: b * hkv * splits * 16 * (d + 4)].view(b, hkv, splits, 16, d + 4)[:, :, :, : hq // hkv].cpu().double()
+        f = torch.exp2(w[..., d] - w[..., d].amax(2, keepdim=True))
+        got = ((w[..., :d] * f[..., None]).sum(2) / (w[..., d + 1] * f).sum(2)[..., None]).reshape(b, hq, d)
+    else:
+        got = out.cpu().double().view(b, hq, d)
+    x = qkv.double().view(b, hq + 2 * hkv, d)
+    worst = 0.0
+    kc, vc = kd.cpu(), vd.cpu()
+    for i, p in enumerate(pasts):
+        q, kn, vn = x[i, :hq], x[i, hq:hq + hkv], x[i, hq + hkv:]
+        if rope:
+            q, kn = _rotate(q, p, table, interleaved), _rotate(kn, p, table, interleaved)
+        # what the call wrote: the value exactly, the key to a rounding of its rotation
+        wk, wv = kc[i, :, p], vc[i, :, :, p]
+        if fp8:
+            wk, wv = wk.view(torch.float8_e5m2).double(), wv.view(torch.float8_e5m2).double()
+            assert torch.equal(wv, vn.half().to(torch.float8_e5m2).double())
+            assert ((wk - kn).abs() <= 0.13 * kn.abs() + 1e-4).all()
+        else:
+            assert torch.equal(wv.double(), vn)
+            assert ((wk.double() - kn).abs() <= 1e-3 * kn.abs() + 1e-4).all()
+        kk = torch.cat([kf[i, :, :p], wk.double()[:, None]], 1)
+        vv = torch.cat([vf[i, :, :, :p].transpose(1, 2), vn.half().to(torch.float8_e5m2).double()[:, None] if fp8 else vn[:, None]], 1)
+        ref = _f64(q, kk, vv, scale, slopes=slopes, mask=None if mask is None else mask[i, 0], **opt)
+        worst = max(worst, ((got[i] - ref).norm() / ref.norm()).item())
+    # nothing else of the caches has changed
+    before_k, before_v = before_k.cpu(), before_v.cpu()
+    for i, p in enumerate(pasts):
+        before_k[i, :, p], before_v[i, :, :, p] = kc[i, :, p], vc[i, :, :, p]
+    assert torch.equal(before_k.view(raw), kc.view(raw)) and torch.equal(before_v.view(raw), vc.view(raw))
+    assert int(counters.abs().sum()) == 0
+    # fp16 operands: q, the weights and the result round to 2^-11 each; an error e of a score (|score| < 8 in these cases, mask included)
+    # changes its weight by a factor 1 + e: 8 x 2^-11 + 2 x 2^-11 < 5e-3.  Two e4m3 terms hold q and the weights to 2^-8 each, of q
+    # averaged over the channels of a score (a quarter of it): 8 / 4 x 2^-8 + 2^-8 < 1.2e-2
+    assert worst < (1.2e-2 if fp8 and d == 128 else 5e-3), worst
+
+
+EDGES = [0, 1, 30, 31, 32, 33, 63, 64, 65, 126, 127, 128, 129, 191, 255, 256, 257, 300, 511, 512, 700, 1022, 1023]
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("hq,hkv,splits", [(2, 2, 2), (8, 2, 3), (7, 1, 1), (16, 1, 2), (40, 40, 1), (32, 16, 2)])
+def test_lengths(d, fp8, hq, hkv, splits):
+    _case(d, fp8, hq, hkv, EDGES, splits)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("opt", [dict(softcap=20.0), dict(window=100), dict(alibi=True), dict(mask=True), dict(interleaved=True),
+                                 dict(interleaved=True, rot=32), dict(rope=False), dict(defer=True)], ids=lambda o: next(iter(o)) + str(len(o)))
+def test_options(d, fp8, opt):
+    _case(d, fp8, 6, 2, [5, 127, 128, 400, 1000], 3, **opt)
+    _case(d, fp8, 96, 96, [0, 63, 64, 200, 256, 777, 1023], 1, **{**opt, "defer": False})

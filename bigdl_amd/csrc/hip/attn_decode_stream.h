@@ -343,7 +343,8 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
       for (int j = 0; j < DTW; ++j) {
         const int ch = 16 * j + (lane >> 2), ck = 4 * (at >> 6) + (lane & 3);
         const uint4v w = *(const uint4v*)(svt + ch * RV + ((ck ^ (ch & 7)) << 4));
-        *(uint4v*)(vc + (int64_t)(wave * CH + ch) * a.Lmax * ES + (int64_t)kb * ES + 16 * ck) = w;
+        __builtin_amdgcn_raw_buffer_store_b128(w, vbuf, (uint32_t)(wave * CH + ch) * (uint32_t)(a.Lmax * ES) + (uint32_t)(kb * ES + 16 * ck), 0,
+                                               17 /* written through: 64 x 32 heads, 1000 e5m2 keys 107 -> 103 us */);
       }
     }
     float mw[NW], m_next = m_all;

@@ -362,7 +362,7 @@ __global__ __launch_bounds__(256) void rep_penalty_kernel(void* scores, const in
 
 // argmax over the last dim; ties -> lowest index.  A row is split over gridDim.y workgroups (a single workgroup reads a
 // 32000-entry fp32 row at the rate of one CU: 6 us); each writes its (value, index) candidate, the last one to arrive
-// (agent-scope ticket) picks the winner.  The same launch can add `inc_alpha * inc_src[i]` to `inc_dst[i]` for
+// (agent-scope ticket) picks the winner, a lane a candidate (one after the other they were eight trips to memory: 32000 fp32 6.8 -> 5.4 us a launch, 64 rows 8.9 -> 7.5).  The same launch can add `inc_alpha * inc_src[i]` to `inc_dst[i]` for
 // i < inc_n: the decode graph advances its per-sequence cache lengths here instead of in a launch of its own.
 struct ArgmaxArgs {
   const void* x; int64_t* out; float* part_v; int* part_i; int* tickets;
@@ -407,30 +407,38 @@ __global__ __launch_bounds__(1024) void argmax_kernel(ArgmaxArgs a) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) { sv[wave] = best; si[wave] = bi; }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < 16; ++w)
-      if (sv[w] > best || (sv[w] == best && si[w] < bi)) { best = sv[w]; bi = si[w]; }
-    if (nch == 1) {
-      a.out[row] = bi == 0x7fffffff ? 0 : bi;
-    } else {
-      // candidates and ticket as device-scope atomics: written through, read by the last arriver past its own L1
+  if (wave != 0) return;
+  auto better = [&](int o) {
+    const float ov = __shfl_xor(best, o);
+    const int oi = __shfl_xor(bi, o);
+    if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
+  };
+  best = sv[lane & 15];
+  bi = si[lane & 15];
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) better(o);
+  if (nch > 1) {
+    // candidates and ticket as device-scope atomics: written through, read by the last arriver past its own L1
+    int ticket = 0;
+    if (lane == 0) {
       __hip_atomic_store(&a.part_v[row * nch + ch], best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(&a.part_i[row * nch + ch], bi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      const int ticket = __hip_atomic_fetch_add(&a.tickets[row], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (ticket == nch - 1) {
-        float bv = -INFINITY;
-        int bj = 0x7fffffff;
-        for (int c = 0; c < nch; ++c) {
-          const float v = __hip_atomic_load(&a.part_v[row * nch + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          const int j = __hip_atomic_load(&a.part_i[row * nch + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          if (v > bv || (v == bv && j < bj)) { bv = v; bj = j; }
-        }
-        a.out[row] = bj == 0x7fffffff ? 0 : bj;
-        __hip_atomic_store(&a.tickets[row], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // ready for the next launch
-      }
+      ticket = __hip_atomic_fetch_add(&a.tickets[row], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    if (__builtin_amdgcn_readfirstlane(ticket) != nch - 1) return;
+    best = -INFINITY;
+    bi = 0x7fffffff;
+    for (int c = lane; c < nch; c += 64) {
+      const float v = __hip_atomic_load(&a.part_v[row * nch + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const int j = __hip_atomic_load(&a.part_i[row * nch + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (v > best || (v == best && j < bi)) { best = v; bi = j; }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) better(o);
+    if (lane == 0) __hip_atomic_store(&a.tickets[row], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // ready for the next launch
   }
+  if (lane == 0) a.out[row] = bi == 0x7fffffff ? 0 : bi;
 }
 
 }  // namespace bigdl

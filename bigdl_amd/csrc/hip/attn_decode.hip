@@ -823,16 +823,16 @@ static int launch_one(const AttnArgs& a, size_t, hipStream_t st) {
   return HIP_CHECK_LAUNCH();
 }
 
-template <int D, bool FP8, int NW>
+template <int D, bool FP8, int NW, int RT>
 static int launch_stream(const AttnArgs& a, hipStream_t st) {
-  const size_t smem = attn_stream_lds<D, FP8, NW>(a.Hq / a.Hkv);
+  const size_t smem = attn_stream_lds<D, FP8, NW, RT>(a.Hq / a.Hkv * a.q_cnt);
   static bool attr = false;
   if (!attr && smem > 65536) {
-    if (hipFuncSetAttribute((const void*)attn_stream_kernel<D, FP8, NW>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
+    if (hipFuncSetAttribute((const void*)attn_stream_kernel<D, FP8, NW, RT>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
       return -5;
     attr = true;
   }
-  hipLaunchKernelGGL((attn_stream_kernel<D, FP8, NW>), dim3(a.splits, a.Hkv, a.B), dim3(NW * 64), smem, st, a.past_len, a.qkv, a.ld, a.splits,
+  hipLaunchKernelGGL((attn_stream_kernel<D, FP8, NW, RT>), dim3(a.splits, a.Hkv, a.B), dim3(NW * 64), smem, st, a.past_len, a.qkv, a.ld, a.splits,
                      a.Hq, a.Hkv, a.Lmax, a.kc, a.vc, a);
   return HIP_CHECK_LAUNCH();
 }
@@ -847,22 +847,30 @@ static int launch_rt(const AttnArgs& a, hipStream_t st) {
     if (rt == 2) return launch_one<D, false, 2, 32, true>(a, smem, st);
     return -4;
   }
-  if (rt == 1) {
-    static const char* force = getenv("BIGDL_ATTN_KEYS");      // "32" / "64": the register form, with so many keys (measurements)
-    // One new token, heads of 64 or 128: the form whose K / V^T come through LDS in whole lines (attn_decode_stream.h).  Us a launch,
-    // caches cold, register form -> two / four wavefronts a workgroup, at (sequence, KV head, range) groups x keys a range:
-    //   fp16 128:  32 x 40 7.2 -> 5.6 / 6.1     192 x 2000 50 -> 50 / 44    256 x 1100 36 -> 31 / 30    512 x 1100 68 -> 53 / 54    1024 x 1100 127 -> 101 / 106
-    //   e5m2 128:  160 x 220 8.2 -> 8.4 / 7.5   192 x 2000 32 -> 39 / 28    256 x 1100 26 -> 25 / 21    512 x 1100 43 -> 33 / 33    1024 x 1100 73 -> 57 / 62
-    //   fp16 64:   20 x 220 6.5 -> 7.6 / 6.5    160 x 1100 19 -> 23 / 17    512 x 1100 38 -> 31 / 30    640 x 1100 50 -> 37 / 38
-    //   e5m2 64:   96 x 2000 21 -> 28 / 19      160 x 4000 35 -> 54 / 37    512 x 1100 27 -> 24 / 20    640 x 1100 34 -> 25 / 26
-    // From two workgroups a CU on the two-wavefront form has as many bytes under way in smaller pieces, below it the longer block fills the
-    // CU.  What stays in the register form: e5m2 heads of 64 with few long ranges (half the bytes a wavefront: 160 x 4000 above).
-    if constexpr (D == 64 || D == 128) {
-      const int64_t groups = (int64_t)a.B * a.Hkv * a.splits;
-      const bool fits = a.q_total == 1 && a.nchunk == 1 && (int64_t)a.Lmax * D * (FP8 ? 1 : 2) < (1ll << 31) && ((uintptr_t)a.rope & 15) == 0;
-      if (!force && fits && !(FP8 && D == 64 && a.splits == 1 && groups < 512))
-        return groups >= (D == 64 ? 640 : 512) ? launch_stream<D, FP8, 2>(a, st) : launch_stream<D, FP8, 4>(a, st);
+  static const char* force = getenv("BIGDL_ATTN_KEYS");      // "32" / "64": the register form, with so many keys (measurements)
+  // Heads of 64 or 128: the form whose K / V^T come through LDS in whole lines (attn_decode_stream.h).  One new token, us a launch,
+  // caches cold, register form -> two / four wavefronts a workgroup, at (sequence, KV head, range) groups x keys a range:
+  //   fp16 128:  32 x 40 7.2 -> 5.6 / 6.1     192 x 2000 50 -> 50 / 44    256 x 1100 36 -> 31 / 30    512 x 1100 68 -> 53 / 54    1024 x 1100 127 -> 101 / 106
+  //   e5m2 128:  160 x 220 8.2 -> 8.4 / 7.5   192 x 2000 32 -> 39 / 28    256 x 1100 26 -> 25 / 21    512 x 1100 43 -> 33 / 33    1024 x 1100 73 -> 57 / 62
+  //   fp16 64:   20 x 220 6.5 -> 7.6 / 6.5    160 x 1100 19 -> 23 / 17    512 x 1100 38 -> 31 / 30    640 x 1100 50 -> 37 / 38
+  //   e5m2 64:   96 x 2000 21 -> 28 / 19      160 x 4000 35 -> 54 / 37    512 x 1100 27 -> 24 / 20    640 x 1100 34 -> 25 / 26
+  // From two workgroups a CU on the two-wavefront form has as many bytes under way in smaller pieces, below it the longer block fills the
+  // CU.  Several tokens (a draft's check) with heads of 128 round as the decode steps that they stand for; 64 x 32 heads, 2 / 8 tokens: fp16
+  // 300 keys 101 -> 79 / 116 -> 90, e5m2 1000 keys 130 -> 124 / 146 -> 141, 300 keys 57 -> 55 / 66 -> 70.  What stays in the register form:
+  // several tokens with heads of 64 (64 groups x 1000, 4 tokens 14.0 -> 14.8), two row tiles of e5m2 (widened to fp16 there: more exact), and
+  // e5m2 heads of 64 with few long ranges (half the bytes a wavefront: 160 x 4000 above).
+  if constexpr (D == 64 || D == 128) {
+    const int64_t groups = (int64_t)a.B * a.Hkv * a.splits;
+    const bool fits = a.nchunk == 1 && rt <= (FP8 ? 1 : 2) && (a.q_total == 1 || D == 128) &&
+                      (int64_t)a.Lmax * D * (FP8 ? 1 : 2) < (1ll << 31) && ((uintptr_t)a.rope & 15) == 0;
+    if (!force && fits && !(FP8 && D == 64 && a.splits == 1 && groups < 512)) {
+      const bool two = groups >= (D == 64 ? 640 : 512);
+      if constexpr (!FP8)
+        if (rt == 2) return two ? launch_stream<D, FP8, 2, 2>(a, st) : launch_stream<D, FP8, 4, 2>(a, st);
+      return two ? launch_stream<D, FP8, 2, 1>(a, st) : launch_stream<D, FP8, 4, 1>(a, st);
     }
+  }
+  if (rt == 1) {
     // 64 keys per wavefront (16-byte fragments).  With one KV split and fewer than 512 (sequence, head) pairs the
     // workgroup has ATT_NW wavefronts; with several splits or 512 pairs and more it has four (below).
     if constexpr (FP8 && D % 128 == 0) {

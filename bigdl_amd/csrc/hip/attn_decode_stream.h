@@ -1,4 +1,4 @@
-// Decode attention of one new token whose K and V^T arrive in whole 128-byte lines, by DMA into LDS (included by attn_decode.hip,
+// Decode attention whose K and V^T arrive in whole 128-byte lines, by DMA into LDS (included by attn_decode.hip,
 // which also states the cache layout and the products' operand order).
 //
 // What bounds it is the K / V stream, and what decides the rate of that stream is the pattern: fragments loaded straight into
@@ -28,12 +28,13 @@ __device__ __forceinline__ void attn_dma16(__amdgpu_buffer_rsrc_t b, char* lds, 
 }
 constexpr int attn_vm_lgkm0(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4); }       // s_waitcnt vmcnt(n) lgkmcnt(0)
 
-template <int D, bool FP8, int NW>
+template <int D, bool FP8, int NW, int RT>
 constexpr size_t attn_stream_lds(int rows) {
-  return (size_t)NW * (D * 128) + 2 * NW * rows * (FP8 ? 128 : 64) + 2 * NW * 64 + NW * 64;
+  return (size_t)NW * (D * 128) + 2 * NW * rows * (FP8 ? 128 : 64) + 3 * NW * RT * 64;
 }
 
-template <int D, bool FP8, int NW>
+// RT = 16-row tiles of query rows (G query heads x the launch's new tokens).  A row's result does not depend on the rows beside it.
+template <int D, bool FP8, int NW, int RT>
 __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_past, _Float16* p_qkv, int p_ld, int p_splits, int p_Hq,
                                                                               int p_Hkv, int p_Lmax, void* p_kc, void* p_vc, AttnArgs a) {
   a.past_len = p_past; a.qkv = p_qkv; a.ld = p_ld; a.splits = p_splits; a.Hq = p_Hq; a.Hkv = p_Hkv; a.Lmax = p_Lmax;
@@ -54,16 +55,16 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rr = lane & 15, g = lane >> 4;
   const int split = blockIdx.x, hkv = blockIdx.y, b = blockIdx.z;
-  const int G = a.Hq / a.Hkv, rows = G;
+  const int G = a.Hq / a.Hkv, rows = G * a.q_cnt;
   constexpr int PB = FP8 ? 128 : 64;         // LDS bytes of a row's probabilities, one wavefront's keys
   char* sk = smem + wave * (D * 128);                                   // this wavefront's keys of a block, then its V^T rows
   char* svt = sk + D * 64;
   char* sp = smem + NW * (D * 128);                                    // [2][NW][row][PB]
-  float* s_m = (float*)(sp + 2 * NW * rows * PB);                       // [2][NW][16]
-  float* s_l = s_m + 2 * NW * 16;                                       // [NW][16]
+  float* s_m = (float*)(sp + 2 * NW * rows * PB);                       // [2][NW][RT * 16]
+  float* s_l = s_m + 2 * NW * RT * 16;                                  // [NW][RT * 16]
 
   const int past = a.past_len[b];
-  const int kv_len = min(past + 1, a.Lmax);
+  const int kv_len = min(past + a.q_total, a.Lmax);
   const int nblk = (kv_len + BK - 1) / BK;
   const int per = (nblk + a.splits - 1) / a.splits;
   const int blk0 = split * per, blk1 = min(nblk, blk0 + per);
@@ -71,7 +72,8 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
   char* kc = (char*)p_kc + base;
   char* vc = (char*)p_vc + base;
   const int half_rot = a.rot >> 1;
-  const bool append = (a.rope != nullptr || a.rot == 0) && past < a.Lmax && past >= blk0 * BK && past < blk1 * BK;
+  const bool appends = a.rope != nullptr || a.rot == 0;
+  const bool append = appends && a.q_total == 1 && past < a.Lmax && past >= blk0 * BK && past < blk1 * BK;     // one token: into its block in LDS
   const int kw_new = (past % BK) / KW;       // the wavefront with the new key
 
   // ---- requests ----
@@ -101,49 +103,87 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
 
   // first head channel of this lane's 8 values in k-step c (as in the register form: the rotate-half partner is k-step c + DC / 2)
   auto chan = [](int c, int g) { return F8M ? 64 * (c >> 1) + 16 * g + 8 * (c & 1) : 32 * c + 8 * g; };
-  // ---- q, its rotation, the new key and value, then the first block (all without a branch: what arrives is counted) ----
-  half8 qraw[DC];
-  const int row = min(rr, rows - 1);
-  const _Float16* qp = a.qkv + (int64_t)b * a.ld + (int64_t)(hkv * G + row) * D;
-#pragma unroll
-  for (int c = 0; c < DC; ++c) qraw[c] = *(const half8*)(qp + chan(c, g));
-  // cs[2 i], cs[2 i + 1]: cosine and sine of 8 / 2 channel pairs each (without a rotation: any readable numbers)
-  const int pos = max(min(a.position_ids ? a.position_ids[b] : past, a.rope_max_pos - 1), 0);
   const bool rotate = a.rope != nullptr;
-  const float* tab = rotate ? a.rope + (int64_t)pos * half_rot * 2 : (const float*)qp;
-  float4v cs[DC][2];
-#pragma unroll
-  for (int i = 0; i < DC; ++i) {
-    const int at = a.interleaved ? (chan(i, g) < a.rot ? chan(i, g) : 0) : 2 * chan(i >> 1, g) + 8 * (i & 1);
-    const float* t = tab + (rotate ? at : 0);
-    cs[i][0] = *(const float4v*)t;
-    cs[i][1] = *(const float4v*)(t + 4);
-  }
-  // the new key's channel pair (i0, i1) of this lane and the new value's channel
-  const _Float16* krow = a.qkv + (int64_t)b * a.ld + (int64_t)(a.Hq + hkv) * D;
+  const _Float16* krow = a.qkv + (int64_t)b * a.q_total * a.ld + (int64_t)(a.Hq + hkv) * D;
+  // the channel pair (i0, i1) of the new keys that this lane rotates
   const int pair = min(lane, D / 2 - 1);
   const bool rot_pair = rotate && pair < half_rot;
   const int i0 = !rot_pair ? max(a.rot, 0) + 2 * (pair - max(half_rot, 0)) : a.interleaved ? 2 * pair : pair;
   const int i1 = rot_pair && !a.interleaved ? pair + half_rot : i0 + 1;
+  auto table_row = [&](int tok) {
+    const int pos = max(min(a.position_ids ? a.position_ids[b * a.q_total + tok] : past + tok, a.rope_max_pos - 1), 0);
+    return a.rope + (int64_t)pos * half_rot * 2;
+  };
+  auto rotated = [&](float u, float w, float2 cs, float& y0, float& y1) {
+    y0 = rot_pair ? fmaf(u, cs.x, -(w * cs.y)) : u;
+    y1 = rot_pair ? fmaf(w, cs.x, u * cs.y) : w;
+  };
+  // several new tokens: those of this range go to the cache first
+  if (appends && a.q_total > 1 && a.q_off == 0) {
+    for (int t = wave; t < a.q_total; t += NW) {
+      const int p = past + t;
+      if (p < blk0 * BK || p >= blk1 * BK || p >= a.Lmax) continue;
+      const _Float16* kt = krow + (int64_t)t * a.ld;
+      const _Float16* vt = kt + (int64_t)a.Hkv * D;
+      if (lane < D / 2) {
+        float y0, y1;
+        rotated((float)kt[i0], (float)kt[i1], rot_pair ? *(const float2*)(table_row(t) + 2 * pair) : float2{1.0f, 0.0f}, y0, y1);
+        if constexpr (FP8) {
+          ((uint8_t*)kc)[(int64_t)p * D + i0] = f16_to_e5m2((_Float16)y0);
+          ((uint8_t*)kc)[(int64_t)p * D + i1] = f16_to_e5m2((_Float16)y1);
+        } else {
+          ((_Float16*)kc)[(int64_t)p * D + i0] = (_Float16)y0;
+          ((_Float16*)kc)[(int64_t)p * D + i1] = (_Float16)y1;
+        }
+      }
+      for (int d = lane; d < D; d += 64) {
+        if constexpr (FP8) ((uint8_t*)vc)[(int64_t)d * a.Lmax + p] = f16_to_e5m2(vt[d]);
+        else ((_Float16*)vc)[(int64_t)d * a.Lmax + p] = vt[d];
+      }
+    }
+    __syncthreads();
+  }
+  // ---- q, its rotation, the new key and value, then the first block (all without a branch: what arrives is counted) ----
+  half8 qraw[RT][DC];
+  float4v cs[RT][DC][2];     // [2 i], [2 i + 1]: cosine and sine of 8 / 2 channel pairs each (without a rotation: any readable numbers)
+  int row[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    row[t] = min(16 * t + rr, rows - 1);
+    const int tok = a.q_off + row[t] / G;
+    const _Float16* qp = a.qkv + ((int64_t)b * a.q_total + tok) * a.ld + (int64_t)(hkv * G + row[t] % G) * D;
+#pragma unroll
+    for (int c = 0; c < DC; ++c) qraw[t][c] = *(const half8*)(qp + chan(c, g));
+    const float* tab = rotate ? table_row(tok) : (const float*)qp;
+#pragma unroll
+    for (int i = 0; i < DC; ++i) {
+      const int at = a.interleaved ? (chan(i, g) < a.rot ? chan(i, g) : 0) : 2 * chan(i >> 1, g) + 8 * (i & 1);
+      const float* p = tab + (rotate ? at : 0);
+      cs[t][i][0] = *(const float4v*)p;
+      cs[t][i][1] = *(const float4v*)(p + 4);
+    }
+  }
   const _Float16 x0 = krow[i0], x1 = krow[i1];
-  const float2 kcs = *(const float2*)(tab + (rot_pair ? 2 * pair : 0));
+  const float2 kcs = *(const float2*)(rot_pair ? table_row(0) + 2 * pair : (const float*)a.qkv);
   const _Float16 nv = krow[(int64_t)a.Hkv * D + wave * CH + min(lane, CH - 1)];
   const int first_end = blk0 < blk1 ? kv_len : 0;
   request_k(blk0 * BK, first_end);
   request_v(blk0 * BK, first_end);
   __builtin_amdgcn_sched_barrier(0);
 
-  const bool valid = rr < rows;
   const float qscale = a.softcap > 0.0f ? a.scale : a.scale * 1.4426950408889634f;
-  half8 qf[F8M ? 1 : DC];
-  uint2v qh[F8M ? DC : 1], ql[F8M ? DC : 1];
-  float q_unscale = 1.0f;
-  {
+  half8 qf[RT][F8M ? 1 : DC];
+  uint2v qh[RT][F8M ? DC : 1], ql[RT][F8M ? DC : 1];
+  float q_unscale[RT], slope[RT];
+  int lim[RT], lo_lim[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    const bool valid = 16 * t + rr < rows;
     float qv[DC][8];
 #pragma unroll
     for (int c = 0; c < DC; ++c)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) qv[c][j] = valid ? (float)qraw[c][j] : 0.0f;
+      for (int j = 0; j < 8; ++j) qv[c][j] = valid ? (float)qraw[t][c][j] : 0.0f;
     if (rotate) {
       if (a.interleaved) {
 #pragma unroll
@@ -151,7 +191,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
           if (chan(c, g) < a.rot) {
 #pragma unroll
             for (int j = 0; j < 8; j += 2) {
-              const float co = cs[c][j >> 2][j & 3], si = cs[c][j >> 2][(j & 3) + 1], u = qv[c][j], w = qv[c][j + 1];
+              const float co = cs[t][c][j >> 2][j & 3], si = cs[t][c][j >> 2][(j & 3) + 1], u = qv[c][j], w = qv[c][j + 1];
               qv[c][j] = u * co - w * si;
               qv[c][j + 1] = w * co + u * si;
             }
@@ -162,14 +202,15 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
         for (int c = 0; c < DC / 2; ++c) {
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
-            const float4v t = cs[2 * c + (j >> 2)][(j >> 1) & 1];
-            const float co = t[2 * (j & 1)], si = t[2 * (j & 1) + 1], u = qv[c][j], w = qv[c + DC / 2][j];
+            const float4v p = cs[t][2 * c + (j >> 2)][(j >> 1) & 1];
+            const float co = p[2 * (j & 1)], si = p[2 * (j & 1) + 1], u = qv[c][j], w = qv[c + DC / 2][j];
             qv[c][j] = u * co - w * si;
             qv[c + DC / 2][j] = w * co + u * si;
           }
         }
       }
     }
+    q_unscale[t] = 1.0f;
     if constexpr (F8M) {
       float am = 0.0f;
 #pragma unroll
@@ -179,13 +220,13 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
       am = fmaxf(am, __shfl_xor(am, 16));
       am = fmaxf(am, __shfl_xor(am, 32));
       const float f = am > 0.0f ? P8_SCALE / am : 0.0f;
-      q_unscale = am * (qscale / P8_SCALE);
+      q_unscale[t] = am * (qscale / P8_SCALE);
 #pragma unroll
       for (int c = 0; c < DC; ++c) {
         float x[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) x[j] = qv[c][j] * f;
-        split_e4m3(x, qh[c], ql[c]);
+        split_e4m3(x, qh[t][c], ql[t][c]);
       }
     } else {
 #pragma unroll
@@ -193,19 +234,24 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
         half8 v;
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = (_Float16)(qv[c][j] * qscale);
-        qf[c] = v;
+        qf[t][c] = v;
       }
     }
+    const int last = past + a.q_off + row[t] / G;
+    lim[t] = valid ? last : -1;
+    lo_lim[t] = a.window > 0 && valid ? max(0, last - a.window + 1) : 0;
+    slope[t] = a.alibi != nullptr ? a.alibi[hkv * G + row[t] % G] * 1.4426950408889634f : 0.0f;
   }
-  const int lim = valid ? past : -1;
-  const int lo_lim = a.window > 0 && valid ? max(0, past - a.window + 1) : 0;
-  const float slope = a.alibi != nullptr ? a.alibi[hkv * G + row] * 1.4426950408889634f : 0.0f;
 
-  float m_all = NEG_BIG;     // running maximum of the row, the same in every wavefront
-  float l_run = 0.0f;        // sum over this lane's keys, relative to m_all
-  float4v o[DTW];
+  float m_all[RT], l_run[RT];      // running maximum of the row, the same in every wavefront; sum over this lane's keys relative to it
+  float4v o[RT][DTW];
 #pragma unroll
-  for (int d = 0; d < DTW; ++d) o[d] = float4v{0, 0, 0, 0};
+  for (int t = 0; t < RT; ++t) {
+    m_all[t] = NEG_BIG;
+    l_run[t] = 0.0f;
+#pragma unroll
+    for (int d = 0; d < DTW; ++d) o[t][d] = float4v{0, 0, 0, 0};
+  }
 
   for (int blk = blk0; blk < blk1; ++blk) {
     const int kb = blk * BK, kbw = kb + wave * KW;
@@ -227,11 +273,11 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
           ((_Float16*)kc)[(int64_t)past * D + c] = (_Float16)x;
         }
       };
-      const float u = (float)x0, w = (float)x1;
-      put(i0, rot_pair ? u * kcs.x - w * kcs.y : u);
-      put(i1, rot_pair ? w * kcs.x + u * kcs.y : w);
+      float y0, y1;
+      rotated((float)x0, (float)x1, kcs, y0, y1);
+      put(i0, y0);
+      put(i1, y1);
     }
-    float sv[KL];
     const bool mine = kbw < kv_len;
     half8 kf[FP8 ? 1 : NU][FP8 ? 1 : DC];
     uint2v kr[FP8 ? NU : 1][FP8 ? DC : 1];
@@ -257,75 +303,83 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
     __builtin_amdgcn_s_waitcnt(attn_vm_lgkm0(63));
     __builtin_amdgcn_sched_barrier(0);
     if (more) request_k(kb + BK, kv_len);
-    float m_new = m_all;
-    char* pw = sp + ((par * NW + wave) * rows + rr) * PB + 16 * g;
-    if (mine) {
+    float m_new[RT];
 #pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        float4v su = {0, 0, 0, 0};
+    for (int t = 0; t < RT; ++t) {
+      const bool valid = 16 * t + rr < rows;
+      m_new[t] = m_all[t];
+      if (mine) {
+        char* pw = sp + ((par * NW + wave) * rows + 16 * t + rr) * PB + 16 * g;
+        float sv[KL];
 #pragma unroll
-        for (int c = 0; c < DC; ++c) {
-          if constexpr (F8M) {
-            su = mfma_bf8_fp8(kr[u][c], qh[c], su);
-            su = mfma_bf8_fp8(kr[u][c], ql[c], su);
-          } else if constexpr (FP8) {
-            su = mfma16(dec_e5m2(kr[u][c].x, kr[u][c].y), qf[c], su);
-          } else {
-            su = mfma16(kf[u][c], qf[c], su);
+        for (int u = 0; u < NU; ++u) {
+          float4v su = {0, 0, 0, 0};
+#pragma unroll
+          for (int c = 0; c < DC; ++c) {
+            if constexpr (F8M) {
+              su = mfma_bf8_fp8(kr[u][c], qh[t][c], su);
+              su = mfma_bf8_fp8(kr[u][c], ql[t][c], su);
+            } else if constexpr (FP8) {
+              su = mfma16(dec_e5m2(kr[u][c].x, kr[u][c].y), qf[t][c], su);
+            } else {
+              su = mfma16(kf[u][c], qf[t][c], su);
+            }
+          }
+#pragma unroll
+          for (int q = 0; q < 4; ++q) sv[4 * u + q] = F8M ? su[q] * q_unscale[t] : su[q];
+        }
+        if (a.softcap > 0.0f) {
+#pragma unroll
+          for (int q = 0; q < KL; ++q) sv[q] = a.softcap * tanhf(sv[q] / a.softcap) * 1.4426950408889634f;
+        }
+        const int kfirst = kbw + KL * g;
+        if (a.alibi != nullptr) {
+#pragma unroll
+          for (int q = 0; q < KL; ++q) sv[q] += slope[t] * (float)(kfirst + q - lim[t]);
+        }
+        if (a.mask && valid) {
+          const _Float16* mp = a.mask + ((int64_t)b * a.q_total + a.q_off + row[t] / G) * a.mask_ld + kfirst;
+#pragma unroll
+          for (int q = 0; q < KL; ++q)
+            if (kfirst + q < a.mask_ld) sv[q] += (float)mp[q] * 1.4426950408889634f;
+        }
+        float mx = m_all[t];
+#pragma unroll
+        for (int q = 0; q < KL; ++q) {
+          const int key = kfirst + q;
+          if (key > lim[t] || key < lo_lim[t]) sv[q] = NEG_BIG;
+          mx = fmaxf(mx, sv[q]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        m_new[t] = mx;
+        float ps = 0.0f;
+#pragma unroll
+        for (int q = 0; q < KL; ++q) {
+          sv[q] = sv[q] <= NEG_BIG ? 0.0f : (F8M ? P8_SCALE : 1.0f) * __builtin_amdgcn_exp2f(sv[q] - mx);
+          ps += sv[q];
+        }
+        l_run[t] = l_run[t] * __builtin_amdgcn_exp2f(m_all[t] - mx) + ps;
+        if constexpr (F8M) {
+          uint2v h0, l0, h1, l1;
+          split_e4m3(*(const float(*)[8]) & sv[0], h0, l0);
+          split_e4m3(*(const float(*)[8]) & sv[8], h1, l1);
+          if (valid) {
+            *(uint4v*)pw = uint4v{h0.x, h0.y, h1.x, h1.y};
+            *(uint4v*)(pw + 64) = uint4v{l0.x, l0.y, l1.x, l1.y};
+          }
+        } else {
+#pragma unroll
+          for (int h = 0; h < KL / 8; ++h) {
+            half8 p;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) p[q] = (_Float16)sv[8 * h + q];
+            if (valid) *(half8*)(pw + 64 * h) = p;
           }
         }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) sv[4 * u + q] = F8M ? su[q] * q_unscale : su[q];
       }
-      if (a.softcap > 0.0f) {
-#pragma unroll
-        for (int q = 0; q < KL; ++q) sv[q] = a.softcap * tanhf(sv[q] / a.softcap) * 1.4426950408889634f;
-      }
-      const int kfirst = kbw + KL * g;
-      if (a.alibi != nullptr) {
-#pragma unroll
-        for (int q = 0; q < KL; ++q) sv[q] += slope * (float)(kfirst + q - lim);
-      }
-      if (a.mask && valid) {
-        const _Float16* mp = a.mask + (int64_t)b * a.mask_ld + kfirst;
-#pragma unroll
-        for (int q = 0; q < KL; ++q)
-          if (kfirst + q < a.mask_ld) sv[q] += (float)mp[q] * 1.4426950408889634f;
-      }
-#pragma unroll
-      for (int q = 0; q < KL; ++q) {
-        const int key = kfirst + q;
-        if (key > lim || key < lo_lim) sv[q] = NEG_BIG;
-        m_new = fmaxf(m_new, sv[q]);
-      }
-      m_new = fmaxf(m_new, __shfl_xor(m_new, 16));
-      m_new = fmaxf(m_new, __shfl_xor(m_new, 32));
-      float ps = 0.0f;
-#pragma unroll
-      for (int q = 0; q < KL; ++q) {
-        sv[q] = sv[q] <= NEG_BIG ? 0.0f : (F8M ? P8_SCALE : 1.0f) * __builtin_amdgcn_exp2f(sv[q] - m_new);
-        ps += sv[q];
-      }
-      l_run = l_run * __builtin_amdgcn_exp2f(m_all - m_new) + ps;
-      if constexpr (F8M) {
-        uint2v h0, l0, h1, l1;
-        split_e4m3(*(const float(*)[8]) & sv[0], h0, l0);
-        split_e4m3(*(const float(*)[8]) & sv[8], h1, l1);
-        if (valid) {
-          *(uint4v*)pw = uint4v{h0.x, h0.y, h1.x, h1.y};
-          *(uint4v*)(pw + 64) = uint4v{l0.x, l0.y, l1.x, l1.y};
-        }
-      } else {
-#pragma unroll
-        for (int h = 0; h < KL / 8; ++h) {
-          half8 p;
-#pragma unroll
-          for (int q = 0; q < 8; ++q) p[q] = (_Float16)sv[8 * h + q];
-          if (valid) *(half8*)(pw + 64 * h) = p;
-        }
-      }
+      if (g == 0) s_m[((par * NW + wave) * RT + t) * 16 + rr] = m_new[t];
     }
-    if (g == 0) s_m[(par * NW + wave) * 16 + rr] = m_new;
     // ---- everybody's probabilities, this wavefront's channels ----
     if (more) __builtin_amdgcn_s_waitcnt(attn_vm_lgkm0(NR));
     else __builtin_amdgcn_s_waitcnt(attn_vm_lgkm0(0));
@@ -347,90 +401,108 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
                                                17 /* written through: 64 x 32 heads, 1000 e5m2 keys 107 -> 103 us */);
       }
     }
-    float mw[NW], m_next = m_all;
+    uint4v vr[DTW][NW], ph[RT][NW], pl[RT][FP8 ? NW : 1];
+    float mw[RT][NW];
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      mw[w] = s_m[(par * NW + w) * 16 + rr];
-      m_next = fmaxf(m_next, mw[w]);
-    }
-    uint4v vr[DTW][NW], ph[NW], pl[FP8 ? NW : 1];
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const char* pr = sp + ((par * NW + w) * rows + row) * PB + 16 * g;
-      ph[w] = *(const uint4v*)pr;
-      if constexpr (FP8) pl[w] = *(const uint4v*)(pr + 64);
+      for (int t = 0; t < RT; ++t) {
+        mw[t][w] = s_m[((par * NW + w) * RT + t) * 16 + rr];
+        const char* pr = sp + ((par * NW + w) * rows + row[t]) * PB + 16 * g;
+        ph[t][w] = *(const uint4v*)pr;
+        if constexpr (FP8) pl[t][w] = *(const uint4v*)(pr + 64);
+      }
 #pragma unroll
       for (int d = 0; d < DTW; ++d) vr[d][w] = *(const uint4v*)(svt + (16 * d + rr) * RV + (((4 * w + g) ^ (rr & 7)) << 4));
     }
     __builtin_amdgcn_s_waitcnt(attn_vm_lgkm0(63));
     __builtin_amdgcn_sched_barrier(0);
     if (more) request_v(kb + BK, kv_len);
-    auto times = [&](int d, int w, float4v c) {
+    auto times = [&](int t, int d, int w) {
+      const float4v zero = {0, 0, 0, 0};
       if constexpr (FP8 && !F8M) {
-        c = mfma16(dec_e5m2(vr[d][w][0], vr[d][w][1]), __builtin_bit_cast(half8, ph[w]), c);
-        return mfma16(dec_e5m2(vr[d][w][2], vr[d][w][3]), __builtin_bit_cast(half8, pl[w]), c);
+        const float4v c = mfma16(dec_e5m2(vr[d][w][0], vr[d][w][1]), __builtin_bit_cast(half8, ph[t][w]), zero);
+        return mfma16(dec_e5m2(vr[d][w][2], vr[d][w][3]), __builtin_bit_cast(half8, pl[t][w]), c);
       } else if constexpr (F8M) {
         const uint2v v0 = {vr[d][w][0], vr[d][w][1]}, v1 = {vr[d][w][2], vr[d][w][3]};
-        c = mfma_bf8_fp8(v0, uint2v{ph[w][0], ph[w][1]}, c);
-        c = mfma_bf8_fp8(v1, uint2v{ph[w][2], ph[w][3]}, c);
-        c = mfma_bf8_fp8(v0, uint2v{pl[w][0], pl[w][1]}, c);
-        return mfma_bf8_fp8(v1, uint2v{pl[w][2], pl[w][3]}, c);
+        float4v c = mfma_bf8_fp8(v0, uint2v{ph[t][w][0], ph[t][w][1]}, zero);
+        c = mfma_bf8_fp8(v1, uint2v{ph[t][w][2], ph[t][w][3]}, c);
+        c = mfma_bf8_fp8(v0, uint2v{pl[t][w][0], pl[t][w][1]}, c);
+        return mfma_bf8_fp8(v1, uint2v{pl[t][w][2], pl[t][w][3]}, c);
       } else {
-        return mfma16(__builtin_bit_cast(half8, vr[d][w]), __builtin_bit_cast(half8, ph[w]), c);
+        return mfma16(__builtin_bit_cast(half8, vr[d][w]), __builtin_bit_cast(half8, ph[t][w]), zero);
       }
     };
-    if (__any(m_next != m_all)) {
-      const float alpha = __builtin_amdgcn_exp2f(m_all - m_next);
 #pragma unroll
-      for (int d = 0; d < DTW; ++d) o[d] *= alpha;
+    for (int t = 0; t < RT; ++t) {
+      float m_next = m_all[t];
 #pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        if (kb + w * KW >= kv_len) continue;      // (bytes that nobody wrote)
-        const float f = __builtin_amdgcn_exp2f(mw[w] - m_next);
+      for (int w = 0; w < NW; ++w) m_next = fmaxf(m_next, mw[t][w]);
+      // (the two forms round alike where no factor differs from 1: a row does not feel its neighbours' maxima)
+      if (__any(m_next != m_all[t])) {
+        const float alpha = __builtin_amdgcn_exp2f(m_all[t] - m_next);
 #pragma unroll
-        for (int d = 0; d < DTW; ++d) o[d] += times(d, w, float4v{0, 0, 0, 0}) * f;
-      }
-      l_run *= __builtin_amdgcn_exp2f(m_new - m_next);
-      m_all = m_next;
-    } else {
+        for (int d = 0; d < DTW; ++d) o[t][d] *= alpha;
 #pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        if (kb + w * KW >= kv_len) continue;
+        for (int w = 0; w < NW; ++w) {
+          if (kb + w * KW >= kv_len) continue;      // (bytes that nobody wrote)
+          const float f = __builtin_amdgcn_exp2f(mw[t][w] - m_next);
 #pragma unroll
-        for (int d = 0; d < DTW; ++d) o[d] = times(d, w, o[d]);
+          for (int d = 0; d < DTW; ++d) {
+            const float4v c = times(t, d, w);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) o[t][d][q] = fmaf(c[q], f, o[t][d][q]);
+          }
+        }
+        l_run[t] *= __builtin_amdgcn_exp2f(m_new[t] - m_next);
+        m_all[t] = m_next;
+      } else {
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+          if (kb + w * KW >= kv_len) continue;
+#pragma unroll
+          for (int d = 0; d < DTW; ++d) o[t][d] += times(t, d, w);
+        }
       }
     }
   }
 
-  // ---- the row's sum ----
-  float l = l_run;
-  l += __shfl_xor(l, 16);
-  l += __shfl_xor(l, 32);
-  if (g == 0) s_l[wave * 16 + rr] = l;
-  __syncthreads();
-  float lt = 0.0f;
+  // ---- the rows' sums ----
 #pragma unroll
-  for (int w = 0; w < NW; ++w) lt += s_l[w * 16 + rr];
-
+  for (int t = 0; t < RT; ++t) {
+    float l = l_run[t];
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (g == 0) s_l[(wave * RT + t) * 16 + rr] = l;
+  }
+  __syncthreads();
   const int bh = b * gridDim.y + hkv;
   const bool single = a.splits == 1;
-  if (valid) {
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    float lt = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) lt += s_l[(w * RT + t) * 16 + rr];
+    if (16 * t + rr >= rows) continue;
     if (single) {
       const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+      const int tok = a.q_off + row[t] / G, head = hkv * G + row[t] % G;
 #pragma unroll
       for (int d = 0; d < DTW; ++d) {
-        const half4 hv = {(_Float16)(o[d][0] * inv), (_Float16)(o[d][1] * inv), (_Float16)(o[d][2] * inv), (_Float16)(o[d][3] * inv)};
-        *(half4*)(a.out + out_at(b, (hkv * G + rr) * D + wave * CH + 16 * d + 4 * g, a.Hq * D, a.frag_mt)) = hv;
+        half4 hv;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) hv[q] = (_Float16)(o[t][d][q] * inv);
+        *(half4*)(a.out + out_at(b * a.q_total + tok, head * D + wave * CH + 16 * d + 4 * g, a.Hq * D, a.frag_mt)) = hv;
       }
     } else {
-      float* dst = a.ws + (((int64_t)bh * a.splits + split) * 16 + rr) * (D + 4);
+      float* dst = a.ws + (((int64_t)bh * a.splits + split) * (RT * 16) + 16 * t + rr) * (D + 4);
 #pragma unroll
-      for (int d = 0; d < DTW; ++d) *(float4v*)(dst + wave * CH + 16 * d + 4 * g) = o[d];
-      if (wave == 0 && g == 0) { dst[D] = m_all; dst[D + 1] = lt; }
+      for (int d = 0; d < DTW; ++d) *(float4v*)(dst + wave * CH + 16 * d + 4 * g) = o[t][d];
+      if (wave == 0 && g == 0) { dst[D] = m_all[t]; dst[D + 1] = lt; }
     }
   }
   if (single || a.defer_combine) return;
-  combine_splits<D, 1, NW * 64>(a, bh, hkv * G, b * a.q_total, rows, G, (int*)s_m);
+  combine_splits<D, RT, NW * 64>(a, bh, hkv * G, b * a.q_total + a.q_off, rows, G, (int*)s_m);
 }
 
 }  // namespace bigdl

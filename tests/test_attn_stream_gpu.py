@@ -1,6 +1,6 @@
-"""Decode attention of one new token with K / V^T through LDS in whole lines (csrc/hip/attn_decode_stream.h) against float64: lengths
+"""Decode attention with K / V^T through LDS in whole lines (csrc/hip/attn_decode_stream.h) against float64: lengths
 around its blocks (64 keys a wavefront in e5m2 caches, 32 in fp16; two or four wavefronts), several lengths in a batch, ranges without
-keys, groups of 1 to 16 query heads, and what changes a score.  The cache behind the last piece that holds a key is NaN: nothing of it
+keys, groups of 1 to 32 query heads, and what changes a score.  The cache behind the last piece that holds a key is NaN: nothing of it
 may reach a result."""
 import math
 
@@ -125,7 +125,7 @@ EDGES = [0, 1, 30, 31, 32, 33, 63, 64, 65, 126, 127, 128, 129, 191, 255, 256, 25
 
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("d", [64, 128])
-@pytest.mark.parametrize("hq,hkv,splits", [(2, 2, 2), (8, 2, 3), (7, 1, 1), (16, 1, 2), (40, 40, 1), (32, 16, 2)])
+@pytest.mark.parametrize("hq,hkv,splits", [(2, 2, 2), (8, 2, 3), (7, 1, 1), (16, 1, 2), (40, 40, 1), (32, 16, 2), (32, 1, 2), (50, 2, 1)])
 def test_lengths(d, fp8, hq, hkv, splits):
     _case(d, fp8, hq, hkv, EDGES, splits)
 
@@ -137,3 +137,38 @@ def test_lengths(d, fp8, hq, hkv, splits):
 def test_options(d, fp8, opt):
     _case(d, fp8, 6, 2, [5, 127, 128, 400, 1000], 3, **opt)
     _case(d, fp8, 96, 96, [0, 63, 64, 200, 256, 777, 1023], 1, **{**opt, "defer": False})
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hq,hkv,n", [(4, 4, 9), (8, 2, 4), (1, 1, 3), (2, 2, 16), (8, 2, 7), (16, 1, 2), (60, 60, 5)])
+@pytest.mark.parametrize("interleaved", [False, True])
+def test_several_tokens_round_as_one_after_the_other(fp8, hq, hkv, n, interleaved):
+    """a draft's check in one call and the decode steps it stands for: the same bits, in the output and in both caches"""
+    if fp8 and hq // hkv * n > 16:
+        pytest.skip("two row tiles of e5m2 take the form that widens them")
+    torch.manual_seed(n)
+    d = 128
+    pasts = [0, 29, 60, 63, 120, 250, 255, 500, 1000]
+    b = len(pasts)
+    dt = torch.float8_e5m2 if fp8 else torch.float16
+    raw = torch.uint8 if fp8 else torch.int16
+    k, v = torch.randn(b, hkv, LMAX, d).half().to(dt).cuda(), torch.randn(b, hkv, d, LMAX).half().to(dt).cuda()
+    qkv = torch.randn(b, n, (hq + 2 * hkv) * d, device="cuda").half()
+    ang = torch.arange(LMAX, device="cuda").float()[:, None] / (10000 ** (torch.arange(d // 2, device="cuda").float() / (d // 2)))
+    table = torch.stack([ang.cos(), ang.sin()], -1).contiguous()
+    counters = torch.zeros(hip.attn_decode_counters(b, hq, hkv), dtype=torch.int32, device="cuda")
+    ws = torch.empty(hip.attn_decode_ws_floats(b, hq, hkv, n, d, 1), dtype=torch.float32, device="cuda")
+
+    def call(x, kc, vc, first, m):
+        out = torch.empty(b * m, hq * d, dtype=torch.float16, device="cuda")
+        past = torch.tensor(pasts, dtype=torch.int32, device="cuda") + first
+        c = (lambda t: t.view(torch.uint8)) if fp8 else (lambda t: t)
+        hip.attn_decode(x.reshape(b * m, -1), c(kc), c(vc), past, out, ws, counters, n_heads=hq, n_kv_heads=hkv, head_dim=d, q_len=m,
+                        batch=b, scale=d ** -0.5, splits=1, rope_table=table, interleaved=interleaved)
+        return out.view(b, m, hq * d)
+
+    k1, v1 = k.clone(), v.clone()
+    many = call(qkv, k1, v1, 0, n)
+    steps = torch.cat([call(qkv[:, t:t + 1].contiguous(), k, v, t, 1) for t in range(n)], 1)
+    assert torch.equal(k1.view(raw), k.view(raw)) and torch.equal(v1.view(raw), v.view(raw))
+    assert torch.equal(many, steps)

@@ -823,16 +823,16 @@ static int launch_one(const AttnArgs& a, size_t, hipStream_t st) {
   return HIP_CHECK_LAUNCH();
 }
 
-template <int D, bool FP8, int NW, int RT>
+template <int D, bool FP8, int NW, int RT, bool MULTI>
 static int launch_stream(const AttnArgs& a, hipStream_t st) {
   const size_t smem = attn_stream_lds<D, FP8, NW, RT>(a.Hq / a.Hkv * a.q_cnt);
   static bool attr = false;
   if (!attr && smem > 65536) {
-    if (hipFuncSetAttribute((const void*)attn_stream_kernel<D, FP8, NW, RT>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
+    if (hipFuncSetAttribute((const void*)attn_stream_kernel<D, FP8, NW, RT, MULTI>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
       return -5;
     attr = true;
   }
-  hipLaunchKernelGGL((attn_stream_kernel<D, FP8, NW, RT>), dim3(a.splits, a.Hkv, a.B), dim3(NW * 64), smem, st, a.past_len, a.qkv, a.ld, a.splits,
+  hipLaunchKernelGGL((attn_stream_kernel<D, FP8, NW, RT, MULTI>), dim3(a.splits, a.Hkv, a.B), dim3(NW * 64), smem, st, a.past_len, a.qkv, a.ld, a.splits,
                      a.Hq, a.Hkv, a.Lmax, a.kc, a.vc, a);
   return HIP_CHECK_LAUNCH();
 }
@@ -865,9 +865,22 @@ static int launch_rt(const AttnArgs& a, hipStream_t st) {
                       (int64_t)a.Lmax * D * (FP8 ? 1 : 2) < (1ll << 31) && ((uintptr_t)a.rope & 15) == 0;
     if (!force && fits && !(FP8 && D == 64 && a.splits == 1 && groups < 512)) {
       const bool two = groups >= (D == 64 ? 640 : 512);
+      auto launch = [&](auto rows16, auto multi) {
+        constexpr int RT = decltype(rows16)::value;
+        constexpr bool MULTI = decltype(multi)::value;
+        return two ? launch_stream<D, FP8, 2, RT, MULTI>(a, st) : launch_stream<D, FP8, 4, RT, MULTI>(a, st);
+      };
+      using One = std::integral_constant<int, 1>;
+      using Two = std::integral_constant<int, 2>;
+      if constexpr (D == 128)
+        if (a.q_total > 1) {
+          if constexpr (!FP8)
+            if (rt == 2) return launch(Two{}, std::true_type{});
+          return launch(One{}, std::true_type{});
+        }
       if constexpr (!FP8)
-        if (rt == 2) return two ? launch_stream<D, FP8, 2, 2>(a, st) : launch_stream<D, FP8, 4, 2>(a, st);
-      return two ? launch_stream<D, FP8, 2, 1>(a, st) : launch_stream<D, FP8, 4, 1>(a, st);
+        if (rt == 2) return launch(Two{}, std::false_type{});
+      return launch(One{}, std::false_type{});
     }
   }
   if (rt == 1) {

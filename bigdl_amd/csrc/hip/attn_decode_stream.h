@@ -33,8 +33,9 @@ constexpr size_t attn_stream_lds(int rows) {
   return (size_t)NW * (D * 128) + 2 * NW * rows * (FP8 ? 128 : 64) + 3 * NW * RT * 64;
 }
 
-// RT = 16-row tiles of query rows (G query heads x the launch's new tokens).  A row's result does not depend on the rows beside it.
-template <int D, bool FP8, int NW, int RT>
+// RT = 16-row tiles of query rows (G query heads x the launch's new tokens, of which MULTI has several).  A row's result does not depend
+// on the rows beside it.
+template <int D, bool FP8, int NW, int RT, bool MULTI>
 __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_past, _Float16* p_qkv, int p_ld, int p_splits, int p_Hq,
                                                                               int p_Hkv, int p_Lmax, void* p_kc, void* p_vc, AttnArgs a) {
   a.past_len = p_past; a.qkv = p_qkv; a.ld = p_ld; a.splits = p_splits; a.Hq = p_Hq; a.Hkv = p_Hkv; a.Lmax = p_Lmax;
@@ -55,7 +56,9 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rr = lane & 15, g = lane >> 4;
   const int split = blockIdx.x, hkv = blockIdx.y, b = blockIdx.z;
-  const int G = a.Hq / a.Hkv, rows = G * a.q_cnt;
+  const int G = a.Hq / a.Hkv, q_total = MULTI ? a.q_total : 1, rows = MULTI ? G * a.q_cnt : G;
+  auto token = [&](int row) { return MULTI ? a.q_off + row / G : 0; };
+  auto head = [&](int row) { return hkv * G + (MULTI ? row % G : row); };
   constexpr int PB = FP8 ? 128 : 64;         // LDS bytes of a row's probabilities, one wavefront's keys
   char* sk = smem + wave * (D * 128);                                   // this wavefront's keys of a block, then its V^T rows
   char* svt = sk + D * 64;
@@ -64,7 +67,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
   float* s_l = s_m + 2 * NW * RT * 16;                                  // [NW][RT * 16]
 
   const int past = a.past_len[b];
-  const int kv_len = min(past + a.q_total, a.Lmax);
+  const int kv_len = min(past + q_total, a.Lmax);
   const int nblk = (kv_len + BK - 1) / BK;
   const int per = (nblk + a.splits - 1) / a.splits;
   const int blk0 = split * per, blk1 = min(nblk, blk0 + per);
@@ -73,7 +76,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
   char* vc = (char*)p_vc + base;
   const int half_rot = a.rot >> 1;
   const bool appends = a.rope != nullptr || a.rot == 0;
-  const bool append = appends && a.q_total == 1 && past < a.Lmax && past >= blk0 * BK && past < blk1 * BK;     // one token: into its block in LDS
+  const bool append = appends && !MULTI && past < a.Lmax && past >= blk0 * BK && past < blk1 * BK;     // one token: into its block in LDS
   const int kw_new = (past % BK) / KW;       // the wavefront with the new key
 
   // ---- requests ----
@@ -104,14 +107,14 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
   // first head channel of this lane's 8 values in k-step c (as in the register form: the rotate-half partner is k-step c + DC / 2)
   auto chan = [](int c, int g) { return F8M ? 64 * (c >> 1) + 16 * g + 8 * (c & 1) : 32 * c + 8 * g; };
   const bool rotate = a.rope != nullptr;
-  const _Float16* krow = a.qkv + (int64_t)b * a.q_total * a.ld + (int64_t)(a.Hq + hkv) * D;
+  const _Float16* krow = a.qkv + (int64_t)b * q_total * a.ld + (int64_t)(a.Hq + hkv) * D;
   // the channel pair (i0, i1) of the new keys that this lane rotates
   const int pair = min(lane, D / 2 - 1);
   const bool rot_pair = rotate && pair < half_rot;
   const int i0 = !rot_pair ? max(a.rot, 0) + 2 * (pair - max(half_rot, 0)) : a.interleaved ? 2 * pair : pair;
   const int i1 = rot_pair && !a.interleaved ? pair + half_rot : i0 + 1;
   auto table_row = [&](int tok) {
-    const int pos = max(min(a.position_ids ? a.position_ids[b * a.q_total + tok] : past + tok, a.rope_max_pos - 1), 0);
+    const int pos = max(min(a.position_ids ? a.position_ids[b * q_total + tok] : past + tok, a.rope_max_pos - 1), 0);
     return a.rope + (int64_t)pos * half_rot * 2;
   };
   auto rotated = [&](float u, float w, float2 cs, float& y0, float& y1) {
@@ -119,8 +122,8 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
     y1 = rot_pair ? fmaf(w, cs.x, u * cs.y) : w;
   };
   // several new tokens: those of this range go to the cache first
-  if (appends && a.q_total > 1 && a.q_off == 0) {
-    for (int t = wave; t < a.q_total; t += NW) {
+  if (MULTI && appends && a.q_off == 0) {
+    for (int t = wave; t < q_total; t += NW) {
       const int p = past + t;
       if (p < blk0 * BK || p >= blk1 * BK || p >= a.Lmax) continue;
       const _Float16* kt = krow + (int64_t)t * a.ld;
@@ -150,8 +153,8 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
     row[t] = min(16 * t + rr, rows - 1);
-    const int tok = a.q_off + row[t] / G;
-    const _Float16* qp = a.qkv + ((int64_t)b * a.q_total + tok) * a.ld + (int64_t)(hkv * G + row[t] % G) * D;
+    const int tok = token(row[t]);
+    const _Float16* qp = a.qkv + ((int64_t)b * q_total + tok) * a.ld + (int64_t)head(row[t]) * D;
 #pragma unroll
     for (int c = 0; c < DC; ++c) qraw[t][c] = *(const half8*)(qp + chan(c, g));
     const float* tab = rotate ? table_row(tok) : (const float*)qp;
@@ -237,10 +240,10 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
         qf[t][c] = v;
       }
     }
-    const int last = past + a.q_off + row[t] / G;
+    const int last = past + token(row[t]);
     lim[t] = valid ? last : -1;
     lo_lim[t] = a.window > 0 && valid ? max(0, last - a.window + 1) : 0;
-    slope[t] = a.alibi != nullptr ? a.alibi[hkv * G + row[t] % G] * 1.4426950408889634f : 0.0f;
+    slope[t] = a.alibi != nullptr ? a.alibi[head(row[t])] * 1.4426950408889634f : 0.0f;
   }
 
   float m_all[RT], l_run[RT];      // running maximum of the row, the same in every wavefront; sum over this lane's keys relative to it
@@ -338,7 +341,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
           for (int q = 0; q < KL; ++q) sv[q] += slope[t] * (float)(kfirst + q - lim[t]);
         }
         if (a.mask && valid) {
-          const _Float16* mp = a.mask + ((int64_t)b * a.q_total + a.q_off + row[t] / G) * a.mask_ld + kfirst;
+          const _Float16* mp = a.mask + ((int64_t)b * q_total + token(row[t])) * a.mask_ld + kfirst;
 #pragma unroll
           for (int q = 0; q < KL; ++q)
             if (kfirst + q < a.mask_ld) sv[q] += (float)mp[q] * 1.4426950408889634f;
@@ -418,19 +421,18 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
     __builtin_amdgcn_s_waitcnt(attn_vm_lgkm0(63));
     __builtin_amdgcn_sched_barrier(0);
     if (more) request_v(kb + BK, kv_len);
-    auto times = [&](int t, int d, int w) {
-      const float4v zero = {0, 0, 0, 0};
+    auto times = [&](int t, int d, int w, float4v c) {
       if constexpr (FP8 && !F8M) {
-        const float4v c = mfma16(dec_e5m2(vr[d][w][0], vr[d][w][1]), __builtin_bit_cast(half8, ph[t][w]), zero);
+        c = mfma16(dec_e5m2(vr[d][w][0], vr[d][w][1]), __builtin_bit_cast(half8, ph[t][w]), c);
         return mfma16(dec_e5m2(vr[d][w][2], vr[d][w][3]), __builtin_bit_cast(half8, pl[t][w]), c);
       } else if constexpr (F8M) {
         const uint2v v0 = {vr[d][w][0], vr[d][w][1]}, v1 = {vr[d][w][2], vr[d][w][3]};
-        float4v c = mfma_bf8_fp8(v0, uint2v{ph[t][w][0], ph[t][w][1]}, zero);
+        c = mfma_bf8_fp8(v0, uint2v{ph[t][w][0], ph[t][w][1]}, c);
         c = mfma_bf8_fp8(v1, uint2v{ph[t][w][2], ph[t][w][3]}, c);
         c = mfma_bf8_fp8(v0, uint2v{pl[t][w][0], pl[t][w][1]}, c);
         return mfma_bf8_fp8(v1, uint2v{pl[t][w][2], pl[t][w][3]}, c);
       } else {
-        return mfma16(__builtin_bit_cast(half8, vr[d][w]), __builtin_bit_cast(half8, ph[t][w]), zero);
+        return mfma16(__builtin_bit_cast(half8, vr[d][w]), __builtin_bit_cast(half8, ph[t][w]), c);
       }
     };
 #pragma unroll
@@ -438,31 +440,36 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
       float m_next = m_all[t];
 #pragma unroll
       for (int w = 0; w < NW; ++w) m_next = fmaxf(m_next, mw[t][w]);
-      // (the two forms round alike where no factor differs from 1: a row does not feel its neighbours' maxima)
-      if (__any(m_next != m_all[t])) {
+      // rows whose maximum stays add to O in the matrix unit; the others' O and each wavefront's share are scaled (every row takes its own
+      // of the two results)
+      const bool grown = m_next != m_all[t];
+      float4v scaled[DTW];
+      const bool some = __any(grown);
+      if (some) {
         const float alpha = __builtin_amdgcn_exp2f(m_all[t] - m_next);
 #pragma unroll
-        for (int d = 0; d < DTW; ++d) o[t][d] *= alpha;
+        for (int d = 0; d < DTW; ++d) scaled[d] = o[t][d] * alpha;
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
           if (kb + w * KW >= kv_len) continue;      // (bytes that nobody wrote)
           const float f = __builtin_amdgcn_exp2f(mw[t][w] - m_next);
 #pragma unroll
-          for (int d = 0; d < DTW; ++d) {
-            const float4v c = times(t, d, w);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) o[t][d][q] = fmaf(c[q], f, o[t][d][q]);
-          }
+          for (int d = 0; d < DTW; ++d) scaled[d] += times(t, d, w, float4v{0, 0, 0, 0}) * f;
         }
         l_run[t] *= __builtin_amdgcn_exp2f(m_new[t] - m_next);
         m_all[t] = m_next;
-      } else {
+      }
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-          if (kb + w * KW >= kv_len) continue;
+      for (int w = 0; w < NW; ++w) {
+        if (kb + w * KW >= kv_len) continue;
 #pragma unroll
-          for (int d = 0; d < DTW; ++d) o[t][d] += times(t, d, w);
-        }
+        for (int d = 0; d < DTW; ++d) o[t][d] = times(t, d, w, o[t][d]);
+      }
+      if (some) {
+#pragma unroll
+        for (int d = 0; d < DTW; ++d)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) o[t][d][q] = grown ? scaled[d][q] : o[t][d][q];
       }
     }
   }
@@ -486,13 +493,12 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
     if (16 * t + rr >= rows) continue;
     if (single) {
       const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-      const int tok = a.q_off + row[t] / G, head = hkv * G + row[t] % G;
 #pragma unroll
       for (int d = 0; d < DTW; ++d) {
         half4 hv;
 #pragma unroll
         for (int q = 0; q < 4; ++q) hv[q] = (_Float16)(o[t][d][q] * inv);
-        *(half4*)(a.out + out_at(b * a.q_total + tok, head * D + wave * CH + 16 * d + 4 * g, a.Hq * D, a.frag_mt)) = hv;
+        *(half4*)(a.out + out_at(b * q_total + token(row[t]), head(row[t]) * D + wave * CH + 16 * d + 4 * g, a.Hq * D, a.frag_mt)) = hv;
       }
     } else {
       float* dst = a.ws + (((int64_t)bh * a.splits + split) * (RT * 16) + 16 * t + rr) * (D + 4);
@@ -502,7 +508,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
     }
   }
   if (single || a.defer_combine) return;
-  combine_splits<D, RT, NW * 64>(a, bh, hkv * G, b * a.q_total + a.q_off, rows, G, (int*)s_m);
+  combine_splits<D, RT, NW * 64>(a, bh, hkv * G, b * q_total + (MULTI ? a.q_off : 0), rows, G, (int*)s_m);
 }
 
 }  // namespace bigdl

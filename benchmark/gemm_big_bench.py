@@ -43,7 +43,7 @@ if __name__ == "__main__":
             ref = torch.nn.functional.linear(x.float(), wd.float())
             forces = [(-1, 0)]
             if args.sweep:
-                forces += [(c, sk) for c in (0, 1, 2) for sk in (1, 2, 4) if sk == 1 or k // 128 // sk >= 8]
+                forces += [(c, sk) for c in range(6) for sk in (1, 2, 4) if sk == 1 or k // 128 // sk >= 8]
             us_dense = us_blas = None
             if not args.no_ref:
                 us_dense = timed(lambda: torch.nn.functional.linear(x, hip.dequant_t16(w, qt, n, k)))

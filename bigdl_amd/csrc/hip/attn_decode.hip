@@ -174,6 +174,7 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
   constexpr bool F8M = FP8 && WIDE;
   static_assert(!WIDE || (FP8 && D % 128 == 0), "16-byte fragments: e5m2 cache, rotate-half partner in k-step c + DC/2");
   static_assert(!I4 || (!FP8 && KW == 32), "int4 caches: 32 keys per wavefront");
+  // (fp16 heads of 64 and 128 with one new token are attn_decode_stream.h's: the figures are of when they came here.)
   // The next block in flight, the new value stored with its block and q requested ahead of the append: one row tile and heads of
   // up to 128 channels.  fp16 caches, 12 sequences x 8 heads of 128, 6000 keys: 113 -> 102 us.  In a step, where caches are cold:
   // 8 layers of 4 kv heads of 64, 4 tokens, 45 / 1900 keys 849 -> 840 / 930 -> 922 us; 16 sequences x 32 heads of 128, 1000 keys

@@ -345,7 +345,7 @@ def lowbit_matmul(x_2d: torch.Tensor, weight: FP4Params, out_features: int, for_
     if weight.is_cuda:
         from ..ops import hip
         t16 = weight.qlayout == "t16"
-        if t16 or (weight.qtype == Q.Q6_K and not for_training):
+        if x_2d.shape[0] <= GEMM_MAX_ROWS and (t16 or (weight.qtype == Q.Q6_K and not for_training)):
             # fp16 rows that lie as the few-row kernels take them; everything else is declined (None) and takes the way below
             qt = weight.qtype
             y = hip.linear_call()(x_2d, weight, n, k, qt, hip._t16_nbytes(qt, n, k) if t16 else n * (k // 256) * 210, GEMV_MAX_ROWS,

@@ -23,7 +23,7 @@ setup(
     version="0.1.0",
     description="MI355X-native low-bit LLM inference and fine-tuning library (IPEX-LLM compatible API)",
     packages=find_packages(include=["bigdl_amd", "bigdl_amd.*", "ipex_llm", "bigdl"]),
-    package_data={"bigdl_amd": ["lib/*.so", "csrc/host/*", "csrc/hip/*"]},
+    package_data={"bigdl_amd": ["lib/*.so", "csrc/host/*", "csrc/hip/*", "csrc/torch_ext/*"]},
     python_requires=">=3.10",
     install_requires=["torch", "transformers", "numpy", "safetensors", "tokenizers", "pyyaml"],
     extras_require={

@@ -132,6 +132,14 @@ def test_lengths(d, fp8, hq, hkv, splits):
 
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("hq,hkv", [(8, 2), (24, 1)])
+@pytest.mark.parametrize("splits", [4, 5, 16, 17, 33])
+def test_merges_any_number_of_ranges(d, fp8, hq, hkv, splits):
+    _case(d, fp8, hq, hkv, [0, 31, 256, 700, 1023], splits)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("opt", [dict(softcap=20.0), dict(window=100), dict(alibi=True), dict(mask=True), dict(interleaved=True),
                                  dict(interleaved=True, rot=32), dict(rope=False), dict(defer=True)], ids=lambda o: next(iter(o)) + str(len(o)))
 def test_options(d, fp8, opt):

@@ -878,13 +878,18 @@ static int launch_rt(const AttnArgs& a, hipStream_t st) {
   // From two workgroups a CU on the two-wavefront form has as many bytes under way in smaller pieces, below it the longer block fills the
   // CU.  Several tokens (a draft's check) with heads of 128 round as the decode steps that they stand for; 64 x 32 heads, 2 / 8 tokens: fp16
   // 300 keys 101 -> 79 / 116 -> 90, e5m2 1000 keys 130 -> 124 / 146 -> 141, 300 keys 57 -> 55 / 66 -> 70.  What stays in the register form:
-  // several tokens with heads of 64 (64 groups x 1000, 4 tokens 14.0 -> 14.8), two row tiles of e5m2 (widened to fp16 there: more exact), and
-  // e5m2 heads of 64 with few long ranges (half the bytes a wavefront: 160 x 4000 above).
+  // several tokens with heads of 64 (64 groups x 1000, 4 tokens 14.0 -> 14.8), two row tiles of e5m2 (widened to fp16 there: more exact),
+  // e5m2 heads of 64 with few long ranges (half the bytes a wavefront: 160 x 4000 above, 192 x 4500 in two ranges 32.8 -> 34.6, 256 x 2250 in
+  // four 19.8 -> 19.8; merged here, by half the wavefronts, 25.1 -> 26.7, 256 x 750 in twelve 20.3 -> 16.4), and two row tiles of fp16 heads of 64 unless their ranges are short (two tiles' scores and exponentials for half
+  // the bytes; 20 - 32 heads a group: 64 x 1000 16.0 -> 19.1, 256 x 4000 56.6 -> 64.6, 256 x 1125 20.1 -> 21.7, 80 x 562 12.9 -> 13.5; 256 x 500
+  // 13.2 -> 12.3, 64 x 100 7.9 -> 5.8).  How long a range is follows from the cache's capacity: the lengths are not known here.
   if constexpr (D == 64 || D == 128) {
     const int64_t groups = (int64_t)a.B * a.Hkv * a.splits;
     const bool fits = a.nchunk == 1 && rt <= (FP8 ? 1 : 2) && (a.q_total == 1 || D == 128) &&
                       (int64_t)a.Lmax * D * (FP8 ? 1 : 2) < (1ll << 31) && ((uintptr_t)a.rope & 15) == 0;
-    if (!force && fits && !(FP8 && D == 64 && a.splits == 1 && groups < 512)) {
+    const int64_t longest = (int64_t)a.Lmax / a.splits;      // keys of a range at most
+    const bool left = D == 64 && (FP8 ? groups < 512 && (a.splits == 1 || longest > (a.defer_combine ? 3072 : 1024)) : a.gchunk > 16 && longest > 512);
+    if (!force && fits && !left) {
       const bool two = groups >= (D == 64 ? 640 : 512);
       auto launch = [&](auto rows16, auto multi) {
         constexpr int RT = decltype(rows16)::value;

@@ -876,19 +876,23 @@ static int launch_rt(const AttnArgs& a, hipStream_t st) {
   //   fp16 64:   20 x 220 6.5 -> 7.6 / 6.5    160 x 1100 19 -> 23 / 17    512 x 1100 38 -> 31 / 30    640 x 1100 50 -> 37 / 38
   //   e5m2 64:   96 x 2000 21 -> 28 / 19      160 x 4000 35 -> 54 / 37    512 x 1100 27 -> 24 / 20    640 x 1100 34 -> 25 / 26
   // From two workgroups a CU on the two-wavefront form has as many bytes under way in smaller pieces, below it the longer block fills the
-  // CU.  Several tokens (a draft's check) with heads of 128 round as the decode steps that they stand for; 64 x 32 heads, 2 / 8 tokens: fp16
-  // 300 keys 101 -> 79 / 116 -> 90, e5m2 1000 keys 130 -> 124 / 146 -> 141, 300 keys 57 -> 55 / 66 -> 70.  What stays in the register form:
-  // several tokens with heads of 64 (64 groups x 1000, 4 tokens 14.0 -> 14.8), two row tiles of e5m2 (widened to fp16 there: more exact),
-  // e5m2 heads of 64 with few long ranges (half the bytes a wavefront: 160 x 4000 above, 192 x 4500 in two ranges 32.8 -> 34.6, 256 x 2250 in
-  // four 19.8 -> 19.8; merged here, by half the wavefronts, 25.1 -> 26.7, 256 x 750 in twelve 20.3 -> 16.4), and two row tiles of fp16 heads of 64 unless their ranges are short (two tiles' scores and exponentials for half
-  // the bytes; 20 - 32 heads a group: 64 x 1000 16.0 -> 19.1, 256 x 4000 56.6 -> 64.6, 256 x 1125 20.1 -> 21.7, 80 x 562 12.9 -> 13.5; 256 x 500
-  // 13.2 -> 12.3, 64 x 100 7.9 -> 5.8).  How long a range is follows from the cache's capacity: the lengths are not known here.
+  // CU.  Several tokens (a draft's check) round as the decode steps that they stand for; 64 x 32 heads, 2 / 8 tokens: fp16 128
+  // 300 keys 101 -> 79 / 116 -> 90, e5m2 128 1000 keys 130 -> 124 / 146 -> 141, 300 keys 57 -> 55 / 66 -> 70, fp16 64 300 keys 4 tokens 56 -> 40 (16 x 4
+  // groups of two tiles, 1000 keys 16.5 -> 17.6).  What stays in the register form:
+  //  * two row tiles of e5m2, but not of several tokens with heads of 64 (which round as one: widened to fp16 in both forms);
+  //  * e5m2 heads of 64 with few long ranges (half the bytes a wavefront: 160 x 4000 above, 192 x 4500 in two 32.8 -> 34.2, 256 x 2250 in four
+  //    19.2 -> 19.2; merged here, by half the wavefronts, 23.6 -> 26.3, 256 x 750 in twelve 20.3 -> 16.4);
+  //  * groups of 17 - 32 fp16 heads of 64 with long ranges (two tiles' scores and exponentials for half the bytes: 256 x 4500 57.2 -> 61.8, 64 x 1000
+  //    16.4 -> 17.0, 256 x 1000 20.8 -> 17.5, 80 x 562 12.8 -> 12.0; merged here 256 x 1125 27.3 -> 30.3, 256 x 500 46.2 -> 37.6).
+  // How long a range is follows from the cache's capacity: the lengths are not known here.
   if constexpr (D == 64 || D == 128) {
     const int64_t groups = (int64_t)a.B * a.Hkv * a.splits;
-    const bool fits = a.nchunk == 1 && rt <= (FP8 ? 1 : 2) && (a.q_total == 1 || D == 128) &&
+    const bool fits = a.nchunk == 1 && rt <= (FP8 && (D == 128 || a.gchunk > 16) ? 1 : 2) &&
                       (int64_t)a.Lmax * D * (FP8 ? 1 : 2) < (1ll << 31) && ((uintptr_t)a.rope & 15) == 0;
     const int64_t longest = (int64_t)a.Lmax / a.splits;      // keys of a range at most
-    const bool left = D == 64 && (FP8 ? groups < 512 && (a.splits == 1 || longest > (a.defer_combine ? 3072 : 1024)) : a.gchunk > 16 && longest > 512);
+    const bool merges = a.splits > 1 && !a.defer_combine;
+    const bool left = D == 64 && (FP8 ? groups < 512 && (a.splits == 1 || longest > (merges ? 1024 : 3072))
+                                      : a.gchunk > 16 && longest > (merges ? 512 : 4096));
     if (!force && fits && !left) {
       const bool two = groups >= (D == 64 ? 640 : 512);
       auto launch = [&](auto rows16, auto multi) {
@@ -898,12 +902,11 @@ static int launch_rt(const AttnArgs& a, hipStream_t st) {
       };
       using One = std::integral_constant<int, 1>;
       using Two = std::integral_constant<int, 2>;
-      if constexpr (D == 128)
-        if (a.q_total > 1) {
-          if constexpr (!FP8)
-            if (rt == 2) return launch(Two{}, std::true_type{});
-          return launch(One{}, std::true_type{});
-        }
+      if (a.q_total > 1) {
+        if constexpr (!FP8 || D == 64)
+          if (rt == 2) return launch(Two{}, std::true_type{});
+        return launch(One{}, std::true_type{});
+      }
       if constexpr (!FP8)
         if (rt == 2) return launch(Two{}, std::false_type{});
       return launch(One{}, std::false_type{});

@@ -147,11 +147,11 @@ def test_options(d, fp8, opt):
     _case(d, fp8, 96, 96, [0, 63, 64, 200, 256, 777, 1023], 1, **{**opt, "defer": False})
 
 
-SEVERAL = [(4, 4, 9), (8, 2, 4), (1, 1, 3), (2, 2, 16), (8, 2, 7), (16, 1, 2), (60, 60, 5)]
+SEVERAL = [(4, 4, 9), (8, 2, 4), (1, 1, 3), (2, 2, 16), (8, 2, 7), (16, 1, 2), (60, 60, 5), (240, 60, 6), (24, 1, 3)]
 
 
 # (two row tiles of e5m2 with heads of 128 take the form that widens them: more exact than one token's)
-@pytest.mark.parametrize("d,fp8,hq,hkv,n", [(d, fp8, *c) for d in (128,) for fp8 in (False, True) for c in SEVERAL
+@pytest.mark.parametrize("d,fp8,hq,hkv,n", [(d, fp8, *c) for d in (64, 128) for fp8 in (False, True) for c in SEVERAL
                                             if not (fp8 and d == 128 and c[0] // c[1] * c[2] > 16)])
 @pytest.mark.parametrize("interleaved", [False, True])
 def test_several_tokens_round_as_one_after_the_other(d, fp8, hq, hkv, n, interleaved):
@@ -183,10 +183,10 @@ def test_several_tokens_round_as_one_after_the_other(d, fp8, hq, hkv, n, interle
     assert torch.equal(many, steps)
 
 
-# (heads of 64 come here in e5m2 caches of one range from 512 pairs on, with more than 16 to a group in ranges of 512 keys at most)
+# (heads of 64 in an e5m2 cache of one range come here from 512 pairs on)
 @pytest.mark.parametrize("d,fp8,hq,hkv,b,splits", [
     (d, fp8, *c, splits) for d in (64, 128) for fp8 in (False, True) for c in [(8, 2, 2), (40, 40, 2), (40, 40, 16), (40, 2, 3)]
-    for splits in (1, 2) if not (d == 64 and splits == 1 and (c[1] * c[2] < 512 if fp8 else c[0] > 16 * c[1]))])
+    for splits in (1, 2) if not (fp8 and d == 64 and splits == 1 and c[1] * c[2] < 512)])
 def test_weights_far_below_the_largest_keep_their_bits(d, fp8, hq, hkv, b, splits):
     """The first key takes nearly all of the weight, and the values of the first 64 keys are zero: the result is the sum over all the
     others, whose weights are e^-16 of the largest"""

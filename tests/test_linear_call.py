@@ -71,7 +71,28 @@ def test_same_bits(both, qname, n, k, rows):
         a, b, took = both(lin, x)
         assert _same(a, b) and took == (rows <= (128 if qname == "q6_k" else 256))
         a, b, took = both(lin, x.view(1, rows, k))
-        assert _same(a, b) and a.shape == (1, rows, n)
+        assert _same(a, b) and a.shape == (1, rows, n) and took == (rows <= (128 if qname == "q6_k" else 256))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", [torch.enable_grad, torch.no_grad, torch.inference_mode])
+@pytest.mark.parametrize("rows", [1, 18, 100])
+def test_views_take_the_native_call(both, mode, rows):
+    """What a model passes: hidden states of three dimensions, which are flattened by a view, and pieces of larger tensors"""
+    lin = _linear("sym_int4", 128, 512)
+    with mode():
+        wide = torch.randn(2, rows, 1024, device="cuda", dtype=torch.float16)
+        for x in (wide[:1, :, :512].contiguous(), wide[:, :, 512:].contiguous(), wide[0, :, :512], wide.view(-1, 512)[rows:2 * rows],
+                  (wide[:1] * 2).view(1, 2 * rows, 512)):
+            a, b, took = both(lin, x)
+            assert took and _same(a, b) and a.shape == (*x.shape[:-1], 128)
+    with torch.autograd.forward_ad.dual_level():
+        x = torch.randn(1, rows, 512, device="cuda", dtype=torch.float16)
+        a, b, took = both(lin, torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)))
+        assert not took and _same(a, b)
+    x = torch.randn(1, rows, 512, device="cuda", dtype=torch.float16, requires_grad=True)
+    a, b, took = both(lin, x * 1)
+    assert not took and _same(a, b) and a.requires_grad == b.requires_grad
 
 
 @pytest.mark.gpu

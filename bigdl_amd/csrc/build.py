@@ -1,14 +1,15 @@
-"""Builds the two native libraries in-tree.
+"""Builds the native libraries in-tree.
 
   bigdl_amd/lib/libbigdl_host.so   g++  -O3 -fopenmp   (quantizers, re-layout, CPU matmul)
   bigdl_amd/lib/libbigdl_hip.so    hipcc --offload-arch=gfx950  (all device kernels + decode engine)
   bigdl_amd/lib/libbigdl_ragged.so hipcc --offload-arch=gfx950  (csrc/ragged: the kernels of the ragged engine; a library
                                    of its own so that a checkout without built files that only serves such a model
                                    compiles only these few translation units, see ops/ragged.py::build)
-  bigdl_amd/lib/bigdl_linear_call.so  g++, against PyTorch's headers  (csrc/torch_ext: the host side of a linear's call as a
-                                   Python module; without it the same calls are made from Python)
+  bigdl_amd/lib/bigdl_linear_call.<Python and PyTorch build>.so  g++, against PyTorch's headers  (csrc/torch_ext: the host side of a
+                                   linear's call as a Python module; without it the same calls are made from Python, so
+                                   it comes last and may fail)
 
-The first two expose a plain C ABI and are loaded with ctypes, so neither needs the PyTorch
+The others expose a plain C ABI and are loaded with ctypes, so none of them needs the PyTorch
 headers: a full rebuild is a few seconds per file and hipcc cross-compiles gfx950
 without a GPU present.  Objects are cached by source mtime under build/.
 """
@@ -103,26 +104,34 @@ def build_ragged(force=False) -> Path:
     return ragged.build(force=force)
 
 
-def build_calls(force=False) -> Path:
-    out, src = LIB / "bigdl_linear_call.so", CSRC / "torch_ext" / "linear_call.cpp"
-    if force or _newer(src, out, [Path(__file__)]):
+def build_calls(force=False) -> Path | None:
+    """None (and a line on stderr) where this PyTorch cannot be built against: no headers, no ROCm"""
+    try:
         import sysconfig
 
         import torch
-        base = Path(torch.__file__).resolve().parent
-        include = [sysconfig.get_paths()["include"], base / "include", base / "include" / "torch" / "csrc" / "api" / "include",
-                   Path(os.environ.get("ROCM_PATH", "/opt/rocm")) / "include"]
-        LIB.mkdir(exist_ok=True)
-        _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1",
-              f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{p}" for p in include), "-o", str(out), str(src),
-              f"-L{base / 'lib'}", "-lc10", "-ltorch_cpu", "-ltorch_python", "-lc10_hip"])
-    return out
+
+        from ..ops.hip import linear_call_path
+        out, src = linear_call_path(), CSRC / "torch_ext" / "linear_call.cpp"
+        if force or _newer(src, out, [Path(__file__)]):
+            base = Path(torch.__file__).resolve().parent
+            include = [sysconfig.get_paths()["include"], base / "include", base / "include" / "torch" / "csrc" / "api" / "include",
+                       Path(os.environ.get("ROCM_PATH", "/opt/rocm")) / "include"]
+            out.parent.mkdir(exist_ok=True)
+            _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1",
+                  f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{p}" for p in include), "-o", str(out), str(src),
+                  f"-L{base / 'lib'}", "-lc10", "-ltorch_cpu", "-ltorch_python", "-lc10_hip"])
+        return out
+    except (ImportError, OSError, RuntimeError, AttributeError) as e:
+        sys.stderr.write(f"the native linear call is left out: {e}\n")
+        return None
 
 
 def build_all(jobs=8, force=False):
     build_ragged(force)
+    built = build_host(jobs, force), build_hip(jobs, force)
     build_calls(force)
-    return build_host(jobs, force), build_hip(jobs, force)
+    return built
 
 
 if __name__ == "__main__":

@@ -11,9 +11,46 @@ CALL = (64, 256, Q.SYM_INT4, 64 * 256 // 2 + 64 * 8 * 2, 16, 256)
 
 
 def _module():
-    path = hip.Path(hip.__file__).resolve().parent.parent / "lib" / "bigdl_linear_call.so"
-    if not path.exists():
+    if not hip.linear_call_path().exists():
         pytest.skip("not built")
+
+
+@pytest.fixture()
+def fresh():
+    hip.linear_call.cache_clear()
+    yield
+    hip.linear_call.cache_clear()
+
+
+@pytest.mark.parametrize("content", [None, b"", b"not a library"], ids=["missing", "empty", "text"])
+def test_a_module_that_does_not_load_leaves_the_calls_to_python(monkeypatch, tmp_path, fresh, content, recwarn):
+    path = tmp_path / "bigdl_linear_call.so"
+    if content is not None:
+        path.write_bytes(content)
+    monkeypatch.setattr(hip, "linear_call_path", lambda: path)
+    assert hip.linear_call()(torch.zeros(1, 256).half(), torch.zeros(CALL[3], dtype=torch.uint8), *CALL) is None
+    assert hip.linear_call() is hip.linear_call()
+    assert len([w for w in recwarn if "linear_call" in str(w.message)]) == (content is not None)
+
+
+def test_a_module_for_another_pytorch_is_not_looked_at(monkeypatch):
+    path = hip.linear_call_path()
+    monkeypatch.setattr(torch, "__version__", "1.0.0")
+    assert hip.linear_call_path() != path and hip.linear_call_path().parent == path.parent
+
+
+def test_the_other_libraries_are_built_where_this_one_cannot_be(monkeypatch, capsys):
+    from bigdl_amd.csrc import build
+    done = []
+    for name in ("ragged", "host", "hip"):
+        monkeypatch.setattr(build, f"build_{name}", lambda *args, name=name, **kw: done.append(name) or name)
+
+    def fails(cmd):
+        raise RuntimeError("no such header")
+
+    monkeypatch.setattr(build, "_run", fails)
+    assert build.build_all(force=True) == ("host", "hip") and done == ["ragged", "host", "hip"]
+    assert "no such header" in capsys.readouterr().err
 
 
 def test_declines_what_is_not_on_the_gpu():

@@ -48,10 +48,10 @@ constexpr int prompt_lds_tiles(int BM, int BN, int NW, int MTW, int NTW) {
 constexpr int waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
 constexpr int waitcnt_vm_lgkm0(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4); }
 
-// x / (1 + e^-x), rounded as the division: the divisor is 1 at least, so the scaling that a division begins with is not needed, only one
-// correction of the quotient (infinite or NaN where that has nothing to correct)
+// x / (1 + e^-x) by a reciprocal and one correction of the quotient (infinite or NaN where that has nothing to correct).  Both are taken as
+// quarters: the divisor is then 1/4 at least and its reciprocal never below 2^-126, where it would be flushed to zero (x near -88)
 __device__ __forceinline__ float prompt_silu(float x) {
-  const float d = 1.0f + __expf(-x), r = __builtin_amdgcn_rcpf(d), q = x * r, e = fmaf(-q, d, x);
+  const float n = 0.25f * x, d = fmaf(0.25f, __expf(-x), 0.25f), r = __builtin_amdgcn_rcpf(d), q = n * r, e = fmaf(-q, d, n);
   return e == e ? fmaf(e, r, q) : q;
 }
 

@@ -82,3 +82,22 @@ def test_pairs(hip, cfg, act):
     eu = e * u.abs() + 2.0 ** -10 * (xd.abs() @ wu.abs().t())
     bound = 1.13 * eg * u.abs() + f(g).abs() * eu + 1.13 * eg * eu + e * ref.abs() + 1e-4
     assert ((out.double().cpu() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_gate_where_the_exponential_is_largest(hip, dtype):
+    """silu(g) u for g down to where 1 + e^-g overflows: the products of zero rows are the biases"""
+    n, k, qt = 256, 256, Q.SYM_INT4
+    dev, _ = _weight(n, k, qt, 3)
+    g = torch.linspace(-100, 100, n - 64).bfloat16().half()
+    g = torch.cat([torch.arange(-96, -80, 0.25).bfloat16().half(), g])
+    u = torch.full((n,), 2.0 ** 15).half()
+    out = hip.gemm_prompt_pair(torch.zeros(300, k, dtype=torch.float16, device="cuda"), dev, dev, qt, n, k, bias=g.cuda(), bias2=u.cuda(),
+                               act="silu", out_dtype=dtype)
+    ref = g.double() / (1 + torch.exp(-g.double())) * 2.0 ** 15
+    # e^-g overflows fp32 below -88.72, which leaves zero; else the result's rounding, e^x to 2^-17 at 2^7, fp16's smallest steps
+    ref = torch.where(g.double() < -88.72, 0.0, ref).clamp(-torch.finfo(dtype).max, torch.finfo(dtype).max)
+    bound = (2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7) * ref.abs() + (2.0 ** -24 if dtype == torch.float16 else 1e-38)
+    ok = (out.double().cpu() - ref).abs() <= bound
+    big = ref.abs() >= torch.finfo(dtype).max                 # (beyond fp16: infinite)
+    assert (ok | big).all(), (g[~(ok | big).all(0)], out[0].cpu()[~(ok | big).all(0)])

@@ -31,69 +31,79 @@ static int prompt_dispatch(const GemmArgs& a, int qtype, int cfg, hipStream_t st
 
 // Tile configurations (gemm_prompt_launch<QT> instantiates them in this order).  us per 128-deep k tile and us around the loop (first
 // requests, epilogue) of 256 tiles at once, one a CU, fitted with the constants below to 2500 launches of 310 random products (M 257 -
-// 8000, N 1024 - 14336, K 512 - 14336, pairs among them, weights out of the caches) in 10 formats: off by 4 % on average, and the plan
-// taken is 0.2 % slower than the fastest of all plans on average.  With the first three configurations alone the fastest is 4 %
-// slower: 1024 x 8192 x 8192 is 119 us in 256 x 128 tiles, 124 in 256 x 256 with 2 K splits; 1696 x 6544 x 4736 87 in 192 x 256, 96 in
-// 256 x 192.  128 x 256, 192 x 192 and 128 x 192 tiles were measured too: 0.1 % on average.
+// 8000, N 1024 - 14336, K 512 - 14336, pairs among them, weights out of the caches) in 10 formats: off by 4 % on average for one launch
+// by itself.  Launches in a row, as a prompt runs them, are slower (power): of 332 other random products in 6 formats the estimate is 5 %
+// low in the middle, 16 % above 2000 rows (1024 x 12288 x 4096 71 for 90 us); the plan taken is then 0.5 % slower than the fastest of all
+// on average, 11 % at most.  With the first three configurations alone the fastest is 4 % slower: 1024 x 8192 x 8192 is 119 us in
+// 256 x 128 tiles, 124 in 256 x 256 with 2 K splits; 1696 x 6544 x 4736 87 in 192 x 256, 96 in 256 x 192.  128 x 256, 192 x 192 and
+// 128 x 192 tiles were measured too: 0.1 % on average.
 struct PromptCfg { int bm, bn; float kt_us, tile_us; };
 static const PromptCfg kPromptCfgs[PROMPT_NCFG] = {{256, 256, 2.285f, 6.80f}, {256, 192, 1.986f, 5.78f}, {128, 128, 0.806f, 2.46f},
                                                    {256, 128, 1.407f, 4.53f}, {192, 256, 1.853f, 5.72f}, {192, 128, 1.210f, 3.86f}};
+// time of a k tile against the mean of the formats that plans are made with (the size of their slabs is asked for without a format; with
+// the format's own the plan of the 332 products is 0.6 % slower than the fastest)
+constexpr double PLAN_FMT = 1.1;
 
 struct PromptPlan { int cfg, splitk, kt_per_split; double us; };
 static int g_force_cfg = -1, g_force_sk = 0;         // bigdl_gemm_prompt_force (tests / sweeps)
 
-// The fastest plan by its estimated time: turns of 256 tiles, each its k tiles and its first requests and epilogue; K splits add the
-// fp32 slabs' traffic and the reduce launch.  128 x 128 tiles run two to a CU where there are more than 256 (a lone one is 1.24 times
-// as long, not half as long, as two).
+// Turns of 256 tiles, each its k tiles and its first requests and epilogue; K splits add the fp32 slabs' traffic and the reduce launch.
+// 128 x 128 tiles run two to a CU where there are more than 256 (a lone one is 1.24 times as long, not half as long, as two).
+static double plan_us(int M, int N, bool pair, int cfg, int splitk, int kt_per_split, double fmt) {
+  const PromptCfg& pc = kPromptCfgs[cfg];
+  const int bno = pair ? pc.bn / 2 : pc.bn;
+  const int64_t tiles = (int64_t)((M + pc.bm - 1) / pc.bm) * ((N + bno - 1) / bno), turns = (tiles * splitk + 255) / 256;
+  const double lone = pc.bm == 128 && turns == 1 ? 1.24 : 1.0;
+  double us = 1.3 + (double)turns * (pc.kt_us * (pair ? 1.02 : 1.0) * fmt * lone * kt_per_split + pc.tile_us * (pair ? 1.15 : 1.0));
+  if (splitk > 1) us += 5.2 + 1.07e-6 * splitk * (double)M * N;
+  return us;
+}
+
+// The fastest plan by its estimated time.
 // pair: the gate / up form (two products per output column: blocks cover bn / 2 output columns, no K split)
-// forced_cfg >= 0, forced_sk > 0: only plans of these;  fmt: time of a k tile against the mean of the formats
-static PromptPlan prompt_plan_of(int M, int N, int K, bool pair, int forced_cfg, int forced_sk, double fmt) {
+// forced_cfg >= 0, forced_sk > 0: only plans of these
+static PromptPlan prompt_plan_of(int M, int N, int K, bool pair, int forced_cfg, int forced_sk) {
   const int KT = K >> 7;
   PromptPlan best = {0, 1, KT, 1e300};
   for (int c = 0; c < PROMPT_NCFG; ++c) {
     if (forced_cfg >= 0 && c != forced_cfg) continue;
-    const PromptCfg& pc = kPromptCfgs[c];
-    const int bno = pair ? pc.bn / 2 : pc.bn;
-    const int64_t tiles = (int64_t)((M + pc.bm - 1) / pc.bm) * ((N + bno - 1) / bno);
     for (int sk = 1; sk <= (pair ? 1 : 8); ++sk) {
       if (forced_sk ? sk != forced_sk : (sk > 1 && KT / sk < 6)) continue;
       if (sk > KT) continue;
       const int per = (KT + sk - 1) / sk, rsk = (KT + per - 1) / per;
-      const int64_t turns = (tiles * rsk + 255) / 256;
-      const double lone = pc.bm == 128 && turns == 1 ? 1.24 : 1.0;
-      double us = 1.3 + (double)turns * (pc.kt_us * (pair ? 1.02 : 1.0) * fmt * lone * per + pc.tile_us * (pair ? 1.15 : 1.0));
-      if (rsk > 1) us += 5.2 + 1.07e-6 * rsk * (double)M * N;
+      const double us = plan_us(M, N, pair, c, rsk, per, PLAN_FMT);
       // (equal within the estimate: the earlier configuration, the larger tile)
       if (us < (best.cfg == c ? 1.0 : 0.985) * best.us) best = {c, rsk, per, us};
     }
   }
   return best;
 }
-// (one plan for all formats: the size of its slabs is asked for without one)
 static PromptPlan prompt_plan(int M, int N, int K, bool pair = false) {
   static const int env_cfg = getenv("BIGDL_PROMPT_CFG") ? atoi(getenv("BIGDL_PROMPT_CFG")) : -1;
   static const int env_sk = getenv("BIGDL_PROMPT_SPLITK") ? atoi(getenv("BIGDL_PROMPT_SPLITK")) : 0;
-  return prompt_plan_of(M, N, K, pair, g_force_cfg >= 0 ? g_force_cfg : env_cfg, g_force_sk > 0 ? g_force_sk : env_sk, 1.1);
+  return prompt_plan_of(M, N, K, pair, g_force_cfg >= 0 ? g_force_cfg : env_cfg, g_force_sk > 0 ? g_force_sk : env_sk);
 }
 
-// The time in us of the plan that nothing forces (callers remember the choice by the product's sizes), for the choice between this
-// kernel and others at 257 - 512 rows.
+// The time in us, in this format, of the plan that is launched where nothing forces another (callers remember the choice by the product's
+// sizes), for the choice between this kernel and others at 257 - 512 rows.  Large tiles of many splits are 10 - 15 % over the estimate: that
+// is counted here, but not in the choice of the plan (of the 332 products above it would be 0.8 % behind the fastest instead of 0.5:
+// 512 x 4096 x 11008 59.3 us in four splits of 256 x 128, 63.6 in those of 128 x 128 that it would take).
 double prompt_us(int M, int N, int K, int qtype, bool pair) {
-  float fmt = 1.0f;                                    // sym_int4
+  double fmt = 1.0;                                    // sym_int4
   switch (qtype) {
-    case Q_ASYM_INT4: case Q_WOQ_INT4: fmt = 1.08f; break;
-    case Q_FP4: fmt = 1.12f; break;
-    case Q_NF4: fmt = 1.26f; break;
-    case Q_SYM_INT5: fmt = 1.26f; break;
-    case Q_ASYM_INT5: fmt = 1.30f; break;
-    case Q_FP6: fmt = 1.39f; break;
-    case Q_SYM_INT8: fmt = 1.12f; break;
-    case Q_FP8_E4M3: fmt = 1.16f; break;
-    case Q_FP8_E5M2: fmt = 1.08f; break;
+    case Q_ASYM_INT4: case Q_WOQ_INT4: fmt = 1.08; break;
+    case Q_FP4: fmt = 1.12; break;
+    case Q_NF4: fmt = 1.26; break;
+    case Q_SYM_INT5: fmt = 1.26; break;
+    case Q_ASYM_INT5: fmt = 1.30; break;
+    case Q_FP6: fmt = 1.39; break;
+    case Q_SYM_INT8: fmt = 1.12; break;
+    case Q_FP8_E4M3: fmt = 1.16; break;
+    case Q_FP8_E5M2: fmt = 1.08; break;
     default: break;
   }
-  const PromptPlan p = prompt_plan_of(M, N, K, pair, -1, 0, fmt);
-  return p.splitk >= 4 && p.cfg != 2 ? 1.12 * p.us : p.us;      // (large tiles of many splits: 10 - 15 % over the estimate)
+  const PromptPlan p = prompt_plan_of(M, N, K, pair, -1, 0);
+  return (p.splitk >= 4 && p.cfg != 2 ? 1.12 : 1.0) * plan_us(M, N, pair, p.cfg, p.splitk, p.kt_per_split, fmt);
 }
 
 // the staged 16-bit epilogue covers this output; otherwise one fp32 slab + the reduce kernel
@@ -129,6 +139,11 @@ extern "C" int bigdl_gemm_prompt_plan(int M, int N, int K, int* cfg, int* splitk
   if (cfg) *cfg = pl.cfg;
   if (splitk) *splitk = pl.splitk;
   return 0;
+}
+
+// the estimate that the choice of the kernel goes by, for its tests
+extern "C" double bigdl_gemm_prompt_us(int M, int N, int K, int qtype, int pair) {
+  return prompt_us(M, N, K, t16_kernel_qtype(qtype), pair != 0);
 }
 
 // Gate / up pair in one launch: out[M, N] = act(x W^T + bias) * (x W2^T + bias2), both weights [N, K] of one format,

@@ -1,10 +1,8 @@
 """Decode attention alone at a serving batch: ``--layers`` distinct e5m2 caches (so nothing is re-read from the
 memory-side cache), one launch per cache inside a hipGraph, microseconds per launch and TB/s of K / V bytes.
-    PYTHONPATH=. python benchmark/attn_decode_probe.py --batch 64 --ctx 1024 [--no-rope] [--ablate 1]
-``--no-rope``: q already rotated and the new key / value already in the cache (the kernel without its append prologue).
-``--ablate 1``: the kernel issues its K / V loads and skips the products (the load pattern's own rate)."""
+    PYTHONPATH=. python benchmark/attn_decode_probe.py --batch 64 --ctx 1024 [--no-rope]
+``--no-rope``: q already rotated and the new key / value already in the cache (the kernel without its append prologue)."""
 import argparse
-import ctypes
 import json
 import math
 
@@ -23,14 +21,10 @@ if __name__ == "__main__":
     ap.add_argument("--splits", type=int, default=1)
     ap.add_argument("--no-rope", action="store_true")
     ap.add_argument("--separate-rope", action="store_true", help="rope_append kernel + attention without the prologue")
-    ap.add_argument("--ablate", type=int, default=0)
     args = ap.parse_args()
     b, hq, hkv, d = args.batch, args.heads, args.kv_heads, 128
     lmax = (args.ctx + 64 + 255) // 256 * 256
     dev = "cuda"
-    if args.ablate:
-        hip.lib().bigdl_attn_set_ablation.argtypes = [ctypes.c_int]
-        hip.lib().bigdl_attn_set_ablation(args.ablate)
     kcs = [torch.randint(0, 120, (b, hkv, lmax, d), dtype=torch.uint8, device=dev) for _ in range(args.layers)]
     vcs = [torch.randint(0, 120, (b, hkv, d, lmax), dtype=torch.uint8, device=dev) for _ in range(args.layers)]
     qkv = (torch.randn(b, (hq + 2 * hkv) * d, device=dev) * 0.5).half()
@@ -66,4 +60,4 @@ if __name__ == "__main__":
     us = e0.elapsed_time(e1) * 1e3 / (args.reps * args.layers)
     nbytes = 2 * b * hkv * (args.ctx + 1) * d
     print(json.dumps({"batch": b, "heads": hq, "kv_heads": hkv, "ctx": args.ctx, "splits": args.splits, "rope_in_kernel": not (args.no_rope or args.separate_rope), "separate_rope": args.separate_rope,
-                      "ablate": args.ablate, "us_per_launch": round(us, 2), "kv_tb_per_s": round(nbytes / us / 1e6, 3)}), flush=True)
+                      "us_per_launch": round(us, 2), "kv_tb_per_s": round(nbytes / us / 1e6, 3)}), flush=True)

@@ -25,7 +25,6 @@
 // with keys {8g+q} and {8g+4+q} so that lane group g ends up owning 8 consecutive keys, which
 // is exactly the k-slice its P^T fragment must hold for the O^T product.
 #include "common.h"
-#include <stdlib.h>
 #include <type_traits>
 
 namespace bigdl {
@@ -53,7 +52,6 @@ struct AttnArgs {
   int rot, interleaved, rope_max_pos;
   int defer_combine;     // 1: stop after writing the per-split partials (the consumer GEMV combines them)
   int nchunk, gchunk;    // query-head chunks per kv head and heads per chunk (1, Hq/Hkv unless Hq/Hkv > 32)
-  int ablate;            // measurement builds only (bigdl_attn_set_ablation): 1 = K / V loads without the products
   int frag_mt;             // out in fragment order of so many 16-row tiles (0: rows), for the product that reads it
 };
 // place of (row m, column c) of the output
@@ -168,16 +166,15 @@ __device__ __forceinline__ void combine_splits(const AttnArgs& a, int bh, int he
 }
 
 // D = head dim (multiple of 32), RT = number of 16-row tiles, KW = keys per wavefront per iteration.
-// KW = 64 (e5m2 caches, D % 128 == 0): every lane loads 16 bytes of a key row / of a V^T channel row instead of 8, i.e.
-// half as many load instructions and 64-byte instead of 32-byte contiguous pieces per 4 lanes.  With 8-byte pieces the
-// e5m2 path is bound by the number of memory instructions, not by bytes (batch 64, 1024 keys: 184 us per layer where
-// the fp16 cache needs 258 us for twice the bytes).  The MFMA k index <-> head channel assignment is free as long as
-// Q and K agree, so lane group g takes channels [16 (g + 4 c2), +16) of a row for the k-steps 2 c2 and 2 c2 + 1.
+// KW = 64 (e5m2 heads of 256): every lane loads 16 bytes of a key row / of a V^T channel row instead of 8, i.e. half as many load
+// instructions and 64-byte instead of 32-byte contiguous pieces per 4 lanes (in four wavefronts; 32 keys in eight -> 64 in four: 64 x 8 heads,
+// 1000 keys 83 -> 72 us, one sequence of 4, 4000 keys in 16 ranges 13.1 -> 11.6).  The MFMA k index <-> head channel assignment is free as
+// long as Q and K agree, so lane group g takes channels [16 (g + 4 c2), +16) of a row for the k-steps 2 c2 and 2 c2 + 1.
 //
 // The leading arguments arrive in scalar registers (build flag, see gemv_kernel.h): the length is requested at once, and the
 // rest of the arguments returns along with it.
-template <int D, bool FP8, int RT, int KW, bool I4, int NWT = ATT_NW, int MINW = 1>
-__global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* p_past, _Float16* p_qkv, int p_ld, int p_q_total,
+template <int D, bool FP8, int RT, int KW, bool I4, int NWT = ATT_NW>
+__global__ __launch_bounds__(NWT * 64) void attn_decode_kernel(const int* p_past, _Float16* p_qkv, int p_ld, int p_q_total,
                                                                      int p_splits, int p_Hq, int p_Hkv, int p_nchunk, int p_gchunk,
                                                                      int p_Lmax, void* p_kc, AttnArgs a) {
   a.past_len = p_past; a.qkv = p_qkv; a.ld = p_ld; a.q_total = p_q_total; a.splits = p_splits; a.Hq = p_Hq; a.Hkv = p_Hkv;
@@ -189,17 +186,16 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
   constexpr int NU = KW / 16;          // 16-key score tiles per wavefront
   constexpr int KL = KW / 4;           // consecutive keys per lane
   constexpr bool WIDE = KW == 64;
-  // e5m2 bytes straight into the fp8 matrix instruction (below): the many-keys-per-workgroup form.  The latency-bound
-  // batch-1 form keeps fp16 fragments: splitting q into two e4m3 terms in its prologue cost 0.2 us per launch there.
+  // e5m2 bytes straight into the fp8 matrix instruction (below)
   constexpr bool F8M = FP8 && WIDE;
   static_assert(!WIDE || (FP8 && D % 128 == 0), "16-byte fragments: e5m2 cache, rotate-half partner in k-step c + DC/2");
   static_assert(!I4 || (!FP8 && KW == 32), "int4 caches: 32 keys per wavefront");
-  // (fp16 heads of 64 and 128 with one new token are attn_decode_stream.h's: the figures are of when they came here.)
+  // (Heads of 64 and 128 are mostly attn_decode_stream.h's: the figures for them are of when they came here.)
   // The next block in flight, the new value stored with its block and q requested ahead of the append: one row tile and heads of
-  // up to 128 channels.  fp16 caches, 12 sequences x 8 heads of 128, 6000 keys: 113 -> 102 us.  In a step, where caches are cold:
-  // 8 layers of 4 kv heads of 64, 4 tokens, 45 / 1900 keys 849 -> 840 / 930 -> 922 us; 16 sequences x 32 heads of 128, 1000 keys
-  // 1168 -> 1141 (2 layers).  Heads of 256 spilled (4 layers of 8 heads, 500 keys 676 -> 753 us), two row tiles lost registers (20
-  // query heads a group, 1900 keys 11.3 -> 12.1 us a launch).  e5m2 caches take the block in flight (in the 32-key form: 4 heads of
+  // up to 128 channels (in fp16 caches: heads of 96).  fp16 caches, 12 sequences x 8 heads of 128, 6000 keys: 113 -> 102 us.  In a step,
+  // where caches are cold: 8 layers of 4 kv heads of 64, 4 tokens, 45 / 1900 keys 849 -> 840 / 930 -> 922 us; 16 sequences x 32 heads of
+  // 128, 1000 keys 1168 -> 1141 (2 layers).  Heads of 256 spilled (4 layers of 8 heads, 500 keys 676 -> 753 us), two row tiles lost registers
+  // (20 query heads a group, 1900 keys 11.3 -> 12.1 us a launch).  e5m2 caches take the block in flight (in the 32-key form: 4 heads of
   // 64, 1900 keys in eight ranges 5.7 -> 5.3 us) and nothing else: their 8-byte pieces would not make whole 64 bytes of a
   // value column, and q ahead cost 4 - 8 % with several key ranges (14.0 -> 15.1 us).
   constexpr bool AHEAD = RT == 1 && D <= 128;
@@ -593,19 +589,6 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
       for (int d = 0; d < DT; ++d) vf[d][0] = widen(fr.v[d]);
     }
 
-    if constexpr (F8M) {
-      if (a.ablate & 1) {
-#pragma unroll
-        for (int u = 0; u < NU; ++u)
-#pragma unroll
-          for (int c = 0; c < DC; ++c) asm volatile("" ::"v"(kr.w[u][c].x), "v"(kr.w[u][c].y));
-#pragma unroll
-        for (int d = 0; d < DT; ++d)
-#pragma unroll
-          for (int h = 0; h < KL / 8; ++h) asm volatile("" ::"v"(vr.w[d][h].x), "v"(vr.w[d][h].y));
-        return;
-      }
-    }
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
       // lane (row rr, g): tile u, register q  <->  key kb + KL*g + 4*u + q
@@ -826,20 +809,20 @@ __global__ __launch_bounds__(NWT * 64, MINW) void attn_decode_kernel(const int* 
 #include "attn_decode_stream.h"
 namespace bigdl {
 
-template <int D, bool FP8, int RT, int KW, bool I4 = false, int NWT = ATT_NW, int MINW = 1>
-static int launch_one(const AttnArgs& a, size_t, hipStream_t st) {
+template <int D, bool FP8, int RT, int KW, bool I4 = false, int NWT = ATT_NW>
+static int launch_one(const AttnArgs& a, hipStream_t st) {
   const dim3 grid(a.splits, a.Hkv * a.nchunk, a.B), block(NWT * 64);
   const int rows = a.gchunk * a.q_cnt;
   const size_t smem = (size_t)(NWT * RT * 16 * 2 + NWT * rows * D) * 4 + 16;
   // more than 64 KiB of dynamic LDS has to be requested explicitly (once per kernel)
   static bool attr = false;
   if (!attr && smem > 65536) {
-    if (hipFuncSetAttribute((const void*)attn_decode_kernel<D, FP8, RT, KW, I4, NWT, MINW>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    if (hipFuncSetAttribute((const void*)attn_decode_kernel<D, FP8, RT, KW, I4, NWT>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             160 * 1024) != hipSuccess)
       return -5;
     attr = true;
   }
-  hipLaunchKernelGGL((attn_decode_kernel<D, FP8, RT, KW, I4, NWT, MINW>), grid, block, smem, st, a.past_len, a.qkv, a.ld, a.q_total,
+  hipLaunchKernelGGL((attn_decode_kernel<D, FP8, RT, KW, I4, NWT>), grid, block, smem, st, a.past_len, a.qkv, a.ld, a.q_total,
                      a.splits, a.Hq, a.Hkv, a.nchunk, a.gchunk, a.Lmax, a.kc, a);
   return HIP_CHECK_LAUNCH();
 }
@@ -862,13 +845,11 @@ template <int D, bool FP8, bool I4 = false>
 static int launch_rt(const AttnArgs& a, hipStream_t st) {
   const int rows = a.gchunk * a.q_cnt;
   const int rt = (rows + 15) / 16;
-  const size_t smem = (size_t)(ATT_NW * rt * 16 * 2 + ATT_NW * rows * D) * 4 + 16;
   if constexpr (I4) {
-    if (rt == 1) return launch_one<D, false, 1, 32, true>(a, smem, st);
-    if (rt == 2) return launch_one<D, false, 2, 32, true>(a, smem, st);
+    if (rt == 1) return launch_one<D, false, 1, 32, true>(a, st);
+    if (rt == 2) return launch_one<D, false, 2, 32, true>(a, st);
     return -4;
   }
-  static const char* force = getenv("BIGDL_ATTN_KEYS");      // "32" / "64": the register form, with so many keys (measurements)
   // Heads of 64 or 128: the form whose K / V^T come through LDS in whole lines (attn_decode_stream.h).  One new token, us a launch,
   // caches cold, register form -> two / four wavefronts a workgroup, at (sequence, KV head, range) groups x keys a range:
   //   fp16 128:  32 x 40 7.2 -> 5.6 / 6.1     192 x 2000 50 -> 50 / 44    256 x 1100 36 -> 31 / 30    512 x 1100 68 -> 53 / 54    1024 x 1100 127 -> 101 / 106
@@ -888,12 +869,12 @@ static int launch_rt(const AttnArgs& a, hipStream_t st) {
   if constexpr (D == 64 || D == 128) {
     const int64_t groups = (int64_t)a.B * a.Hkv * a.splits;
     const bool fits = a.nchunk == 1 && rt <= (FP8 && (D == 128 || a.gchunk > 16) ? 1 : 2) &&
-                      (int64_t)a.Lmax * D * (FP8 ? 1 : 2) < (1ll << 31) && ((uintptr_t)a.rope & 15) == 0;
+                      (int64_t)a.Lmax * D * (FP8 ? 1 : 2) < (1ll << 31);      // (32-bit offsets into a head)
     const int64_t longest = (int64_t)a.Lmax / a.splits;      // keys of a range at most
     const bool merges = a.splits > 1 && !a.defer_combine;
     const bool left = D == 64 && (FP8 ? groups < 512 && (a.splits == 1 || longest > (merges ? 1024 : 3072))
                                       : a.gchunk > 16 && longest > (merges ? 512 : 4096));
-    if (!force && fits && !left) {
+    if (fits && !left) {
       const bool two = groups >= (D == 64 ? 640 : 512);
       auto launch = [&](auto rows16, auto multi) {
         constexpr int RT = decltype(rows16)::value;
@@ -913,34 +894,13 @@ static int launch_rt(const AttnArgs& a, hipStream_t st) {
     }
   }
   if (rt == 1) {
-    // 64 keys per wavefront (16-byte fragments).  With one KV split and fewer than 512 (sequence, head) pairs the
-    // workgroup has ATT_NW wavefronts; with several splits or 512 pairs and more it has four (below).
-    if constexpr (FP8 && D % 128 == 0) {
-      const bool wide = force ? atoi(force) == 64 : true;
-      // batched decode (512 or more (sequence, head) workgroups, one KV split): four-wavefront workgroups, so
-      // that two of them share a CU and one streams keys while the other is in its softmax / merge phase.  Measured
-      // on Llama-2-7B at 1024-token context: batch 64 9.36 -> 8.65 ms per step, batch 16 4.34 -> 4.20.  Tried on top
-      // and dropped: two-wavefront workgroups (8.94), keys / values kept as bytes in registers (no fewer live
-      // registers: 186 either way), a second register set that prefetches the next block (256 registers, 8.83).
-      static const char* nw4 = getenv("BIGDL_ATTN_NW4");           // "0" / "1": override for measurements
-      // Several KV splits (few pairs, each split a short key range): the same four-wavefront form, one 256-key pass
-      // per wavefront round instead of ATT_NW x 32 keys, and a four-way merge in LDS instead of an ATT_NW-way one.
-      // Measured per decode step on one MI355X, same box, 32-key ATT_NW-wavefront form -> this one: Llama-2-7B batch 1
-      // 1.551 -> 1.511 ms at 1024 keys, 1.875 -> 1.781 at 4096; Llama-3-8B 1.642 -> 1.612 / 1.834 -> 1.756;
-      // Qwen2-7B 1.557 -> 1.532 / 1.714 -> 1.637.  With ONE split and fewer than 512 pairs it loses (Llama-2-7B
-      // batch 2 at 1024 keys 1.857 -> 1.899), so that case keeps ATT_NW wavefronts.
-      const bool small = nw4 ? atoi(nw4) == 1 : (a.splits > 1 || (int64_t)a.B * a.Hkv * a.nchunk >= 512);
-      if constexpr (D == 128) {
-        static const char* occ = getenv("BIGDL_ATTN_OCC");         // wavefronts per SIMD the register budget allows
-        if (wide && small && occ && atoi(occ) == 3) return launch_one<D, FP8, 1, 64, false, 4, 3>(a, smem, st);
-        if (wide && small && occ && atoi(occ) == 4) return launch_one<D, FP8, 1, 64, false, 4, 4>(a, smem, st);
-      }
-      if (wide && small) return launch_one<D, FP8, 1, 64, false, 4, (D <= 128 ? 2 : 1)>(a, smem, st);
-      if (wide) return launch_one<D, FP8, 1, 64>(a, smem, st);
-    }
-    return launch_one<D, FP8, 1, 32>(a, smem, st);
+    // e5m2 heads of 256: 64 keys a wavefront (16-byte fragments), four wavefronts, so that two workgroups share a CU and one streams
+    // keys while the other is in its softmax or merge.  Eight -> four, us a launch: 64 x 8 heads, 1000 keys 89 -> 72, 16 x 8 34.8 -> 30.8,
+    // 4 x 16, 1500 keys in four ranges 25.0 -> 19.9, one sequence of one head, 1000 keys in four 18.5 -> 12.2.
+    if constexpr (FP8 && D == 256) return launch_one<D, FP8, 1, 64, false, 4>(a, st);
+    return launch_one<D, FP8, 1, 32>(a, st);          // (heads of 64 and 128 in fp16, of 128 in e5m2: those of 2 GiB and more)
   }
-  if (rt == 2) return launch_one<D, FP8, 2, 32>(a, smem, st);
+  if (rt == 2) return launch_one<D, FP8, 2, 32>(a, st);
   return -4;
 }
 
@@ -1020,9 +980,6 @@ __global__ __launch_bounds__(64) void rope_append_kernel(RopeAppendArgs a) {
 
 using namespace bigdl;
 
-static int g_attn_ablate = 0;
-extern "C" void bigdl_attn_set_ablation(int v) { g_attn_ablate = v; }
-
 // q tokens [q_off, q_off+q_cnt) of the q_total tokens appended this step; (Hq/Hkv)*q_cnt <= 32.
 // rope != null: q is rotated in registers, k is rotated and k/v appended to the caches by this launch
 // (requires q_off == 0 for the append; rot/2 % 32 == 0 unless interleaved).
@@ -1050,7 +1007,7 @@ extern "C" int bigdl_attn_decode(void* qkv, void* kc, void* vc, void* out, float
   a.rot = rope ? rot : (append ? 0 : -1); a.interleaved = interleaved;
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.ld = ld; a.Lmax = Lmax; a.splits = splits; a.window = window;
   a.q_total = q_total; a.q_off = q_off; a.q_cnt = q_cnt; a.defer_combine = defer_combine;
-  a.nchunk = nchunk; a.gchunk = gchunk; a.ablate = g_attn_ablate;
+  a.nchunk = nchunk; a.gchunk = gchunk;
   a.ks = (_Float16*)k_scale; a.vs = (_Float16*)v_scale;
   if (frag && ((Hq * D) & 127)) return -1;
   a.frag_mt = frag ? (B * q_total + 15) / 16 : 0;

@@ -148,6 +148,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
   }
   // ---- q, its rotation, the new key and value, then the first block (all without a branch: what arrives is counted) ----
   half8 qraw[RT][DC];
+  typedef float __attribute__((ext_vector_type(4), aligned(8))) pairs2;      // two pairs of a table that may start anywhere
   float4v cs[RT][DC][2];     // [2 i], [2 i + 1]: cosine and sine of 8 / 2 channel pairs each (without a rotation: any readable numbers)
   int row[RT];
 #pragma unroll
@@ -162,8 +163,8 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
     for (int i = 0; i < DC; ++i) {
       const int at = a.interleaved ? (chan(i, g) < a.rot ? chan(i, g) : 0) : 2 * chan(i >> 1, g) + 8 * (i & 1);
       const float* p = tab + (rotate ? at : 0);
-      cs[t][i][0] = *(const float4v*)p;
-      cs[t][i][1] = *(const float4v*)(p + 4);
+      cs[t][i][0] = *(const pairs2*)p;
+      cs[t][i][1] = *(const pairs2*)(p + 4);
     }
   }
   const _Float16 x0 = krow[i0], x1 = krow[i1];

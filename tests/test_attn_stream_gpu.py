@@ -214,3 +214,49 @@ def test_weights_far_below_the_largest_keep_their_bits(d, fp8, hq, hkv, b, split
         worst = max(worst, ((out[i].cpu().double().view(hq, d) - ref).norm() / ref.norm()).item())
     # as in _case; the error of the largest score, 16, is in all of the result: 16 x 2^-11 + 2 x 2^-11, or 16 / 4 x 2^-8 + 2^-8
     assert worst < (2e-2 if fp8 and d == 128 else 9e-3), worst
+
+
+def _plain(d, fp8, qkv, kd, vd, past, table, hq, hkv):
+    b = qkv.shape[0]
+    out = torch.empty(b, hq * d, dtype=torch.float16, device="cuda")
+    ws = torch.empty(hip.attn_decode_ws_floats(b, hq, hkv, 1, d, 1), dtype=torch.float32, device="cuda")
+    counters = torch.zeros(hip.attn_decode_counters(b, hq, hkv), dtype=torch.int32, device="cuda")
+    hip.attn_decode(qkv, kd, vd, torch.full((b,), past, dtype=torch.int32, device="cuda"), out, ws, counters, n_heads=hq, n_kv_heads=hkv,
+                    head_dim=d, q_len=1, batch=b, scale=d ** -0.5, splits=1, rope_table=table)
+    return out
+
+
+def _small_cache(d, fp8, hkv, lmax):
+    k, v = torch.randn(1, hkv, lmax, d, device="cuda").half(), torch.randn(1, hkv, d, lmax, device="cuda").half()
+    return (t.to(torch.float8_e5m2).view(torch.uint8) if fp8 else t for t in (k, v))
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("d", [64, 128])
+def test_a_rope_table_may_start_anywhere(d, fp8):
+    torch.manual_seed(d)
+    k, v = _small_cache(d, fp8, 4, LMAX)
+    qkv = torch.randn(1, 24 * d, device="cuda").half()
+    ang = torch.rand(LMAX, d // 2, device="cuda")
+    table = torch.stack([ang.cos(), ang.sin()], -1).contiguous()
+    moved = torch.empty(table.numel() + 2, device="cuda")[2:].view_as(table).copy_(table)
+    assert moved.data_ptr() % 16 == 8
+    assert torch.equal(_plain(d, fp8, qkv, k.clone(), v.clone(), 300, table, 16, 4), _plain(d, fp8, qkv, k.clone(), v.clone(), 300, moved, 16, 4))
+
+
+@pytest.mark.parametrize("d,fp8", [(64, False), (64, True), (128, False), (128, True)])
+def test_heads_of_two_gib(d, fp8):
+    """past what a 32-bit offset reaches: the register form, and the result of a small cache with the same keys"""
+    torch.manual_seed(d)
+    lmax = (1 << 31) // (d * (1 if fp8 else 2))
+    ks, vs = _small_cache(d, fp8, 1, LMAX)
+    kd = torch.zeros(1, 1, lmax, d, dtype=ks.dtype, device="cuda")
+    vd = torch.zeros(1, 1, d, lmax, dtype=vs.dtype, device="cuda")
+    kd[:, :, :LMAX], vd[..., :LMAX] = ks, vs
+    qkv = torch.randn(1, 10 * d, device="cuda").half()
+    ang = torch.rand(LMAX, d // 2, device="cuda")
+    table = torch.stack([ang.cos(), ang.sin()], -1).contiguous()
+    a, b = _plain(d, fp8, qkv, kd, vd, 1000, table, 8, 1), _plain(d, fp8, qkv, ks, vs, 1000, table, 8, 1)
+    assert torch.equal(kd[:, :, :LMAX], ks) and torch.equal(vd[..., :LMAX], vs)
+    # (each within the bound of _case of the exact result)
+    assert ((a.double() - b.double()).norm() / b.double().norm()).item() < 2 * (1.2e-2 if fp8 and d == 128 else 5e-3)

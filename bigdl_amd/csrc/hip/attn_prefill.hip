@@ -26,6 +26,7 @@
 //    group of wavefronts taking alternate key tiles (51 / 588 us on the earlier kernel), tiles requested two phases
 //    ahead through a second register set (29 / 295 us), the normaliser as an extra MFMA row block (no change).
 #include "common.h"
+#include <math.h>
 #include <type_traits>
 
 namespace bigdl {
@@ -1056,29 +1057,58 @@ static int launch_pf_one(const PrefillArgs& a, hipStream_t st) {
   return HIP_CHECK_LAUNCH();
 }
 
-// Which form: 0 = 64 queries a workgroup, several to a CU, 1 / 2 = the long-prompt form of 256 queries / 128 in split groups.  Long prompts: from
-// 321 queries (1025 of 64 channels) and more than 256 blocks of 64 on; us, old -> new: 32 heads of 128 channels 512 tokens 14.8 -> 16.7, 700
-// 26.0 -> 20.1, 3 x 300 16.7 -> 17.8, 3 x 400 22.8 -> 19.7, of 64 channels 512 10.4 -> 12.2, 1300 25.1 -> 21.2, 3 x 700 24.1 -> 24.9.  Between them by
-// the time of the longest workgroup or of all on 256 CUs, with a workgroup's start and end, fitted to 40 shapes: us, 256 / split: 1024 35.4 /
-// 25.0, 2048 62 / 55, 2500 78 / 86, 2 x 900 34.6 / 36.0, 2 x 1500 59 / 67.
+// Which form: 0 = 64 queries a workgroup, several to a CU, 1 / 2 = the long-prompt form of 256 queries / 128 in split groups.
+//  * Causal calls without a window.  Form 0 up to 320 queries (1024 of 64 channels) or 256 blocks of 64; us, form 0 -> 1 or 2: 32 heads of 128
+//    channels 512 tokens 14.8 -> 16.7, 700 26.0 -> 20.1, 3 x 300 16.7 -> 17.8, 3 x 400 22.8 -> 19.7, of 64 channels 512 10.4 -> 12.2, 1300 25.1 ->
+//    21.2, 3 x 700 24.1 -> 24.9.  Between 1 and 2 by the time of the longest workgroup or of all on 256 CUs, with a workgroup's start and
+//    end, fitted to 40 shapes: us, 1 / 2: 1024 35.4 / 25.0, 2048 62 / 55, 2500 78 / 86, 2 x 900 34.6 / 36.0, 2 x 1500 59 / 67.  Of 1285 calls (64 and
+//    128 channels, 4 - 64 heads, 1 - 8 sequences, 200 - 9000 queries, up to 4000 keys before them) 1.9 % behind the fastest form on average.
+//  * Without a causal mask, or with a window of less than half of the keys, the lengths say less: workgroups are alike (the last turn counts)
+//    and short (their ends count, the more so where a window masks both).  By the rule above 110 of 491 such calls were more than 2 % slower in
+//    the new form than in form 0, up to 83 %.  There all three forms are estimated: a launch plus the longer of the longest workgroup (the
+//    slower the more CUs are busy) and of all of them on 256 CUs with an uneven last turn; fitted to 370 of them, off by 4 - 9 %.  The rule's
+//    choice is left where another is expected to be faster: 0.6 % behind the fastest on average (7.3), 6 of 491 more than 3 % slower than
+//    form 0.  us, form 0 -> by the rule alone -> so: 32 heads of 64, window of 700, 3000 queries 44.7 -> 57.6 -> 44.6, 1100 queries not causal
+//    31.4 -> 39.2 -> 31.3.
+struct PromptForm { double launch, ends, lone, tile, uneven, window; };
+static const PromptForm kPromptForms[2][3] = {
+    {{8.268, -0.222, 0.596, 0.438, 1.208, 0.899}, {4.102, 4.807, 1.043, 1.258, 0.903, 4.369}, {3.496, 5.653, 1.244, 1.402, 0.925, 0.511}},      // 64
+    {{7.008, 0.251, 0.888, 0.892, 1.454, 2.146}, {2.895, 9.339, 1.159, 1.679, 0.895, 4.871}, {3.757, 9.599, 1.131, 1.898, 0.803, 0.818}}};      // 128
+
+static int g_force_form = -1;                         // bigdl_attn_prefill_force (tests / sweeps)
+
 static int prompt_form(const PrefillArgs& a, int D) {
-  const int64_t heads = (int64_t)a.Hq * a.B;
-  if (a.Sq <= (D == 64 ? 1024 : 320) || (a.Sq + 63) / 64 * heads <= 256) return 0;
-  double us[2];
-  for (int f = 0; f < 2; ++f) {
-    const int BM = f ? 128 : 256, nqb = (a.Sq + BM - 1) / BM, offset = a.Lk - a.Sq;
-    double total = 0.0, longest = 0.0;
+  if (g_force_form >= 0) return g_force_form;
+  const double heads = (double)a.Hq * a.B;
+  const bool few = a.Sq <= (D == 64 ? 1024 : 320) || (a.Sq + 63) / 64 * heads <= 256;
+  const bool windowed = a.window > 0 && 2ll * a.window < a.Lk, estimate = (!a.causal || windowed) && a.Sq >= 200;
+  if (few && !estimate) return 0;
+  double rule[3] = {0.0, 0.0, 0.0}, us[3];
+  for (int f = 0; f < 3; ++f) {
+    const int BM = f == 0 ? 64 : f == 1 ? 256 : 128, nqb = (a.Sq + BM - 1) / BM, offset = a.Lk - a.Sq;
+    double total = 0.0, pairs = 0.0, longest = 0.0, shortest = 1e30;
     for (int j = 0; j < nqb; ++j) {
       const int kend = a.causal && (j + 1) * BM + offset < a.Lk ? (j + 1) * BM + offset : a.Lk;
       const int first = a.window > 0 ? j * BM + offset - a.window + 1 : 0, kbeg = first > 0 ? first / PF_BN * PF_BN : 0;
-      const double steps = (kend - kbeg + PF_BN - 1) / PF_BN * (f ? 0.5 : 1.0);
-      total += steps;
-      longest = longest > steps ? longest : steps;
+      const double tiles = kend > kbeg ? (kend - kbeg + PF_BN - 1) / PF_BN : 0;
+      total += tiles;
+      pairs += ceil(0.5 * tiles);
+      longest = longest > tiles ? longest : tiles;
+      shortest = shortest < tiles ? shortest : tiles;
     }
-    const double turns = nqb * heads > 256 ? nqb * heads / 256.0 : 1.0, shared = total * heads / 256.0;
-    us[f] = 8.5 * turns + (f ? 2.4 : 1.75) * (longest > shared ? longest : shared);
+    const double turns = nqb * heads / 256.0, part = f == 2 ? 0.5 : 1.0, shared = total * heads / 256.0;
+    rule[f] = 8.5 * (turns > 1.0 ? turns : 1.0) + (f == 2 ? 2.4 : 1.75) * part * (longest > shared ? longest : shared);
+    const PromptForm& p = kPromptForms[D == 128][f];
+    const double ends = p.ends + (windowed ? p.window : 0.0), lng = ceil(part * longest), sht = ceil(part * shortest);
+    const double work = (f == 2 ? pairs : total) * heads / 256.0, busy = work < lng ? work / lng : 1.0;
+    const double one = ends + (p.lone + (p.tile - p.lone) * busy) * lng;
+    const double all = turns * ends + p.tile * work + p.uneven * (ends + p.tile * sht) * (ceil(turns) - turns);
+    us[f] = p.launch + (one > all ? one : all);
   }
-  return us[1] < us[0] ? 2 : 1;
+  const int chosen = few ? 0 : rule[2] < rule[1] ? 2 : 1;
+  if (!estimate) return chosen;
+  const int fast = us[2] < us[1] ? 2 : 1, best = us[fast] < 0.97 * us[0] ? fast : 0;
+  return us[best] < us[chosen] ? best : chosen;
 }
 
 template <int D, bool SPLIT>
@@ -1128,6 +1158,9 @@ static int launch_pf(const PrefillArgs& a, hipStream_t st) {
 // with v_transposed, v is [B, Hkv, D, Lk] (v_ss = stride between d rows; the layout of the engine's V^T cache,
 // which saves the in-kernel transpose).  out [B, Sq, Hq * D] (o_sb, o_ss; heads contiguous).
 // Query i attends to keys <= i + (Lk - Sq) when causal.
+// form >= 0 pins the form of the following calls that can take any of them (-1: planned)
+extern "C" void bigdl_attn_prefill_force(int form) { g_force_form = form > 2 ? -1 : form; }
+
 extern "C" int bigdl_attn_prefill(const void* q, const void* k, const void* v, void* out, const void* mask, int B, int Hq,
                                   int Hkv, int Sq, int Lk, int D, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb,
                                   int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t o_sb,

@@ -7,11 +7,13 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module")
-def hip():
+# the form that the estimates choose, and each of the three
+@pytest.fixture(scope="module", params=[-1, 0, 1, 2])
+def hip(request):
     from bigdl_amd.ops import hip as h
-    h.lib()
-    return h
+    h.lib().bigdl_attn_prefill_force(request.param)
+    yield h
+    h.lib().bigdl_attn_prefill_force(-1)
 
 
 def _inputs(b, hq, hkv, sq, lk, d, spread=1.0):

@@ -432,7 +432,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(PrefillArgs a) {
 // LDS).  The groups (wavefronts w and w + 4 share a SIMD) are one block apart, a barrier
 // behind every block: while one group multiplies the other takes exponentials.
 // SPLIT: the groups take alternate tiles of the same 128 queries, each with its own tile buffers, and are added up at the end.
-// What bounds it: power and the vector unit.  7700 tokens of 32 heads, causal: 798 us of the kernel above -> 508 (960 TFLOP/s), about 4000
+// What bounds it: power and the vector unit.  7700 tokens of 32 heads, causal: 775 us of the kernel above -> 490 in a row (1 PFLOP/s; traced in a prompt 898 -> 498), about 4000
 // cycles for a tile of the 8 wavefronts (2230 of MFMAs) at 1.6 GHz; with 16 x 16 x 32 MFMAs 4550 cycles at 1.8 GHz, the same time.
 // 1024 tokens 28.1 -> 25.0, 2048 86.9 -> 55.4, 4096 254 -> 153.  Measured and dropped: the three parts of a tile in one instruction stream
 // (values of the tile before, softmax, scores of the next; registers for two sets of scores: 7 % slower), tiles through registers

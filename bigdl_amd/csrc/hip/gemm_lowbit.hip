@@ -342,13 +342,15 @@ extern "C" int bigdl_gemm_lowbit(const void* x, const void* w, void* out, const 
 //    terms); the mean speed is 1.15 times the former.  Measured, us, before -> with the pass -> x in fragment order already: sym_int4
 //    4096 x 4096 at 160 / 256 rows 22.7 -> 16.6 -> 12.7, 23.7 -> 19.1 -> 14.6; sym_int8 4672 x 4544 at 203 rows 37.6 -> 24.1 -> 20.7.  Left:
 //    sym_int4 4096 x 4096 at 77 rows 14.6 -> 12.2 -> 9.1, 12288 x 4096 at 64 rows 16.5 -> 18.3 -> 15.4, 14336 x 4096 at 256 rows 45.6 -> 55.1 -> 50.5.
-//  * Rows in bf16 need a pass in any case, their conversion: by 5 %.
+//  * Rows in bf16 need a pass in any case, their conversion: by 5 %.  At 257 - 512 rows too: the prompt way's conversion, 3 - 5 us, is not in
+//    its estimate.  Of 158 random products in a row this choice is 0.6 % behind the faster way on average, 20 % at most (all on the prompt
+//    kernel: 12 and 72).
 //  * x whose producer writes it in that order: in a whole step, against the others with x in rows, it is ahead where both are
 //    alike alone (their split sums take a launch more, and they come back to cold code), so up to 256 rows unless it is expected
 //    to be 15 % behind.  Steps of 8 layers, us, without it / with 3 % ahead asked for / as here: llama3-8b nf4 33 rows 988 / 896 / 857,
 //    q4_k 64 rows 970 / 915 / 871, llama2-7b sym_int4 64 rows 1157 / 1121 / 1074.
 //  * Against the prompt kernel (257 - 512 rows) this kernel's estimate is a tenth too high: at 1.08 of its time for rows the choice among
-//    90 random products loses 0.4 % on average, 9 % at most (at 0.95 1.6 and 22); at 1.14 for produced x prompts of 3 layers take, us, at
+//    90 random products loses 0.4 % on average, 9 % at most (at 0.95 1.6 and 22), of 158 in a row 1.2 and 18; at 1.14 for produced x prompts of 3 layers take, us, at
 //    0.95 / 1.14 / 1.3: llama2-7b sym_int4 300 tokens 699 / 699 / 733, 400 809 / 799 / 831, llama3-8b nf4 300 778 / 765 / 779, q4_k 450 887 /
 //    893 / 910, tinyllama nf4 300 399 / 370 / 376.
 enum XKind { X_ROWS = 0, X_ROWS_BF16 = 1, X_FRAGMENTS = 2, X_PRODUCED = 3 };

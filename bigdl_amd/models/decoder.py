@@ -341,9 +341,10 @@ def attn_decode_splits(batch: int, num_kv_heads: int, capacity: int) -> int:
     One workgroup serves one pair and one range, so a lone sequence needs ranges to fill the chip: as many as keep the
     grid within 256 workgroups, never shorter than 256 keys.  The partial results are merged by every workgroup of the
     output projection, which costs rows x ranges x q_size floats per workgroup, so from 64 pairs on a range is at least
-    1024 keys long.  Measured on one MI355X, before heads of 64 and 128 came to the streaming form, at 1024 keys of context, Llama-2-7B sym_int4 + fp8 cache: 5 sequences
-    2.97 -> 2.34 ms per step, 6 3.06 -> 2.45, 7 3.34 -> 2.73 with one range instead of two; at 4096 keys 2 sequences
-    are fastest with 4 ranges, 3-4 with 2, 6 and more with 1.  ``BIGDL_ATTN_SPLITS`` overrides the count."""
+    1024 keys long.  Measured on one MI355X at 1024 keys of context, Llama-2-7B sym_int4 + fp8 cache, before heads of 64
+    and 128 came to the streaming form of the kernel: 5 sequences 2.97 -> 2.34 ms per step, 6 3.06 -> 2.45, 7 3.34 ->
+    2.73 with one range instead of two; at 4096 keys 2 sequences are fastest with 4 ranges, 3-4 with 2, 6 and more with
+    1.  ``BIGDL_ATTN_SPLITS`` overrides the count."""
     pairs = max(1, batch * num_kv_heads)
     max_splits = max(1, capacity // 256)
     if os.environ.get("BIGDL_ATTN_SPLITS"):

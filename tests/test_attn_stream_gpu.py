@@ -183,6 +183,42 @@ def test_several_tokens_round_as_one_after_the_other(d, fp8, hq, hkv, n, interle
     assert torch.equal(many, steps)
 
 
+@pytest.mark.parametrize("d,fp8", [(64, False), (64, True), (128, False), (128, True)])
+@pytest.mark.parametrize("hq,hkv,b,n", [(8, 2, 3, 3), (12, 4, 130, 5)])
+@pytest.mark.parametrize("opt", ["window", "softcap", "alibi", "mask", "append"])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_several_tokens_with_what_changes_a_score(d, fp8, hq, hkv, b, n, opt, splits):
+    """the same bits as one after the other with one range; with several, whose bounds depend on the length, the same result"""
+    torch.manual_seed(b + n)
+    pasts = [(37 * i) % 900 for i in range(b)]
+    k, v = torch.randn(b, hkv, LMAX, d, device="cuda").half(), torch.randn(b, hkv, d, LMAX, device="cuda").half()
+    if fp8:
+        k, v = (t.to(torch.float8_e5m2).view(torch.uint8) for t in (k, v))
+    qkv = torch.randn(b, n, (hq + 2 * hkv) * d, device="cuda").half()
+    ang = torch.rand(LMAX, d // 2, device="cuda")
+    table = None if opt == "append" else torch.stack([ang.cos(), ang.sin()], -1).contiguous()
+    mask = (2 * torch.randn(b, n, LMAX, device="cuda")).half()
+    ws = torch.empty(hip.attn_decode_ws_floats(b, hq, hkv, n, d, splits), dtype=torch.float32, device="cuda")
+    counters = torch.zeros(hip.attn_decode_counters(b, hq, hkv), dtype=torch.int32, device="cuda")
+    extra = {"window": dict(window=100), "softcap": dict(softcap=20.0), "alibi": dict(alibi=torch.rand(hq, device="cuda") * 0.05)}.get(opt, {})
+
+    def call(kc, vc, first, m):
+        out = torch.empty(b * m, hq * d, dtype=torch.float16, device="cuda")
+        more = dict(extra, mask=mask[:, first:first + m].contiguous()) if opt == "mask" else extra
+        hip.attn_decode(qkv[:, first:first + m].reshape(b * m, -1), kc, vc, torch.tensor(pasts, dtype=torch.int32, device="cuda") + first, out, ws,
+                        counters, n_heads=hq, n_kv_heads=hkv, head_dim=d, q_len=m, batch=b, scale=d ** -0.5, splits=splits, rope_table=table,
+                        append=table is None, **more)
+        return out.view(b, m, hq * d)
+
+    k1, v1 = k.clone(), v.clone()
+    many, steps = call(k1, v1, 0, n), torch.cat([call(k, v, t, 1) for t in range(n)], 1)
+    assert torch.equal(k1, k) and torch.equal(v1, v)
+    if splits == 1:
+        assert torch.equal(many, steps)
+    # (each within the bound of _case of the exact result)
+    assert ((many.double() - steps.double()).norm() / steps.double().norm()).item() < 2 * (1.2e-2 if fp8 and d == 128 else 5e-3)
+
+
 # (heads of 64 in an e5m2 cache of one range come here from 512 pairs on)
 @pytest.mark.parametrize("d,fp8,hq,hkv,b,splits", [
     (d, fp8, *c, splits) for d in (64, 128) for fp8 in (False, True) for c in [(8, 2, 2), (40, 40, 2), (40, 40, 16), (40, 2, 3)]

@@ -38,6 +38,9 @@ __device__ __forceinline__ int64_t frag_at(int m, int k, int mt_all) {
 
 __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t mask, uint32_t orv) { return (a & mask) | orv; }
 
+// the same of three vector registers: v_bitop3_b32 issues at twice the rate of v_and_or_b32 (and of itself with a scalar operand)
+__device__ __forceinline__ uint32_t and_or3(uint32_t a, uint32_t mask, uint32_t orv) { return __builtin_amdgcn_bitop3_b32(a, mask, orv, 0xEA); }
+
 union H8 {
   half8 v;
   uint32_t u[4];
@@ -123,6 +126,13 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
   v += __shfl_xor(v, 16);
   v += __shfl_xor(v, 32);
   return v;
+}
+// sum of a value over the four groups of 16 lanes, in every lane
+__device__ __forceinline__ float row_groups_sum(float v) {
+  const uint2v a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a.x) + __uint_as_float(a.y);
+  const uint2v b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(b.x) + __uint_as_float(b.y);
 }
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll

@@ -196,14 +196,11 @@ __device__ __forceinline__ half8 dec_int4_fast(uint32_t w, float bias) {
   const half2v mulB = {(_Float16)0.0625f, (_Float16)0.0625f};
   const half2v offB = {(_Float16)(-64.0f - bias), (_Float16)(-64.0f - bias)};
   const uint32_t w8 = w >> 8;
-  // v_and_or_b32 takes at most one scalar/literal operand on gfx950: keep the magic exponent in a VGPR
-  uint32_t magic;
+  uint32_t lo, hi, magic;
+  asm("v_mov_b32 %0, 0x000f000f" : "=v"(lo));
+  asm("v_mov_b32 %0, 0x00f000f0" : "=v"(hi));
   asm("v_mov_b32 %0, 0x64006400" : "=v"(magic));
-  uint32_t a0, a1, a2, a3;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(a0) : "v"(w), "s"(0x000F000Fu), "v"(magic));
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(a1) : "v"(w), "s"(0x00F000F0u), "v"(magic));
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(a2) : "v"(w8), "s"(0x000F000Fu), "v"(magic));
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(a3) : "v"(w8), "s"(0x00F000F0u), "v"(magic));
+  const uint32_t a0 = and_or3(w, lo, magic), a1 = and_or3(w, hi, magic), a2 = and_or3(w8, lo, magic), a3 = and_or3(w8, hi, magic);
   r.h2[0] = u2h(a0) - offA;
   r.h2[1] = u2h(a1) * mulB + offB;
   r.h2[2] = u2h(a2) - offA;
@@ -529,7 +526,6 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
   if constexpr (CU) {
     if (cnt * RPN > 2) fetch(tc, sc3, 0);
   }
-
   GEMV_STAMP_AT(1);
   // ---- 3. stage x (optionally scaled by the norm's gamma) in LDS, all wavefronts together ----
   if constexpr (SCLDS) {
@@ -795,9 +791,7 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
     }
   };
   // epilogue of one output element: norm factors, bias, activation / gate, residual, store
-  auto emit = [&](float v, float u, int m, int n) {
-    float rs, mean;
-    row_stats(m, rs, mean);
+  auto emit = [&](float v, float u, int m, int n, float rs, float mean) {
     v *= rs;
     if (lnorm) v += a.ln_c2[n] - rs * mean * a.ln_c1[n];
     if (a.bias) v += (float)((const _Float16*)a.bias)[n];
@@ -822,6 +816,20 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
       store_out<OUT_F32>(a.out, oi, v);
     }
   };
+  // the rows' factors, by the wavefront that writes the outputs, into its own slots of the partial sums: these are complete behind the
+  // staging barrier, and in front of the main loop a wavefront waits for weights anyway (behind it, the sum over the wavefronts, the
+  // division and the root were on the way of every result).  With the sums of up to four rows added up by lane groups, us a launch in a
+  // row, one MI355X, before -> now: sym_int4 pair of 5632 x 2048 6.32 -> 6.01, 2560 x 2048 with a norm 3.57 -> 3.44, 2048 x 5632 4.92 -> 4.79,
+  // 4096 x 4096 4.90 -> 4.73, two rows 5.20 -> 5.06, pair of 11008 x 4096 at two rows 15.84 -> 15.43
+  auto rows_of = [&]() {
+    if (norm && lane < MT * 16) {
+      float rs, mean;
+      row_stats(lane, rs, mean);
+      ssq_sh[lane] = rs;
+      if (lnorm) sum_sh[lane] = mean;
+    }
+  };
+  auto emit_row = [&](float v, float u, int m, int n) { emit(v, u, m, n, norm ? ssq_sh[m] : 1.0f, lnorm ? sum_sh[m] : 0.0f); };
 
   if constexpr (CU) {
     // ---- 3'. all tiles of this workgroup, round after round through the two register sets ----
@@ -859,7 +867,11 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const int m = 4 * g + q;
-          if (m < a.M && n < a.N) emit(o[0][q], o[NACC - 1][q], m, n);
+          if (m < a.M && n < a.N) {
+            float rs, mean;
+            row_stats(m, rs, mean);
+            emit(o[0][q], o[NACC - 1][q], m, n, rs, mean);
+          }
         }
       }
       if (c_i != cnt) __syncthreads();            // the slots are reused by the next chunk
@@ -885,6 +897,9 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
     return;
   }
 
+  if constexpr (XLDS) {
+    if (wave == 0) rows_of();
+  }
   // ---- 3. main loop: ping-pong between two register sets; a set is re-requested as soon as it has been consumed ----
   for (int base = 0; base < (GEMV_PROBE == 2 ? min(ntw, 1) : ntw); base += 2 * U) {
     if (GEMV_PROBE != 2 && base + U < ntw && !(PF2 && base == 0)) fetch(tb, sb, base + U);
@@ -922,6 +937,25 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
   }
 
   const int n = (int)nt * 16 + r;
+  if constexpr (!XLDS) rows_of();
+  if (MT == 1 && a.M <= 4) {
+    // up to four rows (lane group 0 holds them): every lane group adds up a quarter of the wavefronts, then the four meet
+    float4v o[NACC];
+#pragma unroll
+    for (int i = 0; i < NACC; ++i) {
+      o[i] = *(const float4v*)(red + ((g * NACC + i) * 64 + r) * 4);
+#pragma unroll
+      for (int w = 4; w < GEMV_NW; w += 4) o[i] += *(const float4v*)(red + (((w + g) * NACC + i) * 64 + r) * 4);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (q >= a.M) break;
+      const float v = row_groups_sum(o[0][q]), u = NACC == 2 ? row_groups_sum(o[NACC - 1][q]) : 0.0f;
+      if (g == 0 && n < a.N) emit_row(v, u, q, n);
+    }
+    GEMV_STAMP_AT(5);
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < MT; ++j) {
     float4v o[NACC];
@@ -934,7 +968,7 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int m = 16 * j + 4 * g + q;
-      if (m < a.M && n < a.N) emit(o[0][q], o[NACC - 1][q], m, n);
+      if (m < a.M && n < a.N) emit_row(o[0][q], o[NACC - 1][q], m, n);
     }
   }
   GEMV_STAMP_AT(5);

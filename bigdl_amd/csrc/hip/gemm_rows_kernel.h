@@ -195,6 +195,13 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(const 
   constexpr int NS = PAIR ? 2 * NT : NT;             // weight tiles per k-tile
   constexpr bool POST = MT == 1;                     // block scale on the fp32 product instead of the fp16 code (q6_k: always)
   constexpr bool NORM = MT == 1;                     // the folded RMSNorm exists for up to 16 rows
+  constexpr bool MINS = POST && has_min_of(QT);
+  // Pairs of six or eight tiles: the look-ahead is one k-tile, and requested all at once behind it, it came a memory round trip late.  Each
+  // tile is requested again as soon as it has been multiplied (all four steps at once), and seven others hide its way.  With minima or
+  // 8-bit codes only, us before -> now: asym_int4 14336 x 4096 at 4 / 12 rows 23.5 -> 21.5, 25.0 -> 23.9, 11008 x 4096 at 8 rows 19.0 -> 17.5;
+  // sym_int8 14336 x 4096 at 16 rows 28.8 -> 25.7, fp8_e4m3 at 12 rows 31.1 -> 28.2; other formats' tiles are smaller and take it +-1 %,
+  // single products of four tiles, whose look-ahead is two k-tiles, as well.
+  constexpr bool ROLL = POST && QT != Q_Q6_K && PAIR && NS >= 6 && (has_min_of(QT) || lo_bits_of(QT) == 8);
   constexpr int XB = MT * 2048;                      // bytes of half a staged x tile: MT * 16 rows of 64 halves
   constexpr bool TWO = rows_two_phase(MT, NS, NW);
   constexpr int NR = TWO ? NW / 2 : NW;              // wavefronts whose partial sums are in LDS at once
@@ -264,26 +271,59 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(const 
   float ssq[NP];
 #pragma unroll
   for (int p = 0; p < NP; ++p) ssq[p] = 0.0f;
-  auto stage_x = [&](int h) {
+  auto stage_from = [&](auto& xs, auto& gs, int h) {
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-      half8 v = __builtin_bit_cast(half8, xr[h % XH][p]);
+      half8 v = __builtin_bit_cast(half8, xs[h % XH][p]);
       if constexpr (NORM) {
         ssq[p] += frag_sumsq(v);
-        v = v * (__builtin_bit_cast(half8, gr[h]) + goff);
+        v = v * (__builtin_bit_cast(half8, gs[h]) + goff);
       }
       *(half8*)(xt + h * XB + (8 * p + srow) * 128 + ((slot ^ srow) << 4)) = v;
     }
+  };
+  auto stage_x = [&](int h) { stage_from(xr, gr, h); };
+  // ROLL: one weight tile of k-tile i, so that the requests follow each other in the order of their use
+  auto fetch_tile = [&](Tile<QT>& t, int n, int i) {
+    if constexpr (!RAW) {
+      const int kt = kmap(i);
+      const uint32_t out = past(i);
+      if (!PAIR || n < NT) pl.load(t, tbase[n % NT] + kt, lane, out);
+      else if constexpr (PAIR) pl2.load(t, tbase[n % NT] + kt, lane, out);
+    }
+    rows_issued();
   };
 
   // x first (vector loads return in order), then the weights of the first WD k-tiles
   fetch_x(0, 0);
   if constexpr (XH == 2) fetch_x(0, 1);
   rows_issued();
+  uint4v xr0[ROLL ? 2 : 1][NP], gr0[2];
+  if constexpr (ROLL) {
+    // (the loop's order from the start: its waits count what is younger on every way into it)
 #pragma unroll
-  for (int d = 0; d < WD; ++d) {
-    fetch_w(tt[d], d);
-    rows_issued();
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int p = 0; p < NP; ++p) xr0[h][p] = xr[h][p];
+      if constexpr (NORM) gr0[h] = gr[h];
+    }
+#pragma unroll
+    for (int d = 0; d < WD; ++d)
+#pragma unroll
+      for (int n = 0; n < NS; ++n) {
+        fetch_tile(tt[d][n], n, d);
+        if (d == WD - 1 && n == NS / 2) {
+          fetch_x(1, 0);
+          fetch_x(1, 1);
+          rows_issued();
+        }
+      }
+  } else {
+#pragma unroll
+    for (int d = 0; d < WD; ++d) {
+      fetch_w(tt[d], d);
+      rows_issued();
+    }
   }
 
   float4v acc[NS][MT];
@@ -294,6 +334,29 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(const 
 
   auto x_fragment = [&](int h, int s, int j) {
     return *(const half8*)(xt + h * XB + (16 * j + r) * 128 + ((rows_chunk<QT>(s, g) ^ (r & 7)) << 4));
+  };
+  // MINS: block sums of x in the layout of the product: a fragment of ones
+  auto x_sum = [&](half8 xa) {
+    const half8 one8 = {1, 1, 1, 1, 1, 1, 1, 1};
+    return MINS ? mfma16(xa, one8, float4v{0, 0, 0, 0}) : float4v{0, 0, 0, 0};
+  };
+  // one fragment of a weight tile and x: code x x, scaled in fp32, + minimum x block sum.  ROLL: scale and minimum are converted by
+  // themselves; full-rate multiply-adds follow, where the mixed form with a half operand issues at half the rate
+  auto multiply = [&](float4v& c, const Tile<QT>& t, half8 xa, float4v sx, int s) {
+    if constexpr (!RAW) {
+      const half8 code = rows_fragment<QT>(t, s, g);
+      float d = rows_scale<QT>(t, s);
+      if constexpr (ROLL) asm("" : "+v"(d));
+      const float4v p = mfma16(xa, code, float4v{0, 0, 0, 0});
+#pragma unroll
+      for (int q = 0; q < 4; ++q) c[q] = fmaf(p[q], d, c[q]);
+      if constexpr (MINS) {
+        float m = (float)t.m[s];
+        if constexpr (ROLL) asm("" : "+v"(m));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) c[q] = fmaf(sx[q], m, c[q]);
+      }
+    }
   };
   auto half_step = [&](Tile<QT> (&t)[NS], int h) {
     if constexpr (RAW) {
@@ -313,40 +376,25 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(const 
           for (int q = 0; q < 4; ++q) acc[n][j][q] = fmaf(c[q], d, acc[n][j][q]);
         }
       }
+    } else if constexpr (POST) {
+#pragma unroll
+      for (int s = 2 * h; s < 2 * h + 2; ++s) {
+        const half8 xa = x_fragment(h, s, 0);
+        const float4v sx = x_sum(xa);
+#pragma unroll
+        for (int n = 0; n < NS; ++n) multiply(acc[n][0], t[n], xa, sx, s);
+      }
     } else {
 #pragma unroll
       for (int s = 2 * h; s < 2 * h + 2; ++s) {
         half8 xa[MT];
 #pragma unroll
         for (int j = 0; j < MT; ++j) xa[j] = x_fragment(h, s, j);
-        float4v sx[POST ? MT : 1];
-        if constexpr (POST && has_min<QT>()) {
-          // block sums of x in the layout of the product: a fragment of ones
-          const half8 one8 = {1, 1, 1, 1, 1, 1, 1, 1};
-#pragma unroll
-          for (int j = 0; j < MT; ++j) sx[j] = mfma16(xa[j], one8, float4v{0, 0, 0, 0});
-        }
 #pragma unroll
         for (int n = 0; n < NS; ++n) {
-          const half8 code = rows_fragment<QT>(t[n], s, g);
-          if constexpr (POST) {
-            const float d = rows_scale<QT>(t[n], s);
+          const half8 bf = rows_scaled<QT>(t[n], rows_fragment<QT>(t[n], s, g), s);
 #pragma unroll
-            for (int j = 0; j < MT; ++j) {
-              const float4v c = mfma16(xa[j], code, float4v{0, 0, 0, 0});
-#pragma unroll
-              for (int q = 0; q < 4; ++q) acc[n][j][q] = fmaf(c[q], d, acc[n][j][q]);
-              if constexpr (has_min<QT>()) {
-                const float mn = (float)t[n].m[s];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) acc[n][j][q] = fmaf(sx[j][q], mn, acc[n][j][q]);
-              }
-            }
-          } else {
-            const half8 bf = rows_scaled<QT>(t[n], code, s);
-#pragma unroll
-            for (int j = 0; j < MT; ++j) acc[n][j] = mfma16(xa[j], bf, acc[n][j]);
-          }
+          for (int j = 0; j < MT; ++j) acc[n][j] = mfma16(xa[j], bf, acc[n][j]);
         }
       }
     }
@@ -354,41 +402,79 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(const 
   // Half a k-tile of x is staged while the half before it is multiplied: registers -> LDS one half ahead, memory ->
   // registers three halves ahead (one where the accumulators leave no room).  (A wavefront's LDS operations execute in
   // order, so its two buffers need no waits.)
-  stage_x(0);
-  if constexpr (XH == 2) fetch_x(1, 0);
-  else fetch_x(0, 1);
-  rows_issued();
-  for (int i = 0; i < nk; i += WD) {
+  if constexpr (ROLL) {
+    stage_from(xr0, gr0, 0);
+    stage_from(xr0, gr0, 1);
+    for (int i = 0; i < nk; i += WD) {
 #pragma unroll
-    for (int d = 0; d < WD; ++d) {
-      // (only arithmetic stands under a condition: a load there would cost the counts of the waits)
-      const bool live = d == 0 || i + d < nk, next = i + d + 1 < nk;
-      if constexpr (RAW) {
-        if (live)
+      for (int d = 0; d < WD; ++d) {
+        const bool live = d == 0 || i + d < nk;
+        half8 xa[4];
+        float4v sx[4];
+        if (live) {
 #pragma unroll
-          for (int n = 0; n < NT; ++n) pl.settle(tt[d][n], n, kmap(i + d));
+          for (int s = 0; s < 4; ++s) xa[s] = x_fragment(s >> 1, s, 0);
+#pragma unroll
+          for (int s = 0; s < 4; ++s) sx[s] = x_sum(xa[s]);
+        }
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+          // (the empty statements pin the tile's arithmetic between its wait and its next request: moved together, the tiles' spill)
+          asm volatile("" : "+v"(tt[d][n].lo0));
+          if (live) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) multiply(acc[n][0], tt[d][n], xa[s], sx[s], s);
+          }
+          asm volatile("" : "+v"(acc[n][0]));
+          __builtin_amdgcn_sched_barrier(0);
+          fetch_tile(tt[d][n], n, i + d + WD);
+          if (n == NS / 2) {
+            stage_x(0);                              // (past the last k-tile: zeros)
+            stage_x(1);
+            fetch_x(i + d + 2, 0);
+            fetch_x(i + d + 2, 1);
+            rows_issued();
+          }
+        }
       }
-      if constexpr (XH == 2) {
-        if (live) stage_x(1);
-        fetch_x(i + d + 1, 1);
-        rows_issued();
-        if (live) half_step(tt[d], 0);
-        if (next) stage_x(0);
-        fetch_x(i + d + 2, 0);
-        rows_issued();
-        if (live) half_step(tt[d], 1);
-      } else {
-        if (live) half_step(tt[d], 0);
-        if (live) stage_x(1);
-        fetch_x(i + d + 1, 0);
-        rows_issued();
-        if (live) half_step(tt[d], 1);
-        if (next) stage_x(0);
-        fetch_x(i + d + 1, 1);
+    }
+  } else {
+    stage_x(0);
+    if constexpr (XH == 2) fetch_x(1, 0);
+    else fetch_x(0, 1);
+    rows_issued();
+    for (int i = 0; i < nk; i += WD) {
+#pragma unroll
+      for (int d = 0; d < WD; ++d) {
+        // (only arithmetic stands under a condition: a load there would cost the counts of the waits)
+        const bool live = d == 0 || i + d < nk, next = i + d + 1 < nk;
+        if constexpr (RAW) {
+          if (live)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) pl.settle(tt[d][n], n, kmap(i + d));
+        }
+        if constexpr (XH == 2) {
+          if (live) stage_x(1);
+          fetch_x(i + d + 1, 1);
+          rows_issued();
+          if (live) half_step(tt[d], 0);
+          if (next) stage_x(0);
+          fetch_x(i + d + 2, 0);
+          rows_issued();
+          if (live) half_step(tt[d], 1);
+        } else {
+          if (live) half_step(tt[d], 0);
+          if (live) stage_x(1);
+          fetch_x(i + d + 1, 0);
+          rows_issued();
+          if (live) half_step(tt[d], 1);
+          if (next) stage_x(0);
+          fetch_x(i + d + 1, 1);
+          rows_issued();
+        }
+        fetch_w(tt[d], i + d + WD);
         rows_issued();
       }
-      fetch_w(tt[d], i + d + WD);
-      rows_issued();
     }
   }
 

@@ -196,11 +196,14 @@ __device__ __forceinline__ half8 dec_int4_fast(uint32_t w, float bias) {
   const half2v mulB = {(_Float16)0.0625f, (_Float16)0.0625f};
   const half2v offB = {(_Float16)(-64.0f - bias), (_Float16)(-64.0f - bias)};
   const uint32_t w8 = w >> 8;
-  uint32_t lo, hi, magic;
-  asm("v_mov_b32 %0, 0x000f000f" : "=v"(lo));
-  asm("v_mov_b32 %0, 0x00f000f0" : "=v"(hi));
+  // v_and_or_b32 takes at most one scalar/literal operand on gfx950: keep the magic exponent in a VGPR
+  uint32_t magic;
   asm("v_mov_b32 %0, 0x64006400" : "=v"(magic));
-  const uint32_t a0 = and_or3(w, lo, magic), a1 = and_or3(w, hi, magic), a2 = and_or3(w8, lo, magic), a3 = and_or3(w8, hi, magic);
+  uint32_t a0, a1, a2, a3;
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(a0) : "v"(w), "s"(0x000F000Fu), "v"(magic));
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(a1) : "v"(w), "s"(0x00F000F0u), "v"(magic));
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(a2) : "v"(w8), "s"(0x000F000Fu), "v"(magic));
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(a3) : "v"(w8), "s"(0x00F000F0u), "v"(magic));
   r.h2[0] = u2h(a0) - offA;
   r.h2[1] = u2h(a1) * mulB + offB;
   r.h2[2] = u2h(a2) - offA;
@@ -281,12 +284,17 @@ constexpr int XTAIL = 128;   // zero halves after each LDS x row: the k-tile "on
 // is never in the scalar cache, and these kernels last 4 - 14 us.  SLOT (routed experts) is a template parameter for the same
 // reason: as a run-time branch its reads stood in front of the first weight request.  Llama-2-7B shape, batch 1, 8 steps of 4
 // layers: 1775 -> 1718 us (1742 without SLOT).
+// Wavefronts a SIMD that the registers have to allow: where the allocation is near a step of the occupancy, the lower side of it
+constexpr int gemv_occupancy(int qt, int mt, bool pair, bool xlds, int nw, bool att, bool lean, bool slot) {
+  if (lean) return pair || lo_bits_of(qt) == 8 || hi_bits_of(qt) > 0 ? 6 : 8;
+  return mt == 1 && !pair && xlds && nw == 8 && !att && (slot ? lo_bits_of(qt) == 8 : hi_bits_of(qt) == 1) ? 6 : (nw + 3) / 4;
+}
 template <int QT, int MT, bool GATE_UP, bool XLDS, int NW, bool ATT = false, bool CU = false, bool LEAN = false, bool CAT = false,
           bool SLOT = false>
 #ifndef GEMV_GU_OCC
 #define GEMV_GU_OCC 5
 #endif
-__global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_kernel(
+__global__ __launch_bounds__(NW * 64, gemv_occupancy(QT, MT, GATE_UP, XLDS, NW, ATT, LEAN, SLOT)) void gemv_t16_kernel(
     const _Float16* p_x, const void* p_w, const void* p_w2, const _Float16* p_gamma, const int* p_slots, int p_M, int p_N, int p_K,
     int p_ldx, GemvArgs a) {
   a.x = p_x; a.w = p_w; a.w2 = p_w2; a.gamma = p_gamma; a.slot_expert = p_slots; a.M = p_M; a.N = p_N; a.K = p_K; a.ldx = p_ldx;
@@ -526,6 +534,7 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
   if constexpr (CU) {
     if (cnt * RPN > 2) fetch(tc, sc3, 0);
   }
+
   GEMV_STAMP_AT(1);
   // ---- 3. stage x (optionally scaled by the norm's gamma) in LDS, all wavefronts together ----
   if constexpr (SCLDS) {
@@ -829,7 +838,16 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
       if (lnorm) sum_sh[lane] = mean;
     }
   };
-  auto emit_row = [&](float v, float u, int m, int n) { emit(v, u, m, n, norm ? ssq_sh[m] : 1.0f, lnorm ? sum_sh[m] : 0.0f); };
+  auto emit_row = [&](float v, float u, int m, int n) {
+    float rs = 1.0f, mean = 0.0f;
+    if constexpr (XLDS && MT == 1) {
+      if (norm) rs = ssq_sh[m];
+      if (lnorm) mean = sum_sh[m];
+    } else {
+      row_stats(m, rs, mean);
+    }
+    emit(v, u, m, n, rs, mean);
+  };
 
   if constexpr (CU) {
     // ---- 3'. all tiles of this workgroup, round after round through the two register sets ----
@@ -897,7 +915,7 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
     return;
   }
 
-  if constexpr (XLDS) {
+  if constexpr (XLDS && MT == 1) {
     if (wave == 0) rows_of();
   }
   // ---- 3. main loop: ping-pong between two register sets; a set is re-requested as soon as it has been consumed ----
@@ -937,8 +955,7 @@ __global__ __launch_bounds__(NW * 64, LEAN ? 6 : (NW + 3) / 4) void gemv_t16_ker
   }
 
   const int n = (int)nt * 16 + r;
-  if constexpr (!XLDS) rows_of();
-  if (MT == 1 && a.M <= 4) {
+  if (MT == 1 && (LEAN || a.M <= 4)) {
     // up to four rows (lane group 0 holds them): every lane group adds up a quarter of the wavefronts, then the four meet
     float4v o[NACC];
 #pragma unroll

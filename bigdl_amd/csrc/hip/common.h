@@ -90,6 +90,13 @@ __device__ __forceinline__ float act_apply(int act, float x) {
   }
 }
 
+// x / (1 + e^-x) by a reciprocal and one correction of the quotient (infinite or NaN where that has nothing to correct).  Both are taken as
+// quarters: the divisor is then 1/4 at least and its reciprocal never below 2^-126, where it would be flushed to zero (x near -88)
+__device__ __forceinline__ float silu_rcp(float x) {
+  const float n = 0.25f * x, d = fmaf(0.25f, __expf(-x), 0.25f), r = __builtin_amdgcn_rcpf(d), q = n * r, e = fmaf(-q, d, n);
+  return e == e ? fmaf(e, r, q) : q;
+}
+
 __device__ __forceinline__ uint8_t f16_to_e5m2(_Float16 h) {
   // round-to-nearest-even on the dropped 8 mantissa bits, saturate to the largest finite value
   union { _Float16 h; uint16_t u; } c;

@@ -48,13 +48,6 @@ constexpr int prompt_lds_tiles(int BM, int BN, int NW, int MTW, int NTW) {
 constexpr int waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
 constexpr int waitcnt_vm_lgkm0(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4); }
 
-// x / (1 + e^-x) by a reciprocal and one correction of the quotient (infinite or NaN where that has nothing to correct).  Both are taken as
-// quarters: the divisor is then 1/4 at least and its reciprocal never below 2^-126, where it would be flushed to zero (x near -88)
-__device__ __forceinline__ float prompt_silu(float x) {
-  const float n = 0.25f * x, d = fmaf(0.25f, __expf(-x), 0.25f), r = __builtin_amdgcn_rcpf(d), q = n * r, e = fmaf(-q, d, n);
-  return e == e ? fmaf(e, r, q) : q;
-}
-
 // one expansion unit = the 8 codes per lane of one (16-row weight tile, 32-deep k step) -> the fp16 fragment with the
 // block scale (and minimum) folded in.  `s` is the step inside the T16 tile (0 .. 3), static.
 template <int QT, int S>
@@ -416,7 +409,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_prompt_kernel(GemmArgs a
   };
   // act(first) * second on the rounded 16-bit values (what a separate activation kernel would read).  The usual gate has a loop of
   // its own: with the choice of the activation inside, an element took twice the instructions
-  if (pair && a.act == ACT_SILU) rows_out([&](uint4v p, uint4v q) { return chunk(p, q, [](float x, float u) { return prompt_silu(x) * u; }); });
+  if (pair && a.act == ACT_SILU) rows_out([&](uint4v p, uint4v q) { return chunk(p, q, [](float x, float u) { return silu_rcp(x) * u; }); });
   else if (pair) rows_out([&](uint4v p, uint4v q) { return chunk(p, q, [&](float x, float u) { return act_apply(a.act, x) * u; }); });
   else if (plain) rows_out([](uint4v p, uint4v) { return p; });
   else rows_out([&](uint4v p, uint4v q) { return chunk(p, q, [&](float x, float u) { return act_apply(a.act, x) + u; }); });

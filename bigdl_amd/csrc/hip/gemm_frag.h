@@ -17,7 +17,8 @@ struct FragPlan {
   double us;                // what it is expected to take with its reduce launch, without the pass that orders x
 };
 static inline double frag_pack_us(int M, int K) { return 3.4 + 1e-6 * M * K; }
-FragPlan frag_plan(int M, int N, int K, int qtype, bool pair, bool may_split);
+// sums_left: the sums of a split K stay in their slabs, for the norm that follows to add up
+FragPlan frag_plan(int M, int N, int K, int qtype, bool pair, bool may_split, bool sums_left = false);
 // halves of x in fragment order
 static inline int64_t frag_halves(int M, int K) { return (int64_t)((K + 127) / 128) * 4 * ((M + 15) / 16) * 512; }
 int frag_pack(const void* x, void* xp, int M, int K, int ldx, bool bf16, hipStream_t st);

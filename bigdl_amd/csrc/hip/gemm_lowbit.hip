@@ -22,6 +22,8 @@ int gemm_launch_sym_int8(const GemmArgs& a, int bm, int bn, int mblocks, hipStre
 int gemm_launch_fp8_e4m3(const GemmArgs& a, int bm, int bn, int mblocks, hipStream_t st);
 int gemm_launch_fp8_e5m2(const GemmArgs& a, int bm, int bn, int mblocks, hipStream_t st);
 double prompt_us(int M, int N, int K, int qtype, bool pair);        // gemm_prompt.hip
+int prompt_parts(int M, int N, int K);
+int prompt_parts_launch(const void* x, const void* w, float* partial, int M, int N, int K, int ldx, int qtype, hipStream_t st);
 
 // out[m][n] = epilogue(sum_s partial[s][m][n]); pair form: act(first) * second; optional folded RMSNorm factor of the
 // row (row_ssq) and sum of squares of the rows written (ssq_out, for the norm folded into the next product).
@@ -431,6 +433,39 @@ extern "C" int bigdl_gemm_frag_dense(const void* x, const void* w, const void* w
   a.out = out; a.bias = bias; a.residual = residual; a.partial = workspace + xfloats;
   a.M = M; a.N = N; a.K = K; a.ldo = ldo; a.act = act; a.out_type = out_type; a.splitk = p.splitk;
   return launch_reduce(a, stream);
+}
+
+// A product in front of a norm: with K split over workgroups its sums can stay in their slabs, and the norm, which reads every element
+// anyway, adds them up (bigdl_rms_norm_parts).  Returns the splits (0: the product is better off whole).  x_kind 2: x in fragment order;
+// 0: fp16 rows, more than 256 of them, where the prompt kernel runs.
+extern "C" int bigdl_gemm_parts(int M, int N, int K, int ldx, int qtype, int x_kind) {
+  qtype = t16_kernel_qtype(qtype);
+  if (M <= 32 || N <= 0 || K <= 0 || (K & 31) || (N & 7) || !is_t16(qtype)) return 0;
+  int splits = 0;
+  if (x_kind == X_FRAGMENTS) {
+    const FragPlan p = frag_plan(M, N, K, qtype, false, true, true);
+    splits = p.ns == 0 ? 0 : p.splitk;
+  } else if (x_kind == X_ROWS && M > 256 && K >= 256 && (K & 127) == 0 && (ldx & 7) == 0 && (int64_t)M * ldx < (1ll << 31)) {
+    splits = prompt_parts(M, N, K);
+  }
+  return splits > 1 ? splits : 0;
+}
+
+// that product: partial [bigdl_gemm_parts][M][N] fp32, 16-byte aligned.  x as there, 16-byte aligned.
+extern "C" int bigdl_gemm_parts_run(const void* x, const void* w, float* partial, int64_t floats, int M, int N, int K, int ldx, int qtype,
+                                    int x_kind, hipStream_t stream) {
+  const int splits = bigdl_gemm_parts(M, N, K, ldx, qtype, x_kind);
+  if (splits < 2) return -4;
+  if (partial == nullptr || floats < (int64_t)splits * M * N) return -5;
+  if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)partial & 15)) return -1;
+  qtype = t16_kernel_qtype(qtype);
+  if (x_kind != X_FRAGMENTS) return prompt_parts_launch(x, w, partial, M, N, K, ldx, qtype, stream);
+  const FragPlan p = frag_plan(M, N, K, qtype, false, true, true);
+  FragArgs b = {};
+  b.xp = (const _Float16*)x; b.w = w; b.partial = partial;
+  b.M = M; b.N = N; b.K = K; b.mt_all = (M + 15) / 16; b.ldo = N; b.act = ACT_NONE; b.out_type = OUT_F16;
+  b.splitk = p.splitk; b.kt_per_split = p.kt_per_split;
+  return frag_launch(b, p, qtype, stream);
 }
 
 // Extended dense form for batched decode: RMSNorm folded in (gamma + row_ssq of x, see GemmArgs), gate / up pair in one

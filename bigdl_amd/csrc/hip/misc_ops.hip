@@ -130,6 +130,73 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const void* x, const void
   }
 }
 
+// The same of a product whose K was split, fp16: out = norm(sum of the slabs [parts][rows][H] fp32 [+ bias] [+ residual]).  The sums are added
+// here, in fp32, where a launch of its own wrote and re-read them.  What it costs is the slabs' bytes: all of a thread's pieces are requested
+// together, up to four slabs at a time.
+template <int VPT>
+__global__ __launch_bounds__(256) void rms_norm_parts_kernel(const float* x, int parts, int64_t stride, const _Float16* bias, const void* residual,
+                                                             const void* w, void* out, void* res_out, int H, float eps, float offset, int frag_mt) {
+  __shared__ float sh[8];
+  const int64_t row = blockIdx.x;
+  float v[VPT][8];
+  float ss = 0.0f;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int c = (threadIdx.x + i * 256) * 8;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[i][j] = 0.0f;
+    if (c < H) {
+      const float* p = x + row * (int64_t)H + c;
+      if (residual) load8<DT_F16>(residual, row * (int64_t)H + c, v[i]);
+      if (bias) {
+        float b[8];
+        load8<DT_F16>(bias, c, b);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[i][j] += b[j];
+      }
+      float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+      int k = 0;
+      for (; k + 4 <= parts; k += 4) {
+        float a[4][8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) load8<DT_F32>(p, (k + e) * stride, a[e]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s[j] += (a[0][j] + a[1][j]) + (a[2][j] + a[3][j]);
+      }
+      for (; k + 2 <= parts; k += 2) {
+        float a[2][8];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) load8<DT_F32>(p, (k + e) * stride, a[e]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s[j] += a[0][j] + a[1][j];
+      }
+      if (k < parts) {
+        float a[8];
+        load8<DT_F32>(p, k * stride, a);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s[j] += a[j];
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[i][j] += s[j];
+      if (res_out) store8<DT_F16>(res_out, row * (int64_t)H + c, v[i]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss += v[i][j] * v[i][j];
+    }
+  }
+  const float rs = rsqrtf(block_sum(ss, sh) / (float)H + eps);
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int c = (threadIdx.x + i * 256) * 8;
+    if (c < H) {
+      float g[8];
+      load8<DT_F16>(w, c, g);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[i][j] = v[i][j] * rs * (g[j] + offset);
+      store8<DT_F16>(out, frag_mt > 0 ? frag_at((int)row, c, frag_mt) : row * (int64_t)H + c, v[i]);
+    }
+  }
+}
+
 template <int DT, int VPT>
 __global__ __launch_bounds__(256) void layer_norm_kernel(const void* x, const void* w, const void* b, void* out, int H,
                                                          int64_t ldx, float eps) {
@@ -552,6 +619,26 @@ extern "C" int bigdl_rms_norm(const void* x, const void* residual, const void* w
     else if (vpt <= 2) hipLaunchKernelGGL((rms_norm_kernel<DT, 2>), dim3(rows), dim3(256), 0, st, x, residual, w, out, res_out, H, ldx, eps, offset, mt);
     else if (vpt <= 4) hipLaunchKernelGGL((rms_norm_kernel<DT, 4>), dim3(rows), dim3(256), 0, st, x, residual, w, out, res_out, H, ldx, eps, offset, mt);
     else hipLaunchKernelGGL((rms_norm_kernel<DT, 8>), dim3(rows), dim3(256), 0, st, x, residual, w, out, res_out, H, ldx, eps, offset, mt))
+  return HIP_CHECK_LAUNCH();
+}
+
+// x: slabs [parts][rows][H] fp32 (bigdl_gemm_parts_run); bias fp16 [H] or null; residual, res_out (may be the same), w, out fp16
+extern "C" int bigdl_rms_norm_parts(const float* x, int parts, const void* bias, const void* residual, const void* w, void* out, void* res_out,
+                                    int64_t rows, int H, float eps, float offset, int frag, hipStream_t st) {
+  if (parts < 1 || rows <= 0 || H <= 0 || (H & 7) || H > 8 * 256 * 8) return -1;
+  if (!aligned16(x) || !aligned16(w) || !aligned16(out) || (bias && !aligned16(bias)) || (residual && !aligned16(residual)) ||
+      (res_out && !aligned16(res_out))) return -1;
+  if (frag && ((H & 127) || rows > 1 << 20)) return -1;
+  const int mt = frag ? (int)((rows + 15) / 16) : 0;
+  const int vpt = (H / 8 + 255) / 256;
+  const int64_t stride = rows * (int64_t)H;
+#define PARTS_LAUNCH(V) hipLaunchKernelGGL((rms_norm_parts_kernel<V>), dim3(rows), dim3(256), 0, st, x, parts, stride, (const _Float16*)bias, \
+                                           residual, w, out, res_out, H, eps, offset, mt)
+  if (vpt <= 1) PARTS_LAUNCH(1);
+  else if (vpt <= 2) PARTS_LAUNCH(2);
+  else if (vpt <= 4) PARTS_LAUNCH(4);
+  else PARTS_LAUNCH(8);
+#undef PARTS_LAUNCH
   return HIP_CHECK_LAUNCH();
 }
 

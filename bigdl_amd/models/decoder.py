@@ -583,6 +583,28 @@ class NativeDecoder:
             y = y + lin.bias
         return y
 
+    def _norm_adds(self):
+        """whether the norms of this engine can add up what a split product in front of them leaves (``hip.Parts``)"""
+        cfg = self.cfg
+        return self.tp_group is None and cfg.norm != "layer" and not cfg.parallel_residual and cfg.hidden_size % 8 == 0
+
+    def _linear_parts(self, x, lin: Lin, wanted=True):
+        """``_linear_dense``, or with ``wanted`` (an RMSNorm that adds a residual is all that reads the result) the sums of the product with
+        its K split, for that norm to add up, where that is faster"""
+        from ..ops import hip
+        if wanted and lin.fused:
+            if type(x) is hip.Frags:
+                p = hip.gemm_parts(x, lin.w, lin.qtype, lin.n, lin.k, bias=lin.bias)
+            elif (x.shape[0] > GEMM_MAX_ROWS and self.prefill_fused and x.dtype == torch.float16 and x.dim() == 2 and x.is_contiguous()
+                  and not Lin.cache_dense and not self.prefill_fp8
+                  and not hip.gemm_lowbit_frag(x.shape[0], lin.n, lin.k, lin.qtype)):
+                p = hip.gemm_parts(x, lin.w, lin.qtype, lin.n, lin.k, bias=lin.bias)
+            else:
+                p = None
+            if p is not None:
+                return p
+        return self._linear_dense(x, lin)
+
     def _dense_ahead(self, lin: Lin):
         """fp16 form of ``lin``'s weight for a library GEMM on the current stream, valid until the next-but-one call.
         Starts the expansion of the weight that follows ``lin`` in a prompt pass on the side stream."""
@@ -670,7 +692,9 @@ class NativeDecoder:
             if frags:
                 return hip.rms_norm(h, w, self.cfg.rms_eps, offset=self.cfg.norm_offset, frags=True), h
             return self._norm(h, w, b), h
-        if self.cfg.norm == "layer" or add.dtype != h.dtype or not (h.is_contiguous() and add.is_contiguous()):
+        if type(add) is hip.Parts and not h.is_contiguous():
+            add = add.sum()
+        if type(add) is not hip.Parts and (self.cfg.norm == "layer" or add.dtype != h.dtype or not (h.is_contiguous() and add.is_contiguous())):
             h = h + add
             return self._norm(h, w, b), h
         hn = torch.empty_like(h)
@@ -686,7 +710,8 @@ class NativeDecoder:
             h = hip.layer_norm(h, self.embed_norm[0], self.embed_norm[1], self.cfg.rms_eps)
         return h
 
-    def _mlp_dense(self, x, lw):
+    def _mlp_dense(self, x, lw, parts=False):
+        """``parts``: the result may come back as ``hip.Parts`` (``_linear_parts``)"""
         from ..ops import hip
         cfg = self.cfg
         if type(x) is hip.Frags:
@@ -712,7 +737,7 @@ class NativeDecoder:
                 hip.act_mul(g, u, cfg.act)
         else:
             g = _ACT_FNS[cfg.act](self._linear_dense(x, lw.up))
-        return self._tp_reduce(self._linear_dense(g, lw.down))
+        return self._tp_reduce(self._linear_parts(g, lw.down, parts))
 
     @torch.no_grad()
     def prefill(self, input_ids: Optional[torch.Tensor], last_only: bool = True, slot: Optional[int] = None,
@@ -792,6 +817,7 @@ class NativeDecoder:
             assert bool((top == top[0]).all()), "sequences of one batch must end at the same rotary position"
             mrope_delta = int(top[0]) + 1 - s
         pend = None                          # MLP output of the previous layer, added to h by the next norm launch
+        adds = self._norm_adds() and h.dtype == torch.float16
         for li, lw in enumerate(self.layers):
             plain = not cfg.parallel_residual
             x, h = self._add_norm(h, pend, lw.input_norm, lw.input_norm_b,
@@ -853,7 +879,7 @@ class NativeDecoder:
                 vc[:, :, :, nk:cap_] = vc[:, :, :, s - w_: s].clone()
             if nd:
                 attn = torch.cat([attn, attn_d])
-            o = self._tp_reduce(self._linear_dense(attn, lw.o))
+            o = self._tp_reduce(self._linear_parts(attn, lw.o, adds and lw.post_attn_out_norm is None))
             if lw.post_attn_out_norm is not None:
                 o = self._norm(o, lw.post_attn_out_norm)
             if cfg.parallel_residual:
@@ -865,7 +891,7 @@ class NativeDecoder:
             if lw.moe is not None:
                 m = lw.moe.forward_dense(x, self)
             else:
-                m = self._mlp_dense(x, lw)
+                m = self._mlp_dense(x, lw, adds and lw.post_ffn_out_norm is None and li + 1 < len(self.layers))
             if lw.post_ffn_out_norm is not None:
                 m = self._norm(m, lw.post_ffn_out_norm)
             pend = m
@@ -1227,14 +1253,28 @@ class NativeDecoder:
         st["att_partials"] = (st["ws"], splits, cfg.head_dim, g, cfg.num_kv_heads, q_len, (rows + 15) // 16 * 16)
         return st
 
+    def _norm_first(self, m, lin: Lin, w2: Optional[Lin] = None):
+        """whether ``_gemv`` with a gamma runs an RMSNorm of its own in front of the product of m rows (and could add a split product's sums)"""
+        if m <= GEMV_MAX_ROWS or self.fold_batched_norm or not lin.fused:
+            return False
+        return w2 is None or (w2.fused and w2.qtype == lin.qtype and w2.n == lin.n and not os.environ.get("BIGDL_NO_PAIR_GEMM"))
+
     def _gemv(self, x, lin: Lin, out, *, gamma=None, residual=None, w2: Lin = None, act=None, att_partials=None,
-              beta=False, then: Lin = None):
+              beta=False, then: Lin = None, add=None):
         """out = epilogue(norm?(x) @ W^T): fused kernel for T16 weights, unfused torch ops otherwise.  ``beta``
         (a tensor or None, instead of the default False) selects LayerNorm(gamma, beta) as the norm.  ``then``: the product that alone
-        reads a pair's result; where it takes x in fragment order the result comes back so, and not in ``out``."""
+        reads a pair's result; where it takes x in fragment order the result comes back so, and not in ``out``.  ``add`` (``hip.Parts``, where
+        ``_norm_first``): what is still to be added to x, by the norm in front."""
         from ..ops import hip
         cfg = self.cfg
         m = x.shape[0]
+
+        def normed(frags=False):
+            if add is not None:
+                return hip.rms_norm(add, gamma, cfg.rms_eps, offset=cfg.norm_offset, residual=x, res_out=x, frags=frags)
+            return hip.rms_norm(x, gamma, cfg.rms_eps, offset=cfg.norm_offset, frags=frags)
+
+        assert add is None or (gamma is not None and beta is False and self._norm_first(m, lin, w2))
         if beta is not False:
             if lin.fused and (w2 is None or w2.fused) and m <= GEMV_MAX_ROWS and hip.gemv_x_in_lds(m, lin.k):
                 return hip.gemv_lowbit_ln(x, lin.w, lin.qtype, lin.n, lin.k, gamma, lin.ln_fold(gamma, beta),
@@ -1247,7 +1287,7 @@ class NativeDecoder:
             # batched decode (17 .. 256 rows): gate and up in one launch, act(g) * u in the few-row kernel's epilogue or, where
             # the tile kernel runs, in its reduce kernel (at 64 rows of 11008 x 4096: 23 and 33 us)
             frags = gamma is not None and self._takes_frags(m, lin, w2, False, then)
-            xin = x if gamma is None else hip.rms_norm(x, gamma, cfg.rms_eps, offset=cfg.norm_offset, frags=frags)
+            xin = x if gamma is None else normed(frags)
             if frags and then is not None and self._takes_frags(m, then, prompt=False):
                 return hip.gemm_lowbit_ex(xin, lin.w, lin.qtype, lin.n, lin.k, w2=w2.w, bias=lin.bias, bias2=w2.bias, act=act, out_frags=True)
             return hip.gemm_lowbit_ex(xin, lin.w, lin.qtype, lin.n, lin.k, w2=w2.w, bias=lin.bias, bias2=w2.bias, act=act, out=out)
@@ -1265,8 +1305,7 @@ class NativeDecoder:
                                       act=act, out=out)
         if lin.fused and (w2 is None or w2.fused) and m > GEMV_MAX_ROWS and att_partials is None:
             # batched decode (17 .. 64 rows): RMSNorm kernel + MFMA GEMM with the epilogue fused
-            xin = x if gamma is None else hip.rms_norm(x, gamma, cfg.rms_eps, offset=cfg.norm_offset,
-                                                       frags=w2 is None and self._takes_frags(m, lin, prompt=False))
+            xin = x if gamma is None else normed(w2 is None and self._takes_frags(m, lin, prompt=False))
             if w2 is None:
                 return hip.gemm_lowbit(xin, lin.w, lin.qtype, lin.n, lin.k, bias=lin.bias, residual=residual, act=act, out=out)
             g = hip.gemm_lowbit(xin, lin.w, lin.qtype, lin.n, lin.k, bias=lin.bias, out=out)
@@ -1330,12 +1369,12 @@ class NativeDecoder:
         self._ssq_owner = (x.data_ptr(), x.shape[1], slot)
         return slot
 
-    def _mlp_in(self, h, lw, a, gamma, beta):
+    def _mlp_in(self, h, lw, a, gamma, beta, add=None):
         """act(gate(norm(h))) * up(norm(h))  or  act(up(norm(h))): in a, or as the down projection takes it (see ``_gemv``)"""
         cfg = self.cfg
         if cfg.gated_mlp:
-            return self._gemv(h, lw.gate, a, gamma=gamma, beta=beta, w2=lw.up, act=cfg.act, then=lw.down)
-        return self._gemv(h, lw.up, a, gamma=gamma, beta=beta, act=cfg.act)
+            return self._gemv(h, lw.gate, a, gamma=gamma, beta=beta, w2=lw.up, act=cfg.act, then=lw.down, add=add)
+        return self._gemv(h, lw.up, a, gamma=gamma, beta=beta, act=cfg.act, add=add)
 
     def _decode_body(self, st, batch: int, q_len: int, chain: bool):
         from ..ops import hip
@@ -1352,6 +1391,13 @@ class NativeDecoder:
         else:
             torch.index_select(self.embed, 0, st["tokens"].view(-1), out=h)      # gather straight into the residual stream
         layer_norm = cfg.norm == "layer"
+        # a split product's sums, added to h by the norm that follows (``_gemv``): o and down in front of a norm of its own
+        adds, pend = self._norm_adds() and h.dtype == torch.float16, None
+
+        def parts(x, lin, first, w2=None):
+            if adds and type(x) is hip.Frags and lin.fused and self._norm_first(h.shape[0], first, w2):
+                return hip.gemm_parts(x, lin.w, lin.qtype, lin.n, lin.k, bias=lin.bias)
+            return None
         if self.stage_first and (self.pos_embed is not None or self.embed_norm is not None):
             pos = cache.past_len.to(torch.int64)[:, None] + torch.arange(q_len, device=self.device)[None]
             h.copy_(self._embed_extras(h, pos.reshape(-1)))
@@ -1364,7 +1410,8 @@ class NativeDecoder:
             elif layer_norm:
                 self._gemv(h, lw.qkv, qkv, gamma=lw.input_norm, beta=lw.input_norm_b)
             else:
-                self._gemv(h, lw.qkv, qkv, gamma=lw.input_norm)
+                self._gemv(h, lw.qkv, qkv, gamma=lw.input_norm, add=pend)
+            pend = None
             if not self.fused_rope:
                 hip.rope_append(qkv, cache.k[li], cache.v[li], cache.past_len, self.inv_freq, n_heads=cfg.num_heads,
                                 n_kv_heads=cfg.num_kv_heads, head_dim=cfg.head_dim, q_len=q_len, batch=batch,
@@ -1389,7 +1436,10 @@ class NativeDecoder:
                 else:
                     a = self._mlp_in(h, lw, a, lw.post_norm, lw.post_norm_b)
             if lw.post_attn_out_norm is None and self.tp_group is None:
-                self._gemv(attn, lw.o, h, residual=h, att_partials=att_partials)
+                if att_partials is None and lw.moe is None:
+                    pend = parts(attn, lw.o, *((lw.gate, lw.up) if cfg.gated_mlp else (lw.up,)))
+                if pend is None:
+                    self._gemv(attn, lw.o, h, residual=h, att_partials=att_partials)
             else:
                 self._tp_reduce(self._gemv(attn, lw.o, tmp, att_partials=att_partials))
                 if lw.post_attn_out_norm is not None:
@@ -1403,9 +1453,16 @@ class NativeDecoder:
                 continue
             if not (layer_norm and cfg.parallel_residual):
                 a = act[:, : lw.up.n]
-                a = self._mlp_in(h, lw, a, ffn_norm, lw.post_norm_b if layer_norm else False)
+                a = self._mlp_in(h, lw, a, ffn_norm, lw.post_norm_b if layer_norm else False, pend)
+                pend = None
             if lw.post_ffn_out_norm is None and self.tp_group is None:
-                self._gemv(a, lw.down, h, residual=h)
+                after = self.layers[li_ + 1] if li_ + 1 < len(self.layers) else None
+                if after is not None and after.mla is None:
+                    pend = parts(a, lw.down, after.qkv)
+                elif after is None and self.stage_last:
+                    pend = parts(a, lw.down, self.lm_head)
+                if pend is None:
+                    self._gemv(a, lw.down, h, residual=h)
             else:
                 self._tp_reduce(self._gemv(a, lw.down, tmp))
                 if lw.post_ffn_out_norm is not None:
@@ -1415,7 +1472,7 @@ class NativeDecoder:
         if not self.stage_last:
             cache.past_len.add_(cache.active, alpha=q_len)
             return
-        self._gemv(h, self.lm_head, st["logits"], gamma=self.final_norm, beta=self.final_norm_b if layer_norm else False)
+        self._gemv(h, self.lm_head, st["logits"], gamma=self.final_norm, beta=self.final_norm_b if layer_norm else False, add=pend)
         if cfg.logit_scale != 1.0 or cfg.final_softcap > 0:
             st["logits"].copy_(self._finish_logits(st["logits"]))
         # the argmax launch also advances the cache lengths (past_len += q_len * active)

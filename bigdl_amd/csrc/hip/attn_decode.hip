@@ -104,6 +104,29 @@ __device__ __forceinline__ void split_e4m3(const float (&x)[8], uint2v& hi, uint
 }
 constexpr float P8_SCALE = 256.0f;     // probabilities are carried as 256 p (and the row sums with them)
 
+// The partial results of a row group's ranges, [splits][RT * 16][D + 4] floats.  Whichever workgroup arrives last reads what the others wrote,
+// perhaps behind another XCD's L2: stores that go through the caches (agent scope) and loads that go around them need no fence.  A fence
+// writes back and invalidates a whole L2, once per workgroup.  12 sequences x 8 heads, 1900 fp16 keys: two ranges 23.4 -> 20.8 us a launch,
+// 1515 -> 1466 us for four steps of four layers, with three, four, five ranges 1697 -> 1549, 1722 -> 1511, 1748 -> 1500.
+// Partials that the output projection adds up are stored plainly: the launch's end writes them back (llama2-7b, one sequence: 0.3 %).
+constexpr int AGENT_SCOPE = 16;        // cache policy bits of a buffer access (sc1)
+template <int D, int RT>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t partials_of(const AttnArgs& a, int bh) {
+  const uint32_t bytes = (uint32_t)a.splits * (RT * 16) * (D + 4) * 4;
+  return __builtin_amdgcn_make_buffer_rsrc(a.ws + (int64_t)bh * (bytes / 4), 0, bytes, 0x00027000);
+}
+// (byte offsets: of row `row` of range `split`, column `col`)
+template <int D, int RT>
+__device__ __forceinline__ uint32_t partial_at(int split, int row, int col) { return (((uint32_t)split * (RT * 16) + row) * (D + 4) + col) * 4; }
+template <int D, int RT, int SCOPE>
+__device__ __forceinline__ void put_partial(__amdgpu_buffer_rsrc_t parts, int split, int row, int col, float4v v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v, v), parts, partial_at<D, RT>(split, row, col), 0, SCOPE);
+}
+template <int D, int RT, int SCOPE>
+__device__ __forceinline__ void put_partial(__amdgpu_buffer_rsrc_t parts, int split, int row, int col, float2 v) {
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, v), parts, partial_at<D, RT>(split, row, col), 0, SCOPE);
+}
+
 // Cross-split combine by the last-arriving workgroup of a (sequence, KV head, chunk) `bh`: row r of its partials is query head
 // head0 + r % Gc of token tok0 + r / Gc.  `s_flag`: one int of LDS.
 template <int D, int RT, int NT>
@@ -111,15 +134,9 @@ __device__ __forceinline__ void combine_splits(const AttnArgs& a, int bh, int he
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const int ticket = __hip_atomic_fetch_add(&a.counters[bh], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int last = ticket == a.splits - 1;
-    if (last) {
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __hip_atomic_store(&a.counters[bh], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (last) __hip_atomic_store(&a.counters[bh], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     *s_flag = last;
   }
   __syncthreads();
@@ -128,23 +145,25 @@ __device__ __forceinline__ void combine_splits(const AttnArgs& a, int bh, int he
   // A row's partials are requested together, up to 16: one after the other, by the four wavefronts of the streaming form, they took 15 ranges
   // of 32 heads of 128 on one KV head, 4000 keys, from 35.8 us with eight wavefronts to 43.9; so 19.3.  Four ranges of 32 heads, 1024
   // e5m2 keys 13.4 -> 12.0, two of 12 x 8 heads, 1900 fp16 keys 23.4 -> 23.1.
-  const float* wbase = a.ws + (int64_t)bh * a.splits * (RT * 16) * (D + 4);
+  const __amdgpu_buffer_rsrc_t parts = partials_of<D, RT>(a, bh);
   auto combine = [&](auto at) {
     constexpr int AT = decltype(at)::value;
     for (int idx = threadIdx.x; idx < rows * (D / 4); idx += NT) {
       const int row = idx / (D / 4), d4 = (idx % (D / 4)) * 4;
       float mm = NEG_BIG, lt = 0.0f;
       float4v acc = {0, 0, 0, 0};
-      auto part = [&](int s) { return wbase + ((int64_t)min(s, a.splits - 1) * RT * 16 + row) * (D + 4); };
+      auto sums = [&](int s) {
+        return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(parts, partial_at<D, RT>(min(s, a.splits - 1), row, D), 0, AGENT_SCOPE));
+      };
       if (a.splits > AT)
-        for (int s = 0; s < a.splits; ++s) mm = fmaxf(mm, part(s)[D]);
+        for (int s = 0; s < a.splits; ++s) mm = fmaxf(mm, sums(s).x);
       for (int s = 0; s < a.splits; s += AT) {
         float4v o[AT];
         float2 ml[AT];
 #pragma unroll
         for (int j = 0; j < AT; ++j) {                // (behind the end: the last one again)
-          o[j] = *(const float4v*)(part(s + j) + d4);
-          ml[j] = *(const float2*)(part(s + j) + D);
+          o[j] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(parts, partial_at<D, RT>(min(s + j, a.splits - 1), row, d4), 0, AGENT_SCOPE));
+          ml[j] = sums(s + j);
         }
 #pragma unroll
         for (int j = 0; j < AT; ++j) mm = fmaxf(mm, ml[j].x);
@@ -773,7 +792,7 @@ __global__ __launch_bounds__(NWT * 64) void attn_decode_kernel(const int* p_past
 
   const int bh = b * gridDim.y + blockIdx.y;
   const bool single = a.splits == 1;
-  float* wsp = a.ws + ((int64_t)bh * a.splits + split) * (RT * 16) * (D + 4);
+  const __amdgpu_buffer_rsrc_t parts = partials_of<D, RT>(a, bh);
   // thread -> (row, d-chunk): merge the NW wavefronts; with one split this is the final result
   for (int idx = threadIdx.x; idx < rows * (D / 4); idx += NW * 64) {
     const int row = idx / (D / 4), d4 = (idx % (D / 4)) * 4;
@@ -795,9 +814,12 @@ __global__ __launch_bounds__(NWT * 64) void attn_decode_kernel(const int* p_past
       half4 hv = {(_Float16)(acc[0] * inv), (_Float16)(acc[1] * inv), (_Float16)(acc[2] * inv), (_Float16)(acc[3] * inv)};
       *(half4*)dst = hv;
     } else {
-      float* dst = wsp + row * (D + 4);
-      *(float4v*)(dst + d4) = acc;
-      if (d4 == 0) { dst[D] = mm; dst[D + 1] = lt; }
+      auto leave = [&](auto scope) {
+        put_partial<D, RT, decltype(scope)::value>(parts, split, row, d4, acc);
+        if (d4 == 0) put_partial<D, RT, decltype(scope)::value>(parts, split, row, D, float2{mm, lt});
+      };
+      if (a.defer_combine) leave(std::integral_constant<int, 0>{});
+      else leave(std::integral_constant<int, AGENT_SCOPE>{});
     }
   }
   if (single || a.defer_combine) return;

@@ -510,10 +510,14 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_stream_kernel(const int* p_pa
         *(half4*)(a.out + out_at(b * q_total + token(row[t]), head(row[t]) * D + wave * CH + 16 * d + 4 * g, a.Hq * D, a.frag_mt)) = hv;
       }
     } else {
-      float* dst = a.ws + (((int64_t)bh * a.splits + split) * (RT * 16) + 16 * t + rr) * (D + 4);
+      const __amdgpu_buffer_rsrc_t parts = partials_of<D, RT>(a, bh);
+      auto leave = [&](auto scope) {
 #pragma unroll
-      for (int d = 0; d < DTW; ++d) *(float4v*)(dst + wave * CH + 16 * d + 4 * g) = o[t][d];
-      if (wave == 0 && g == 0) { dst[D] = m_all[t]; dst[D + 1] = lt; }
+        for (int d = 0; d < DTW; ++d) put_partial<D, RT, decltype(scope)::value>(parts, split, 16 * t + rr, wave * CH + 16 * d + 4 * g, o[t][d]);
+        if (wave == 0 && g == 0) put_partial<D, RT, decltype(scope)::value>(parts, split, 16 * t + rr, D, float2{m_all[t], lt});
+      };
+      if (a.defer_combine) leave(std::integral_constant<int, 0>{});
+      else leave(std::integral_constant<int, AGENT_SCOPE>{});
     }
   }
   if (single || a.defer_combine) return;

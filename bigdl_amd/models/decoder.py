@@ -25,6 +25,7 @@ import torch
 import torch.nn.functional as F
 
 from .. import qtypes as Q
+from ..ops import hip
 from ..transformers.low_bit_linear import FP4Params, GEMM_MAX_ROWS, GEMV_MAX_ROWS, dequant_weight
 
 
@@ -183,7 +184,6 @@ class Lin:
         """(W @ gamma, W @ beta) for the LayerNorm-folding GEMV, computed once per (weight, norm) pair."""
         key = (gamma.data_ptr(), None if beta is None else beta.data_ptr())
         if getattr(self, "_ln_key", None) != key:
-            from ..ops import hip
             dense, keep = Lin.cache_dense, getattr(self, "_dense", None)
             Lin.cache_dense = False                       # a transient dequantized copy, not the resident one
             try:
@@ -202,7 +202,6 @@ class Lin:
 
     def dense(self, dtype=torch.float16):
         if self.fused:
-            from ..ops import hip
             if Lin.cache_dense and dtype == torch.float16:
                 d = getattr(self, "_dense", None)
                 if d is None:
@@ -217,7 +216,6 @@ class Lin:
         low-bit tiles, which decode keeps using)."""
         w8 = getattr(self, "_fp8", None)
         if w8 is None:
-            from ..ops import hip
             d = hip.dequant_t16(self.w, self.qtype, self.n, self.k, dtype=torch.float16) if self.fused else self.w
             sw = d.abs().amax(dim=1, keepdim=True).float().clamp_min(1e-12) / 448.0
             w8 = self._fp8 = ((d.float() / sw).to(torch.float8_e4m3fn), sw)
@@ -277,7 +275,6 @@ class KVCache:
         self.batch = batch
         self.k_scale = self.v_scale = None
         if self.int4:
-            from ..ops import hip
             if cfg.head_dim not in hip.KV_INT4_HEAD_DIMS:
                 raise ValueError(f"the int4 KV cache needs head_dim in {hip.KV_INT4_HEAD_DIMS}, got {cfg.head_dim}")
             sk, sv, ssk, ssv = hip.kv_int4_shapes(batch, cfg.num_kv_heads, capacity, cfg.head_dim)
@@ -533,7 +530,6 @@ class NativeDecoder:
             return False
         if rows > GEMM_MAX_ROWS and not (prompt and self.prefill_fused and not Lin.cache_dense and not self.prefill_fp8):
             return False
-        from ..ops import hip
         return hip.gemm_lowbit_frag(rows, lin.n, lin.k, lin.qtype, None, w2 is not None, 3,
                                     then is not None and self._takes_frags(rows, then, None, prompt))
 
@@ -542,7 +538,6 @@ class NativeDecoder:
                 and self._takes_frags(rows, lw.gate, lw.up, True, lw.down))
 
     def _linear_dense(self, x, lin: Lin):
-        from ..ops import hip
         if type(x) is hip.Frags:
             return hip.gemm_lowbit(x, lin.w, lin.qtype, lin.n, lin.k, bias=lin.bias)
         if lin.fused and x.shape[0] <= GEMV_MAX_ROWS:
@@ -591,7 +586,6 @@ class NativeDecoder:
     def _linear_parts(self, x, lin: Lin, wanted=True):
         """``_linear_dense``, or with ``wanted`` (an RMSNorm that adds a residual is all that reads the result) the sums of the product with
         its K split, for that norm to add up, where that is faster"""
-        from ..ops import hip
         if wanted and lin.fused:
             if type(x) is hip.Frags:
                 p = hip.gemm_parts(x, lin.w, lin.qtype, lin.n, lin.k, bias=lin.bias)
@@ -608,7 +602,6 @@ class NativeDecoder:
     def _dense_ahead(self, lin: Lin):
         """fp16 form of ``lin``'s weight for a library GEMM on the current stream, valid until the next-but-one call.
         Starts the expansion of the weight that follows ``lin`` in a prompt pass on the side stream."""
-        from ..ops import hip
         a = self._ahead
         if a is None:
             plain = [lw for lw in self.layers if lw.mla is None and lw.moe is None]
@@ -677,7 +670,6 @@ class NativeDecoder:
         return torch.distributed.get_backend(self.tp_group) == "nccl"
 
     def _norm(self, x, w, b=None, residual=None, res_out=None):
-        from ..ops import hip
         if self.cfg.norm == "layer":
             return hip.layer_norm(x, w, b, self.cfg.rms_eps)
         return hip.rms_norm(x, w, self.cfg.rms_eps, offset=self.cfg.norm_offset, residual=residual, res_out=res_out)
@@ -686,7 +678,6 @@ class NativeDecoder:
         """(norm(h + add), h + add): the residual add rides in the RMSNorm launch (the prompt pass otherwise spends one
         elementwise launch per add: 64 of them, 0.37 ms, on a 1024-token Llama-2-7B prompt).  ``add`` None: (norm(h), h).
         ``frags``: an RMSNorm's result in fragment order, for the product that reads it."""
-        from ..ops import hip
         frags = frags and self.cfg.norm != "layer" and h.dtype == torch.float16
         if add is None:
             if frags:
@@ -703,7 +694,6 @@ class NativeDecoder:
 
     def _embed_extras(self, h, pos):
         """learned absolute positions and the embedding LayerNorm; h [rows, hidden], pos [rows] (device, int64)"""
-        from ..ops import hip
         if self.pos_embed is not None:
             h = h + F.embedding(pos + self.cfg.pos_offset, self.pos_embed)
         if self.embed_norm is not None:
@@ -712,7 +702,6 @@ class NativeDecoder:
 
     def _mlp_dense(self, x, lw, parts=False):
         """``parts``: the result may come back as ``hip.Parts`` (``_linear_parts``)"""
-        from ..ops import hip
         cfg = self.cfg
         if type(x) is hip.Frags:
             gt, up = lw.gate, lw.up
@@ -754,7 +743,6 @@ class NativeDecoder:
         S + slots rows together; attention runs per kind (flash kernel for the prompt, split-KV decode kernel for the
         slots).  Returns (prompt logits, decode logits [slots, V], next tokens [slots]) and advances every active
         slot by one token exactly like ``decode(None, 1, chain=True)``."""
-        from ..ops import hip
         cfg, cache = self.cfg, self.cache
         if not self.stage_first:
             assert hidden is not None and not with_decode, "a later pipeline stage is fed hidden states [B, S, hidden]"
@@ -941,7 +929,6 @@ class NativeDecoder:
         Pipeline stages: a later stage passes ``prompts=None`` with ``hidden`` [rows, hidden] (the previous stage's
         output for the same packed rows) and ``lens``; a stage that is not the last returns its [rows, hidden] output
         instead of logits."""
-        from ..ops import hip
         cfg, cache = self.cfg, self.cache
         if not self.stage_first:
             assert hidden is not None and lens is not None and not with_decode, "a later stage is fed packed hidden rows"
@@ -1035,7 +1022,6 @@ class NativeDecoder:
 
     def _mla_qkv_dense(self, x, m: MLAWeights):
         """prompt rows: normed hidden [rows, hidden] -> qkv [rows, 3 * heads * head_dim] (un-rotated)"""
-        from ..ops import hip
         cfg = self.cfg
         rows, qs, r = x.shape[0], cfg.q_size, cfg.rot_dim
         qkv = torch.empty(rows, 3 * qs, dtype=torch.float16, device=self.device)
@@ -1069,7 +1055,6 @@ class NativeDecoder:
     def _decode_attention(self, qkv, li, lw, st, batch):
         """split-KV decode attention (+ RoPE and cache append) of one token per slot, outside the graph; qkv
         [batch, q + 2 kv] rows of a larger pass.  Returns [batch, q_size]."""
-        from ..ops import hip
         cfg, cache = self.cfg, self.cache
         qkv = qkv.contiguous()
         out = torch.empty(batch, cfg.q_size, dtype=torch.float16, device=self.device)
@@ -1093,7 +1078,6 @@ class NativeDecoder:
         cache per layer, attention runs per chunk over the keys before it.  ``input_ids`` [1, S] is the full prompt on
         every rank, S a multiple of 2 * world; the cache must be empty.  Returns the last token's logits [1, 1, V] on
         every rank; afterwards every rank holds the complete KV cache and can decode."""
-        from ..ops import hip
         from ..parallel import context_parallel as cp
         cfg, cache = self.cfg, self.cache
         assert not cache.int4, "context-parallel prefill gathers fp16 / e5m2 caches"
@@ -1161,7 +1145,6 @@ class NativeDecoder:
 
     def _read_cache(self, li, length, slot=None):
         """-> (K [B,Hkv,L,D], V^T [B,Hkv,D,L]) in fp16"""
-        from ..ops import hip
         c = self.cache
         rows = slice(None) if slot is None else slice(slot, slot + 1)
         if c.int4:
@@ -1181,7 +1164,6 @@ class NativeDecoder:
         views of the fp8 cache (bytes).  ``frags``: in fragment order where the kernel of this package runs"""
         cfg = self.cfg
         if cfg.head_dim in (64, 96, 128, 256) and vt.stride(2) % 8 == 0 and vt.data_ptr() % 16 == 0:
-            from ..ops import hip
             return hip.attn_prefill(q, k, vt, scale=self.attn_scale, causal=True, softcap=cfg.attn_softcap, window=window,
                                     v_transposed=True, alibi=self.alibi, kv_e5m2=kv_e5m2, frags=frags)
         assert not kv_e5m2
@@ -1214,7 +1196,6 @@ class NativeDecoder:
 
     # ------------------------------------------------------------------ decode (graph)
     def _build_static(self, batch: int, q_len: int):
-        from ..ops import hip
         cfg = self.cfg
         m = batch * q_len
         dev = self.device
@@ -1265,7 +1246,6 @@ class NativeDecoder:
         (a tensor or None, instead of the default False) selects LayerNorm(gamma, beta) as the norm.  ``then``: the product that alone
         reads a pair's result; where it takes x in fragment order the result comes back so, and not in ``out``.  ``add`` (``hip.Parts``, where
         ``_norm_first``): what is still to be added to x, by the norm in front."""
-        from ..ops import hip
         cfg = self.cfg
         m = x.shape[0]
 
@@ -1377,7 +1357,6 @@ class NativeDecoder:
         return self._gemv(h, lw.up, a, gamma=gamma, beta=beta, act=cfg.act, add=add)
 
     def _decode_body(self, st, batch: int, q_len: int, chain: bool):
-        from ..ops import hip
         cfg, cache = self.cfg, self.cache
         h, qkv, attn, act, tmp = st["h"], st["qkv"], st["attn"], st["act"], st["tmp"]
         self.fold_batched_norm = (batch * q_len > GEMV_MAX_ROWS and cfg.norm != "layer" and self.tp_group is None
@@ -1588,7 +1567,6 @@ class NativeDecoder:
         padding (left or right): every row becomes a cache slot with its own length -- the prompts run packed in one
         pass without their pad tokens, positions count from each row's first real token, and the decode steps read
         the per-slot lengths on the device."""
-        from ..ops import hip
         dev = self.device
         input_ids = input_ids.to(dev)
         b, s = input_ids.shape

@@ -78,6 +78,15 @@ __device__ __forceinline__ float block_sum(float v, float* sh) {
   __syncthreads();
   return t;
 }
+// of 256 threads, called once: the barrier waits for LDS alone, not for the stores in front of it
+__device__ __forceinline__ float block_sum_once(float v, float* sh) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  return ((sh[0] + sh[1]) + sh[2]) + sh[3];
+}
 __device__ __forceinline__ float block_max(float v, float* sh) {
   v = wave_max(v);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -93,105 +102,122 @@ __device__ __forceinline__ float block_max(float v, float* sh) {
 // summed residual stream back (res_out) -- one row per workgroup, row kept in registers.  frag_mt > 0: the result goes out in
 // fragment order (gemm_frag_kernel.h) of frag_mt 16-row tiles, 16 bytes a thread and 256 bytes apart: it saves the pass of 3.5 us
 // that would order it, at no change of its own time (64 x 4096: 5.1 us) ----
-template <int DT, int VPT>  // VPT: 8-element vectors per thread
+// A few rows are latencies one behind the other: x, the residual and the weight are requested together, without a branch (places behind the end
+// read the row's last ones and store nothing), in front of the first store, which would hold up the loads behind it; the barrier does not
+// wait for that store.  With a residual, us in a row of launches: 64 x 4096 3.3 -> 2.7, 512 x 4096 4.6 -> 4.1, 1024 x 4096 6.0, 256 x 8192
+// 5.4 -> 4.4, 64 x 16384 7.2 -> 5.0; without 2.9 -> 2.6, 3.5 -> 3.3, 4.4 -> 4.2, 4.2 -> 3.5, 5.6 -> 4.5.
+template <int DT, int VPT, bool ADD>  // VPT: 8-element vectors per thread; ADD: a residual
 __global__ __launch_bounds__(256) void rms_norm_kernel(const void* x, const void* residual, const void* w, void* out,
                                                        void* res_out, int H, int64_t ldx, float eps, float offset, int frag_mt) {
   __shared__ float sh[8];
   const int64_t row = blockIdx.x;
-  float v[VPT][8];
+  float v[VPT][8], r[VPT][8], g[VPT][8];
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int c = min((int)(threadIdx.x + i * 256) * 8, H - 8);
+    load8<DT>(x, row * ldx + c, v[i]);
+    if constexpr (ADD) load8<DT>(residual, row * (int64_t)H + c, r[i]);
+    load8<DT>(w, c, g[i]);
+  }
   float ss = 0.0f;
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    const int c = (threadIdx.x + i * 256) * 8;
-    if (c < H) {
-      load8<DT>(x, row * ldx + c, v[i]);
-      if (residual) {
-        float r[8];
-        load8<DT>(residual, row * (int64_t)H + c, r);
+    const bool on = (threadIdx.x + i * 256) * 8 < H;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[i][j] += r[j];
-      }
-      if (res_out) store8<DT>(res_out, row * (int64_t)H + c, v[i]);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ss += v[i][j] * v[i][j];
+    for (int j = 0; j < 8; ++j) {
+      if constexpr (ADD) v[i][j] += r[i][j];
+      ss += on ? v[i][j] * v[i][j] : 0.0f;
     }
+    if (res_out && on) store8<DT>(res_out, row * (int64_t)H + (threadIdx.x + i * 256) * 8, v[i]);
   }
-  const float rs = rsqrtf(block_sum(ss, sh) / (float)H + eps);
+  const float rs = rsqrtf(block_sum_once(ss, sh) / (float)H + eps);
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
     const int c = (threadIdx.x + i * 256) * 8;
     if (c < H) {
-      float g[8];
-      load8<DT>(w, c, g);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[i][j] = v[i][j] * rs * (g[j] + offset);
+      for (int j = 0; j < 8; ++j) v[i][j] = v[i][j] * rs * (g[i][j] + offset);
       store8<DT>(out, frag_mt > 0 ? frag_at((int)row, c, frag_mt) : row * (int64_t)H + c, v[i]);
     }
   }
 }
 
 // The same of a product whose K was split, fp16: out = norm(sum of the slabs [parts][rows][H] fp32 [+ bias] [+ residual]).  The sums are added
-// here, in fp32, where a launch of its own wrote and re-read them.  What it costs is the slabs' bytes: all of a thread's pieces are requested
-// together, up to four slabs at a time.
-template <int VPT>
+// here, in fp32, where a launch of its own wrote and re-read them.  P: the parts, all of them requested together with everything else (77 x
+// 4096, 2 / 3 / 4 parts 3.7 / 4.1 / 4.1 -> 3.2 / 3.4 / 3.5 us; 1024 x 4096, bound by the slabs, 10.8 / 13.7 / 16.1 -> 10.3 / 12.7 / 15.1); 0: any
+// number, up to four at a time.
+template <int VPT, int P>
 __global__ __launch_bounds__(256) void rms_norm_parts_kernel(const float* x, int parts, int64_t stride, const _Float16* bias, const void* residual,
                                                              const void* w, void* out, void* res_out, int H, float eps, float offset, int frag_mt) {
   __shared__ float sh[8];
   const int64_t row = blockIdx.x;
-  float v[VPT][8];
-  float ss = 0.0f;
+  float v[VPT][8], g[VPT][8], s[VPT][8];
+  half8 r[VPT], b[VPT];
+  // (no residual, no bias: the weight in their place, not added)
+  const _Float16* rp = residual ? (const _Float16*)residual + row * (int64_t)H : (const _Float16*)w;
+  const _Float16* bp = bias ? bias : (const _Float16*)w;
+  auto at = [&](int i) { return min((int)(threadIdx.x + i * 256) * 8, H - 8); };
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    const int c = (threadIdx.x + i * 256) * 8;
+    r[i] = *(const half8*)(rp + at(i));
+    b[i] = *(const half8*)(bp + at(i));
+  }
+  if constexpr (P > 0) {
+    float a[VPT][P][8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[i][j] = 0.0f;
-    if (c < H) {
-      const float* p = x + row * (int64_t)H + c;
-      if (residual) load8<DT_F16>(residual, row * (int64_t)H + c, v[i]);
-      if (bias) {
-        float b[8];
-        load8<DT_F16>(bias, c, b);
+    for (int i = 0; i < VPT; ++i)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[i][j] += b[j];
-      }
-      float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+      for (int e = 0; e < P; ++e) load8<DT_F32>(x + row * (int64_t)H + at(i), e * stride, a[i][e]);
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) load8<DT_F16>(w, at(i), g[i]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < VPT; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        s[i][j] = P == 4 ? (a[i][0][j] + a[i][1][j]) + (a[i][2][j] + a[i][P - 1][j])
+                         : P == 3 ? (a[i][0][j] + a[i][1][j]) + a[i][P - 1][j] : a[i][0][j] + a[i][P - 1][j];
+  } else {
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      const float* p = x + row * (int64_t)H + at(i);
+      load8<DT_F16>(w, at(i), g[i]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s[i][j] = 0.0f;
       int k = 0;
       for (; k + 4 <= parts; k += 4) {
         float a[4][8];
 #pragma unroll
         for (int e = 0; e < 4; ++e) load8<DT_F32>(p, (k + e) * stride, a[e]);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) s[j] += (a[0][j] + a[1][j]) + (a[2][j] + a[3][j]);
+        for (int j = 0; j < 8; ++j) s[i][j] += (a[0][j] + a[1][j]) + (a[2][j] + a[3][j]);
       }
-      for (; k + 2 <= parts; k += 2) {
-        float a[2][8];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) load8<DT_F32>(p, (k + e) * stride, a[e]);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) s[j] += a[0][j] + a[1][j];
-      }
-      if (k < parts) {
+      for (; k < parts; ++k) {
         float a[8];
         load8<DT_F32>(p, k * stride, a);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) s[j] += a[j];
+        for (int j = 0; j < 8; ++j) s[i][j] += a[j];
       }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[i][j] += s[j];
-      if (res_out) store8<DT_F16>(res_out, row * (int64_t)H + c, v[i]);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ss += v[i][j] * v[i][j];
     }
   }
-  const float rs = rsqrtf(block_sum(ss, sh) / (float)H + eps);
+  float ss = 0.0f;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const bool on = (threadIdx.x + i * 256) * 8 < H;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      v[i][j] = ((residual ? (float)r[i][j] : 0.0f) + (bias ? (float)b[i][j] : 0.0f)) + s[i][j];
+      ss += on ? v[i][j] * v[i][j] : 0.0f;
+    }
+    if (res_out && on) store8<DT_F16>(res_out, row * (int64_t)H + at(i), v[i]);
+  }
+  const float rs = rsqrtf(block_sum_once(ss, sh) / (float)H + eps);
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
     const int c = (threadIdx.x + i * 256) * 8;
     if (c < H) {
-      float g[8];
-      load8<DT_F16>(w, c, g);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[i][j] = v[i][j] * rs * (g[j] + offset);
+      for (int j = 0; j < 8; ++j) v[i][j] = v[i][j] * rs * (g[i][j] + offset);
       store8<DT_F16>(out, frag_mt > 0 ? frag_at((int)row, c, frag_mt) : row * (int64_t)H + c, v[i]);
     }
   }
@@ -614,11 +640,15 @@ extern "C" int bigdl_rms_norm(const void* x, const void* residual, const void* w
   if (frag && (dtype != DT_F16 || (H & 127) || rows > 1 << 20)) return -1;
   const int mt = frag ? (int)((rows + 15) / 16) : 0;
   const int vpt = (H / 8 + 255) / 256;
+#define NORM_LAUNCH(V, ADD) hipLaunchKernelGGL((rms_norm_kernel<DT, V, ADD>), dim3(rows), dim3(256), 0, st, x, residual, w, out, res_out, H, ldx, eps, offset, mt)
+#define NORM_OF(V) { if (residual) NORM_LAUNCH(V, true); else NORM_LAUNCH(V, false); }
   DISPATCH_DT(dtype,
-    if (vpt <= 1) hipLaunchKernelGGL((rms_norm_kernel<DT, 1>), dim3(rows), dim3(256), 0, st, x, residual, w, out, res_out, H, ldx, eps, offset, mt);
-    else if (vpt <= 2) hipLaunchKernelGGL((rms_norm_kernel<DT, 2>), dim3(rows), dim3(256), 0, st, x, residual, w, out, res_out, H, ldx, eps, offset, mt);
-    else if (vpt <= 4) hipLaunchKernelGGL((rms_norm_kernel<DT, 4>), dim3(rows), dim3(256), 0, st, x, residual, w, out, res_out, H, ldx, eps, offset, mt);
-    else hipLaunchKernelGGL((rms_norm_kernel<DT, 8>), dim3(rows), dim3(256), 0, st, x, residual, w, out, res_out, H, ldx, eps, offset, mt))
+    if (vpt <= 1) NORM_OF(1)
+    else if (vpt <= 2) NORM_OF(2)
+    else if (vpt <= 4) NORM_OF(4)
+    else NORM_OF(8))
+#undef NORM_OF
+#undef NORM_LAUNCH
   return HIP_CHECK_LAUNCH();
 }
 
@@ -632,12 +662,20 @@ extern "C" int bigdl_rms_norm_parts(const float* x, int parts, const void* bias,
   const int mt = frag ? (int)((rows + 15) / 16) : 0;
   const int vpt = (H / 8 + 255) / 256;
   const int64_t stride = rows * (int64_t)H;
-#define PARTS_LAUNCH(V) hipLaunchKernelGGL((rms_norm_parts_kernel<V>), dim3(rows), dim3(256), 0, st, x, parts, stride, (const _Float16*)bias, \
-                                           residual, w, out, res_out, H, eps, offset, mt)
-  if (vpt <= 1) PARTS_LAUNCH(1);
-  else if (vpt <= 2) PARTS_LAUNCH(2);
-  else if (vpt <= 4) PARTS_LAUNCH(4);
-  else PARTS_LAUNCH(8);
+#define PARTS_LAUNCH(V, P) hipLaunchKernelGGL((rms_norm_parts_kernel<V, P>), dim3(rows), dim3(256), 0, st, x, parts, stride, (const _Float16*)bias, \
+                                              residual, w, out, res_out, H, eps, offset, mt)
+#define PARTS_OF(V)                  \
+  switch (parts) {                   \
+    case 2: PARTS_LAUNCH(V, 2); break; \
+    case 3: PARTS_LAUNCH(V, 3); break; \
+    case 4: PARTS_LAUNCH(V, 4); break; \
+    default: PARTS_LAUNCH(V, 0);     \
+  }
+  if (vpt <= 1) { PARTS_OF(1) }
+  else if (vpt <= 2) { PARTS_OF(2) }
+  else if (vpt <= 4) PARTS_LAUNCH(4, 0);
+  else PARTS_LAUNCH(8, 0);
+#undef PARTS_OF
 #undef PARTS_LAUNCH
   return HIP_CHECK_LAUNCH();
 }

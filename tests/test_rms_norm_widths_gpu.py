@@ -1,0 +1,47 @@
+"""RMSNorm at the edges of a thread's pieces (256 threads of eight elements): against 64 bits, sums in place, with and without a residual."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,h", [(1, 8), (5, 2040), (5, 2048), (3, 2056), (2, 4096), (3, 8184), (2, 16384)])
+def test_widths(rows, h, dtype):
+    from bigdl_amd.ops import hip
+    g = torch.Generator(device="cuda").manual_seed(h)
+    x, r, w = (torch.randn(*s, device="cuda", generator=g).to(dtype) for s in ((rows, h), (rows, h), (h,)))
+    ulp = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -23}[dtype]
+
+    def ref(t):
+        return t * torch.rsqrt(t.pow(2).mean(-1, keepdim=True) + 1e-5) * (w.double() + 1.0)
+
+    # one rounding of the result; fp32 sums of squares (2^-24 times the depth of the sum) and a handful of fp32 operations: 2^-20
+    plain = ref(x.double())
+    assert ((hip.rms_norm(x, w, 1e-5, offset=1.0).double() - plain).abs() <= plain.abs() * (ulp + 2.0 ** -20) + 1e-7).all()
+    total = x.double() + r.double()
+    want = ref(total)
+    added = r.clone()
+    got = hip.rms_norm(x, w, 1e-5, offset=1.0, residual=added, res_out=added)          # the residual stream is summed in place
+    assert ((got.double() - want).abs() <= want.abs() * (ulp + 2.0 ** -20) + 1e-7).all()
+    assert ((added.double() - total).abs() <= total.abs() * ulp + 1e-7).all()
+
+
+@pytest.mark.parametrize("parts", [1, 2, 3, 4, 5, 9])
+@pytest.mark.parametrize("rows,h", [(1, 8), (5, 2056), (3, 4096), (2, 8200)])
+def test_parts(rows, h, parts):
+    from bigdl_amd.ops import hip
+    g = torch.Generator(device="cuda").manual_seed(h + parts)
+    slabs = torch.randn(parts, rows, h, device="cuda", generator=g)
+    r, w, bias = (torch.randn(*s, device="cuda", generator=g).half() for s in ((rows, h), (h,), (h,)))
+    for b in (None, bias):
+        for res in (None, r):
+            total = slabs.double().sum(0) + (0 if b is None else b.double()) + (0 if res is None else res.double())
+            want = total * torch.rsqrt(total.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
+            added = torch.empty_like(r)
+            got = hip.rms_norm(hip.Parts(slabs, b), w, 1e-5, residual=res, res_out=added)
+            # as above; a sum that cancels keeps the error of its terms: 2^-23 of their magnitudes, scaled like the result
+            mag = slabs.double().abs().sum(0) + 8
+            scale = (want / total).abs().nan_to_num(0, 0, 0)
+            assert ((got.double() - want).abs() <= want.abs() * (2.0 ** -11 + 2.0 ** -20) + mag * scale * 2.0 ** -22 + 1e-7).all()
+            assert ((added.double() - total).abs() <= total.abs() * 2.0 ** -11 + mag * 2.0 ** -22).all()

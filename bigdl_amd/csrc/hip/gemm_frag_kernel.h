@@ -1,9 +1,10 @@
 // Dequant-fused product on x in fragment order for gfx950:  y[M,N] = f(x[M,K] . dequant(W)[N,K]^T), 33 to 512 rows, and up to
 // FRAG_MAX_ROWS where K is no multiple of 128: short prompts, wide decode batches, module calls.
 //
-// What bounds products of so many rows is neither the weights (28 MB for Llama-2-7B's qkv, 6 us) nor the matrix cores (64 rows:
-// 5 us) but x, which every workgroup pulls through its CU's L1.  Measured rates per CU, x in L2: 70 GB/s for requests of 8 rows x
-// 128 bytes, 29 for MFMA fragments straight from rows (16 rows x 64 bytes), 105 - 120 for whole contiguous KiB.  Hence:
+// What bounds products of so many rows is neither the weights (28 MB for Llama-2-7B's qkv, 6 us) nor the matrix cores alone (64 rows: 5 us).
+// In rows it is x, which every workgroup pulls through its CU's L1: rates per CU, x in L2, 70 GB/s for requests of 8 rows x 128 bytes, 29
+// for MFMA fragments straight from rows (16 rows x 64 bytes), 105 - 120 for whole contiguous KiB.  In the last form what remains is mostly
+// instructions: without any memory access 73 - 87 % of the time (77 x 14336 pair 30.4 of 35.1 us, 203 x 4672 x 4544 19.6 of 26).  Hence:
 //  * x comes in fragment order: [k / 32][row / 16][lane][8 halves], 1 KiB that a wavefront requests at once and multiplies as it
 //    arrives -- no LDS, no swizzle, no barrier in the loop.  A pass of 3.5 us puts rows into that order (frag_pack_kernel; for
 //    bf16 rows in place of their conversion), unless the producer of x writes it so.
@@ -16,9 +17,8 @@
 //    which it does not keep, are for the only row block: 203 rows, three blocks: 24.0 -> 22.4 us; 64 rows, one: 16.0 <- 15.6).
 // One MI355X, us, kernels of before (few-row / tile kernel) -> this one, without the pass over x: gate / up pair of 14336 x 4096,
 // 77 rows, asym_int4 67.6 -> 32; 4672 x 4544, 203 rows, sym_int8 38.7 -> 22; sym_int4 4096 x 4096 at 64 / 256 / 400 rows 12.4 -> 9.6,
-// 23.1 -> 14.3, 31.3 -> 20.1; 4096 x 11008 at 256 rows 39.2 -> 29.1.  The rest: 60 GB/s a CU with weights from memory in between (an L1
-// that returns loads in order lets x wait behind them), 4 us of launch and first loads, 2 us of the exchange.  Depth of look-ahead,
-// 4 / 8 / 16 wavefronts and the order of arithmetic and loads change it by 3 %.
+// 23.1 -> 14.3, 31.3 -> 20.1; 4096 x 11008 at 256 rows 39.2 -> 29.1.  Depth of look-ahead, 4 / 8 / 16
+// wavefronts, the order of arithmetic and loads and decoding between the products of the fragment before change it by 3 %.
 #pragma once
 #include "gemm_rows_kernel.h"
 

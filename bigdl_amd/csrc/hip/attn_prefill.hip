@@ -741,7 +741,7 @@ struct PrefillRopeArgs {
   int hpb, qk_blocks;                                  // q / k heads per workgroup (0: the general form, one), workgroups of q / k heads per 64 tokens
 };
 
-constexpr int PR_TOK = 64;
+constexpr int PR_TOK = 64, PR_FEW = 16;       // tokens of a workgroup; of a small launch's
 
 // Rotate-half over a whole head of D channels: a thread holds the cosines and sines of its 8 channel pairs of 64 / TP tokens and takes
 // the workgroup's heads one after the other, two requested at a time.  (The general form below reads the table for every head, twice
@@ -819,10 +819,10 @@ __device__ __forceinline__ void rope_whole_heads(const PrefillRopeArgs& a, int t
 
 // WHOLE: q and k heads as above, where the workgroups of a launch are many; a kernel of its own, since its registers leave fewer wavefronts
 // to the general form (3 x 16 + 2 heads of 128, 1024 tokens 10.7 us in one kernel, 9.0 in two)
-template <bool WHOLE>
+template <bool WHOLE, int TOK>
 __global__ __launch_bounds__(256) void prefill_rope_append_kernel(PrefillRopeArgs a) {
-  __shared__ __attribute__((aligned(16))) _Float16 tile[PR_TOK * (256 + 8)];   // V transpose staging, D <= 256
-  const int t0 = blockIdx.x * PR_TOK, b = blockIdx.z;
+  __shared__ __attribute__((aligned(16))) _Float16 tile[TOK * (256 + 8)];   // V transpose staging, D <= 256
+  const int t0 = blockIdx.x * TOK, b = blockIdx.z;
   if (WHOLE && (int)blockIdx.y < a.qk_blocks) {
     const int head0 = blockIdx.y * a.hpb, n = min(a.hpb, a.Hq + a.Hkv - head0);
     if (a.D == 64) rope_whole_heads<64>(a, t0, head0, n, b);
@@ -836,7 +836,7 @@ __global__ __launch_bounds__(256) void prefill_rope_append_kernel(PrefillRopeArg
   if (is_q || is_k) {
     const int hk = head - a.Hq;
     const int half_rot = a.rot / 2;
-    for (int it = threadIdx.x; it < PR_TOK * CH; it += 256) {
+    for (int it = threadIdx.x; it < TOK * CH; it += 256) {
       const int tl = it / CH, c = it % CH, t = t0 + tl;
       if (t >= a.S) continue;
       const int d0 = 8 * c;
@@ -897,17 +897,17 @@ __global__ __launch_bounds__(256) void prefill_rope_append_kernel(PrefillRopeArg
   // rows 8 apart are a multiple of 32 banks apart, so the 16-byte chunk index is XOR-ed with the token group to
   // spread the 8 groups over all banks (needs the chunk count to be a multiple of 8)
   const int swz = (CH & 7) == 0 ? 7 : 0;
-  for (int it = threadIdx.x; it < PR_TOK * CH; it += 256) {
+  for (int it = threadIdx.x; it < TOK * CH; it += 256) {
     const int tl = it / CH, c = it % CH, t = t0 + tl;
     half8 v = {0, 0, 0, 0, 0, 0, 0, 0};
     if (t < a.S) v = *(const half8*)(base + (int64_t)t * a.ld + 8 * c);
     *(half8*)(tile + tl * TS + 8 * (c ^ ((tl >> 3) & swz))) = v;
   }
   __syncthreads();
-  const int ntok = min(PR_TOK, a.S - t0);
+  const int ntok = min(TOK, a.S - t0);
   // each item: one d row, 8 consecutive tokens
-  for (int it = threadIdx.x; it < D * (PR_TOK / 8); it += 256) {
-    const int d = it / (PR_TOK / 8), tc = it % (PR_TOK / 8);
+  for (int it = threadIdx.x; it < D * (TOK / 8); it += 256) {
+    const int d = it / (TOK / 8), tc = it % (TOK / 8);
     if (8 * tc >= ntok) continue;
     half8 v;
 #pragma unroll
@@ -1036,9 +1036,16 @@ extern "C" int bigdl_prefill_rope_append(void* qkv, void* kc, void* vc, void* vt
   const bool whole = per >= 1 && rot == D && !interleaved && (D == 64 || D == 128) && ((uintptr_t)table & 15) == 0;
   a.hpb = !whole ? 0 : per > 8 ? 8 : (int)per;
   a.qk_blocks = whole ? (Hq + Hkv + a.hpb - 1) / a.hpb : Hq + Hkv;
-  const dim3 grid((S + PR_TOK - 1) / PR_TOK, a.qk_blocks + Hkv, B);
-  if (whole) hipLaunchKernelGGL(prefill_rope_append_kernel<true>, grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL(prefill_rope_append_kernel<false>, grid, dim3(256), 0, st, a);
+  // Few workgroups: a quarter of the tokens each, so that what a thread does is one round of loads and stores and not four (two at 64
+  // channels), one behind the other.  us, 64 -> 16 tokens, 32 + 2 x 8 heads of 128, fp16 / e5m2 cache: 16 tokens 3.4 -> 2.4 / 4.9 -> 2.9, 77 5.4 -> 2.9 /
+  // 11.8 -> 3.8, 320 4.9 -> 3.8 / 6.9 -> 4.4, 700 6.9 -> 5.7 / 10.5 -> 6.8, 3 x 300 (720 workgroups of 64) 7.9 -> 6.9 / 12.1 -> 8.1; of 256, 600 tokens (480)
+  // 11.8 -> 8.4 / 15.5 -> 10.9, 1000 (768) 13.0 -> 13.5 / 16.8 -> 17.1; of 64, 1000 (640) 3.8 -> 4.1 / 4.5 -> 4.6; 4 x 400 of 128 (2688) 16.6 -> 17.6 / 19.1 -> 20.6.
+  const bool few = !whole && (int64_t)((S + PR_TOK - 1) / PR_TOK) * B * (Hq + 2 * Hkv) < 6 * (D < 128 ? D : 128);
+  const int tok = few ? PR_FEW : PR_TOK;
+  const dim3 grid((S + tok - 1) / tok, a.qk_blocks + Hkv, B);
+  if (whole) hipLaunchKernelGGL((prefill_rope_append_kernel<true, PR_TOK>), grid, dim3(256), 0, st, a);
+  else if (few) hipLaunchKernelGGL((prefill_rope_append_kernel<false, PR_FEW>), grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((prefill_rope_append_kernel<false, PR_TOK>), grid, dim3(256), 0, st, a);
   return HIP_CHECK_LAUNCH();
 }
 

@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const void* x, const void
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       if constexpr (ADD) v[i][j] += r[i][j];
-      ss += on ? v[i][j] * v[i][j] : 0.0f;
+      ss = on ? fmaf(v[i][j], v[i][j], ss) : ss;      // (the sum is selected, not the square: that would be rounded by itself)
     }
     if (res_out && on) store8<DT>(res_out, row * (int64_t)H + (threadIdx.x + i * 256) * 8, v[i]);
   }
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(256) void rms_norm_parts_kernel(const float* x, int
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       v[i][j] = ((residual ? (float)r[i][j] : 0.0f) + (bias ? (float)b[i][j] : 0.0f)) + s[i][j];
-      ss += on ? v[i][j] * v[i][j] : 0.0f;
+      ss = on ? fmaf(v[i][j], v[i][j], ss) : ss;
     }
     if (res_out && on) store8<DT_F16>(res_out, row * (int64_t)H + at(i), v[i]);
   }

@@ -451,12 +451,13 @@ extern "C" int bigdl_gemm_parts(int M, int N, int K, int ldx, int qtype, int x_k
   return splits > 1 ? splits : 0;
 }
 
-// that product: partial [bigdl_gemm_parts][M][N] fp32, 16-byte aligned.  x as there, 16-byte aligned.
+// that product: partial [bigdl_gemm_parts][M][N] fp32, 16-byte aligned, `floats` of them.  x as there, 16-byte aligned.  (A scratch of any
+// other size is refused, a larger one too: the norm adds up all the slabs that it is given.)
 extern "C" int bigdl_gemm_parts_run(const void* x, const void* w, float* partial, int64_t floats, int M, int N, int K, int ldx, int qtype,
                                     int x_kind, hipStream_t stream) {
   const int splits = bigdl_gemm_parts(M, N, K, ldx, qtype, x_kind);
   if (splits < 2) return -4;
-  if (partial == nullptr || floats < (int64_t)splits * M * N) return -5;
+  if (partial == nullptr || floats != (int64_t)splits * M * N) return -5;
   if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)partial & 15)) return -1;
   qtype = t16_kernel_qtype(qtype);
   if (x_kind != X_FRAGMENTS) return prompt_parts_launch(x, w, partial, M, N, K, ldx, qtype, stream);

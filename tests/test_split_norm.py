@@ -33,6 +33,40 @@ def test_rule(qt):
     assert L.bigdl_gemm_parts(64, 4096, 14336, 14336, qt, 2) > 1          # 128 column tiles of a long K: half the chip without
 
 
+@needs_library
+@pytest.mark.parametrize("m,n,k,kind", [(64, 4096, 14336, 2), (1024, 4096, 11008, 0)])
+def test_only_the_planned_scratch(m, n, k, kind):
+    """a scratch of fewer or more slabs than the plan writes is refused, by the first of the checks (the addresses are odd ones, which the
+    next refuses: no launch comes of this)"""
+    L = hip.lib()
+    s = L.bigdl_gemm_parts(m, n, k, k, Q.SYM_INT4, kind)
+    assert s > 1
+    for floats in (0, (s - 1) * m * n, s * m * n - 1, s * m * n + 1, (s + 1) * m * n):
+        assert L.bigdl_gemm_parts_run(4104, 4104, 4104, floats, m, n, k, k, Q.SYM_INT4, kind, None) == -5
+    assert L.bigdl_gemm_parts_run(4104, 4104, 4104, s * m * n, m, n, k, k, Q.SYM_INT4, kind, None) == -1
+
+
+@pytest.mark.gpu
+def test_another_plan_between_two_calls():
+    m, n, k = 700, 1024, 14336
+    dev, w = _weight(n, k, Q.SYM_INT4, 8)
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(9)).half()
+    ref, mag = x.double() @ w.t(), x.double().abs() @ w.abs().t()
+    xg = x.cuda()
+    try:
+        for splits in (0, 2, 3, 1, 0):
+            hip.gemm_prompt_force(-1, splits)
+            torch.full((16 << 20,), float("nan"), device="cuda")               # (what the next allocation holds)
+            p = hip.gemm_parts(xg, dev, Q.SYM_INT4, n, k)
+            if splits == 1:
+                assert p is None
+                continue
+            assert p.data.shape[0] == (splits or hip.lib().bigdl_gemm_parts(m, n, k, k, Q.SYM_INT4, 0))
+            assert ((p.data.double().sum(0).cpu() - ref).abs() <= 2.0 ** -9 * mag + 1e-5).all(), splits
+    finally:
+        hip.gemm_prompt_force()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("parts", [1, 2, 3, 4, 7])
 @pytest.mark.parametrize("rows,h", [(1, 8), (5, 128), (33, 2304), (70, 4096), (3, 16384)])

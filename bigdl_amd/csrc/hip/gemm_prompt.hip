@@ -49,20 +49,20 @@ static int g_force_cfg = -1, g_force_sk = 0;         // bigdl_gemm_prompt_force 
 
 // Turns of 256 tiles, each its k tiles and its first requests and epilogue; K splits add the fp32 slabs' traffic and the reduce launch.
 // 128 x 128 tiles run two to a CU where there are more than 256 (a lone one is 1.24 times as long, not half as long, as two).
-static double plan_us(int M, int N, bool pair, int cfg, int splitk, int kt_per_split, double fmt, bool sums_left = false) {
+static double plan_us(int M, int N, bool pair, int cfg, int splitk, int kt_per_split, double fmt) {
   const PromptCfg& pc = kPromptCfgs[cfg];
   const int bno = pair ? pc.bn / 2 : pc.bn;
   const int64_t tiles = (int64_t)((M + pc.bm - 1) / pc.bm) * ((N + bno - 1) / bno), turns = (tiles * splitk + 255) / 256;
   const double lone = pc.bm == 128 && turns == 1 ? 1.24 : 1.0;
   double us = 1.3 + (double)turns * (pc.kt_us * (pair ? 1.02 : 1.0) * fmt * lone * kt_per_split + pc.tile_us * (pair ? 1.15 : 1.0));
-  if (splitk > 1) us += sums_left ? 0.5 + 0.9e-6 * splitk * (double)M * N : 5.2 + 1.07e-6 * splitk * (double)M * N;
+  if (splitk > 1) us += 5.2 + 1.07e-6 * splitk * (double)M * N;
   return us;
 }
 
 // The fastest plan by its estimated time.
 // pair: the gate / up form (two products per output column: blocks cover bn / 2 output columns, no K split)
 // forced_cfg >= 0, forced_sk > 0: only plans of these
-static PromptPlan prompt_plan_of(int M, int N, int K, bool pair, int forced_cfg, int forced_sk, bool sums_left = false) {
+static PromptPlan prompt_plan_of(int M, int N, int K, bool pair, int forced_cfg, int forced_sk) {
   const int KT = K >> 7;
   PromptPlan best = {0, 1, KT, 1e300};
   for (int c = 0; c < PROMPT_NCFG; ++c) {
@@ -71,17 +71,17 @@ static PromptPlan prompt_plan_of(int M, int N, int K, bool pair, int forced_cfg,
       if (forced_sk ? sk != forced_sk : (sk > 1 && KT / sk < 6)) continue;
       if (sk > KT) continue;
       const int per = (KT + sk - 1) / sk, rsk = (KT + per - 1) / per;
-      const double us = plan_us(M, N, pair, c, rsk, per, PLAN_FMT, sums_left);
+      const double us = plan_us(M, N, pair, c, rsk, per, PLAN_FMT);
       // (equal within the estimate: the earlier configuration, the larger tile)
       if (us < (best.cfg == c ? 1.0 : 0.985) * best.us) best = {c, rsk, per, us};
     }
   }
   return best;
 }
-static PromptPlan prompt_plan(int M, int N, int K, bool pair = false, bool sums_left = false) {
+static PromptPlan prompt_plan(int M, int N, int K, bool pair = false) {
   static const int env_cfg = getenv("BIGDL_PROMPT_CFG") ? atoi(getenv("BIGDL_PROMPT_CFG")) : -1;
   static const int env_sk = getenv("BIGDL_PROMPT_SPLITK") ? atoi(getenv("BIGDL_PROMPT_SPLITK")) : 0;
-  return prompt_plan_of(M, N, K, pair, g_force_cfg >= 0 ? g_force_cfg : env_cfg, g_force_sk > 0 ? g_force_sk : env_sk, sums_left);
+  return prompt_plan_of(M, N, K, pair, g_force_cfg >= 0 ? g_force_cfg : env_cfg, g_force_sk > 0 ? g_force_sk : env_sk);
 }
 
 // The time in us, in this format, of the plan that is launched where nothing forces another (callers remember the choice by the product's
@@ -106,11 +106,15 @@ double prompt_us(int M, int N, int K, int qtype, bool pair) {
   return (p.splitk >= 4 && p.cfg != 2 ? 1.12 : 1.0) * plan_us(M, N, pair, p.cfg, p.splitk, p.kt_per_split, fmt);
 }
 
-// Splits of K whose sums are left to the norm that follows (1: none), and the product that writes them, [splits][M][N] fp32
-int prompt_parts(int M, int N, int K) { return prompt_plan(M, N, K, false, true).splitk; }
+// Splits of K whose sums are left to the norm that follows (1: none), and the product that writes them, [splits][M][N] fp32.  The plan is the
+// one without a norm: what is split there saves its reduce launch and a pass over the result, with its norm 7 % on average, 2 to 18 (150 random
+// products of 257 - 8000 rows, four formats; 1024 x 4096 x 11008 sym_int4 109.1 -> 102.5 us).  What is whole there stays whole: 90 random products of 513 - 8000 rows
+// that a price of left sums (0.5 us + 0.9 ps an element and split) would split were 1.2 % slower on average, 39 of them by 2 - 17 % (844 x
+// 5120 x 4096 sym_int8 57.4 -> 63.3), and took slabs of up to 150 MB.
+int prompt_parts(int M, int N, int K) { return prompt_plan(M, N, K).splitk; }
 int prompt_parts_launch(const void* x, const void* w, float* partial, int M, int N, int K, int ldx, int qtype, hipStream_t st) {
   GemmArgs a = {};
-  const PromptPlan pl = prompt_plan(M, N, K, false, true);
+  const PromptPlan pl = prompt_plan(M, N, K);
   a.x = (const _Float16*)x; a.w = w; a.partial = partial; a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldo = N; a.out_type = OUT_F16;
   a.splitk = pl.splitk; a.kt_per_split = pl.kt_per_split;
   return prompt_dispatch(a, qtype, pl.cfg, st);

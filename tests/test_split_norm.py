@@ -1,5 +1,7 @@
 """Products whose K is split and whose sums the RMSNorm behind adds up (csrc/hip/gemm_lowbit.hip ``bigdl_gemm_parts``, misc_ops.hip
 ``rms_norm_parts_kernel``)."""
+import random
+
 import pytest
 import torch
 
@@ -31,6 +33,19 @@ def test_rule(qt):
             s = L.bigdl_gemm_parts(m, n, k, k, qt, 2)
             assert s in (0, 2, 3, 4) and (s == 0 or (k + 127) // 128 >= 4 * s), (m, n, k, s)
     assert L.bigdl_gemm_parts(64, 4096, 14336, 14336, qt, 2) > 1          # 128 column tiles of a long K: half the chip without
+
+
+@needs_library
+def test_rule_of_rows():
+    """a product of rows leaves the sums of the splits that it has without a norm too: six k-tiles a split at least, none where it is whole"""
+    L, seen, rng = hip.lib(), set(), random.Random(1)
+    sizes = [(300, 4096, 11008), (844, 5120, 4096), (3000, 2048, 5632)]
+    sizes += [(rng.randint(257, 8000), 128 * rng.randint(4, 64), 128 * rng.randint(2, 112)) for _ in range(400)]
+    for m, n, k in sizes:
+        splits, s = hip.gemm_prompt_plan(m, n, k)[1], L.bigdl_gemm_parts(m, n, k, k, Q.SYM_INT4, 0)
+        assert s == (splits if splits > 1 else 0) and (s == 0 or k // 128 >= 6 * s), (m, n, k, s)
+        seen.add(s)
+    assert seen >= {0, 2, 3, 4, 5, 6, 7, 8}
 
 
 @needs_library

@@ -76,15 +76,15 @@ FragPlan frag_plan(int M, int N, int K, int qtype, bool pair, bool may_split, bo
         const int per = (KT + sk - 1) / sk;
         if (sk > 1 && (KT < 8 * sk || (KT + per - 1) / per != sk)) break;
         const double load = (double)(blocks * sk) / cus;
-        const bool left = sums_left && sk > 1;
-        double us = c.a + ceil(load) * (c.turn + (left ? 0.7 : 1.0) * c.tile * mt * ns + per * (c.x * mt + c.w * ns + c.xw * mt * ns)) + load * per * c.mem * ns;
+        double us = c.a + ceil(load) * (c.turn + c.tile * mt * ns + per * (c.x * mt + c.w * ns + c.xw * mt * ns)) + load * per * c.mem * ns;
         // partial sums, and the launch that adds them up: 4 us on the GPU.  Where the host is behind it costs 3.5 us there, so a split has
         // to be ahead by that much (34 rows of 2048 x 5632 nf4 in a prompt of two layers: 282 us a pass, without the split 273)
-        // Sums that are left to the norm behind cost what it takes to write and read them (with fewer instructions on a tile than an epilogue).
-        // 45 products of 36 - 400 rows in front of a norm (2048 and 4096 columns, K 2048 - 14336, three formats): the plan taken is 0.4 % behind
-        // the fastest of all, 7 % at most, and takes 0.86 of the time without a split (64 x 4096 x 11008 sym_int4 20.7 -> 15.5 us, 77 x 4096 x
-        // 14336 asym_int4 26.5 -> 19.9, 36 x 4096 x 14336 27.2 -> 14.6; 4 % slower at most)
-        if (left) us += 1.0 + 0.7e-6 * sk * M * N;
+        // Sums that are left to the norm behind cost what it takes to write and read them, and have to be 4 % ahead, for
+        // the estimate's own error.  Of 400 random products of 33 - 512 rows in six formats that this splits, with their norm, none is more
+        // than 1 % slower than whole, 17 % faster on average (64 x 4096 x 11008 sym_int4 23.1 -> 19.7 us, 77 x 4096 x 14336 asym_int4 29.6 -> 24.7,
+        // 36 x 4096 x 14336 23.0 -> 20.1).  Priced at 1.0 us + 0.7 ps with 0.7 of a tile's exchange, 86 of 550 were 2 - 20 % slower than
+        // whole (80 x 5120 x 2048 asym_int5 14.5 -> 17.5), nearly all of them whole in 160 - 256 workgroups and split into larger tiles.
+        if (sums_left && sk > 1) us = (us + 2.0 + 0.4e-6 * sk * M * N) / 0.96;
         else if (sk > 1) us += 7.5 + 1e-6 * sk * M * N * (c.part + 1.0);
         if (us < best.us) best = {mt, ns, sk, per, us};
       }

@@ -284,10 +284,10 @@ constexpr int XTAIL = 128;   // zero halves after each LDS x row: the k-tile "on
 // is never in the scalar cache, and these kernels last 4 - 14 us.  SLOT (routed experts) is a template parameter for the same
 // reason: as a run-time branch its reads stood in front of the first weight request.  Llama-2-7B shape, batch 1, 8 steps of 4
 // layers: 1775 -> 1718 us (1742 without SLOT).
-// Wavefronts a SIMD that the registers have to allow: where the allocation is near a step of the occupancy, the lower side of it
+// Wavefronts a SIMD that the registers have to allow.  asym_int5 takes one register more than three workgroups a CU leave, by itself: 27760 x 4096,
+// three rows, 34.8 -> 31.6 us with the bound, 14672 x 5632, two rows, 26.1 -> 24.4; no other format's allocation is next to a step.
 constexpr int gemv_occupancy(int qt, int mt, bool pair, bool xlds, int nw, bool att, bool lean, bool slot) {
-  if (lean) return pair || lo_bits_of(qt) == 8 || hi_bits_of(qt) > 0 ? 6 : 8;
-  return mt == 1 && !pair && xlds && nw == 8 && !att && (slot ? lo_bits_of(qt) == 8 : hi_bits_of(qt) == 1) ? 6 : (nw + 3) / 4;
+  return lean || (qt == Q_ASYM_INT5 && mt == 1 && !pair && xlds && nw == 8 && !att && !slot) ? 6 : (nw + 3) / 4;
 }
 template <int QT, int MT, bool GATE_UP, bool XLDS, int NW, bool ATT = false, bool CU = false, bool LEAN = false, bool CAT = false,
           bool SLOT = false>
@@ -780,7 +780,8 @@ __global__ __launch_bounds__(NW * 64, gemv_occupancy(QT, MT, GATE_UP, XLDS, NW, 
 #endif
     }
   };
-  // row statistics of the fused norm, from the per-wavefront partials (valid after the barrier that ends the main loop)
+  // row statistics of the fused norm, from the per-wavefront partials: behind the staging barrier where x is staged in LDS, else (the partials are
+  // left by the main loop) behind the barrier that ends it
   auto row_stats = [&](int m, float& rs, float& mean) {
     rs = 1.0f;
     mean = 0.0f;
@@ -825,28 +826,39 @@ __global__ __launch_bounds__(NW * 64, gemv_occupancy(QT, MT, GATE_UP, XLDS, NW, 
       store_out<OUT_F32>(a.out, oi, v);
     }
   };
+  // The lane, counted again: around the main loop nothing of it stays in a register for what stands outside.  (Held, it took asym_int4's lean form
+  // over 64 registers: 12352 x 2048 6.6 -> 7.1 us; a bound on them instead changed its schedule: 5184 x 3072 7.1 -> 7.4.)
+  auto lane_anew = []() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0)); };
   // the rows' factors, by the wavefront that writes the outputs, into its own slots of the partial sums: these are complete behind the
   // staging barrier, and in front of the main loop a wavefront waits for weights anyway (behind it, the sum over the wavefronts, the
-  // division and the root were on the way of every result).  With the sums of up to four rows added up by lane groups, us a launch in a
-  // row, one MI355X, before -> now: sym_int4 pair of 5632 x 2048 6.32 -> 6.01, 2560 x 2048 with a norm 3.57 -> 3.44, 2048 x 5632 4.92 -> 4.79,
-  // 4096 x 4096 4.90 -> 4.73, two rows 5.20 -> 5.06, pair of 11008 x 4096 at two rows 15.84 -> 15.43
+  // division and the root were on the way of every result).  One to eight rows with a norm: 3 - 10 % (fp4 1 x 2048 x 4096 5.02 -> 4.7 us)
   auto rows_of = [&]() {
-    if (norm && lane < MT * 16) {
+    const int m = lane_anew();
+    if (norm && m < MT * 16) {
       float rs, mean;
-      row_stats(lane, rs, mean);
-      ssq_sh[lane] = rs;
-      if (lnorm) sum_sh[lane] = mean;
+      row_stats(m, rs, mean);
+      ssq_sh[m] = rs;
+      if (lnorm) sum_sh[m] = mean;
     }
   };
-  auto emit_row = [&](float v, float u, int m, int n) {
-    float rs = 1.0f, mean = 0.0f;
-    if constexpr (XLDS && MT == 1) {
-      if (norm) rs = ssq_sh[m];
-      if (lnorm) mean = sum_sh[m];
-    } else {
-      row_stats(m, rs, mean);
+  // factors of the rows m0 .., R of them, as rows_of left them (rows past the last one: anything), behind one branch: asked for row by row a product
+  // without a norm of 5 - 16 rows took 2 - 3 % longer
+  constexpr bool KEPT = XLDS && MT == 1;
+  auto rows_kept = [&](auto& rs, auto& mean, int m0) {
+    constexpr int R = sizeof(rs) / 4;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      rs[q] = 1.0f;
+      mean[q] = 0.0f;
     }
-    emit(v, u, m, n, rs, mean);
+    if (norm) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) rs[q] = ssq_sh[m0 + q];
+      if (lnorm) {
+#pragma unroll
+        for (int q = 0; q < R; ++q) mean[q] = sum_sh[m0 + q];
+      }
+    }
   };
 
   if constexpr (CU) {
@@ -915,11 +927,19 @@ __global__ __launch_bounds__(NW * 64, gemv_occupancy(QT, MT, GATE_UP, XLDS, NW, 
     return;
   }
 
-  if constexpr (XLDS && MT == 1) {
+  if constexpr (KEPT) {
     if (wave == 0) rows_of();
   }
   // ---- 3. main loop: ping-pong between two register sets; a set is re-requested as soon as it has been consumed ----
   for (int base = 0; base < (GEMV_PROBE == 2 ? min(ntw, 1) : ntw); base += 2 * U) {
+    // fp4: the first set is waited for in front of the second one's request, as the compiler has it for the other formats by itself.  Behind it the
+    // wait is for both (two rows of 2400 x 8192 6.9 -> 7.8 us, eight of 3952 x 4096 7.2 -> 8.0)
+    if constexpr (QT == Q_FP4 && !LEAN && !GATE_UP && !ATT) {
+#pragma unroll
+      for (int st = 0; st < NSTREAM; ++st)
+#pragma unroll
+        for (int u = 0; u < U; ++u) asm volatile("" : "+v"(ta[st][u].lo0), "+v"(ta[st][u].d));
+    }
     if (GEMV_PROBE != 2 && base + U < ntw && !(PF2 && base == 0)) fetch(tb, sb, base + U);
     consume(ta, sa, base);
     if (GEMV_PROBE != 2 && base + U < ntw) {
@@ -948,28 +968,37 @@ __global__ __launch_bounds__(NW * 64, gemv_occupancy(QT, MT, GATE_UP, XLDS, NW, 
       }
     }
   }
+  int lane_e = lane_anew();                        // (in front of the barrier: behind it everything waits for it)
+  asm volatile("" : "+v"(lane_e));
+  const int r_e = lane_e & 15, g_e = lane_e >> 4;
   __syncthreads();
   if (wave != 0) {
     GEMV_STAMP_AT(5);
     return;
   }
 
-  const int n = (int)nt * 16 + r;
+  const int n = (int)nt * 16 + r_e;
+  // Up to four rows lie in lane group 0: every lane group adds up a quarter of the wavefronts, the four meet, and group q goes on with row q.  us,
+  // every lane adding up all wavefronts and lane group 0 writing row after row -> now: four rows of 1568 x 1024 sym_int4 5.0 -> 4.2, 18944 x 4096
+  // asym_int4 20.2 -> 18.8, three of 3616 x 4096 fp4 with a norm 7.5 -> 6.5, one 3568 x 4096 sym_int4 4.95 -> 4.8
   if (MT == 1 && (LEAN || a.M <= 4)) {
-    // up to four rows (lane group 0 holds them): every lane group adds up a quarter of the wavefronts, then the four meet
-    float4v o[NACC];
+    float rs[1], mean[1], y[NACC];
+    if constexpr (KEPT) rows_kept(rs, mean, g_e);
+    else row_stats(g_e, rs[0], mean[0]);
 #pragma unroll
     for (int i = 0; i < NACC; ++i) {
-      o[i] = *(const float4v*)(red + ((g * NACC + i) * 64 + r) * 4);
+      float4v p = *(const float4v*)(red + ((g_e * NACC + i) * 64 + r_e) * 4);
 #pragma unroll
-      for (int w = 4; w < GEMV_NW; w += 4) o[i] += *(const float4v*)(red + (((w + g) * NACC + i) * 64 + r) * 4);
-    }
+      for (int w = 4; w < GEMV_NW; w += 4) p += *(const float4v*)(red + (((w + g_e) * NACC + i) * 64 + r_e) * 4);
+      y[i] = row_groups_sum(p[0]);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (q >= a.M) break;
-      const float v = row_groups_sum(o[0][q]), u = NACC == 2 ? row_groups_sum(o[NACC - 1][q]) : 0.0f;
-      if (g == 0 && n < a.N) emit_row(v, u, q, n);
+      for (int q = 1; q < 4; ++q) {
+        if (q >= a.M) break;
+        const float t = row_groups_sum(p[q]);
+        if (g_e == q) y[i] = t;
+      }
     }
+    if (g_e < a.M && n < a.N) emit(y[0], y[NACC - 1], g_e, n, rs[0], mean[0]);
     GEMV_STAMP_AT(5);
     return;
   }
@@ -978,14 +1007,19 @@ __global__ __launch_bounds__(NW * 64, gemv_occupancy(QT, MT, GATE_UP, XLDS, NW, 
     float4v o[NACC];
 #pragma unroll
     for (int i = 0; i < NACC; ++i) {
-      o[i] = *(const float4v*)(red + ((i * MT + j) * 64 + lane) * 4);
+      o[i] = *(const float4v*)(red + ((i * MT + j) * 64 + lane_e) * 4);
 #pragma unroll
-      for (int w = 1; w < GEMV_NW; ++w) o[i] += *(const float4v*)(red + ((w * NACC * MT + i * MT + j) * 64 + lane) * 4);
+      for (int w = 1; w < GEMV_NW; ++w) o[i] += *(const float4v*)(red + ((w * NACC * MT + i * MT + j) * 64 + lane_e) * 4);
     }
+    float rs[4], mean[4];
+    if constexpr (KEPT) rows_kept(rs, mean, 4 * g_e);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int m = 16 * j + 4 * g + q;
-      if (m < a.M && n < a.N) emit_row(o[0][q], o[NACC - 1][q], m, n);
+      const int m = 16 * j + 4 * g_e + q;
+      if (m < a.M && n < a.N) {
+        if constexpr (!KEPT) row_stats(m, rs[q], mean[q]);
+        emit(o[0][q], o[NACC - 1][q], m, n, rs[q], mean[q]);
+      }
     }
   }
   GEMV_STAMP_AT(5);

@@ -15,10 +15,11 @@ def _weight(n, k, qt, seed):
     return host.relayout_to_device(raw, qt, n, k).cuda(), host.dequantize(raw, qt, w.shape).double()
 
 
-# K of the lean form, of 8 wavefronts with a staging loop, of 16 wavefronts; N with a last tile that is cut
-@pytest.mark.parametrize("name", ["sym_int4", "asym_int4", "sym_int8"])
-@pytest.mark.parametrize("n,k", [(72, 1024), (40, 4096), (24, 9216)])
-@pytest.mark.parametrize("m", [1, 2, 3, 4, 5])
+# K of the lean form, of 8 wavefronts with a staging loop, of 16 wavefronts, of x that is not staged (four rows and more); N with a last tile that
+# is cut; rows of one lane group (up to four) and of all
+@pytest.mark.parametrize("name", ["sym_int4", "asym_int4", "sym_int8", "fp4", "asym_int5"])
+@pytest.mark.parametrize("n,k", [(72, 1024), (40, 4096), (24, 9216), (24, 20480)])
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 16])
 def test_rows_norm_bias_residual_pair(name, n, k, m):
     from bigdl_amd.ops import hip
     eps, qt = 1e-5, Q.ggml_tensor_qtype[name]

@@ -186,7 +186,21 @@ __device__ __forceinline__ int rows_chunk<Q_Q6_K>(int s, int g) { return 2 * g +
 // MT = 16-row tiles of x, NT = 16-column tiles of a weight per workgroup, WD = k-tiles of weights requested ahead.  What the
 // first requests need is preloaded into scalar registers (build flag, see gemv_kernel.h).  4 decode steps of 4 layers, 12 sequences,
 // Llama-3-8B shape: 1676 -> 1641 us; of 3 layers, 64 sequences, Llama-2-7B shape: 2798 -> 2772.
-template <int QT, int MT, int NT, bool PAIR, int NW = ROWS_NW, int WD = rows_ahead(QT, MT, PAIR ? 2 * NT : NT)>
+// Pairs of six or eight tiles: the look-ahead is one k-tile, and requested all at once behind it, it came a memory round trip late.  Each
+// tile is requested again as soon as it has been multiplied (all four steps at once), and the other five or seven hide its way.  With minima or
+// 8-bit codes only, us before -> now: asym_int4 14336 x 4096 at 4 / 12 rows 23.5 -> 21.5, 25.0 -> 23.9, 11008 x 4096 at 8 rows 19.0 -> 17.5;
+// sym_int8 14336 x 4096 at 16 rows 28.8 -> 25.7, fp8_e4m3 at 12 rows 31.1 -> 28.2; other formats' tiles are smaller and take it +-1 %,
+// single products of four tiles, whose look-ahead is two k-tiles, as well.
+// (fp8_e5m2's six tiles take 171 registers so, with which no workgroup starts beside the last wavefront of another: 16.6 us for 15.9 where CUs
+// have two workgroups, 21440 x 1024 at 6 rows.)
+constexpr bool rows_rolls(int qt, int mt, int ns, bool pair) {
+  return mt == 1 && qt != Q_Q6_K && pair && ns >= 6 && (has_min_of(qt) || lo_bits_of(qt) == 8) && !(qt == Q_FP8_E5M2 && ns == 6);
+}
+// ... and with 8-bit codes not where some wavefronts have no k-tile at all and the others one, with nothing to request again: SHORT.  fp8_e4m3
+// 20896 x 768 at 12 rows, six / eight tiles, 15.2 / 19.2 us rolling 16.2 / 20.1, sym_int8 14.5 / 18.5 and 15.0 / 18.6, 23296 x 512 at 4 rows 11.9 and
+// 12.2; 11000 x 1024 at 16 rows, a k-tile for each, 9.9 and 9.5.  With minima it pays there too (asym_int4 23296 x 512 12.7, rolling 11.6).
+constexpr bool rows_has_short(int qt, int mt, int ns, bool pair) { return rows_rolls(qt, mt, ns, pair) && lo_bits_of(qt) == 8; }
+template <int QT, int MT, int NT, bool PAIR, bool SHORT = false, int NW = ROWS_NW, int WD = rows_ahead(QT, MT, PAIR ? 2 * NT : NT)>
 __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(const _Float16* p_x, const void* p_w, const void* p_w2,
                                                                           const _Float16* p_gamma, int p_M, int p_N, int p_K,
                                                                           int p_ldx, int p_kt_per_split, float p_goff, RowsArgs a) {
@@ -196,12 +210,7 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(const 
   constexpr bool POST = MT == 1;                     // block scale on the fp32 product instead of the fp16 code (q6_k: always)
   constexpr bool NORM = MT == 1;                     // the folded RMSNorm exists for up to 16 rows
   constexpr bool MINS = POST && has_min_of(QT);
-  // Pairs of six or eight tiles: the look-ahead is one k-tile, and requested all at once behind it, it came a memory round trip late.  Each
-  // tile is requested again as soon as it has been multiplied (all four steps at once), and seven others hide its way.  With minima or
-  // 8-bit codes only, us before -> now: asym_int4 14336 x 4096 at 4 / 12 rows 23.5 -> 21.5, 25.0 -> 23.9, 11008 x 4096 at 8 rows 19.0 -> 17.5;
-  // sym_int8 14336 x 4096 at 16 rows 28.8 -> 25.7, fp8_e4m3 at 12 rows 31.1 -> 28.2; other formats' tiles are smaller and take it +-1 %,
-  // single products of four tiles, whose look-ahead is two k-tiles, as well.
-  constexpr bool ROLL = POST && QT != Q_Q6_K && PAIR && NS >= 6 && (has_min_of(QT) || lo_bits_of(QT) == 8);
+  constexpr bool ROLL = !SHORT && rows_rolls(QT, MT, NS, PAIR);
   constexpr int XB = MT * 2048;                      // bytes of half a staged x tile: MT * 16 rows of 64 halves
   constexpr bool TWO = rows_two_phase(MT, NS, NW);
   constexpr int NR = TWO ? NW / 2 : NW;              // wavefronts whose partial sums are in LDS at once
@@ -562,11 +571,13 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void gemm_rows_kernel(const 
   }
 }
 
-template <int QT, int MT, int NT, bool PAIR>
+template <int QT, int MT, int NT, bool PAIR, bool SHORT = false>
 static int gemm_rows_launch_t(const RowsArgs& a, hipStream_t st) {
-  constexpr int lds = rows_lds(MT, PAIR ? 2 * NT : NT, ROWS_NW);
+  constexpr int NS = PAIR ? 2 * NT : NT, lds = rows_lds(MT, NS, ROWS_NW);
   static_assert(lds <= 160 * 1024, "LDS of a CU");
-  auto k = gemm_rows_kernel<QT, MT, NT, PAIR>;
+  if constexpr (!SHORT && rows_has_short(QT, MT, NS, PAIR))
+    if (a.kt_per_split < ROWS_NW) return gemm_rows_launch_t<QT, MT, NT, PAIR, true>(a, st);
+  auto k = gemm_rows_kernel<QT, MT, NT, PAIR, SHORT>;
   if (!gemv_allow_lds((const void*)k, lds)) return -101;
   const int nblocks = ((a.N + 15) / 16 + NT - 1) / NT;
   hipLaunchKernelGGL(k, dim3(nblocks, (a.M + MT * 16 - 1) / (MT * 16), a.splitk), dim3(ROWS_NW * 64), lds, st, a.x, a.w, a.w2, a.gamma,

@@ -15,9 +15,9 @@ def _weight(n, k, qt, seed):
     return host.relayout_to_device(raw, qt, n, k).cuda(), host.dequantize(raw, qt, w.shape).double()
 
 
-# K: fewer k-tiles than wavefronts, a cut last one, wavefronts with one and two, with two and three; N: a cut tile, a cut workgroup
+# K: fewer k-tiles than wavefronts, one less, a cut last one, wavefronts with one and two, with two and three; N: a cut tile, a cut workgroup
 @pytest.mark.parametrize("name", ["asym_int4", "woq_int4", "asym_int5", "sym_int8", "fp8_e4m3", "fp8_e5m2"])
-@pytest.mark.parametrize("n,k", [(40, 128), (136, 1184), (72, 2304), (264, 4096)])
+@pytest.mark.parametrize("n,k", [(40, 128), (136, 896), (136, 1184), (72, 2304), (264, 4096)])
 @pytest.mark.parametrize("m,norm", [(1, False), (3, True), (16, True), (16, False)])
 def test_pair_matches_float64(name, n, k, m, norm):
     from bigdl_amd.ops import hip

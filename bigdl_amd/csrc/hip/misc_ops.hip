@@ -78,14 +78,14 @@ __device__ __forceinline__ float block_sum(float v, float* sh) {
   __syncthreads();
   return t;
 }
-// of 256 threads, called once: the barrier waits for LDS alone, not for the stores in front of it
-__device__ __forceinline__ float block_sum_once(float v, float* sh) {
+// of up to four wavefronts, called once: the barrier waits for LDS alone, not for the stores in front of it
+__device__ __forceinline__ float block_sum_once(float v, float* sh, int waves = 4) {
   v = wave_sum(v);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  return ((sh[0] + sh[1]) + sh[2]) + sh[3];
+  return ((sh[0] + (waves > 1 ? sh[1] : 0.0f)) + (waves > 2 ? sh[2] : 0.0f)) + (waves > 3 ? sh[3] : 0.0f);
 }
 __device__ __forceinline__ float block_max(float v, float* sh) {
   v = wave_max(v);
@@ -106,7 +106,12 @@ __device__ __forceinline__ float block_max(float v, float* sh) {
 // read the row's last ones and store nothing), in front of the first store, which would hold up the loads behind it; the barrier does not
 // wait for that store.  With a residual, us in a row of launches: 64 x 4096 3.3 -> 2.7, 512 x 4096 4.6 -> 4.1, 1024 x 4096 6.0, 256 x 8192
 // 5.4 -> 4.4, 64 x 16384 7.2 -> 5.0; without 2.9 -> 2.6, 3.5 -> 3.3, 4.4 -> 4.2, 4.2 -> 3.5, 5.6 -> 4.5.
-template <int DT, int VPT, bool ADD>  // VPT: 8-element vectors per thread; ADD: a residual
+// NARROW: rows of 1536 elements and less have only the wavefronts that lie in front of their end.  With four for all of them many rows were
+// slower than they were with loads under a condition: 7492 x 136 fp32 and a residual 7.7 us, 9.6, now 5.6.  (A form of its own: the count in the sum
+// costs 33 x 2048 0.1 of 2.2 us, and so does a scalar branch in front of the first loads.)
+constexpr int NORM_NARROW = 1536;
+__device__ __host__ __forceinline__ int norm_waves(int H) { return (H + 511) / 512; }
+template <int DT, int VPT, bool ADD, bool NARROW = false>  // VPT: 8-element vectors per thread; ADD: a residual
 __global__ __launch_bounds__(256) void rms_norm_kernel(const void* x, const void* residual, const void* w, void* out,
                                                        void* res_out, int H, int64_t ldx, float eps, float offset, int frag_mt) {
   __shared__ float sh[8];
@@ -130,7 +135,7 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const void* x, const void
     }
     if (res_out && on) store8<DT>(res_out, row * (int64_t)H + (threadIdx.x + i * 256) * 8, v[i]);
   }
-  const float rs = rsqrtf(block_sum_once(ss, sh) / (float)H + eps);
+  const float rs = rsqrtf(block_sum_once(ss, sh, NARROW ? norm_waves(H) : 4) / (float)H + eps);
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
     const int c = (threadIdx.x + i * 256) * 8;
@@ -640,10 +645,12 @@ extern "C" int bigdl_rms_norm(const void* x, const void* residual, const void* w
   if (frag && (dtype != DT_F16 || (H & 127) || rows > 1 << 20)) return -1;
   const int mt = frag ? (int)((rows + 15) / 16) : 0;
   const int vpt = (H / 8 + 255) / 256;
-#define NORM_LAUNCH(V, ADD) hipLaunchKernelGGL((rms_norm_kernel<DT, V, ADD>), dim3(rows), dim3(256), 0, st, x, residual, w, out, res_out, H, ldx, eps, offset, mt)
-#define NORM_OF(V) { if (residual) NORM_LAUNCH(V, true); else NORM_LAUNCH(V, false); }
+#define NORM_LAUNCH(V, ...) hipLaunchKernelGGL((rms_norm_kernel<DT, V, __VA_ARGS__>), dim3(rows), dim3(threads), 0, st, x, residual, w, out, res_out, H, ldx, eps, offset, mt)
+#define NORM_OF(V, ...) { if (residual) NORM_LAUNCH(V, true, ##__VA_ARGS__); else NORM_LAUNCH(V, false, ##__VA_ARGS__); }
+  const int threads = H <= NORM_NARROW ? 64 * norm_waves(H) : 256;
   DISPATCH_DT(dtype,
-    if (vpt <= 1) NORM_OF(1)
+    if (H <= NORM_NARROW) NORM_OF(1, true)
+    else if (vpt <= 1) NORM_OF(1)
     else if (vpt <= 2) NORM_OF(2)
     else if (vpt <= 4) NORM_OF(4)
     else NORM_OF(8))

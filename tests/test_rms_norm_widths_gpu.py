@@ -1,4 +1,4 @@
-"""RMSNorm at the edges of a thread's pieces (256 threads of eight elements): against 64 bits, sums in place, with and without a residual."""
+"""RMSNorm at the edges of a thread's pieces (256 threads of eight elements, fewer wavefronts for narrow rows): against 64 bits, sums in place, with and without a residual."""
 import numpy as np
 import pytest
 import torch
@@ -7,7 +7,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("rows,h", [(1, 8), (5, 2040), (5, 2048), (3, 2056), (2, 4096), (3, 8184), (2, 16384)])
+@pytest.mark.parametrize("rows,h", [(1, 8), (5, 512), (3, 520), (700, 1024), (3, 1032), (2, 1536), (3, 1544), (5, 2040), (5, 2048), (3, 2056), (2, 4096),
+                                    (3, 8184), (2, 16384)])
 def test_widths(rows, h, dtype):
     from bigdl_amd.ops import hip
     g = torch.Generator(device="cuda").manual_seed(h)

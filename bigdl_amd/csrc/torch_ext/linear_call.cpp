@@ -40,6 +40,20 @@ bool bound = false;
 
 constexpr int Q_Q6_K = 26;
 
+// A signature as text, the result in front: p an address (of any type, a stream too), i int, l int64_t, f float.  The entry points' addresses are
+// cast to types that stand here, where no compiler sees csrc/hip: Python holds the texts against the ones it calls them by and binds no other.
+template <class T> constexpr char KIND = 0;
+template <class T> constexpr char KIND<T*> = 'p';
+template <> constexpr char KIND<int> = 'i';
+template <> constexpr char KIND<int64_t> = 'l';
+template <> constexpr char KIND<float> = 'f';
+template <class F> struct Signature;
+template <class R, class... A>
+struct Signature<R (*)(A...)> {
+  static_assert(KIND<R> != 0 && ((KIND<A> != 0) && ...), "a type without a letter");
+  static constexpr char text[] = {KIND<R>, KIND<A>..., 0};
+};
+
 // an ordinary tensor in GPU memory that nothing but the caller looks at: no subclass, wrapper, graph, tangent.  (Views are: the rows of a
 // [batch, tokens, hidden] input are one, and outside inference mode it knows its base.)
 bool plain(const at::Tensor& t) {
@@ -150,14 +164,20 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// bind({name: address}) of the seven entry points above
+// the seven entry points above
+struct Bound { const char* name; void** to; const char* signature; };
+template <class F>
+Bound bound_to(const char* name, F* to) {
+  return {name, (void**)to, Signature<F>::text};
+}
+const Bound bound_of[] = {
+    bound_to("bigdl_gemv_lowbit", &gemv_lowbit), bound_to("bigdl_gemm_lowbit", &gemm_lowbit), bound_to("bigdl_gemm_lowbit_frag", &frag_rule),
+    bound_to("bigdl_gemm_frag_workspace", &frag_floats), bound_to("bigdl_gemm_lowbit_workspace", &gemm_floats),
+    bound_to("bigdl_gemm_frag_dense", &frag_dense), bound_to("bigdl_gemm_rows", &gemm_rows)};
+
+// bind({name: address}) of all of them
 PyObject* bind(PyObject*, PyObject* table) {
-  struct { const char* name; void** to; } want[] = {
-      {"bigdl_gemv_lowbit", (void**)&gemv_lowbit}, {"bigdl_gemm_lowbit", (void**)&gemm_lowbit},
-      {"bigdl_gemm_lowbit_frag", (void**)&frag_rule}, {"bigdl_gemm_frag_workspace", (void**)&frag_floats},
-      {"bigdl_gemm_lowbit_workspace", (void**)&gemm_floats}, {"bigdl_gemm_frag_dense", (void**)&frag_dense},
-      {"bigdl_gemm_rows", (void**)&gemm_rows}};
-  for (auto& e : want) {
+  for (auto& e : bound_of) {
     PyObject* at = PyDict_Check(table) ? PyDict_GetItemString(table, e.name) : nullptr;
     void* p = at ? PyLong_AsVoidPtr(at) : nullptr;
     if (p == nullptr) {
@@ -173,7 +193,7 @@ PyObject* bind(PyObject*, PyObject* table) {
 // ---- launchers: entry points of libbigdl_hip.so called with Python's arguments as they are ----
 // A prompt of 77 tokens is forty launches of a few microseconds each, and ctypes takes 2.5 us of the host for the 19 arguments of a
 // product (pointers asked for in Python included): the pass waits for the host.  Here a call converts by the C signature, with tensors in
-// place of their pointers: 0.4 us.  Four layers, 77 tokens: host 521 -> 417 us, the pass 520 -> 446 (450 of kernels), on a faster host 483 -> 453.
+// place of their pointers: 0.5 us.  Four layers, 77 tokens: host 521 -> 417 us, the pass 520 -> 446 (450 of kernels), on a faster host 483 -> 453.
 template <class T>
 struct From {                                        // int, int64_t
   static bool get(PyObject* o, T& v) {
@@ -212,8 +232,10 @@ struct From<T*> {
   }
 };
 
-template <int ID, class... A>
-struct Launcher {
+template <class F, int ID>
+struct Launcher;
+template <class... A, int ID>
+struct Launcher<int (*)(A...), ID> {
   static inline int (*entry)(A...) = nullptr;
 
   template <size_t... I>
@@ -238,30 +260,30 @@ typedef const void* In;
 typedef void* Out;
 typedef hipStream_t St;
 typedef int64_t L;
-struct Known { const char* name; void** entry; PyCFunction call; };
-template <int ID, class... A>
+struct Known { const char* name; void** entry; PyCFunction call; const char* signature; };
+template <int ID, class F>
 Known known(const char* name) {
-  return {name, (void**)&Launcher<ID, A...>::entry, (PyCFunction)(void (*)(void))Launcher<ID, A...>::call};
+  return {name, (void**)&Launcher<F, ID>::entry, (PyCFunction)(void (*)(void))Launcher<F, ID>::call, Signature<F>::text};
 }
+template <class... A> using Fn = int (*)(A...);
 // (the signatures of csrc/hip)
 const Known launchers_of[] = {
-    known<0, In, In, In, Out, Out, L, int, L, float, float, int, int, St>("bigdl_rms_norm"),
-    known<1, const float*, int, In, In, In, Out, Out, L, int, float, float, int, St>("bigdl_rms_norm_parts"),
-    known<2, Out, Out, Out, Out, const float*, const L*, int, int, int, int, int, int, int, int, int, int, L, L, int, St>("bigdl_prefill_rope_append"),
-    known<3, In, In, In, Out, In, int, int, int, int, int, int, L, L, L, L, L, L, L, L, L, L, L, L, L, L, const float*, float, float, int, int, int, int,
-          int, St>("bigdl_attn_prefill"),
-    known<4, In, In, In, Out, In, In, In, In, float, float, const float*, float*, float*, L, int, int, int, int, int, int, int, int, St>(
+    known<0, Fn<In, In, In, Out, Out, L, int, L, float, float, int, int, St>>("bigdl_rms_norm"),
+    known<1, Fn<const float*, int, In, In, In, Out, Out, L, int, float, float, int, St>>("bigdl_rms_norm_parts"),
+    known<2, Fn<Out, Out, Out, Out, const float*, const L*, int, int, int, int, int, int, int, int, int, int, L, L, int, St>>("bigdl_prefill_rope_append"),
+    known<3, Fn<In, In, In, Out, In, int, int, int, int, int, int, L, L, L, L, L, L, L, L, L, L, L, L, L, L, const float*, float, float, int, int, int,
+                int, int, St>>("bigdl_attn_prefill"),
+    known<4, Fn<In, In, In, Out, In, In, In, In, float, float, const float*, float*, float*, L, int, int, int, int, int, int, int, int, St>>(
         "bigdl_gemm_lowbit_ex"),
-    known<5, In, In, float*, L, int, int, int, int, int, int, St>("bigdl_gemm_parts_run"),
-    known<6, In, In, In, Out, In, In, In, float*, L, int, int, int, int, int, int, int, int, int, St>("bigdl_gemm_frag_dense"),
-    known<7, In, In, Out, In, In, float*, L, int, int, int, int, int, int, int, int, St>("bigdl_gemm_prompt"),
-    known<8, In, In, In, Out, In, In, int, int, int, int, int, int, int, int, St>("bigdl_gemm_prompt_pair"),
-    known<9, In, In, In, Out, In, In, In, In, float, float, int, int, int, int, int, int, int, int, const float*, int, int, int, int, int, int, St>(
-        "bigdl_gemv_lowbit"),
-    known<10, In, In, Out, In, In, float*, L, int, int, int, int, int, int, int, int, St>("bigdl_gemm_lowbit"),
-    known<11, In, In, Out, int, int, int, L, L, int, float, int, St>("bigdl_lora_down"),
-    known<12, In, In, Out, In, int, int, int, L, L, L, int, float, int, int, St>("bigdl_lora_up"),
-    known<13, In, Out, int, int, L, int, int, int, int, St>("bigdl_dequant_t16"),
+    known<5, Fn<In, In, float*, L, int, int, int, int, int, int, St>>("bigdl_gemm_parts_run"),
+    known<6, FragFn>("bigdl_gemm_frag_dense"),
+    known<7, Fn<In, In, Out, In, In, float*, L, int, int, int, int, int, int, int, int, St>>("bigdl_gemm_prompt"),
+    known<8, Fn<In, In, In, Out, In, In, int, int, int, int, int, int, int, int, St>>("bigdl_gemm_prompt_pair"),
+    known<9, GemvFn>("bigdl_gemv_lowbit"),
+    known<10, GemmFn>("bigdl_gemm_lowbit"),
+    known<11, Fn<In, In, Out, int, int, int, L, L, int, float, int, St>>("bigdl_lora_down"),
+    known<12, Fn<In, In, Out, In, int, int, int, L, L, L, int, float, int, int, St>>("bigdl_lora_up"),
+    known<13, Fn<In, Out, int, int, L, int, int, int, int, St>>("bigdl_dequant_t16"),
 };
 constexpr int LAUNCHERS = sizeof(launchers_of) / sizeof(launchers_of[0]);
 PyMethodDef launcher_defs[LAUNCHERS];
@@ -286,7 +308,21 @@ PyObject* launchers(PyObject*, PyObject* table) {
   return out;
 }
 
-PyMethodDef methods[] = {{"launchers", launchers, METH_O, nullptr},
+// signatures() -> {name: text} of all that bind and launchers take
+PyObject* signatures(PyObject*, PyObject*) {
+  PyObject* out = PyDict_New();
+  auto add = [&](const char* name, const char* text) {
+    PyObject* t = out != nullptr ? PyUnicode_FromString(text) : nullptr;
+    if (t == nullptr || PyDict_SetItemString(out, name, t) != 0) Py_CLEAR(out);
+    Py_XDECREF(t);
+  };
+  for (auto& e : bound_of) add(e.name, e.signature);
+  for (auto& k : launchers_of) add(k.name, k.signature);
+  return out;
+}
+
+PyMethodDef methods[] = {{"signatures", signatures, METH_NOARGS, nullptr},
+                         {"launchers", launchers, METH_O, nullptr},
                          {"product", (PyCFunction)(void (*)(void))product, METH_FASTCALL, nullptr}, {"bind", bind, METH_O, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "bigdl_linear_call", nullptr, -1, methods};

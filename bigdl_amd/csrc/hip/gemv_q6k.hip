@@ -183,12 +183,13 @@ static int launch_as(const RowsArgs& a, hipStream_t st, int per_cu, size_t lds) 
   return HIP_CHECK_LAUNCH();
 }
 // As many workgroups of eight wavefronts as a CU's LDS and registers hold (32000 x 4096, one row: 2 / 3 / 4 of them 29.8 / 30.8 /
-// 28.6 us); where only one fits, sixteen wavefronts share its x (4096 x 11008, three rows: 17.6 -> 16.2 us).
+// 28.6 us); where only one fits, sixteen wavefronts share its x (4096 x 11008, three rows: 17.6 -> 16.2 us), unless eight a CU have
+// a row each: sixteen would stand on half of the CUs (300 x 8192, four rows: 8.9 us, with sixteen 12.1, before 10.4).
 template <int M>
 static int launch(const RowsArgs& a, hipStream_t st) {
   const size_t x = q6k_x(M, a.K), lds = x + 8 * 2 * Q6K_PATCH;
   const int fit = (int)(160 * 1024 / lds), most = M <= 2 ? 4 : 3, per_cu = fit < most ? fit : most;
-  return per_cu == 1 ? launch_as<M, 16>(a, st, 1, x + 16 * 2 * Q6K_PATCH) : launch_as<M, 8>(a, st, per_cu, lds);
+  return per_cu == 1 && a.N > 8 * gemv_cu_count() ? launch_as<M, 16>(a, st, 1, x + 16 * 2 * Q6K_PATCH) : launch_as<M, 8>(a, st, per_cu, lds);
 }
 int gemv_q6k_launch(const RowsArgs& a, hipStream_t st) {
   switch (a.M) {

@@ -22,7 +22,7 @@ def _exact(raw, n, k):
     return torch.cat(out, 1).view(n, k)
 
 
-@pytest.mark.parametrize("n,k", [(1, 256), (333, 256), (40, 768), (96, 2048), (17, 2304), (40, 9984), (33, 16640), (8500, 512)])
+@pytest.mark.parametrize("n,k", [(1, 256), (333, 256), (40, 768), (96, 2048), (17, 2304), (40, 9984), (33, 16640), (2064, 8192), (8500, 512)])
 def test_rows_between_dwords(n, k):
     from bigdl_amd.ops import hip
     g = torch.Generator().manual_seed(n + k)

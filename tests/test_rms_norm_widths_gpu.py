@@ -1,4 +1,5 @@
-"""RMSNorm at the edges of a thread's pieces (256 threads of eight elements, fewer wavefronts for narrow rows): against 64 bits, sums in place, with and without a residual."""
+"""RMSNorm at the edges of a thread's pieces (256 threads of eight elements, fewer wavefronts for narrow rows): against 64 bits, sums in place,
+with and without a residual."""
 import numpy as np
 import pytest
 import torch

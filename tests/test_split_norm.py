@@ -172,3 +172,48 @@ def test_engine_with_and_without(monkeypatch, batch, tokens, bias):
     assert any(made[:made.index(None)]) and not any(made[made.index(None):])
     for a, b in zip(*outs):
         assert (a - b).norm() <= 4e-3 * b.norm()            # an fp16 rounding of the products less: 2^-11 of them, three layers
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,tokens", [(1, 70), (36, 3), (1, 600)])
+@pytest.mark.parametrize("kind", ["ungated", "output norms", "experts", "dense head", "gate and up of two formats"])
+def test_engines_of_other_designs(monkeypatch, kind, batch, tokens):
+    """the same of engines where only some products stand in front of a norm that adds: o and down of the layers around are split"""
+    from dataclasses import replace
+
+    from bigdl_amd.models.decoder import DecoderConfig, NativeDecoder, build_random_decoder
+    cfg = DecoderConfig(vocab_size=512, hidden_size=1024, intermediate_size=6144, num_layers=3, num_heads=32, num_kv_heads=4, head_dim=128,
+                        max_position=1024, gated_mlp=kind != "ungated")
+    eng = build_random_decoder(cfg, Q.SYM_INT4, device="cuda", seed=0, lm_head_qtype=Q.FP16 if kind == "dense head" else None)
+    layers = list(eng.layers)
+    if kind == "output norms":
+        ones = [(1 + 0.1 * torch.randn(1024, generator=torch.Generator().manual_seed(i))).half().cuda() for i in range(3)]
+        layers[0].post_ffn_out_norm, layers[1].post_attn_out_norm, layers[2].pre_ffn_norm = ones
+    elif kind == "experts":
+        # (both experts for every token: a choice between them could fall either way)
+        cfg = replace(cfg, num_experts=2, top_k=2, moe_intermediate_size=512)
+        layers[1] = build_random_decoder(cfg, Q.SYM_INT4, device="cuda", seed=1).layers[1]
+    elif kind == "gate and up of two formats":
+        layers[1].up = build_random_decoder(cfg, Q.NF4, device="cuda", seed=1).layers[1].up
+    ids = torch.randint(0, 512, (batch, tokens), generator=torch.Generator().manual_seed(5)).cuda()
+    step = torch.randint(0, 512, (batch, 1), generator=torch.Generator().manual_seed(6)).cuda()
+    real, made, outs = hip.gemm_parts, [], []
+
+    def counted(x, w, qtype, n, k, **kw):
+        p = real(x, w, qtype, n, k, **kw)
+        made.append((k, p is not None))
+        return p
+
+    monkeypatch.setattr(hip, "gemm_parts", counted)
+    for adds in (True, False):
+        if not adds:
+            monkeypatch.setattr(NativeDecoder, "_norm_adds", lambda self: False)
+            # o, and down where its x comes in fragment order or is a long prompt's
+            assert (4096, True) in made and ((6144, True) in made) == (kind != "ungated" or tokens > 512)
+            made.clear()
+        e = NativeDecoder(cfg, eng.embed, layers, eng.final_norm, eng.lm_head, device="cuda")
+        e.ensure_cache(batch, tokens + 16, fp8=False)
+        outs.append([e.prefill(ids).float(), *(e.decode(step, 1)[0].float().clone() for _ in range(3))])
+    assert not any(split for _, split in made)
+    for a, b in zip(*outs):
+        assert (a - b).norm() <= 4e-3 * b.norm()            # (as above)
